@@ -25,9 +25,8 @@ using gl::E2;
 using gl::u32;
 using gl::u64;
 
-// Work area of dps_mle_evaluate_noalloc, the one entry point that allocates nothing: eq tables of the two halves of
-// the point, per-workgroup partial sums and a ticket counter (dpk::WS_WORDS words, 144 KiB).  File-scope device
-// memory: every GPU the library runs on holds its own copy, at its own address, until the process ends.  In host
+// Work area of dps_mle_evaluate_noalloc, the one entry point that allocates nothing: per-workgroup partial sums and a
+// ticket counter (dpk::WS_WORDS words, 16 KiB), zero between calls.  File-scope device memory: every GPU the library runs on holds its own copy, at its own address, until the process ends.  In host
 // code the name below is only a handle for hipGetSymbolAddress; kernels are given the address that call returns.
 static __device__ __align__(256) uint64_t scratch[dpk::WS_WORDS];
 
@@ -92,6 +91,7 @@ struct dps_ctx {
     u64 seq = 0;                // last sequence number handed to a launch
     struct dps_sc *tail_owner = nullptr;  // session whose tail kernel is resident on the stream
     u32 units_held = 0;         // compute units of the device's ledger that launch holds (admit_waiting_launch)
+    u64 *d_eval = nullptr;      // work area of dps_mle_evaluate (dpk::WS_WORDS words)
     u64 *ws = nullptr;          // this device's copy of the allocation-free entry point's work area
     bool profiling = false;
     std::vector<ProfRec> recs;
@@ -296,7 +296,7 @@ struct ProfScope {
     dps_ctx *ctx;
     ProfRec rec;
     bool on;
-    ProfScope(dps_ctx *c, int kernel, double bytes) : ctx(c), on(c->profiling)
+    ProfScope(dps_ctx *c, int kernel, double bytes, bool wanted = true) : ctx(c), on(c->profiling && wanted)
     {
         if (!on) return;
         rec.kernel = kernel;
@@ -548,11 +548,12 @@ extern "C" int32_t dps_ctx_create(int32_t device, dps_ctx **out)
             ctx->h_inv_den[d][k] = h_inv(den);
         }
     const size_t lag_bytes = round_up(lag.size() * 8, 256);
-    if (hipMalloc((void **)&ctx->d_lagrange, lag_bytes + COUNTER_BYTES) != hipSuccess) return bail(DPS_ERR_OOM);
+    if (hipMalloc((void **)&ctx->d_lagrange, lag_bytes + COUNTER_BYTES + dpk::WS_WORDS * 8) != hipSuccess) return bail(DPS_ERR_OOM);
     if (hipMemcpy(ctx->d_lagrange, lag.data(), lag.size() * 8, hipMemcpyHostToDevice) != hipSuccess) return bail(DPS_ERR_HIP);
     ctx->d_counter = (u32 *)((char *)ctx->d_lagrange + lag_bytes);
     ctx->d_slice_ctr = (u64 *)((char *)ctx->d_counter + 256);
-    if (hipMemset(ctx->d_counter, 0, COUNTER_BYTES) != hipSuccess) return bail(DPS_ERR_HIP);
+    ctx->d_eval = (u64 *)((char *)ctx->d_counter + COUNTER_BYTES);
+    if (hipMemset(ctx->d_counter, 0, COUNTER_BYTES + dpk::WS_WORDS * 8) != hipSuccess) return bail(DPS_ERR_HIP);
     {
         int khz = 0;
         if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) == hipSuccess && khz > 0)
@@ -1259,39 +1260,65 @@ int32_t axis_dot(dps_ctx *ctx, const AxisJob &j)
 
 }  // namespace
 
+namespace {
+
+int32_t wait_result(dps_ctx *ctx, u64 seq, u32 slot0, u32 n, u64 *out);
+
+// The value of a table at a point: one launch, whose last workgroup hands it to the host (`area`: the words the launch
+// keeps its partial sums and its ticket counter in, WS_WORDS of them, one such launch at a time).
+int32_t evaluate_at(dps_ctx *ctx, const dps_mle *mle, const uint64_t *point, u32 n, u64 *area, uint64_t out[2])
+{
+    if (mle->eq && !(mle->eq->built & 1)) {
+        // An eq table whose entries nobody has read yet is not in memory, and need not be: the multilinear extension of
+        // eq(rho, .) at z is prod_i eq1(rho_i, z_i).
+        E2 v = gl::e2_one();
+        for (u32 i = 0; i < n; i++) v = gl::mul(v, h_eq1(mle->eq->point[i], gl::e2(point[2 * i], point[2 * i + 1])));
+        out[0] = v.c0;
+        out[1] = v.c1;
+        return DPS_OK;
+    }
+    dpk::EvalArgs a;
+    memset(&a, 0, sizeof a);
+    // (views of 16-bit tensors do not exist: the storage is the table)
+    a.t0 = mle->kind == DPS_I16 ? (const void *)mle->st->c0 : (const void *)mle->p0();
+    a.t1 = mle->p1();
+    a.n = n;
+    a.lo = std::min<u32>(n, dpk::EVAL_LO_BITS);
+    a.n_rows = 1ull << (n - a.lo);
+    const u32 blocks = (u32)std::min<u64>(a.n_rows, dpk::EVAL_MAX_BLOCKS);
+    a.rows_per_block = a.n_rows / blocks;
+    if (n) memcpy(a.p, point, 16 * (size_t)n);
+    dpk::FastFin ff;
+    memset(&ff, 0, sizeof ff);
+    ff.partial = area + dpk::WS_OFF_PARTIAL;
+    ff.n_blocks = blocks;
+    ff.out_host = ctx->d_pinned + ctx->res_off;
+    ff.seq = ++ctx->seq;
+    ff.counter = reinterpret_cast<u32 *>(area + dpk::WS_OFF_COUNTER);
+    // (no timing events in the entry point that allocates nothing: creating one is an allocation of the runtime's)
+    ProfScope ps(ctx, DPS_K_AXIS_DOT, (double)mle->len * (mle->p1() ? 16.0 : mle->kind == DPS_I16 ? 2.0 : 8.0), area != ctx->ws);
+    switch (mle->kind) {
+    case DPS_BASE: dpk::eval_point_kernel<0><<<blocks, dpk::BLOCK, 0, ctx->stream>>>(a, ff); break;
+    case DPS_EXT2: dpk::eval_point_kernel<1><<<blocks, dpk::BLOCK, 0, ctx->stream>>>(a, ff); break;
+    case DPS_I64: dpk::eval_point_kernel<8><<<blocks, dpk::BLOCK, 0, ctx->stream>>>(a, ff); break;
+    case DPS_I16: dpk::eval_point_kernel<2><<<blocks, dpk::BLOCK, 0, ctx->stream>>>(a, ff); break;
+    default: return fail(ctx, DPS_ERR_INVALID, "evaluate: unknown table kind");
+    }
+    HIPCHK(ctx, hipGetLastError());
+    return wait_result(ctx, ff.seq, 0, 2, out);
+}
+
+}  // namespace
+
 extern "C" int32_t dps_mle_evaluate(dps_ctx *ctx, const dps_mle *mle, const uint64_t *point, uint32_t n, uint64_t out[2])
 {
-    if (!ctx || !mle || !out || (n && !point)) return fail(ctx, DPS_ERR_INVALID, "dps_mle_evaluate: bad argument");
+    if (!ctx || !mle || !out || (n && !point) || n > dpk::EQ_MAX_VARS) return fail(ctx, DPS_ERR_INVALID, "dps_mle_evaluate: bad argument");
     if (mle->pad_vars) return fail(ctx, DPS_ERR_UNSUPPORTED, "dps_mle_evaluate: the table is a zero-padded view");
     if (!is_pow2(mle->len) || (1ull << n) != mle->len) return fail(ctx, DPS_ERR_INVALID, "dps_mle_evaluate: point length does not match the table");
+    if (!canonical(point, 2 * (size_t)n)) return fail(ctx, DPS_ERR_INVALID, "dps_mle_evaluate: point not canonical");
     DeviceGuard g(ctx->device);
     tail_abort(ctx);
-    CHK(plain_ready(mle));
-    dps_mle *eq = nullptr;
-    CHK(dps_eq_build(ctx, point, n, &eq));
-    if (int32_t rc_ = plain_ready(eq); rc_ != DPS_OK) {
-        delete eq;
-        return rc_;
-    }
-    AxisJob j;
-    j.in0 = mle->p0();
-    j.in1 = mle->p1();
-    j.in_int = raw_bytes(mle->kind);
-    j.b0 = eq->p0();
-    j.b1 = eq->p1();
-    j.K = mle->len;
-    j.stride_k = 1;
-    // the result lands in the second half of the pinned buffer (the first half staged the point)
-    j.o0 = ctx->d_pinned + ctx->pinned_words / 2;
-    j.o1 = j.o0 + 1;
-    int32_t rc = axis_dot(ctx, j);
-    hipError_t e = hipStreamSynchronize(ctx->stream);
-    delete eq;
-    if (rc != DPS_OK) return rc;
-    if (e != hipSuccess) return fail(ctx, DPS_ERR_HIP, "evaluate: %s", hipGetErrorString(e));
-    out[0] = ctx->h_pinned[ctx->pinned_words / 2];
-    out[1] = ctx->h_pinned[ctx->pinned_words / 2 + 1];
-    return DPS_OK;
+    return evaluate_at(ctx, mle, point, n, ctx->d_eval, out);
 }
 
 extern "C" int32_t dps_mle_fix_high(dps_ctx *ctx, const dps_mle *mle, const uint64_t *point, uint32_t k, dps_mle **out)
@@ -4566,19 +4593,6 @@ extern "C" int32_t dps_sc_prove(dps_sc *sc, dps_round_fn fn, void *user, uint64_
 // pinned result area like a round message, and the call returns when it is there (the host polls for it, so this is
 // not a call to make under stream capture).
 // ---------------------------------------------------------------------------
-namespace {
-
-template <int KIND>
-void launch_ws_dot(dps_ctx *ctx, bool full, u32 blocks, const void *t0, const u64 *t1, u32 lo, u32 hi, const dpk::FastFin &ff)
-{
-    if (full)
-        dpk::ws_dot_kernel<KIND, true><<<blocks, dpk::BLOCK, 0, ctx->stream>>>(t0, t1, lo, hi, ctx->ws, ff);
-    else
-        dpk::ws_dot_kernel<KIND, false><<<blocks, dpk::BLOCK, 0, ctx->stream>>>(t0, t1, lo, hi, ctx->ws, ff);
-}
-
-}  // namespace
-
 extern "C" int32_t dps_mle_evaluate_noalloc(dps_ctx *ctx, const dps_mle *mle, const uint64_t *point, uint32_t n, uint64_t out[2])
 {
     if (!ctx || !mle || !out || (n && !point)) return fail(ctx, DPS_ERR_INVALID, "dps_mle_evaluate_noalloc: bad argument");
@@ -4593,50 +4607,12 @@ extern "C" int32_t dps_mle_evaluate_noalloc(dps_ctx *ctx, const dps_mle *mle, co
     if (!ctx->ws) return fail(ctx, DPS_ERR_STATE, "dps_mle_evaluate_noalloc: the context has no work area");
     // (ending a launch that waits on the GPU for a session of this context would mean a stream wait and a memset)
     if (ctx->tail_owner) return fail(ctx, DPS_ERR_STATE, "dps_mle_evaluate_noalloc: a session of this context has a launch waiting on the GPU");
-    if (mle->eq && !(mle->eq->built & 1)) {
-        // An eq table whose entries nobody has read yet is not in memory (building it takes a scratch block and host
-        // vectors), and need not be: the multilinear extension of eq(rho, .) at z is prod_i eq1(rho_i, z_i).
-        E2 v = gl::e2_one();
-        for (u32 i = 0; i < n; i++) v = gl::mul(v, h_eq1(mle->eq->point[i], gl::e2(point[2 * i], point[2 * i + 1])));
-        out[0] = v.c0;
-        out[1] = v.c1;
-        return DPS_OK;
-    }
     DeviceGuard g(ctx->device);
     // every context on a GPU shares that GPU's work area: one call at a time per device, from the first launch until the
     // result is here
     static std::mutex area_in_use[WS_MAX_DEVICES];
     std::lock_guard<std::mutex> lock(area_in_use[ctx->device]);
-    dpk::WsPoint pt;
-    memset(&pt, 0, sizeof pt);
-    if (n) memcpy(pt.p, point, 16 * (size_t)n);
-    pt.n = n;
-    pt.lo = std::min<u32>(n, dpk::WS_LO_BITS);
-    const u32 lo = pt.lo, hi = n - lo;
-    const u32 eq_entries = (1u << lo) + (1u << hi);
-    dpk::ws_eq_kernel<<<(eq_entries + dpk::BLOCK - 1) / dpk::BLOCK, dpk::BLOCK, 0, ctx->stream>>>(pt, ctx->ws);
-    HIPCHK(ctx, hipGetLastError());
-    const u32 blocks = std::min<u32>(1u << hi, MAX_BLOCKS);
-    static_assert(MAX_BLOCKS <= dpk::WS_MAX_BLOCKS, "one partial per workgroup fits the work area");
-    dpk::FastFin ff;
-    memset(&ff, 0, sizeof ff);
-    ff.partial = ctx->ws + dpk::WS_OFF_PARTIAL;
-    ff.n_blocks = blocks;
-    ff.out_host = ctx->d_pinned + ctx->res_off;
-    ff.seq = ++ctx->seq;
-    ff.counter = reinterpret_cast<u32 *>(ctx->ws + dpk::WS_OFF_COUNTER);
-    const bool full = lo == dpk::WS_LO_BITS;
-    const void *t0 = mle->kind == DPS_I16 ? (const void *)mle->st->c0 : (const void *)mle->p0();
-    // (no timing events here: creating one is an allocation of the runtime's)
-    switch (mle->kind) {
-    case DPS_BASE: launch_ws_dot<0>(ctx, full, blocks, t0, nullptr, lo, hi, ff); break;
-    case DPS_EXT2: launch_ws_dot<1>(ctx, full, blocks, t0, mle->p1(), lo, hi, ff); break;
-    case DPS_I64: launch_ws_dot<8>(ctx, full, blocks, t0, nullptr, lo, hi, ff); break;
-    case DPS_I16: launch_ws_dot<2>(ctx, full, blocks, t0, nullptr, lo, hi, ff); break;
-    default: return fail(ctx, DPS_ERR_INVALID, "dps_mle_evaluate_noalloc: unknown table kind");
-    }
-    HIPCHK(ctx, hipGetLastError());
-    return wait_result(ctx, ff.seq, 0, 2, out);
+    return evaluate_at(ctx, mle, point, n, ctx->ws, out);
 }
 
 // ---------------------------------------------------------------------------

@@ -2767,119 +2767,132 @@ __global__ void __launch_bounds__(BLOCK) axis_dot_row_kernel(AxisArgs a)
 }
 
 // ---------------------------------------------------------------------------
-// evaluation of a table at a point without any memory of its own making: everything beyond the table and the two
-// result words lives in one work area the caller of the kernels passes in (`ws`, WS_WORDS words)
+// evaluation of a table at a point, one launch and no memory beyond a partial sum per workgroup
 //
-//   value = sum_h eq_hi[h] * ( sum_l eq_lo[l] * table[h * 2^lo + l] ),   eq_lo over the lo lowest coordinates of the
-// point, eq_hi over the others: two tables of at most 2^WS_LO_BITS entries instead of one of 2^n.  ws_eq_kernel
-// writes them (and zeroes the ticket counter); ws_dot_kernel streams the table once, one row h per workgroup and
-// step, a thread's eq_lo weights staying in registers across its rows, every sum unreduced until its end.
+//   value = sum_row eq_hi[row] * ( sum_l eq_lo[l] * table[row * 2^lo + l] ),   eq_lo over the lo lowest coordinates of the
+// point, eq_hi over the others.  No eq table is ever in memory: the point travels in the kernel arguments, every workgroup
+// makes four tables of at most 64 entries in LDS (the low coordinates in two parts, the next twelve in two parts), a
+// thread's eq_lo weights are products of two of their entries and stay in registers across its rows, and a row's weight is
+// a product of two entries (of three beyond 23 variables: the top coordinates' product changes every 4096 rows at most).
+// Every sum is unreduced until its end; the last workgroup gathers the partial sums and hands the value to the host.
+// Rows of 2^EVAL_LO_BITS = 2048 entries, so that 2^20 entries already make 512 workgroups (8 entries a thread and row).
+// Bound: the latency of one launch up to 2^20 entries (8 MB), HBM above.  Through the eq table in memory (three launches),
+// a dot product and a pass over its partial sums 2^20 base entries took 170 us, 122 of them in the last pass, whose one
+// thread added 1024 partial sums one behind the other; now 20 us with the way to the host and back.
 // ---------------------------------------------------------------------------
-constexpr u32 WS_MAX_VARS = 24;
-constexpr u32 WS_LO_BITS = 12;
-constexpr u32 WS_MAX_BLOCKS = 1024;
-// layout of the work area, in 64-bit words
-constexpr u32 WS_OFF_COUNTER = 0;  // ticket counter (32 bits used)
-constexpr u32 WS_OFF_LO0 = 32, WS_OFF_LO1 = WS_OFF_LO0 + (1u << WS_LO_BITS);
-constexpr u32 WS_OFF_HI0 = WS_OFF_LO1 + (1u << WS_LO_BITS), WS_OFF_HI1 = WS_OFF_HI0 + (1u << WS_LO_BITS);
-constexpr u32 WS_OFF_PARTIAL = WS_OFF_HI1 + (1u << WS_LO_BITS);  // 2 words per workgroup, word-major
-constexpr u32 WS_WORDS = WS_OFF_PARTIAL + 2 * WS_MAX_BLOCKS;
+constexpr u32 EVAL_LO_BITS = 11;
+constexpr u32 EVAL_MAX_BLOCKS = 1024;
+constexpr u32 EVAL_TOP_SHIFT = 12;  // rows that share a product of the top coordinates (log2)
+// layout of a work area (64-bit words): the ticket counter (32 bits used), zero between launches, and a partial sum per workgroup
+constexpr u32 WS_OFF_COUNTER = 0, WS_OFF_PARTIAL = 32;
+constexpr u32 WS_WORDS = WS_OFF_PARTIAL + 2 * EVAL_MAX_BLOCKS;
+constexpr u32 WS_MAX_VARS = 24;  // largest table of the entry point that allocates nothing
 
-struct WsPoint {
-    u64 p[2 * WS_MAX_VARS];  // 2 limbs per coordinate
-    u32 n, lo;               // coordinates; how many of them eq_lo covers
+struct EvalArgs {
+    const void *t0;
+    const u64 *t1;
+    u64 n_rows, rows_per_block;  // powers of two
+    u32 n, lo;                   // coordinates; how many of them a row covers
+    u64 p[2 * EQ_MAX_VARS];      // 2 limbs per coordinate
 };
 
-__global__ void __launch_bounds__(BLOCK) ws_eq_kernel(WsPoint pt, u64 *__restrict__ ws)
+// KIND: 0 base-field entries, 1 extension entries, 8 raw int64, 2 raw int16
+template <int KIND>
+__global__ void __launch_bounds__(BLOCK) eval_point_kernel(EvalArgs a, FastFin ff)
 {
-    const u32 i = blockIdx.x * BLOCK + threadIdx.x;
-    // the ticket counter of the launch that follows starts at zero whatever an earlier call left behind
-    if (i == 0) *reinterpret_cast<u32 *>(ws + WS_OFF_COUNTER) = 0;
-    const u32 n_lo = 1u << pt.lo, n_hi = 1u << (pt.n - pt.lo);
-    u32 first, bits, e;
-    u64 *o0, *o1;
-    if (i < n_lo) {
-        first = 0, bits = pt.lo, e = i, o0 = ws + WS_OFF_LO0, o1 = ws + WS_OFF_LO1;
-    } else if (i - n_lo < n_hi) {
-        first = pt.lo, bits = pt.n - pt.lo, e = i - n_lo, o0 = ws + WS_OFF_HI0, o1 = ws + WS_OFF_HI1;
-    } else {
-        return;
-    }
-    E2 acc = gl::e2_one();
-    for (u32 b = 0; b < bits; b++) {
-        const E2 r = gl::e2(pt.p[2 * (first + b)], pt.p[2 * (first + b) + 1]);
-        acc = gl::mul(acc, ((e >> b) & 1) ? r : gl::sub(gl::e2_one(), r));
-    }
-    o0[e] = acc.c0;
-    o1[e] = acc.c1;
-}
-
-// KIND: 0 base-field entries, 1 extension entries, 8 raw int64, 2 raw int16.  FULL: rows of exactly 2^WS_LO_BITS entries
-// (a thread's weights then sit in registers and its loads are 16 bytes wide).
-template <int KIND, bool FULL>
-__global__ void __launch_bounds__(BLOCK) ws_dot_kernel(const void *__restrict__ t0, const u64 *__restrict__ t1, u32 lo, u32 hi, u64 *ws, FastFin ff)
-{
+    static_assert(BLOCK == 4 * WAVE, "four wavefronts make the four small tables");
+    constexpr int STEPS = (1 << EVAL_LO_BITS) / (2 * BLOCK);
+    __shared__ u64 part0[4][64], part1[4][64];
     __shared__ u32 lds[(BLOCK / WAVE) * 6];
     __shared__ int last_flag;
-    const u64 *lo0 = ws + WS_OFF_LO0, *lo1 = ws + WS_OFF_LO1, *hi0 = ws + WS_OFF_HI0, *hi1 = ws + WS_OFF_HI1;
-    const u32 rows = 1u << hi, cols = 1u << lo, tid = threadIdx.x;
-    auto entry = [&](u64 i) -> E2 {
-        if (KIND == 8) return gl::e2(gl::from_i64(reinterpret_cast<const int64_t *>(t0)[i]), 0);
-        if (KIND == 2) return gl::e2(gl::from_i64(reinterpret_cast<const int16_t *>(t0)[i]), 0);
-        if (KIND == 1) return gl::e2(reinterpret_cast<const u64 *>(t0)[i], t1[i]);
-        return gl::e2(reinterpret_cast<const u64 *>(t0)[i], 0);
+    const u32 tid = threadIdx.x, w = tid / WAVE, lane = tid % WAVE;
+    // coordinates of the four tables: the low ones as la + lb, then ha + hb of the others; what is left is `top`
+    const u32 la = a.lo / 2, lb = a.lo - la, hi = a.n - a.lo;
+    const u32 ha = hi < 6 ? hi : 6, hb = hi - ha < 6 ? hi - ha : 6, top = hi - ha - hb;
+    const u32 bits_w = w == 0 ? la : w == 1 ? lb : w == 2 ? ha : hb;
+    const u32 first_w = w == 0 ? 0 : w == 1 ? la : w == 2 ? a.lo : a.lo + ha;
+    auto eq_at = [&](u32 first, u32 bits, u32 e) {
+        E2 v = gl::e2_one();
+        for (u32 b = 0; b < bits; b++) {
+            const E2 r = gl::e2(a.p[2 * (first + b)], a.p[2 * (first + b) + 1]);
+            v = gl::mul(v, ((e >> b) & 1) ? r : gl::sub(gl::e2_one(), r));
+        }
+        return v;
     };
-    gl::E2Acc total = gl::e2acc_zero();
-    if (FULL) {
-        // columns 2 (tid + BLOCK k), 2 (tid + BLOCK k) + 1 for k = 0..STEPS-1
-        constexpr int STEPS = (1 << WS_LO_BITS) / (2 * BLOCK);
-        E2 w[2 * STEPS];
+    if (lane < (1u << bits_w)) {
+        const E2 v = eq_at(first_w, bits_w, lane);
+        part0[w][lane] = v.c0;
+        part1[w][lane] = v.c1;
+    }
+    const u32 cols = 1u << a.lo;
+    const u64 row0 = (u64)blockIdx.x * a.rows_per_block;
+    // columns 2 (tid + BLOCK k), 2 (tid + BLOCK k) + 1 for k = 0..STEPS-1, as far as a row has them
+    auto entry = [&](u64 i) -> E2 {
+        if (KIND == 8) return gl::e2(gl::from_i64(reinterpret_cast<const int64_t *>(a.t0)[i]), 0);
+        if (KIND == 2) return gl::e2(gl::from_i64(reinterpret_cast<const int16_t *>(a.t0)[i]), 0);
+        if (KIND == 1) return gl::e2(reinterpret_cast<const u64 *>(a.t0)[i], a.t1[i]);
+        return gl::e2(reinterpret_cast<const u64 *>(a.t0)[i], 0);
+    };
+    E2 v[2 * STEPS];
+    auto load_row = [&](u64 row) {
+        const u64 base = row << a.lo;
 #pragma unroll
         for (int k = 0; k < STEPS; k++) {
-            const U64x2 a = ld2(lo0 + 2 * (tid + BLOCK * k)), b = ld2(lo1 + 2 * (tid + BLOCK * k));
-            w[2 * k] = gl::e2(a.x, b.x);
-            w[2 * k + 1] = gl::e2(a.y, b.y);
-        }
-        for (u32 row = blockIdx.x; row < rows; row += gridDim.x) {
-            const u64 base = (u64)row << WS_LO_BITS;
-            E2 v[2 * STEPS];
-#pragma unroll
-            for (int k = 0; k < STEPS; k++) {
-                const u64 i = base + 2 * (tid + BLOCK * k);
-                if (KIND == 0 || KIND == 1) {
-                    const U64x2 a = ld2(reinterpret_cast<const u64 *>(t0) + i);
-                    U64x2 b = U64x2{0, 0};
-                    if (KIND == 1) b = ld2(t1 + i);
-                    v[2 * k] = gl::e2(a.x, b.x);
-                    v[2 * k + 1] = gl::e2(a.y, b.y);
-                } else {
-                    v[2 * k] = entry(i);
-                    v[2 * k + 1] = entry(i + 1);
+            const u32 c = 2 * (tid + BLOCK * k);
+            v[2 * k] = v[2 * k + 1] = gl::e2_zero();
+            if (KIND == 0 || KIND == 1) {
+                if (c + 1 < cols) {
+                    const U64x2 x = ld2(reinterpret_cast<const u64 *>(a.t0) + base + c);
+                    U64x2 y = U64x2{0, 0};
+                    if (KIND == 1) y = ld2(a.t1 + base + c);
+                    v[2 * k] = gl::e2(x.x, y.x);
+                    v[2 * k + 1] = gl::e2(x.y, y.y);
+                } else if (c < cols) {
+                    v[2 * k] = entry(base + c);
                 }
+            } else {
+                if (c < cols) v[2 * k] = entry(base + c);
+                if (c + 1 < cols) v[2 * k + 1] = entry(base + c + 1);
             }
-            gl::E2Acc a = gl::e2acc_zero();
+        }
+    };
+    // (the first row is asked for before the tables are there: its loads and their products overlap)
+    load_row(row0);
+    __syncthreads();
+    E2 lw[2 * STEPS];
 #pragma unroll
-            for (int k = 0; k < 2 * STEPS; k++) {
-                if (KIND == 1)
-                    gl::acc_mul(a, v[k], gl::prep(w[k]));
-                else
-                    gl::acc_mul_base(a, w[k], v[k].c0);
-            }
-            gl::acc_mul(total, gl::acc_reduce(a), gl::prep(gl::e2(hi0[row], hi1[row])));
+    for (int k = 0; k < 2 * STEPS; k++) {
+        const u32 c = 2 * (tid + BLOCK * (k / 2)) + (k & 1);
+        lw[k] = gl::e2_zero();
+        if (c < cols) {
+            const u32 x = c & ((1u << la) - 1), y = c >> la;
+            lw[k] = gl::mul(gl::e2(part0[0][x], part1[0][x]), gl::e2(part0[1][y], part1[1][y]));
         }
-    } else {
-        for (u32 row = blockIdx.x; row < rows; row += gridDim.x) {
-            const u64 base = (u64)row << lo;
-            gl::E2Acc a = gl::e2acc_zero();
-            for (u32 l = tid; l < cols; l += BLOCK) {
-                const E2 wv = gl::e2(lo0[l], lo1[l]), v = entry(base + l);
-                if (KIND == 1)
-                    gl::acc_mul(a, v, gl::prep(wv));
-                else
-                    gl::acc_mul_base(a, wv, v.c0);
-            }
-            gl::acc_mul(total, gl::acc_reduce(a), gl::prep(gl::e2(hi0[row], hi1[row])));
+    }
+    gl::E2Acc total = gl::e2acc_zero();
+    E2 top_w = gl::e2_one();
+    u64 top_of = ~0ull;
+    for (u64 r = 0; r < a.rows_per_block; r++) {
+        const u64 row = row0 + r;
+        gl::E2Acc s = gl::e2acc_zero();
+#pragma unroll
+        for (int k = 0; k < 2 * STEPS; k++) {
+            if (KIND == 1)
+                gl::acc_mul(s, v[k], gl::prep(lw[k]));
+            else
+                gl::acc_mul_base(s, lw[k], v[k].c0);
         }
+        if (r + 1 < a.rows_per_block) load_row(row + 1);
+        const u32 x = (u32)row & ((1u << ha) - 1), y = (u32)(row >> ha) & ((1u << hb) - 1);
+        E2 hw = gl::mul(gl::e2(part0[2][x], part1[2][x]), gl::e2(part0[3][y], part1[3][y]));
+        if (top) {
+            if ((row >> EVAL_TOP_SHIFT) != top_of) {
+                top_of = row >> EVAL_TOP_SHIFT;
+                top_w = eq_at(a.lo + ha + hb, top, (u32)top_of);
+            }
+            hw = gl::mul(hw, top_w);
+        }
+        gl::acc_mul(total, gl::acc_reduce(s), gl::prep(hw));
     }
     E2 acc[1] = {gl::acc_reduce(total)};
     block_reduce<1>(acc, lds);
@@ -2888,7 +2901,7 @@ __global__ void __launch_bounds__(BLOCK) ws_dot_kernel(const void *__restrict__ 
         return;
     }
     if (tid == 0) {
-        u64 *o = ws + WS_OFF_PARTIAL + blockIdx.x;
+        u64 *o = const_cast<u64 *>(ff.partial) + blockIdx.x;
         st_agent(o, acc[0].c0);
         st_agent(o + gridDim.x, acc[0].c1);
     }
