@@ -2668,16 +2668,18 @@ int32_t SessionSetup::plan_and_ready_tables()
         sc->slice_ids.assign(sc->fast_order, sc->fast_order + sc->fast_nf);
         plan_resident_rounds(sc, sc->fast_nf, n_mles);
     }
-    // A sum of several terms over full-size tables (a fraction-sum layer, a claim merge, the stacked products of an
-    // einsum): the same launches.  One group of tables from the first round that fits; more tables than a group holds
-    // (up to SL_MAX_TABS) when every round is resident, so that the groups' own launches are never needed.
+    // A sum of several terms (a fraction-sum layer, a claim merge, the stacked products of an einsum): the same launches,
+    // from the first round that fits, as long as its tables and terms fit a launch (SL_MAX_TABS, SL_MAX_TERMS).  Tables of
+    // fewer variables are repeated as the launch takes them up.  Sums of more tables than a group of poly_kernel holds take
+    // these launches too: 12 products over 24 tables of 2^8 entries ran 20 us a round with a workgroup per group of 7 tables,
+    // 5 us this way; several workgroups share the pairs, not the tables.
     if (sc->poly && sc->fast_nf <= 4 && sc->n_terms <= (u32)dpk::SL_MAX_TERMS) {
         std::vector<u32> ids;
         for (const auto &g : sc->poly_tabs)
             for (u32 k : g)
                 if (std::find(ids.begin(), ids.end(), k) == ids.end()) ids.push_back(k);
         bool ok = n_mles == ids.size() + (sc->fast_eq >= 0 ? 1 : 0) && ids.size() <= (size_t)dpk::SL_MAX_TABS;
-        for (u32 k : ids) ok = ok && nv0[k] == n_vars && !mles[k]->pad_vars;
+        for (u32 k : ids) ok = ok && !mles[k]->pad_vars;
         if (ok) {
             sc->slice_ids = ids;
             for (const dps_term &t : sc->terms) {
@@ -2689,15 +2691,6 @@ int32_t SessionSetup::plan_and_ready_tables()
                 sc->slice_terms.push_back(tm);
             }
             plan_resident_rounds(sc, (u32)ids.size(), n_mles);
-            if (sc->poly_tabs.size() > 1 && sc->tail_j0 != 1) {
-                // several groups and not every round resident: the groups' launches take the session
-                sc->stages.clear();
-                sc->tail_j0 = 0;
-                sc->fin_len = 0;
-                sc->host_rounds = 0;
-                sc->round_kind.assign(n_vars + 2, 0);
-                sc->round_wide.assign(n_vars + 2, 0);
-            }
         }
     }
     // A small sum over tables the host has copies of (the small levels of fraction trees): every round is the host's.
@@ -3723,13 +3716,19 @@ int32_t FusedRound::launch_stages_at(u64 seq0, u32 first_go)
                 if (si > 0) {
                     sa.s0[f] = sc->stages[si - 1].h0[f];
                     sa.s1[f] = sc->stages[si - 1].h1[f];
-                } else if (sc->poly && first == 1) {
-                    sa.s0[f] = sc->m[sc->slice_ids[f]].c0;
-                    sa.s1[f] = sc->m[sc->slice_ids[f]].c1;
                 } else if (sc->poly) {
-                    const dpk::PolyTab &tb = sc->h_poly_groups[first - 1].tab[f];
+                    // (where the launch of round `first` in the owner's group would find the table)
+                    const u32 id = sc->slice_ids[f], g = (u32)sc->poly_owner[id];
+                    const auto &tabs = sc->poly_tabs[g];
+                    const u32 slot = (u32)(std::find(tabs.begin(), tabs.end(), id) - tabs.begin());
+                    const dpk::PolyTab &tb = sc->h_poly_groups[(size_t)(first - 1) * sc->poly_tabs.size() + g].tab[slot];
                     sa.s0[f] = tb.s0;
                     sa.s1[f] = tb.s1;
+                    if (tb.mode == dpk::POLY_BCAST || (tb.mode == dpk::POLY_PAIR && first > 1)) {
+                        // fewer variables than the round (POLY_BCAST: a pair's value is entry pair >> shift), or as many, not folded
+                        sa.lacks[f] = (uint8_t)(tb.mode == dpk::POLY_BCAST ? tb.shift + 2 : 1);
+                        sa.any_lacks = 1;
+                    }
                 } else if (!sc->quads.empty()) {
                     // the state of two rounds ago, as the last launch of two rounds left it
                     sa.s0[f] = sc->quads.back().d0[f];

@@ -1484,10 +1484,12 @@ constexpr int SL_AREA_WORDS = SL_GROUP_WORDS * (int)SL_MAX_GROUPS + 32;
 // (behind the sets: where the first workgroup says which mail it is waiting for and which it has had last -- read by the
 // host only to say more when a result does not come)
 constexpr int SL_WAITING_SLOT = SL_GROUP_WORDS * (int)SL_MAX_GROUPS, SL_HAD_SLOT = SL_WAITING_SLOT + 1;
-constexpr int SL_FIN_MAX_WORDS = 1024, SL_FIN_SEQ_SLOT = SL_FIN_MAX_WORDS, SL_FIN_CHK_SLOT = SL_FIN_MAX_WORDS + 1, SL_FIN_AREA_WORDS = SL_FIN_MAX_WORDS + 2;
+constexpr int SL_FIN_MAX_WORDS = 2048, SL_FIN_SEQ_SLOT = SL_FIN_MAX_WORDS, SL_FIN_CHK_SLOT = SL_FIN_MAX_WORDS + 1, SL_FIN_AREA_WORDS = SL_FIN_MAX_WORDS + 2;
 constexpr int SL_MAX_TRIPS = 32;
-constexpr int SL_MAX_TABS = 16;   // tables of a sum of several terms (a product has at most 3)
-constexpr int SL_MAX_TERMS = 24;
+// Tables and terms of a sum of several terms (a product has at most 3 tables).  What they cost a launch that does not use
+// them is the kernel arguments' copy; 32 tables of 64 pairs still fit a workgroup's LDS.
+constexpr int SL_MAX_TABS = 32;
+constexpr int SL_MAX_TERMS = 64;
 static_assert(2 * 4 * SL_MAX_TABS <= SL_FIN_MAX_WORDS, "the last entries of every table fit their area");
 // the check word's share of word i of that area
 __host__ __device__ __forceinline__ u64 sl_fin_mix(u64 word, u32 i) { return rotl64(word, (i & 31) + 1); }
@@ -1532,7 +1534,13 @@ struct SliceArgs {
     // a sum of several terms (TERMS): the tables are those of all terms, the polynomial summed is sum_k coeff_k prod table
     u32 n_tabs, n_terms;
     SliceTerm terms[SL_MAX_TERMS];
+    // Tables of fewer variables than the round the launch starts with (they depend on the highest ones): 1 + the number of low
+    // variables they lack.  No fold is pending on them; their entries are repeated as they are taken into LDS, and from then on
+    // they are tables like the others (a fold of two equal entries is that entry).  0: a table that folds with the rest.
+    uint8_t lacks[SL_MAX_TABS];
+    u32 any_lacks;
 };
+static_assert(sizeof(SliceArgs) <= 4096, "kernel arguments");
 
 // dynamic LDS of slice_kernel, in 64-bit words: counters per wavefront, mailbox copy, flags, the terms, then the two table buffers
 // (`blk`: threads of a workgroup)
@@ -1654,7 +1662,7 @@ __global__ void __launch_bounds__(BLK) slice_kernel(SliceArgs a)
         // but not yet its challenges: the entries this thread will fold are asked for before it waits for the mail, so
         // that they cross from device memory during the wait (up to SL_PRE items a thread; more are loaded after the mail).
         U64x2 pre[SL_PRE][4];
-        const bool have_pre = k == 0 && !a.first_go && pend >= 1 && (nt << len_log) <= (u32)(SL_PRE * BLOCK);
+        const bool have_pre = k == 0 && !a.first_go && pend >= 1 && (nt << len_log) <= (u32)(SL_PRE * BLOCK) && !(TERMS && a.any_lacks);
         if (have_pre) {
             const u64 base = (u64)wg * src_each;
 #pragma unroll
@@ -1716,7 +1724,10 @@ __global__ void __launch_bounds__(BLK) slice_kernel(SliceArgs a)
                 const u32 f = u >> len_log, i = u & (len - 1);
                 const u64 *p0 = regroup ? a.h0[f] : a.s0[f], *p1 = regroup ? a.h1[f] : a.s1[f];
                 E2 v;
-                if (pend == 0) {
+                if (TERMS && k == 0 && a.any_lacks && a.lacks[f]) {
+                    const u64 e = ((base >> pend) + i) >> (a.lacks[f] - 1);
+                    v = gl::e2(p0[e], p1 ? p1[e] : 0);
+                } else if (pend == 0) {
                     v = gl::e2(p0[base + i], p1 ? p1[base + i] : 0);
                 } else if (pend == 1) {
                     const U64x2 x0 = ld2(p0 + base + 2 * (u64)i);
