@@ -887,12 +887,8 @@ extern "C" int32_t dps_mle_zero_pad(const dps_mle *src, uint32_t n_vars, dps_mle
     dps_ctx *ctx = src->ctx;
     if (is_raw(src->kind) || !is_pow2(src->len)) return fail(ctx, DPS_ERR_INVALID, "dps_mle_zero_pad: not a power-of-two field table");
     if (n_vars > 40 || (1ull << n_vars) < src->len) return fail(ctx, DPS_ERR_INVALID, "dps_mle_zero_pad: %u variables are fewer than the table has", n_vars);
-    if (src->eq) {
-        DeviceGuard g(ctx->device);
-        tail_abort(ctx);
-        CHK(plain_ready(src));
-    }
-    *out = new (std::nothrow) dps_mle{ctx, src->st, src->kind, src->offset, src->len, nullptr, n_vars};
+    // (an eq table's entries are built when something reads them)
+    *out = new (std::nothrow) dps_mle{ctx, src->st, src->kind, src->offset, src->len, src->eq, n_vars};
     return *out ? DPS_OK : fail(ctx, DPS_ERR_OOM, "host allocation failed");
 }
 
@@ -1063,6 +1059,68 @@ int32_t plain_ready(const dps_mle *t)
     return eq_ensure(t->ctx, *t->eq, t->st->c0, t->st->c1, 1, false);
 }
 
+// The staging region of the pinned buffer (descriptors of launches that read them from there), h_pinned[STAGE_LO ..
+// pinned_words / 2): the previous launch that read it must be done with it.
+constexpr size_t STAGE_LO = 1024;
+int32_t stage_region(dps_ctx *ctx)
+{
+    if (ctx->stage_pending) {
+        HIPCHK(ctx, hipEventSynchronize(ctx->stage_event));
+        ctx->stage_pending = false;
+    }
+    return DPS_OK;
+}
+int32_t stage_region_read(dps_ctx *ctx)
+{
+    HIPCHK(ctx, hipEventRecord(ctx->stage_event, ctx->stream));
+    ctx->stage_pending = true;
+    return DPS_OK;
+}
+
+// The same for several tables, those of at most 2^16 entries in one launch (a launch each is 10 us of the host's and the
+// GPU's time, whatever is in it)
+int32_t eq_ready_many(dps_ctx *ctx, const std::vector<const dps_mle *> &tables)
+{
+    std::vector<const dps_mle *> small;
+    for (const dps_mle *t : tables) {
+        if (!t->eq || (t->eq->built & 1)) continue;
+        bool seen = false;
+        for (const dps_mle *q : small) seen = seen || q->eq == t->eq;
+        if (seen) continue;
+        if (t->eq->m <= 16)
+            small.push_back(t);
+        else
+            CHK(plain_ready(t));
+    }
+    if (small.size() == 1) return plain_ready(small[0]);
+    for (size_t at = 0; at < small.size();) {
+        std::vector<dpk::EqJobM> jobs;
+        std::vector<u64> pts;
+        u32 max_bits = 0;
+        const size_t first = at;
+        for (; at < small.size() && jobs.size() < 65535; at++) {
+            const EqInfo &e = *small[at]->eq;
+            if (STAGE_LO + ((jobs.size() + 1) * sizeof(dpk::EqJobM)) / 8 + pts.size() + 2 * (size_t)e.m > ctx->pinned_words / 2) break;
+            jobs.push_back(dpk::EqJobM{small[at]->st->c0, small[at]->st->c1, 0, e.m, (u32)pts.size(), 0});
+            for (const E2 &r : e.point) pts.push_back(r.c0), pts.push_back(r.c1);
+            max_bits = std::max(max_bits, e.m);
+        }
+        CHK(stage_region(ctx));
+        const size_t job_words = jobs.size() * sizeof(dpk::EqJobM) / 8;
+        memcpy(ctx->h_pinned + STAGE_LO, jobs.data(), job_words * 8);
+        if (!pts.empty()) memcpy(ctx->h_pinned + STAGE_LO + job_words, pts.data(), pts.size() * 8);
+        {
+            ProfScope ps(ctx, DPS_K_EQ, 0.0);
+            dpk::eq_define_many_kernel<<<dim3((u32)(((1ull << max_bits) + dpk::BLOCK - 1) / dpk::BLOCK), (u32)jobs.size()), dpk::BLOCK, 0, ctx->stream>>>(
+                reinterpret_cast<const dpk::EqJobM *>(ctx->d_pinned + STAGE_LO), ctx->d_pinned + STAGE_LO + job_words);
+            HIPCHK(ctx, hipGetLastError());
+        }
+        CHK(stage_region_read(ctx));
+        for (size_t i = first; i < at; i++) small[i]->eq->built |= 1;
+    }
+    return DPS_OK;
+}
+
 }  // namespace
 
 extern "C" int32_t dps_eq_build(dps_ctx *ctx, const uint64_t *point, uint32_t m, dps_mle **out)
@@ -1110,67 +1168,18 @@ extern "C" int32_t dps_eq_build_many(dps_ctx *ctx, const uint64_t *const *points
         }
         return rc;
     };
-    // staging region of the pinned buffer: job descriptors, then the points
-    const size_t stage_lo = 1024, stage_hi = ctx->pinned_words / 2;
-    std::vector<dpk::EqJobM> jobs;
-    std::vector<u64> pts;
-    u32 max_bits = 0;
-    auto flush = [&]() -> int32_t {
-        if (jobs.empty()) return DPS_OK;
-        // the previous launch that read the region must be done with it
-        if (ctx->stage_pending) {
-            HIPCHK(ctx, hipEventSynchronize(ctx->stage_event));
-            ctx->stage_pending = false;
-        }
-        const size_t job_words = jobs.size() * sizeof(dpk::EqJobM) / 8;
-        memcpy(ctx->h_pinned + stage_lo, jobs.data(), job_words * 8);
-        memcpy(ctx->h_pinned + stage_lo + job_words, pts.data(), pts.size() * 8);
-        ProfScope ps(ctx, DPS_K_EQ, 0.0);
-        dpk::eq_define_many_kernel<<<dim3((u32)(((1ull << max_bits) + dpk::BLOCK - 1) / dpk::BLOCK), (u32)jobs.size()), dpk::BLOCK, 0, ctx->stream>>>(
-            reinterpret_cast<const dpk::EqJobM *>(ctx->d_pinned + stage_lo), ctx->d_pinned + stage_lo + job_words);
-        HIPCHK(ctx, hipGetLastError());
-        HIPCHK(ctx, hipEventRecord(ctx->stage_event, ctx->stream));
-        ctx->stage_pending = true;
-        jobs.clear();
-        pts.clear();
-        max_bits = 0;
-        return DPS_OK;
-    };
+    // nothing is built here: a session that reads several of them builds them together (eq_ready_many), one that takes them in
+    // closed form never reads entries
     for (u32 i = 0; i < count; i++) {
         dps_mle *t = nullptr;
-        int32_t rc = new_table(ctx, DPS_EXT2, eq_storage_entries(m[i]), &t);
-        if (rc != DPS_OK) return undo(rc);
+        if (const int32_t rc = new_table(ctx, DPS_EXT2, eq_storage_entries(m[i]), &t); rc != DPS_OK) return undo(rc);
         out[i] = t;
         t->len = 1ull << m[i];
         t->eq = std::make_shared<EqInfo>();
         t->eq->m = m[i];
-        t->eq->fact_levels = eq_fact_levels(m[i]);  // (only tables of more than 16 variables have any: built by eq_build_dev)
+        t->eq->fact_levels = eq_fact_levels(m[i]);
         for (u32 k = 0; k < m[i]; k++) t->eq->point.push_back(gl::e2(points[i][2 * k], points[i][2 * k + 1]));
-        if (m[i] > 16) {
-            // large tables are built by expansion, one at a time
-            const u64 small = ((2ull << m[i]) - 1) & ~((1ull << eq_first_direct(m[i])) - 1);
-            rc = eq_ensure(ctx, *t->eq, t->st->c0, t->st->c1, small, true);
-            if (rc != DPS_OK) return undo(rc);
-            continue;
-        }
-        t->eq->built = (2ull << m[i]) - 1;  // every level, by the launch below
-        const size_t need = ((jobs.size() + m[i] + 1) * sizeof(dpk::EqJobM)) / 8 + pts.size() + 2 * (size_t)m[i];
-        if (stage_lo + need > stage_hi || jobs.size() + m[i] + 1 > 65535) {
-            rc = flush();
-            if (rc != DPS_OK) return undo(rc);
-        }
-        // every level eq(rho_{l..m-1}, .), l = 0..m, straight from the definition
-        const u32 point_off = (u32)pts.size();
-        pts.insert(pts.end(), points[i], points[i] + 2 * (size_t)m[i]);
-        for (u32 l = 0; l <= m[i]; l++) {
-            const u64 off = eq_level_off(m[i], l);
-            jobs.push_back(dpk::EqJobM{t->st->c0 + off, t->st->c1 + off, l, m[i] - l, point_off, 0});
-            max_bits = std::max(max_bits, m[i] - l);
-        }
     }
-    // the point offsets are relative to the start of the points, which follow the jobs of the same launch
-    int32_t rc = flush();
-    if (rc != DPS_OK) return undo(rc);
     return DPS_OK;
 }
 
@@ -1283,8 +1292,7 @@ int32_t evaluate_at(dps_ctx *ctx, const dps_mle *mle, const uint64_t *point, u32
     a.t0 = mle->kind == DPS_I16 ? (const void *)mle->st->c0 : (const void *)mle->p0();
     a.t1 = mle->p1();
     a.n = n;
-    a.lo = std::min<u32>(n, dpk::EVAL_LO_BITS);
-    a.n_rows = 1ull << (n - a.lo);
+    a.n_rows = 1ull << (n - std::min<u32>(n, dpk::EVAL_LO_BITS));
     const u32 blocks = (u32)std::min<u64>(a.n_rows, dpk::EVAL_MAX_BLOCKS);
     a.rows_per_block = a.n_rows / blocks;
     if (n) memcpy(a.p, point, 16 * (size_t)n);
@@ -1711,6 +1719,20 @@ struct dps_sc {
     std::vector<dpk::PolyOp> h_poly_ops;      // nested programs of the groups (empty: term by term)
     dpk::PolyOp *d_poly_ops;
     std::vector<char> stage;                  // descriptor upload in flight (no wait at set-up)
+    // A sum rewritten over fewer tables (combine_terms): the rounds are those of a session over these, and what is left to this
+    // one are the final evaluations of the tables that are in it no more
+    struct Outside {
+        u32 k, nv;                    // table as registered, its variables
+        bool zpad;
+        const u64 *c0, *c1;
+        std::shared_ptr<EqInfo> eq;   // an eq table: evaluated in closed form
+    };
+    dps_sc *inner = nullptr;
+    std::vector<dps_mle *> made;      // the tables combine_kernel made, given back with the session
+    std::vector<int> inner_of;        // per table as registered: its index in the inner session, or -1
+    std::vector<Outside> outside;
+    std::vector<u64> point;           // challenges so far, 2 limbs each
+    void *eval_block = nullptr;       // partial sums of the evaluations at the end
 };
 
 namespace {
@@ -1739,6 +1761,7 @@ void reset_device_words(dps_ctx *ctx) { (void)hipMemsetAsync(ctx->d_counter, 0, 
 // by a 7-bit tag, so a word nobody took must not stay for the trip that carries the same tag 128 sequence numbers later
 size_t slice_area_off(const dps_ctx *ctx);
 size_t slice_fin_off(const dps_ctx *ctx);
+int32_t wait_slice_entries(dps_ctx *ctx, u64 seq, u32 n, u64 *out);
 // the area of the pinned buffer for the outputs of a fraction tree (16 words each, behind the resident launches' result area)
 size_t logup_out_off(const dps_ctx *ctx, u32 slot) { return slice_area_off(ctx) + dpk::SL_AREA_WORDS + 64 + 16 * (size_t)slot; }
 int32_t wait_result_at(dps_ctx *ctx, size_t base_off, u64 seq, u32 slot0, u32 n, u64 *out, int seq_slot = dpk::HOST_SEQ_SLOT,
@@ -2737,6 +2760,7 @@ int32_t SessionSetup::plan_and_ready_tables()
     // What this session reads of its tables: an eq table taken in closed form is read level by level -- level j in round j,
     // except in the large rounds of a product, which take the low table of level j and level j + 16 instead -- and
     // anything else as ordinary entries.  Whatever of that an eq table has not built yet is built now, on the stream.
+    std::vector<const dps_mle *> plain;
     for (u32 k = 0; k < n_mles; k++) {
         if ((int)k == sc->fast_eq) {
             u32 first_level = 1;
@@ -2745,16 +2769,16 @@ int32_t SessionSetup::plan_and_ready_tables()
                 if (sc->tail_j0) first_level = std::min(first_level, sc->tail_j0);
             } else if (sc->poly) {
                 // the large rounds of a sum of several terms read level j + 16 and the low table of level j
+                CHK(eq_ensure(ctx, *sc->eq_info, const_cast<u64 *>(sc->eq_c0), const_cast<u64 *>(sc->eq_c1), 0, sc->tail_j0 != 1));
                 while (first_level <= n_vars && poly_round_weights_factored(sc, first_level)) first_level++;
             }
             const u64 need = ((2ull << n_vars) - 1) & ~((1ull << first_level) - 1);
             CHK(eq_ensure(ctx, *sc->eq_info, const_cast<u64 *>(sc->eq_c0), const_cast<u64 *>(sc->eq_c1), need, sc->fast));
         } else {
-            CHK(plain_ready(mles[k]));
+            plain.push_back(mles[k]);
         }
     }
-
-    return DPS_OK;
+    return eq_ready_many(ctx, plain);
 }
 
 int32_t SessionSetup::layout_scratch()
@@ -3124,6 +3148,241 @@ int32_t SessionSetup::run()
 
 }  // namespace
 
+namespace {
+
+// Sums of products of two tables that share factors, rewritten over fewer tables (same polynomial, so the same messages):
+//   - every term has the table X (several claims on one table, several uses of one input): sum_k c_k X Y_k = X M with
+//     M = sum_k c_k Y_k -- one product of two tables;
+//   - every term has an eq table E_g (claims of many chunks at a few points): sum_g M_g E_g, M_g = sum over the terms of E_g.
+// What it saves: M costs one read of every Y_k and one write of M, and no Y_k is folded from round to round; eq tables among
+// the Y_k are never in memory at all.  What it costs: the launch that makes M and, for tables other than eq tables, a launch
+// that evaluates them at the final point, about 15 us.  Taken
+//   - for a common X always when every Y_k is an eq table, otherwise from the sizes on whose rounds are not all resident
+//     (2^17 entries; merging four claims on 2^20 entries: 450 -> 250 us), and wherever a sum has more tables than
+//     the resident launches take or zero-padded ones, which only the general launches read (a launch for every fold and 430 us a
+//     round for 67 tables);
+//   - by eq tables only in that last case, when it leaves fewer tables or the sum has zero-padded ones.
+struct CombinedTable {
+    u32 factor;                                // X, or the eq table E_g
+    std::vector<std::pair<u32, E2>> items;     // tables and coefficients
+};
+
+bool plan_combination(const dps_sc *sc, const dps_mle *const *mles, const std::vector<u32> &nv0, std::vector<CombinedTable> *plan)
+{
+    const u32 n_vars = sc->n_vars, n_mles = sc->n_mles;
+    if (sc->n_terms < 2 || n_vars < 1 || n_vars > dpk::EQ_MAX_VARS) return false;
+    bool any_zpad = false;
+    for (u32 k = 0; k < n_mles; k++)
+        if (nv0[k] != n_vars && !mles[k]->pad_vars) return false;  // (constant in its low variables)
+    for (const dps_term &t : sc->terms) {
+        if (t.n_factors != 2 || t.factors[0] == t.factors[1]) return false;
+        any_zpad = any_zpad || nv0[t.factors[0]] != n_vars || nv0[t.factors[1]] != n_vars;
+    }
+    const bool too_many = n_mles > (u32)dpk::SL_MAX_TABS;
+    auto is_eq = [&](u32 k) { return mles[k]->eq != nullptr && mles[k]->kind == DPS_EXT2; };
+    auto coeff_of = [](const dps_term &t) { return gl::e2(t.coeff[0], t.coeff[1]); };
+    for (u32 c = 0; c < 2; c++) {
+        const u32 x = sc->terms[0].factors[c];
+        if (nv0[x] != n_vars) continue;
+        bool all = true, others_eq = true;
+        for (const dps_term &t : sc->terms) {
+            all = all && (t.factors[0] == x || t.factors[1] == x);
+            others_eq = others_eq && is_eq(t.factors[0] == x ? t.factors[1] : t.factors[0]);
+        }
+        if (!all || !(others_eq || too_many || any_zpad || n_vars >= 17)) continue;
+        plan->assign(1, CombinedTable{x, {}});
+        for (const dps_term &t : sc->terms) plan->back().items.emplace_back(t.factors[0] == x ? t.factors[1] : t.factors[0], coeff_of(t));
+        return true;
+    }
+    if (!too_many && !any_zpad) return false;
+    plan->clear();
+    std::map<u32, u32> at;
+    for (const dps_term &t : sc->terms) {
+        const u32 f = is_eq(t.factors[1]) ? 1 : 0;
+        if (!is_eq(t.factors[f])) return false;
+        auto [it, is_new] = at.emplace(t.factors[f], (u32)plan->size());
+        if (is_new) plan->push_back(CombinedTable{t.factors[f], {}});
+        (*plan)[it->second].items.emplace_back(t.factors[f ^ 1], coeff_of(t));
+    }
+    return any_zpad || 2 * plan->size() < n_mles;
+}
+
+// Carries the plan out: the tables M (and eq tables with their padding), and the session over them.
+int32_t combine_terms(dps_ctx *ctx, dps_sc *sc, const dps_mle *const *mles, const std::vector<u32> &nv0, const std::vector<CombinedTable> &plan, bool *fits)
+{
+    const u32 n_vars = sc->n_vars;
+    std::vector<dpk::CombItem> items;
+    std::vector<dpk::CombJob> jobs;
+    std::vector<u64> points;
+    std::map<u32, u32> point_of;
+    std::vector<const dps_mle *> in_mles;
+    std::vector<dps_term> in_terms;
+    sc->inner_of.assign(sc->n_mles, -1);
+    auto add_item = [&](u32 k, E2 c) {
+        const dps_mle *h = mles[k];
+        dpk::CombItem it;
+        memset(&it, 0, sizeof it);
+        it.c0 = c.c0, it.c1 = c.c1;
+        it.len = h->len;
+        it.n_bits = nv0[k];
+        if (h->eq && !(h->eq->built & 1)) {
+            auto [pos, is_new] = point_of.emplace(k, (u32)points.size());
+            if (is_new)
+                for (const E2 &r : h->eq->point) points.push_back(r.c0), points.push_back(r.c1);
+            it.point_off = pos->second;
+        } else {
+            it.t0 = h->p0();
+            it.t1 = h->p1();
+        }
+        items.push_back(it);
+    };
+    auto make = [&](const std::vector<std::pair<u32, E2>> &from, u32 *index) -> int32_t {
+        dps_mle *m = nullptr;
+        CHK(new_table(ctx, DPS_EXT2, 1ull << n_vars, &m));
+        sc->made.push_back(m);
+        jobs.push_back(dpk::CombJob{m->st->c0, m->st->c1, (u32)items.size(), (u32)from.size()});
+        for (const auto &f : from) add_item(f.first, f.second);
+        *index = (u32)in_mles.size();
+        in_mles.push_back(m);
+        return DPS_OK;
+    };
+    auto registered = [&](u32 k) {
+        if (sc->inner_of[k] < 0) {
+            sc->inner_of[k] = (int)in_mles.size();
+            in_mles.push_back(mles[k]);
+        }
+        return (u32)sc->inner_of[k];
+    };
+    for (const CombinedTable &c : plan) {
+        dps_term t;
+        memset(&t, 0, sizeof t);
+        t.coeff[0] = 1;
+        t.n_factors = 2;
+        if (nv0[c.factor] == n_vars)
+            t.factors[0] = registered(c.factor);
+        else
+            CHK(make({{c.factor, gl::e2_one()}}, &t.factors[0]));
+        CHK(make(c.items, &t.factors[1]));
+        in_terms.push_back(t);
+    }
+    if (!(sc->const_sum.c0 == 0 && sc->const_sum.c1 == 0)) {
+        dps_term t;
+        memset(&t, 0, sizeof t);
+        t.coeff[0] = sc->const_sum.c0, t.coeff[1] = sc->const_sum.c1;
+        in_terms.push_back(t);
+    }
+    for (u32 k = 0; k < sc->n_mles; k++)
+        if (sc->inner_of[k] < 0) sc->outside.push_back(dps_sc::Outside{k, nv0[k], mles[k]->pad_vars != 0, mles[k]->p0(), mles[k]->p1(), mles[k]->eq});
+    const size_t job_words = jobs.size() * sizeof(dpk::CombJob) / 8, item_words = items.size() * sizeof(dpk::CombItem) / 8;
+    static_assert(sizeof(dpk::CombJob) % 8 == 0 && sizeof(dpk::CombItem) % 8 == 0 && sizeof(dpk::EvalTable) % 8 == 0, "descriptors are staged as words");
+    const size_t eval_words = sc->outside.size() * sizeof(dpk::EvalTable) / 8;
+    *fits = STAGE_LO + std::max(job_words + item_words + points.size(), eval_words) <= ctx->pinned_words / 2 && jobs.size() <= 65535 &&
+            2 * sc->outside.size() <= (size_t)dpk::SL_FIN_MAX_WORDS;
+    if (!*fits) return DPS_OK;
+    CHK(stage_region(ctx));
+    u64 *h = ctx->h_pinned + STAGE_LO;
+    memcpy(h, jobs.data(), job_words * 8);
+    memcpy(h + job_words, items.data(), item_words * 8);
+    if (!points.empty()) memcpy(h + job_words + item_words, points.data(), points.size() * 8);
+    const u64 *d = ctx->d_pinned + STAGE_LO;
+    const u64 n_out = 1ull << n_vars;
+    {
+        double bytes = (double)jobs.size() * (double)n_out * 16.0;
+        for (const dpk::CombItem &it : items)
+            if (it.t0) bytes += (double)it.len * (it.t1 ? 16.0 : 8.0);
+        ProfScope ps(ctx, DPS_K_EQ, bytes);
+        dpk::combine_kernel<<<dim3((u32)std::min<u64>(std::max<u64>(n_out >> dpk::EVAL_LO_BITS, 1), 1024), (u32)jobs.size()), dpk::BLOCK, 0, ctx->stream>>>(
+            reinterpret_cast<const dpk::CombJob *>(d), reinterpret_cast<const dpk::CombItem *>(d + job_words), d + job_words + item_words, n_out);
+        HIPCHK(ctx, hipGetLastError());
+    }
+    CHK(stage_region_read(ctx));
+    return dps_sc_begin(ctx, n_vars, in_mles.data(), (u32)in_mles.size(), in_terms.data(), (u32)in_terms.size(), &sc->inner);
+}
+
+// The final evaluations of a sum whose rounds were another session's (combine_terms)
+int32_t finish_combined(dps_sc *sc, const u64 *challenge, u64 *final_evals_out)
+{
+    dps_ctx *ctx = sc->ctx;
+    sc->point.insert(sc->point.end(), challenge, challenge + 2);
+    std::vector<u64> inner(2 * (size_t)std::max<u32>(sc->inner->n_mles, 1));
+    // Tables other than eq tables are evaluated on the GPU: the launch is queued before the inner session's end is looked
+    // at, unless that session still has a launch of its own to make
+    std::vector<const dps_sc::Outside *> dev;
+    for (const dps_sc::Outside &o : sc->outside)
+        if (!o.eq) dev.push_back(&o);
+    CHK(dps_sc_finish(sc->inner, challenge, inner.data()));
+    u64 seq = 0;
+    if (!dev.empty()) {
+        u32 most = 0;
+        for (const dps_sc::Outside *o : dev) most = std::max(most, o->nv);
+        const u32 shares = (u32)std::min<u64>(1ull << (most > dpk::EVAL_LO_BITS ? most - dpk::EVAL_LO_BITS : 0), 256);
+        CHK(pool_alloc(ctx, dev.size() * shares * 16, &sc->eval_block));
+        CHK(stage_region(ctx));
+        std::vector<dpk::EvalTable> tabs;
+        double bytes = 0;
+        for (const dps_sc::Outside *o : dev) {
+            tabs.push_back(dpk::EvalTable{o->c0, o->c1, o->nv, 0});
+            bytes += (double)(1ull << o->nv) * (o->c1 ? 16.0 : 8.0);
+        }
+        memcpy(ctx->h_pinned + STAGE_LO, tabs.data(), tabs.size() * sizeof(dpk::EvalTable));
+        dpk::EvalTablesArgs a;
+        memset(&a, 0, sizeof a);
+        a.tables = reinterpret_cast<const dpk::EvalTable *>(ctx->d_pinned + STAGE_LO);
+        a.n_tables = (u32)tabs.size();
+        a.shares = shares;
+        a.partial = (u64 *)sc->eval_block;
+        a.counter = ctx->d_counter;
+        a.fin_out = ctx->d_pinned + slice_fin_off(ctx);
+        a.seq = seq = ++ctx->seq;
+        memcpy(a.p, sc->point.data(), sc->point.size() * 8);
+        {
+            ProfScope ps(ctx, DPS_K_AXIS_DOT, bytes);
+            dpk::eval_tables_kernel<<<dim3(shares, a.n_tables), dpk::BLOCK, 0, ctx->stream>>>(a);
+            HIPCHK(ctx, hipGetLastError());
+        }
+        CHK(stage_region_read(ctx));
+    }
+    for (u32 k = 0; k < sc->n_mles; k++) {
+        if (sc->inner_of[k] < 0) continue;
+        final_evals_out[2 * k] = inner[2 * sc->inner_of[k]];
+        final_evals_out[2 * k + 1] = inner[2 * sc->inner_of[k] + 1];
+    }
+    auto coord = [&](u32 i) { return gl::e2(sc->point[2 * i], sc->point[2 * i + 1]); };
+    auto put = [&](const dps_sc::Outside &o, E2 v) {
+        // a zero-padded table: the value of what there is, times prod (1 - r) over the variables it lacks
+        for (u32 i = o.nv; i < sc->n_vars && o.zpad; i++) v = gl::mul(v, gl::sub(gl::e2_one(), coord(i)));
+        final_evals_out[2 * o.k] = v.c0;
+        final_evals_out[2 * o.k + 1] = v.c1;
+    };
+    for (const dps_sc::Outside &o : sc->outside) {
+        if (!o.eq) continue;
+        E2 v = gl::e2_one();
+        for (u32 i = 0; i < o.nv; i++) v = gl::mul(v, h_eq1(o.eq->point[i], coord(i)));
+        put(o, v);
+    }
+    if (!dev.empty()) {
+        std::vector<u64> w(2 * dev.size());
+        CHK(wait_slice_entries(ctx, seq, (u32)w.size(), w.data()));
+        for (size_t i = 0; i < dev.size(); i++) put(*dev[i], gl::e2(w[2 * i], w[2 * i + 1]));
+    }
+    sc->finished = true;
+    return DPS_OK;
+}
+
+// What a session holds beyond its own blocks when it was rewritten
+void drop_combined(dps_sc *sc)
+{
+    if (sc->inner) (void)dps_sc_free(sc->inner);
+    sc->inner = nullptr;
+    for (dps_mle *m : sc->made) delete m;
+    sc->made.clear();
+    sc->outside.clear();
+    pool_free(sc->ctx, sc->eval_block);
+    sc->eval_block = nullptr;
+}
+
+}  // namespace
+
 extern "C" int32_t dps_sc_begin(dps_ctx *ctx, uint32_t n_vars, const dps_mle *const *mles, uint32_t n_mles,
                                 const dps_term *terms, uint32_t n_terms, dps_sc **out)
 {
@@ -3171,6 +3430,18 @@ extern "C" int32_t dps_sc_begin(dps_ctx *ctx, uint32_t n_vars, const dps_mle *co
     }
     sc->n_terms = (u32)sc->terms.size();
 
+    if (std::vector<CombinedTable> plan; plan_combination(sc.get(), mles, nv0, &plan)) {
+        bool fits = false;
+        if (const int32_t rc = combine_terms(ctx, sc.get(), mles, nv0, plan, &fits); rc != DPS_OK) {
+            drop_combined(sc.get());
+            return rc;
+        }
+        if (fits) {
+            *out = sc.release();
+            return DPS_OK;
+        }
+        drop_combined(sc.get());
+    }
     if (const int32_t rc = su.run(); rc != DPS_OK) {
         pool_free(ctx, sc->scratch);
         pool_free(ctx, sc->dev_block);
@@ -3186,6 +3457,7 @@ extern "C" int32_t dps_sc_set_claim(dps_sc *sc, const uint64_t *claim)
     dps_ctx *ctx = sc->ctx;
     if (sc->round != 0 || sc->finished) return fail(ctx, DPS_ERR_STATE, "dps_sc_set_claim: the session has started");
     if (!canonical(claim, 2)) return fail(ctx, DPS_ERR_INVALID, "dps_sc_set_claim: claim not canonical");
+    if (sc->inner) return dps_sc_set_claim(sc->inner, claim);
     sc->claim = gl::e2(claim[0], claim[1]);
     sc->have_claim = true;
     return DPS_OK;
@@ -4401,6 +4673,12 @@ extern "C" int32_t dps_sc_round(dps_sc *sc, const uint64_t *challenge, uint64_t 
     if ((j == 1) != (challenge == nullptr)) return fail(ctx, DPS_ERR_STATE, "dps_sc_round: round %u %s a challenge", j, j == 1 ? "takes no" : "needs");
     if (challenge && !canonical(challenge, 2)) return fail(ctx, DPS_ERR_INVALID, "dps_sc_round: challenge not canonical");
     if (sc->broken) return fail(ctx, DPS_ERR_STATE, "dps_sc_round: the session was interrupted by another call on its context");
+    if (sc->inner) {
+        CHK(dps_sc_round(sc->inner, challenge, evals_out));
+        if (challenge) sc->point.insert(sc->point.end(), challenge, challenge + 2);
+        sc->round = j;
+        return DPS_OK;
+    }
     DeviceGuard g(ctx->device);
     if (ctx->tail_owner != sc) tail_abort(ctx);
     const u32 live = sc->n_vars - j + 1;
@@ -4471,6 +4749,7 @@ extern "C" int32_t dps_sc_finish(dps_sc *sc, const uint64_t *challenge, uint64_t
     if (challenge && !canonical(challenge, 2)) return fail(ctx, DPS_ERR_INVALID, "dps_sc_finish: challenge not canonical");
     if (sc->broken) return fail(ctx, DPS_ERR_STATE, "dps_sc_finish: the session was interrupted by another call on its context");
     DeviceGuard g(ctx->device);
+    if (sc->inner) return finish_combined(sc, challenge, final_evals_out);
     if (ctx->tail_owner != sc) tail_abort(ctx);
     if (sc->pairs_seq) {
         // the resident launch published value and slope of every table's last pair with its last round: the final
@@ -4537,6 +4816,7 @@ extern "C" int32_t dps_sc_abort(dps_sc *sc)
     if (!sc) return DPS_ERR_INVALID;
     dps_ctx *ctx = sc->ctx;
     DeviceGuard g(ctx->device);
+    if (sc->inner) (void)dps_sc_abort(sc->inner);
     if (ctx->tail_owner == sc) tail_abort(ctx);
     sc->broken = true;
     return DPS_OK;
@@ -4551,6 +4831,7 @@ extern "C" int32_t dps_sc_free(dps_sc *sc)
     // a descriptor upload may still be reading the session's staging vector; the device blocks need no wait,
     // whoever gets them next uses them in stream order
     if (sc->descs_uploaded) (void)hipStreamSynchronize(ctx->stream);
+    drop_combined(sc);
     pool_free(ctx, sc->scratch);
     pool_free(ctx, sc->dev_block);
     delete sc;
@@ -4572,8 +4853,8 @@ extern "C" int32_t dps_sc_prove(dps_sc *sc, dps_round_fn fn, void *user, uint64_
             // which round of which kind of session it was
             char where[160];
             snprintf(where, sizeof where, " [round %u of %u: %s, round kind %u, resident from %u%s%s]", j, sc->n_vars,
-                     sc->fast ? "one product" : sc->poly ? "several terms" : "general", j < sc->round_kind.size() ? (u32)sc->round_kind[j] : 0u, sc->tail_j0,
-                     sc->host_only ? ", on the host" : "", poly_round_weights_factored(sc, j) ? ", factored weights" : "");
+                     sc->inner ? "rewritten over fewer tables" : sc->fast ? "one product" : sc->poly ? "several terms" : "general", j < sc->round_kind.size() ? (u32)sc->round_kind[j] : 0u, sc->tail_j0,
+                     sc->host_only ? ", on the host" : "", !sc->inner && poly_round_weights_factored(sc, j) ? ", factored weights" : "");
             ctx->err += where;
             return rc;
         }

@@ -2803,107 +2803,144 @@ struct EvalArgs {
     const void *t0;
     const u64 *t1;
     u64 n_rows, rows_per_block;  // powers of two
-    u32 n, lo;                   // coordinates; how many of them a row covers
+    u32 n, pad;                  // coordinates
     u64 p[2 * EQ_MAX_VARS];      // 2 limbs per coordinate
 };
 
-// KIND: 0 base-field entries, 1 extension entries, 8 raw int64, 2 raw int16
-template <int KIND>
-__global__ void __launch_bounds__(BLOCK) eval_point_kernel(EvalArgs a, FastFin ff)
+// How the coordinates of a point are shared out: rows of 2^lo entries (la + lb coordinates), then ha + hb, then `top`
+struct PointSplit {
+    u32 lo, la, lb, ha, hb, top;
+};
+__device__ __forceinline__ PointSplit split_point(u32 n)
+{
+    PointSplit s;
+    s.lo = n < EVAL_LO_BITS ? n : EVAL_LO_BITS;
+    s.la = s.lo / 2;
+    s.lb = s.lo - s.la;
+    const u32 hi = n - s.lo;
+    s.ha = hi < 6 ? hi : 6;
+    s.hb = hi - s.ha < 6 ? hi - s.ha : 6;
+    s.top = hi - s.ha - s.hb;
+    return s;
+}
+// prod_b (bit_b(e) ? p[first + b] : 1 - p[first + b]), b < bits (`p`: 2 limbs per coordinate)
+__device__ __forceinline__ E2 eq_entry(const u64 *p, u32 first, u32 bits, u32 e)
+{
+    E2 v = gl::e2_one();
+    for (u32 b = 0; b < bits; b++) {
+        const E2 r = gl::e2(p[2 * (first + b)], p[2 * (first + b) + 1]);
+        v = gl::mul(v, ((e >> b) & 1) ? r : gl::sub(gl::e2_one(), r));
+    }
+    return v;
+}
+// the four small tables of a point, one wavefront each (visible after a barrier)
+typedef u64 SmallEq[4][64];
+__device__ __forceinline__ void small_eq_tables(const u64 *p, const PointSplit &s, SmallEq &part0, SmallEq &part1)
 {
     static_assert(BLOCK == 4 * WAVE, "four wavefronts make the four small tables");
-    constexpr int STEPS = (1 << EVAL_LO_BITS) / (2 * BLOCK);
-    __shared__ u64 part0[4][64], part1[4][64];
-    __shared__ u32 lds[(BLOCK / WAVE) * 6];
-    __shared__ int last_flag;
-    const u32 tid = threadIdx.x, w = tid / WAVE, lane = tid % WAVE;
-    // coordinates of the four tables: the low ones as la + lb, then ha + hb of the others; what is left is `top`
-    const u32 la = a.lo / 2, lb = a.lo - la, hi = a.n - a.lo;
-    const u32 ha = hi < 6 ? hi : 6, hb = hi - ha < 6 ? hi - ha : 6, top = hi - ha - hb;
-    const u32 bits_w = w == 0 ? la : w == 1 ? lb : w == 2 ? ha : hb;
-    const u32 first_w = w == 0 ? 0 : w == 1 ? la : w == 2 ? a.lo : a.lo + ha;
-    auto eq_at = [&](u32 first, u32 bits, u32 e) {
-        E2 v = gl::e2_one();
-        for (u32 b = 0; b < bits; b++) {
-            const E2 r = gl::e2(a.p[2 * (first + b)], a.p[2 * (first + b) + 1]);
-            v = gl::mul(v, ((e >> b) & 1) ? r : gl::sub(gl::e2_one(), r));
-        }
-        return v;
-    };
-    if (lane < (1u << bits_w)) {
-        const E2 v = eq_at(first_w, bits_w, lane);
+    const u32 w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+    const u32 bits = w == 0 ? s.la : w == 1 ? s.lb : w == 2 ? s.ha : s.hb;
+    const u32 first = w == 0 ? 0 : w == 1 ? s.la : w == 2 ? s.lo : s.lo + s.ha;
+    if (lane < (1u << bits)) {
+        const E2 v = eq_entry(p, first, bits, lane);
         part0[w][lane] = v.c0;
         part1[w][lane] = v.c1;
     }
-    const u32 cols = 1u << a.lo;
-    const u64 row0 = (u64)blockIdx.x * a.rows_per_block;
-    // columns 2 (tid + BLOCK k), 2 (tid + BLOCK k) + 1 for k = 0..STEPS-1, as far as a row has them
+}
+__device__ __forceinline__ E2 small_eq(const SmallEq &part0, const SmallEq &part1, u32 w, u32 i) { return gl::e2(part0[w][i], part1[w][i]); }
+// the weight of a row's first entry over the coordinates above `lo`, without those of `top`
+__device__ __forceinline__ E2 row_weight(const PointSplit &s, const SmallEq &part0, const SmallEq &part1, u64 row)
+{
+    return gl::mul(small_eq(part0, part1, 2, (u32)row & ((1u << s.ha) - 1)), small_eq(part0, part1, 3, (u32)(row >> s.ha) & ((1u << s.hb) - 1)));
+}
+// A thread's entries of a row: columns 2 (tid + BLOCK k), 2 (tid + BLOCK k) + 1 for k = 0..ROW_STEPS-1, as far as the row has them
+constexpr int ROW_STEPS = (1 << EVAL_LO_BITS) / (2 * BLOCK);
+__device__ __forceinline__ u32 row_col(int k) { return 2 * (threadIdx.x + BLOCK * (k / 2)) + (k & 1); }
+// KIND: 0 base-field entries, 1 extension entries, 8 raw int64, 2 raw int16
+template <int KIND>
+__device__ __forceinline__ void load_row(const void *t0, const u64 *t1, u64 base, u32 cols, E2 (&v)[2 * ROW_STEPS])
+{
     auto entry = [&](u64 i) -> E2 {
-        if (KIND == 8) return gl::e2(gl::from_i64(reinterpret_cast<const int64_t *>(a.t0)[i]), 0);
-        if (KIND == 2) return gl::e2(gl::from_i64(reinterpret_cast<const int16_t *>(a.t0)[i]), 0);
-        if (KIND == 1) return gl::e2(reinterpret_cast<const u64 *>(a.t0)[i], a.t1[i]);
-        return gl::e2(reinterpret_cast<const u64 *>(a.t0)[i], 0);
+        if (KIND == 8) return gl::e2(gl::from_i64(reinterpret_cast<const int64_t *>(t0)[i]), 0);
+        if (KIND == 2) return gl::e2(gl::from_i64(reinterpret_cast<const int16_t *>(t0)[i]), 0);
+        if (KIND == 1) return gl::e2(reinterpret_cast<const u64 *>(t0)[i], t1[i]);
+        return gl::e2(reinterpret_cast<const u64 *>(t0)[i], 0);
     };
-    E2 v[2 * STEPS];
-    auto load_row = [&](u64 row) {
-        const u64 base = row << a.lo;
 #pragma unroll
-        for (int k = 0; k < STEPS; k++) {
-            const u32 c = 2 * (tid + BLOCK * k);
-            v[2 * k] = v[2 * k + 1] = gl::e2_zero();
-            if (KIND == 0 || KIND == 1) {
-                if (c + 1 < cols) {
-                    const U64x2 x = ld2(reinterpret_cast<const u64 *>(a.t0) + base + c);
-                    U64x2 y = U64x2{0, 0};
-                    if (KIND == 1) y = ld2(a.t1 + base + c);
-                    v[2 * k] = gl::e2(x.x, y.x);
-                    v[2 * k + 1] = gl::e2(x.y, y.y);
-                } else if (c < cols) {
-                    v[2 * k] = entry(base + c);
-                }
-            } else {
-                if (c < cols) v[2 * k] = entry(base + c);
-                if (c + 1 < cols) v[2 * k + 1] = entry(base + c + 1);
+    for (int k = 0; k < ROW_STEPS; k++) {
+        const u32 c = row_col(2 * k);
+        v[2 * k] = v[2 * k + 1] = gl::e2_zero();
+        if (KIND == 0 || KIND == 1) {
+            if (c + 1 < cols) {
+                const U64x2 x = ld2(reinterpret_cast<const u64 *>(t0) + base + c);
+                U64x2 y = U64x2{0, 0};
+                if (KIND == 1) y = ld2(t1 + base + c);
+                v[2 * k] = gl::e2(x.x, y.x);
+                v[2 * k + 1] = gl::e2(x.y, y.y);
+            } else if (c < cols) {
+                v[2 * k] = entry(base + c);
             }
-        }
-    };
-    // (the first row is asked for before the tables are there: its loads and their products overlap)
-    load_row(row0);
-    __syncthreads();
-    E2 lw[2 * STEPS];
-#pragma unroll
-    for (int k = 0; k < 2 * STEPS; k++) {
-        const u32 c = 2 * (tid + BLOCK * (k / 2)) + (k & 1);
-        lw[k] = gl::e2_zero();
-        if (c < cols) {
-            const u32 x = c & ((1u << la) - 1), y = c >> la;
-            lw[k] = gl::mul(gl::e2(part0[0][x], part1[0][x]), gl::e2(part0[1][y], part1[1][y]));
+        } else {
+            if (c < cols) v[2 * k] = entry(base + c);
+            if (c + 1 < cols) v[2 * k + 1] = entry(base + c + 1);
         }
     }
+}
+// sum_k w_k v_k of a thread's entries of a row
+template <int KIND>
+__device__ __forceinline__ E2 weigh_row(const E2 (&w)[2 * ROW_STEPS], const E2 (&v)[2 * ROW_STEPS])
+{
+    gl::E2Acc s = gl::e2acc_zero();
+#pragma unroll
+    for (int k = 0; k < 2 * ROW_STEPS; k++) {
+        if (KIND == 1)
+            gl::acc_mul(s, v[k], gl::prep(w[k]));
+        else
+            gl::acc_mul_base(s, w[k], v[k].c0);
+    }
+    return gl::acc_reduce(s);
+}
+__device__ __forceinline__ void low_weights(const PointSplit &s, const SmallEq &part0, const SmallEq &part1, E2 (&w)[2 * ROW_STEPS])
+{
+#pragma unroll
+    for (int k = 0; k < 2 * ROW_STEPS; k++) {
+        const u32 c = row_col(k);
+        w[k] = gl::e2_zero();
+        if (c < (1u << s.lo)) w[k] = gl::mul(small_eq(part0, part1, 0, c & ((1u << s.la) - 1)), small_eq(part0, part1, 1, c >> s.la));
+    }
+}
+
+template <int KIND>
+__global__ void __launch_bounds__(BLOCK) eval_point_kernel(EvalArgs a, FastFin ff)
+{
+    __shared__ SmallEq part0, part1;
+    __shared__ u32 lds[(BLOCK / WAVE) * 6];
+    __shared__ int last_flag;
+    const u32 tid = threadIdx.x;
+    const PointSplit s = split_point(a.n);
+    small_eq_tables(a.p, s, part0, part1);
+    const u64 row0 = (u64)blockIdx.x * a.rows_per_block;
+    // (the first row is asked for before the tables are there: its loads and their products overlap)
+    E2 v[2 * ROW_STEPS], lw[2 * ROW_STEPS];
+    load_row<KIND>(a.t0, a.t1, row0 << s.lo, 1u << s.lo, v);
+    __syncthreads();
+    low_weights(s, part0, part1, lw);
     gl::E2Acc total = gl::e2acc_zero();
     E2 top_w = gl::e2_one();
     u64 top_of = ~0ull;
     for (u64 r = 0; r < a.rows_per_block; r++) {
         const u64 row = row0 + r;
-        gl::E2Acc s = gl::e2acc_zero();
-#pragma unroll
-        for (int k = 0; k < 2 * STEPS; k++) {
-            if (KIND == 1)
-                gl::acc_mul(s, v[k], gl::prep(lw[k]));
-            else
-                gl::acc_mul_base(s, lw[k], v[k].c0);
-        }
-        if (r + 1 < a.rows_per_block) load_row(row + 1);
-        const u32 x = (u32)row & ((1u << ha) - 1), y = (u32)(row >> ha) & ((1u << hb) - 1);
-        E2 hw = gl::mul(gl::e2(part0[2][x], part1[2][x]), gl::e2(part0[3][y], part1[3][y]));
-        if (top) {
+        const E2 x = weigh_row<KIND>(lw, v);
+        if (r + 1 < a.rows_per_block) load_row<KIND>(a.t0, a.t1, (row + 1) << s.lo, 1u << s.lo, v);
+        E2 hw = row_weight(s, part0, part1, row);
+        if (s.top) {
             if ((row >> EVAL_TOP_SHIFT) != top_of) {
                 top_of = row >> EVAL_TOP_SHIFT;
-                top_w = eq_at(a.lo + ha + hb, top, (u32)top_of);
+                top_w = eq_entry(a.p, s.lo + s.ha + s.hb, s.top, (u32)top_of);
             }
             hw = gl::mul(hw, top_w);
         }
-        gl::acc_mul(total, gl::acc_reduce(s), gl::prep(hw));
+        gl::acc_mul(total, x, gl::prep(hw));
     }
     E2 acc[1] = {gl::acc_reduce(total)};
     block_reduce<1>(acc, lds);
@@ -2920,6 +2957,170 @@ __global__ void __launch_bounds__(BLOCK) eval_point_kernel(EvalArgs a, FastFin f
         E2 q[1];
         gather_partials<1>(ff, lds, q);
         publish_sums<1>(ff.out_host, ff.seq, ff.counter, q);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// A sum whose terms share factors, rewritten over fewer tables:  sum_k c_k X Y_k = X * M,  M = sum_k c_k Y_k.
+//
+// combine_kernel writes the tables M (grid row = table).  An item is a table times its coefficient -- its entries, zero
+// behind its end where it is zero-padded -- or the eq table of a point, whose entries are made here from the point and never
+// stored.  A workgroup writes rows of 2^EVAL_LO_BITS entries, 8 a thread, every entry one unreduced sum over the items.
+// Bound: each table once in, M once out; for eq tables one extension product an entry and table (2^20 entries of four eq
+// tables 9 us) where building, folding and weighting them as tables of their own moved eight times the bytes.
+// Descriptors and points lie in host-visible memory, written just before the launch.
+//
+// eval_tables_kernel evaluates the tables that are in no product any more at the sum's final point (grid: a workgroup per
+// table and share of its rows); the last workgroup adds the shares and hands the values to the host.
+// ---------------------------------------------------------------------------
+struct CombItem {
+    const u64 *t0, *t1;  // t0 nullptr: eq table of the point at `point_off`; t1 nullptr: base field
+    u64 c0, c1;          // coefficient
+    u64 len;             // entries: a power of two
+    u32 point_off;       // words from `points`
+    u32 n_bits;          // log2(len)
+};
+struct CombJob {
+    u64 *o0, *o1;
+    u32 first, count;    // items
+};
+__global__ void __launch_bounds__(BLOCK) combine_kernel(const CombJob *__restrict__ jobs, const CombItem *__restrict__ items, const u64 *__restrict__ points,
+                                                        u64 n_out)
+{
+    __shared__ SmallEq part0, part1;
+    __shared__ u64 high0[64], high1[64];
+    const CombJob job = jobs[blockIdx.y];
+    const u32 tid = threadIdx.x;
+    const u32 cols = n_out < (1ull << EVAL_LO_BITS) ? (u32)n_out : 1u << EVAL_LO_BITS;
+    const u64 n_rows = n_out / cols;
+    for (u64 row = blockIdx.x; row < n_rows; row += gridDim.x) {
+        const u64 base = row * cols;
+        gl::E2Acc acc[2 * ROW_STEPS];
+#pragma unroll
+        for (int k = 0; k < 2 * ROW_STEPS; k++) acc[k] = gl::e2acc_zero();
+        for (u32 it = 0; it < job.count; it++) {
+            const CombItem m = items[job.first + it];
+            if (base >= m.len) continue;  // (the whole workgroup: zero from here on)
+            const u32 have = m.len - base < cols ? (u32)(m.len - base) : cols;
+            const gl::E2P c = gl::prep(gl::e2(m.c0, m.c1));
+            if (m.t0) {
+                E2 v[2 * ROW_STEPS];
+                if (m.t1) {
+                    load_row<1>(m.t0, m.t1, base, have, v);
+#pragma unroll
+                    for (int k = 0; k < 2 * ROW_STEPS; k++) gl::acc_mul(acc[k], v[k], c);
+                } else {
+                    load_row<0>(m.t0, nullptr, base, have, v);
+#pragma unroll
+                    for (int k = 0; k < 2 * ROW_STEPS; k++) gl::acc_mul_base(acc[k], gl::e2(c.c0, c.c1), v[k].c0);
+                }
+                continue;
+            }
+            // (a point of fewer coordinates than a row's: `have` entries, and the point's row is shorter than this one's)
+            const PointSplit s = split_point(m.n_bits);
+            const u64 *p = points + m.point_off;
+            __syncthreads();  // the tables of the item before have been read
+            small_eq_tables(p, s, part0, part1);
+            __syncthreads();
+            if (tid < (1u << s.lb)) {
+                // the row's weight and the coefficient, taken into the upper low table
+                E2 hw = gl::mulp(row_weight(s, part0, part1, row), c);
+                if (s.top) hw = gl::mul(hw, eq_entry(p, s.lo + s.ha + s.hb, s.top, (u32)(row >> EVAL_TOP_SHIFT)));
+                const E2 v = gl::mul(small_eq(part0, part1, 1, tid), hw);
+                high0[tid] = v.c0;
+                high1[tid] = v.c1;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < 2 * ROW_STEPS; k++) {
+                const u32 col = row_col(k);
+                if (col < have) gl::acc_mul(acc[k], small_eq(part0, part1, 0, col & ((1u << s.la) - 1)), gl::prep(gl::e2(high0[col >> s.la], high1[col >> s.la])));
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < ROW_STEPS; k++) {
+            const u32 col = row_col(2 * k);
+            const E2 x = gl::acc_reduce(acc[2 * k]), y = gl::acc_reduce(acc[2 * k + 1]);
+            if (col + 1 < cols) {
+                st2(job.o0 + base + col, x.c0, y.c0);
+                st2(job.o1 + base + col, x.c1, y.c1);
+            } else if (col < cols) {
+                job.o0[base + col] = x.c0;
+                job.o1[base + col] = x.c1;
+            }
+        }
+    }
+}
+
+struct EvalTable {
+    const u64 *t0, *t1;  // t1 nullptr: base field
+    u32 n;               // variables: the first n coordinates of the point
+    u32 pad;
+};
+struct EvalTablesArgs {
+    const EvalTable *tables;
+    u32 n_tables, shares;        // workgroups per table, a power of two
+    u64 *partial;                // 2 words per table and share
+    u32 *counter;                // ticket counter, zero between launches
+    u64 *fin_out;                // area of SL_FIN_AREA_WORDS words: the values, then sequence number and check word
+    u64 seq;
+    u64 p[2 * EQ_MAX_VARS];
+};
+template <int KIND>
+__device__ __forceinline__ E2 eval_rows(const EvalTable &t, const PointSplit &s, const u64 *p, u64 row0, u64 row1, u64 step, const SmallEq &part0, const SmallEq &part1)
+{
+    E2 v[2 * ROW_STEPS], lw[2 * ROW_STEPS];
+    low_weights(s, part0, part1, lw);
+    gl::E2Acc total = gl::e2acc_zero();
+    for (u64 row = row0; row < row1; row += step) {
+        load_row<KIND>(t.t0, t.t1, row << s.lo, 1u << s.lo, v);
+        E2 hw = row_weight(s, part0, part1, row);
+        if (s.top) hw = gl::mul(hw, eq_entry(p, s.lo + s.ha + s.hb, s.top, (u32)(row >> EVAL_TOP_SHIFT)));
+        gl::acc_mul(total, weigh_row<KIND>(lw, v), gl::prep(hw));
+    }
+    return gl::acc_reduce(total);
+}
+__global__ void __launch_bounds__(BLOCK) eval_tables_kernel(EvalTablesArgs a)
+{
+    __shared__ SmallEq part0, part1;
+    __shared__ u32 lds[(BLOCK / WAVE) * 6];
+    __shared__ u64 xr[BLOCK / WAVE];
+    __shared__ int last_flag;
+    const u32 tid = threadIdx.x;
+    const EvalTable t = a.tables[blockIdx.y];
+    const PointSplit s = split_point(t.n);
+    small_eq_tables(a.p, s, part0, part1);
+    __syncthreads();
+    const u64 n_rows = 1ull << (t.n - s.lo);
+    E2 acc[1];
+    acc[0] = t.t1 ? eval_rows<1>(t, s, a.p, blockIdx.x, n_rows, gridDim.x, part0, part1) : eval_rows<0>(t, s, a.p, blockIdx.x, n_rows, gridDim.x, part0, part1);
+    block_reduce<1>(acc, lds);
+    if (tid == 0) {
+        u64 *o = a.partial + 2 * ((u64)blockIdx.y * a.shares + blockIdx.x);
+        st_agent(o, acc[0].c0);
+        st_agent(o + 1, acc[0].c1);
+    }
+    if (!take_ticket(a.counter, a.shares * a.n_tables, &last_flag)) return;
+    u64 x = 0;
+    for (u32 k = tid; k < a.n_tables; k += BLOCK) {
+        E2 v = gl::e2_zero();
+        for (u32 q = 0; q < a.shares; q++) {
+            const u64 *o = a.partial + 2 * ((u64)k * a.shares + q);
+            v = gl::add(v, gl::e2(ld_agent(o), ld_agent(o + 1)));
+        }
+        st_sys(a.fin_out + 2 * k, v.c0);
+        st_sys(a.fin_out + 2 * k + 1, v.c1);
+        x ^= sl_fin_mix(v.c0, 2 * k) ^ sl_fin_mix(v.c1, 2 * k + 1);
+    }
+#pragma unroll
+    for (int off = WAVE / 2; off >= 1; off >>= 1) x ^= __shfl_xor(x, off, WAVE);
+    if (tid % WAVE == 0) xr[tid / WAVE] = x;
+    __syncthreads();
+    if (tid == 0) {
+        for (int w = 1; w < BLOCK / WAVE; w++) x ^= xr[w];
+        *a.counter = 0;
+        st_sys(a.fin_out + SL_FIN_CHK_SLOT, x ^ a.seq);
+        st_sys(a.fin_out + SL_FIN_SEQ_SLOT, a.seq);
     }
 }
 
