@@ -35,6 +35,7 @@ namespace {
 // 3 workgroups per CU on 256 CUs: measured best for the streaming kernels (each workgroup pays a fixed
 // reduction + ticket epilogue, so more, thinner workgroups lose more than they gain in latency hiding)
 constexpr u32 MAX_BLOCKS = 768;
+constexpr u64 COMPUTE_UNITS = 256;
 // areas of pinned memory for the outputs (and the small levels) of the fraction trees built last
 constexpr u32 LOGUP_OUT_AREAS = 8;
 constexpr size_t LOGUP_SHADOW_STRIDE = 2048;  // words per tree: dpk::LOGUP_SHADOW_WORDS rounded up
@@ -1293,7 +1294,8 @@ int32_t evaluate_at(dps_ctx *ctx, const dps_mle *mle, const uint64_t *point, u32
     a.t1 = mle->p1();
     a.n = n;
     a.n_rows = 1ull << (n - std::min<u32>(n, dpk::EVAL_LO_BITS));
-    const u32 blocks = (u32)std::min<u64>(a.n_rows, dpk::EVAL_MAX_BLOCKS);
+    // a row a workgroup up to a workgroup a compute unit, two from there on
+    const u32 blocks = (u32)std::min<u64>(a.n_rows > COMPUTE_UNITS ? a.n_rows / 2 : a.n_rows, dpk::EVAL_MAX_BLOCKS);
     a.rows_per_block = a.n_rows / blocks;
     if (n) memcpy(a.p, point, 16 * (size_t)n);
     dpk::FastFin ff;
@@ -3274,28 +3276,54 @@ int32_t combine_terms(dps_ctx *ctx, dps_sc *sc, const dps_mle *const *mles, cons
     for (u32 k = 0; k < sc->n_mles; k++)
         if (sc->inner_of[k] < 0) sc->outside.push_back(dps_sc::Outside{k, nv0[k], mles[k]->pad_vars != 0, mles[k]->p0(), mles[k]->p1(), mles[k]->eq});
     const size_t job_words = jobs.size() * sizeof(dpk::CombJob) / 8, item_words = items.size() * sizeof(dpk::CombItem) / 8;
-    static_assert(sizeof(dpk::CombJob) % 8 == 0 && sizeof(dpk::CombItem) % 8 == 0 && sizeof(dpk::EvalTable) % 8 == 0, "descriptors are staged as words");
+    static_assert(sizeof(dpk::EvalTable) % 8 == 0, "descriptors are staged as words");
+    const size_t words = job_words + item_words + points.size();
     const size_t eval_words = sc->outside.size() * sizeof(dpk::EvalTable) / 8;
-    *fits = STAGE_LO + std::max(job_words + item_words + points.size(), eval_words) <= ctx->pinned_words / 2 && jobs.size() <= 65535 &&
-            2 * sc->outside.size() <= (size_t)dpk::SL_FIN_MAX_WORDS;
+    *fits = STAGE_LO + std::max(words, eval_words) <= ctx->pinned_words / 2 && jobs.size() <= 65535 && 2 * sc->outside.size() <= (size_t)dpk::SL_FIN_MAX_WORDS;
     if (!*fits) return DPS_OK;
-    CHK(stage_region(ctx));
-    u64 *h = ctx->h_pinned + STAGE_LO;
+    const u64 n_out = 1ull << n_vars;
+    // rows of 1024 entries from a workgroup a compute unit on, of 512 below
+    const bool wide = (n_out >> 10) * jobs.size() >= COMPUTE_UNITS;
+    const dim3 grid((u32)std::min<u64>(std::max<u64>(n_out >> (wide ? 10 : 9), 1), 1024), (u32)jobs.size());
+    dpk::CombArgs a;
+    a.n_out = n_out;
+    a.n_jobs = (u32)jobs.size();
+    a.n_items = (u32)items.size();
+    a.src = nullptr;
+    u64 *h = a.words;
+    const bool inside = words <= dpk::COMB_INLINE_WORDS;
+    if (!inside) {
+        CHK(stage_region(ctx));
+        h = ctx->h_pinned + STAGE_LO;
+        a.src = ctx->d_pinned + STAGE_LO;
+    }
     memcpy(h, jobs.data(), job_words * 8);
     memcpy(h + job_words, items.data(), item_words * 8);
     if (!points.empty()) memcpy(h + job_words + item_words, points.data(), points.size() * 8);
-    const u64 *d = ctx->d_pinned + STAGE_LO;
-    const u64 n_out = 1ull << n_vars;
+    void *on_device = nullptr;
+    if (!inside && (u64)grid.x * grid.y > COMPUTE_UNITS) {
+        CHK(pool_alloc(ctx, words * 8, &on_device));
+        if (const hipError_t e = hipMemcpyAsync(on_device, h, words * 8, hipMemcpyHostToDevice, ctx->stream); e != hipSuccess) {
+            pool_free(ctx, on_device);
+            return fail(ctx, DPS_ERR_HIP, "descriptor copy: %s", hipGetErrorString(e));
+        }
+        a.src = (const u64 *)on_device;
+    }
+    hipError_t e;
     {
         double bytes = (double)jobs.size() * (double)n_out * 16.0;
         for (const dpk::CombItem &it : items)
             if (it.t0) bytes += (double)it.len * (it.t1 ? 16.0 : 8.0);
         ProfScope ps(ctx, DPS_K_EQ, bytes);
-        dpk::combine_kernel<<<dim3((u32)std::min<u64>(std::max<u64>(n_out >> dpk::EVAL_LO_BITS, 1), 1024), (u32)jobs.size()), dpk::BLOCK, 0, ctx->stream>>>(
-            reinterpret_cast<const dpk::CombJob *>(d), reinterpret_cast<const dpk::CombItem *>(d + job_words), d + job_words + item_words, n_out);
-        HIPCHK(ctx, hipGetLastError());
+        if (wide)
+            dpk::combine_kernel<2><<<grid, dpk::BLOCK, 0, ctx->stream>>>(a);
+        else
+            dpk::combine_kernel<1><<<grid, dpk::BLOCK, 0, ctx->stream>>>(a);
+        e = hipGetLastError();
     }
-    CHK(stage_region_read(ctx));
+    pool_free(ctx, on_device);  // (reused in stream order)
+    if (e != hipSuccess) return fail(ctx, DPS_ERR_HIP, "combine launch: %s", hipGetErrorString(e));
+    if (!inside) CHK(stage_region_read(ctx));
     return dps_sc_begin(ctx, n_vars, in_mles.data(), (u32)in_mles.size(), in_terms.data(), (u32)in_terms.size(), &sc->inner);
 }
 

@@ -2780,20 +2780,18 @@ __global__ void __launch_bounds__(BLOCK) axis_dot_row_kernel(AxisArgs a)
 // ---------------------------------------------------------------------------
 // evaluation of a table at a point, one launch and no memory beyond a partial sum per workgroup
 //
-//   value = sum_row eq_hi[row] * ( sum_l eq_lo[l] * table[row * 2^lo + l] ),   eq_lo over the lo lowest coordinates of the
-// point, eq_hi over the others.  No eq table is ever in memory: the point travels in the kernel arguments, every workgroup
-// makes four tables of at most 64 entries in LDS (the low coordinates in two parts, the next twelve in two parts), a
-// thread's eq_lo weights are products of two of their entries and stay in registers across its rows, and a row's weight is
-// a product of two entries (of three beyond 23 variables: the top coordinates' product changes every 4096 rows at most).
-// Every sum is unreduced until its end; the last workgroup gathers the partial sums and hands the value to the host.
-// Rows of 2^EVAL_LO_BITS = 2048 entries, so that 2^20 entries already make 512 workgroups (8 entries a thread and row).
-// Bound: the latency of one launch up to 2^20 entries (8 MB), HBM above.  Through the eq table in memory (three launches),
-// a dot product and a pass over its partial sums 2^20 base entries took 170 us, 122 of them in the last pass, whose one
-// thread added 1024 partial sums one behind the other; now 20 us with the way to the host and back.
+//   value = sum_row eq_hi[row] * ( sum_l eq_lo[l] * table[row * 2^11 + l] ),   eq_lo over the 11 lowest coordinates of the
+// point, eq_hi over the others.  No eq table is ever in memory: the point travels in the kernel arguments and every workgroup
+// makes the weights of EqGroups from it.  An entry costs its product with one of eight weights that all threads share, a row
+// one product more, a thread one at its end; every sum is unreduced until then.  The last workgroup gathers the partial sums and
+// hands the value to the host.  Rows of 2^EVAL_LO_BITS = 2048 entries (8 a thread), two a workgroup from 512 rows on: 2^20
+// entries 11.9 us with 256 workgroups, 14.3 with 512.
+// Bound: the latency of one launch up to 2^20 entries (8 MB), HBM above.  With tables of up to 64 entries made by a wavefront
+// each and a weight per entry in registers (about 17 field products one behind the other, 0.26 us each) a launch took
+// 8.9 / 15.2 / 27.5 us at 2^10 / 2^16 / 2^20 base entries; now 6.0 / 8.5 / 11.9.
 // ---------------------------------------------------------------------------
 constexpr u32 EVAL_LO_BITS = 11;
 constexpr u32 EVAL_MAX_BLOCKS = 1024;
-constexpr u32 EVAL_TOP_SHIFT = 12;  // rows that share a product of the top coordinates (log2)
 // layout of a work area (64-bit words): the ticket counter (32 bits used), zero between launches, and a partial sum per workgroup
 constexpr u32 WS_OFF_COUNTER = 0, WS_OFF_PARTIAL = 32;
 constexpr u32 WS_WORDS = WS_OFF_PARTIAL + 2 * EVAL_MAX_BLOCKS;
@@ -2807,55 +2805,8 @@ struct EvalArgs {
     u64 p[2 * EQ_MAX_VARS];      // 2 limbs per coordinate
 };
 
-// How the coordinates of a point are shared out: rows of 2^lo entries (la + lb coordinates), then ha + hb, then `top`
-struct PointSplit {
-    u32 lo, la, lb, ha, hb, top;
-};
-__device__ __forceinline__ PointSplit split_point(u32 n)
-{
-    PointSplit s;
-    s.lo = n < EVAL_LO_BITS ? n : EVAL_LO_BITS;
-    s.la = s.lo / 2;
-    s.lb = s.lo - s.la;
-    const u32 hi = n - s.lo;
-    s.ha = hi < 6 ? hi : 6;
-    s.hb = hi - s.ha < 6 ? hi - s.ha : 6;
-    s.top = hi - s.ha - s.hb;
-    return s;
-}
-// prod_b (bit_b(e) ? p[first + b] : 1 - p[first + b]), b < bits (`p`: 2 limbs per coordinate)
-__device__ __forceinline__ E2 eq_entry(const u64 *p, u32 first, u32 bits, u32 e)
-{
-    E2 v = gl::e2_one();
-    for (u32 b = 0; b < bits; b++) {
-        const E2 r = gl::e2(p[2 * (first + b)], p[2 * (first + b) + 1]);
-        v = gl::mul(v, ((e >> b) & 1) ? r : gl::sub(gl::e2_one(), r));
-    }
-    return v;
-}
-// the four small tables of a point, one wavefront each (visible after a barrier)
-typedef u64 SmallEq[4][64];
-__device__ __forceinline__ void small_eq_tables(const u64 *p, const PointSplit &s, SmallEq &part0, SmallEq &part1)
-{
-    static_assert(BLOCK == 4 * WAVE, "four wavefronts make the four small tables");
-    const u32 w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-    const u32 bits = w == 0 ? s.la : w == 1 ? s.lb : w == 2 ? s.ha : s.hb;
-    const u32 first = w == 0 ? 0 : w == 1 ? s.la : w == 2 ? s.lo : s.lo + s.ha;
-    if (lane < (1u << bits)) {
-        const E2 v = eq_entry(p, first, bits, lane);
-        part0[w][lane] = v.c0;
-        part1[w][lane] = v.c1;
-    }
-}
-__device__ __forceinline__ E2 small_eq(const SmallEq &part0, const SmallEq &part1, u32 w, u32 i) { return gl::e2(part0[w][i], part1[w][i]); }
-// the weight of a row's first entry over the coordinates above `lo`, without those of `top`
-__device__ __forceinline__ E2 row_weight(const PointSplit &s, const SmallEq &part0, const SmallEq &part1, u64 row)
-{
-    return gl::mul(small_eq(part0, part1, 2, (u32)row & ((1u << s.ha) - 1)), small_eq(part0, part1, 3, (u32)(row >> s.ha) & ((1u << s.hb) - 1)));
-}
 // A thread's entries of a row: columns 2 (tid + BLOCK k), 2 (tid + BLOCK k) + 1 for k = 0..ROW_STEPS-1, as far as the row has them
 constexpr int ROW_STEPS = (1 << EVAL_LO_BITS) / (2 * BLOCK);
-__device__ __forceinline__ u32 row_col(int k) { return 2 * (threadIdx.x + BLOCK * (k / 2)) + (k & 1); }
 // KIND: 0 base-field entries, 1 extension entries, 8 raw int64, 2 raw int16
 template <int KIND>
 __device__ __forceinline__ void load_row(const void *t0, const u64 *t1, u64 base, u32 cols, E2 (&v)[2 * ROW_STEPS])
@@ -2868,7 +2819,7 @@ __device__ __forceinline__ void load_row(const void *t0, const u64 *t1, u64 base
     };
 #pragma unroll
     for (int k = 0; k < ROW_STEPS; k++) {
-        const u32 c = row_col(2 * k);
+        const u32 c = 2 * (threadIdx.x + BLOCK * k);
         v[2 * k] = v[2 * k + 1] = gl::e2_zero();
         if (KIND == 0 || KIND == 1) {
             if (c + 1 < cols) {
@@ -2886,69 +2837,119 @@ __device__ __forceinline__ void load_row(const void *t0, const u64 *t1, u64 base
         }
     }
 }
-// sum_k w_k v_k of a thread's entries of a row
-template <int KIND>
-__device__ __forceinline__ E2 weigh_row(const E2 (&w)[2 * ROW_STEPS], const E2 (&v)[2 * ROW_STEPS])
+// ---------------------------------------------------------------------------
+// The eq table of a point a row of 2^EVAL_LO_BITS = 2048 entries at a time, a thread holding the columns 2 (tid + BLOCK k) + par,
+// k < 4, par < 2: a column's bits are par (bit 0), the thread's (1 .. 8) and k's (9, 10), so an entry is the product of
+//   - a weight of the row (coordinates 11 and up),
+//   - a weight of the thread (coordinates 1 .. 8),
+//   - a weight of (par, k) (coordinates 0, 9, 10), the same for all threads.
+// All are products of entries of the tables of three coordinates each, which a workgroup makes from the point, one entry a
+// thread: two field products one behind the other instead of the six of a 64-entry table, and no weight per entry.  (A
+// product of the extension is 0.26 us as a link of a chain and 0.16 us a wavefront and SIMD of throughput.)  Coordinates the
+// point does not have count as zero: weight 1 where the bit is 0, and no entry has it set.
+// ---------------------------------------------------------------------------
+constexpr u32 EQG_LOW = 4;                                            // {0, 9, 10}, {1, 2, 3}, {4, 5, 6}, {7, 8}
+constexpr u32 EQG_MAX = EQG_LOW + (EQ_MAX_VARS - EVAL_LO_BITS + 2) / 3;
+struct EqGroups {
+    u64 c0[EQG_MAX][8], c1[EQG_MAX][8];
+    __device__ __forceinline__ E2 at(u32 g, u32 e) const { return gl::e2(c0[g][e], c1[g][e]); }
+};
+__device__ __forceinline__ u32 eq_groups(u32 n) { return n > EVAL_LO_BITS ? EQG_LOW + (n - EVAL_LO_BITS + 2) / 3 : EQG_LOW; }
+// entry e of group g of the point of n coordinates at `p` (2 limbs each)
+__device__ __forceinline__ void eq_group_entry(const u64 *p, u32 n, u32 g, u32 e, EqGroups &out)
 {
-    gl::E2Acc s = gl::e2acc_zero();
+    E2 v = gl::e2_one();
 #pragma unroll
-    for (int k = 0; k < 2 * ROW_STEPS; k++) {
-        if (KIND == 1)
-            gl::acc_mul(s, v[k], gl::prep(w[k]));
-        else
-            gl::acc_mul_base(s, w[k], v[k].c0);
+    for (u32 b = 0; b < 3; b++) {
+        const u32 c = g == 0 ? (b == 0 ? 0 : 8 + b) : g < EQG_LOW ? 3 * g - 2 + b : EVAL_LO_BITS + 3 * (g - EQG_LOW) + b;
+        const bool there = c < n && !(g == EQG_LOW - 1 && b == 2);  // (coordinate 9 is the first group's)
+        const E2 r = there ? gl::e2(p[2 * c], p[2 * c + 1]) : gl::e2_zero();
+        const E2 x = ((e >> b) & 1) ? r : gl::sub(gl::e2_one(), r);
+        v = b == 0 ? x : gl::mul(v, x);
     }
-    return gl::acc_reduce(s);
+    out.c0[g][e] = v.c0;
+    out.c1[g][e] = v.c1;
 }
-__device__ __forceinline__ void low_weights(const PointSplit &s, const SmallEq &part0, const SmallEq &part1, E2 (&w)[2 * ROW_STEPS])
+__device__ __forceinline__ E2 eq_thread_weight(const EqGroups &t)
 {
-#pragma unroll
-    for (int k = 0; k < 2 * ROW_STEPS; k++) {
-        const u32 c = row_col(k);
-        w[k] = gl::e2_zero();
-        if (c < (1u << s.lo)) w[k] = gl::mul(small_eq(part0, part1, 0, c & ((1u << s.la) - 1)), small_eq(part0, part1, 1, c >> s.la));
+    const u32 i = threadIdx.x;
+    return gl::mul(gl::mul(t.at(1, i & 7), t.at(2, (i >> 3) & 7)), t.at(3, i >> 6));
+}
+// the weight of a row over the coordinates from EVAL_LO_BITS on
+__device__ __forceinline__ E2 eq_row_weight(const EqGroups &t, u32 n_groups, u64 row)
+{
+    if (n_groups == EQG_LOW) return gl::e2_one();
+    E2 v = t.at(EQG_LOW, (u32)row & 7);
+    for (u32 g = EQG_LOW + 1; g < n_groups; g++) v = gl::mul(v, t.at(g, (u32)(row >> (3 * (g - EQG_LOW))) & 7));
+    return v;
+}
+
+// The weights (par, k) of a thread's entries of a row, prepared (EqGroups group 0: entry par + 2 k); one wavefront makes them
+struct RowWeights {
+    u64 c0[2 * ROW_STEPS], c1[2 * ROW_STEPS], w[2 * ROW_STEPS];
+};
+static_assert(2 * ROW_STEPS == 8, "a table of three coordinates");
+
+// The sum over rows first, first + step, ... (`count` of them) of the products of a table's entries and eq weights; the result
+// is this thread's share.  Entries and (par, k) weights first, unreduced; the row's weight once a row, worked out by one
+// thread a row beforehand; the thread's weight once at the end.  The first row is asked for before the weights are made.
+template <int KIND>
+__device__ __forceinline__ E2 eval_rows(const void *t0, const u64 *t1, const u64 *p, u32 n, u64 first, u64 step, u64 count, EqGroups &groups, RowWeights &rw,
+                                        u64 (&hw0)[BLOCK], u64 (&hw1)[BLOCK])
+{
+    const u32 tid = threadIdx.x, lo = n < EVAL_LO_BITS ? n : EVAL_LO_BITS, n_groups = eq_groups(n);
+    E2 v[2 * ROW_STEPS];
+    if (count) load_row<KIND>(t0, t1, first << lo, 1u << lo, v);
+    static_assert(8 * EQG_MAX <= BLOCK, "an entry a thread");
+    if (tid < 8 * n_groups) {
+        eq_group_entry(p, n, tid / 8, tid % 8, groups);
+        if (tid < 8) rw.c0[tid] = groups.c0[0][tid], rw.c1[tid] = groups.c1[0][tid], rw.w[tid] = gl::mul_small(groups.c1[0][tid], (u32)gl::W);
     }
+    gl::E2Acc total = gl::e2acc_zero();
+    for (u64 at = 0; at < count; at += BLOCK) {
+        __syncthreads();  // the groups are there; the row weights before have been read
+        const u32 here = count - at < BLOCK ? (u32)(count - at) : BLOCK;
+        if (tid < here) {
+            const E2 h = eq_row_weight(groups, n_groups, first + (at + tid) * step);
+            hw0[tid] = h.c0;
+            hw1[tid] = h.c1;
+        }
+        __syncthreads();
+        for (u32 r = 0; r < here; r++) {
+            gl::E2Acc s = gl::e2acc_zero();
+#pragma unroll
+            for (int k = 0; k < 2 * ROW_STEPS; k++) {
+                if (KIND == 1) {
+                    gl::E2P w;
+                    w.c0 = rw.c0[k], w.c1 = rw.c1[k], w.w = rw.w[k];
+                    gl::acc_mul(s, v[k], w);
+                } else {
+                    gl::acc_mul_base(s, gl::e2(rw.c0[k], rw.c1[k]), v[k].c0);
+                }
+            }
+            if (at + r + 1 < count) load_row<KIND>(t0, t1, (first + (at + r + 1) * step) << lo, 1u << lo, v);
+            gl::acc_mul(total, gl::acc_reduce(s), gl::prep(gl::e2(hw0[r], hw1[r])));
+        }
+    }
+    if (!count) return gl::e2_zero();
+    return gl::mul(gl::acc_reduce(total), eq_thread_weight(groups));
 }
 
 template <int KIND>
 __global__ void __launch_bounds__(BLOCK) eval_point_kernel(EvalArgs a, FastFin ff)
 {
-    __shared__ SmallEq part0, part1;
+    __shared__ EqGroups groups;
+    __shared__ RowWeights rw;
+    __shared__ u64 hw0[BLOCK], hw1[BLOCK];
     __shared__ u32 lds[(BLOCK / WAVE) * 6];
     __shared__ int last_flag;
-    const u32 tid = threadIdx.x;
-    const PointSplit s = split_point(a.n);
-    small_eq_tables(a.p, s, part0, part1);
-    const u64 row0 = (u64)blockIdx.x * a.rows_per_block;
-    // (the first row is asked for before the tables are there: its loads and their products overlap)
-    E2 v[2 * ROW_STEPS], lw[2 * ROW_STEPS];
-    load_row<KIND>(a.t0, a.t1, row0 << s.lo, 1u << s.lo, v);
-    __syncthreads();
-    low_weights(s, part0, part1, lw);
-    gl::E2Acc total = gl::e2acc_zero();
-    E2 top_w = gl::e2_one();
-    u64 top_of = ~0ull;
-    for (u64 r = 0; r < a.rows_per_block; r++) {
-        const u64 row = row0 + r;
-        const E2 x = weigh_row<KIND>(lw, v);
-        if (r + 1 < a.rows_per_block) load_row<KIND>(a.t0, a.t1, (row + 1) << s.lo, 1u << s.lo, v);
-        E2 hw = row_weight(s, part0, part1, row);
-        if (s.top) {
-            if ((row >> EVAL_TOP_SHIFT) != top_of) {
-                top_of = row >> EVAL_TOP_SHIFT;
-                top_w = eq_entry(a.p, s.lo + s.ha + s.hb, s.top, (u32)top_of);
-            }
-            hw = gl::mul(hw, top_w);
-        }
-        gl::acc_mul(total, x, gl::prep(hw));
-    }
-    E2 acc[1] = {gl::acc_reduce(total)};
+    E2 acc[1] = {eval_rows<KIND>(a.t0, a.t1, a.p, a.n, (u64)blockIdx.x * a.rows_per_block, 1, a.rows_per_block, groups, rw, hw0, hw1)};
     block_reduce<1>(acc, lds);
     if (gridDim.x == 1) {
         publish_sums<1>(ff.out_host, ff.seq, ff.counter, acc);
         return;
     }
-    if (tid == 0) {
+    if (threadIdx.x == 0) {
         u64 *o = const_cast<u64 *>(ff.partial) + blockIdx.x;
         st_agent(o, acc[0].c0);
         st_agent(o + gridDim.x, acc[0].c1);
@@ -2965,10 +2966,15 @@ __global__ void __launch_bounds__(BLOCK) eval_point_kernel(EvalArgs a, FastFin f
 //
 // combine_kernel writes the tables M (grid row = table).  An item is a table times its coefficient -- its entries, zero
 // behind its end where it is zero-padded -- or the eq table of a point, whose entries are made here from the point and never
-// stored.  A workgroup writes rows of 2^EVAL_LO_BITS entries, 8 a thread, every entry one unreduced sum over the items.
-// Bound: each table once in, M once out; for eq tables one extension product an entry and table (2^20 entries of four eq
-// tables 9 us) where building, folding and weighting them as tables of their own moved eight times the bytes.
-// Descriptors and points lie in host-visible memory, written just before the launch.
+// stored.  A workgroup writes rows, every entry one unreduced sum over the items; of an eq table it makes the weights of
+// EqGroups, of four items at the same time, and an entry costs the products of its sum alone.  Descriptors and points travel
+// in the kernel arguments where they fit; otherwise they are taken into LDS together, from host-visible memory or, for a grid
+// of more than a workgroup a compute unit, from a copy on the device.  Rows are of 512 entries (STEPS = 1, four tables' loads
+// in flight) where rows of 1024 (STEPS = 2) would not make a workgroup a compute unit (four eq tables of 2^16 entries 13.0
+// and 13.7 us, of 2^19 27 and 18 us; rows of 2048 take 256 registers: 17 and 19 us).
+// Bound: each table once in, M once out; for eq tables one extension product an entry and table.  Four eq tables of 2^20
+// entries: 77 -> 33 us; 34 tables of 2^11 entries from about 100 others: 41 -> 19 us (kernel trace).  (Before, descriptors were read one item after
+// the other and every item cost the workgroup a chain of about 20 field products and a weight per entry.)
 //
 // eval_tables_kernel evaluates the tables that are in no product any more at the sum's final point (grid: a workgroup per
 // table and share of its rows); the last workgroup adds the shares and hands the values to the host.
@@ -2977,69 +2983,131 @@ struct CombItem {
     const u64 *t0, *t1;  // t0 nullptr: eq table of the point at `point_off`; t1 nullptr: base field
     u64 c0, c1;          // coefficient
     u64 len;             // entries: a power of two
-    u32 point_off;       // words from `points`
+    u32 point_off;       // words from the first point
     u32 n_bits;          // log2(len)
 };
 struct CombJob {
     u64 *o0, *o1;
     u32 first, count;    // items
 };
-__global__ void __launch_bounds__(BLOCK) combine_kernel(const CombJob *__restrict__ jobs, const CombItem *__restrict__ items, const u64 *__restrict__ points,
-                                                        u64 n_out)
+constexpr u32 COMB_JOB_WORDS = sizeof(CombJob) / 8, COMB_ITEM_WORDS = sizeof(CombItem) / 8;
+constexpr u32 COMB_INLINE_WORDS = 496;
+constexpr u32 COMB_STAGE = 64;  // items taken into LDS together
+struct CombArgs {
+    const u64 *src;      // jobs, items, points; nullptr: in `words`
+    u64 n_out;
+    u32 n_jobs, n_items;
+    u64 words[COMB_INLINE_WORDS];
+};
+static_assert(sizeof(CombJob) % 8 == 0 && sizeof(CombItem) % 8 == 0 && sizeof(CombArgs) <= 4096, "descriptors are copied as words, in the kernel arguments too");
+template <int STEPS>
+__global__ void __launch_bounds__(BLOCK) combine_kernel(CombArgs a)
 {
-    __shared__ SmallEq part0, part1;
-    __shared__ u64 high0[64], high1[64];
-    const CombJob job = jobs[blockIdx.y];
+    static_assert(STEPS == 1 || STEPS == 2, "rows of 512 or 1024 entries");
+    constexpr u32 STEP_BITS = STEPS - 1;
+    constexpr u32 LO_BITS = EVAL_LO_BITS - 2 + STEP_BITS;
+    constexpr u32 PART_BITS = EVAL_LO_BITS - LO_BITS;  // a row of this launch is one of 2^PART_BITS parts of a row of EqGroups
+    constexpr u32 BATCH = BLOCK / WAVE;                // items whose eq weights are made at the same time
+    constexpr u32 GROUP = STEPS == 1 ? BATCH : 1;      // tables whose loads are in flight together
+    __shared__ u64 staged[COMB_STAGE * COMB_ITEM_WORDS];
+    __shared__ EqGroups groups[BATCH];
+    __shared__ u64 row0[BATCH], row1[BATCH];
+    const CombItem *its = reinterpret_cast<const CombItem *>(staged);
+    const u64 *src = a.src ? a.src : a.words;
+    const CombJob job = reinterpret_cast<const CombJob *>(src)[blockIdx.y];
+    const u64 *items = src + (u64)a.n_jobs * COMB_JOB_WORDS;
+    const u64 *points = items + (u64)a.n_items * COMB_ITEM_WORDS;
     const u32 tid = threadIdx.x;
-    const u32 cols = n_out < (1ull << EVAL_LO_BITS) ? (u32)n_out : 1u << EVAL_LO_BITS;
-    const u64 n_rows = n_out / cols;
+    const u32 cols = a.n_out < (1ull << LO_BITS) ? (u32)a.n_out : 1u << LO_BITS;
+    const u64 n_rows = a.n_out / cols;
     for (u64 row = blockIdx.x; row < n_rows; row += gridDim.x) {
         const u64 base = row * cols;
-        gl::E2Acc acc[2 * ROW_STEPS];
+        gl::E2Acc acc[2 * STEPS];
 #pragma unroll
-        for (int k = 0; k < 2 * ROW_STEPS; k++) acc[k] = gl::e2acc_zero();
-        for (u32 it = 0; it < job.count; it++) {
-            const CombItem m = items[job.first + it];
-            if (base >= m.len) continue;  // (the whole workgroup: zero from here on)
-            const u32 have = m.len - base < cols ? (u32)(m.len - base) : cols;
-            const gl::E2P c = gl::prep(gl::e2(m.c0, m.c1));
-            if (m.t0) {
-                E2 v[2 * ROW_STEPS];
-                if (m.t1) {
-                    load_row<1>(m.t0, m.t1, base, have, v);
-#pragma unroll
-                    for (int k = 0; k < 2 * ROW_STEPS; k++) gl::acc_mul(acc[k], v[k], c);
-                } else {
-                    load_row<0>(m.t0, nullptr, base, have, v);
-#pragma unroll
-                    for (int k = 0; k < 2 * ROW_STEPS; k++) gl::acc_mul_base(acc[k], gl::e2(c.c0, c.c1), v[k].c0);
+        for (int k = 0; k < 2 * STEPS; k++) acc[k] = gl::e2acc_zero();
+        for (u32 first = 0; first < job.count; first += COMB_STAGE) {
+            const u32 count = job.count - first < COMB_STAGE ? job.count - first : COMB_STAGE;
+            __syncthreads();  // the items and weights before have been read
+            for (u32 w = tid; w < count * COMB_ITEM_WORDS; w += BLOCK) staged[w] = items[(u64)(job.first + first) * COMB_ITEM_WORDS + w];
+            __syncthreads();
+            for (u32 b = 0; b < count; b += BATCH) {
+                const u32 n_batch = count - b < BATCH ? count - b : BATCH;
+                bool any_eq = false;
+                for (u32 q = 0; q < n_batch; q++) any_eq = any_eq || (!its[b + q].t0 && base < its[b + q].len);
+                if (any_eq) {  // (the same for the whole workgroup)
+                    __syncthreads();
+                    for (u32 j = tid; j < n_batch * EQG_MAX * 8; j += BLOCK) {
+                        const u32 q = j / (EQG_MAX * 8), g = j / 8 % EQG_MAX;
+                        const CombItem &m = its[b + q];
+                        if (!m.t0 && base < m.len && g < eq_groups(m.n_bits)) eq_group_entry(points + m.point_off, m.n_bits, g, j % 8, groups[q]);
+                    }
+                    __syncthreads();
+                    if (tid < n_batch) {
+                        const CombItem &m = its[b + tid];
+                        if (!m.t0 && base < m.len) {
+                            const E2 v = gl::mul(eq_row_weight(groups[tid], eq_groups(m.n_bits), row >> PART_BITS), gl::e2(m.c0, m.c1));
+                            row0[tid] = v.c0;
+                            row1[tid] = v.c1;
+                        }
+                    }
+                    __syncthreads();
                 }
-                continue;
-            }
-            // (a point of fewer coordinates than a row's: `have` entries, and the point's row is shorter than this one's)
-            const PointSplit s = split_point(m.n_bits);
-            const u64 *p = points + m.point_off;
-            __syncthreads();  // the tables of the item before have been read
-            small_eq_tables(p, s, part0, part1);
-            __syncthreads();
-            if (tid < (1u << s.lb)) {
-                // the row's weight and the coefficient, taken into the upper low table
-                E2 hw = gl::mulp(row_weight(s, part0, part1, row), c);
-                if (s.top) hw = gl::mul(hw, eq_entry(p, s.lo + s.ha + s.hb, s.top, (u32)(row >> EVAL_TOP_SHIFT)));
-                const E2 v = gl::mul(small_eq(part0, part1, 1, tid), hw);
-                high0[tid] = v.c0;
-                high1[tid] = v.c1;
-            }
-            __syncthreads();
+                for (u32 g = 0; g < n_batch; g += GROUP) {
+                    E2 v[GROUP][2 * STEPS];
 #pragma unroll
-            for (int k = 0; k < 2 * ROW_STEPS; k++) {
-                const u32 col = row_col(k);
-                if (col < have) gl::acc_mul(acc[k], small_eq(part0, part1, 0, col & ((1u << s.la) - 1)), gl::prep(gl::e2(high0[col >> s.la], high1[col >> s.la])));
+                    for (u32 q = 0; q < GROUP; q++) {
+                        if (g + q >= n_batch) break;
+                        const CombItem &m = its[b + g + q];
+                        if (!m.t0 || base >= m.len) continue;
+                        const u32 have = m.len - base < cols ? (u32)(m.len - base) : cols;
+#pragma unroll
+                        for (int k = 0; k < STEPS; k++) {
+                            const u32 c = 2 * (tid + BLOCK * k);
+                            E2 x = gl::e2_zero(), y = gl::e2_zero();
+                            if (c + 1 < have) {
+                                const U64x2 s = ld2(m.t0 + base + c);
+                                U64x2 t = U64x2{0, 0};
+                                if (m.t1) t = ld2(m.t1 + base + c);
+                                x = gl::e2(s.x, t.x);
+                                y = gl::e2(s.y, t.y);
+                            } else if (c < have) {
+                                x = gl::e2(m.t0[base + c], m.t1 ? m.t1[base + c] : 0);
+                            }
+                            v[q][2 * k] = x;
+                            v[q][2 * k + 1] = y;
+                        }
+                    }
+#pragma unroll
+                    for (u32 q = 0; q < GROUP; q++) {
+                        if (g + q >= n_batch) break;
+                        const CombItem &m = its[b + g + q];
+                        if (base >= m.len) continue;
+                        if (m.t0) {
+                            const gl::E2P c = gl::prep(gl::e2(m.c0, m.c1));
+#pragma unroll
+                            for (int k = 0; k < 2 * STEPS; k++) {
+                                if (m.t1)
+                                    gl::acc_mul(acc[k], v[q][k], c);
+                                else
+                                    gl::acc_mul_base(acc[k], gl::e2(c.c0, c.c1), v[q][k].c0);
+                            }
+                            continue;
+                        }
+                        // (behind the end of a point's table shorter than a row the weights are zero)
+                        const EqGroups &t = groups[g + q];
+                        const gl::E2P w = gl::prep(gl::mul(eq_thread_weight(t), gl::e2(row0[g + q], row1[g + q])));
+#pragma unroll
+                        for (int k = 0; k < 2 * STEPS; k++) {
+                            const u32 e = (u32)k | ((u32)row & ((1u << PART_BITS) - 1)) << (1 + STEP_BITS);
+                            gl::acc_mul(acc[k], t.at(0, e), w);
+                        }
+                    }
+                }
             }
         }
 #pragma unroll
-        for (int k = 0; k < ROW_STEPS; k++) {
-            const u32 col = row_col(2 * k);
+        for (int k = 0; k < STEPS; k++) {
+            const u32 col = 2 * (tid + BLOCK * k);
             const E2 x = gl::acc_reduce(acc[2 * k]), y = gl::acc_reduce(acc[2 * k + 1]);
             if (col + 1 < cols) {
                 st2(job.o0 + base + col, x.c0, y.c0);
@@ -3066,34 +3134,21 @@ struct EvalTablesArgs {
     u64 seq;
     u64 p[2 * EQ_MAX_VARS];
 };
-template <int KIND>
-__device__ __forceinline__ E2 eval_rows(const EvalTable &t, const PointSplit &s, const u64 *p, u64 row0, u64 row1, u64 step, const SmallEq &part0, const SmallEq &part1)
-{
-    E2 v[2 * ROW_STEPS], lw[2 * ROW_STEPS];
-    low_weights(s, part0, part1, lw);
-    gl::E2Acc total = gl::e2acc_zero();
-    for (u64 row = row0; row < row1; row += step) {
-        load_row<KIND>(t.t0, t.t1, row << s.lo, 1u << s.lo, v);
-        E2 hw = row_weight(s, part0, part1, row);
-        if (s.top) hw = gl::mul(hw, eq_entry(p, s.lo + s.ha + s.hb, s.top, (u32)(row >> EVAL_TOP_SHIFT)));
-        gl::acc_mul(total, weigh_row<KIND>(lw, v), gl::prep(hw));
-    }
-    return gl::acc_reduce(total);
-}
 __global__ void __launch_bounds__(BLOCK) eval_tables_kernel(EvalTablesArgs a)
 {
-    __shared__ SmallEq part0, part1;
+    __shared__ EqGroups groups;
+    __shared__ RowWeights rw;
+    __shared__ u64 hw0[BLOCK], hw1[BLOCK];
     __shared__ u32 lds[(BLOCK / WAVE) * 6];
     __shared__ u64 xr[BLOCK / WAVE];
     __shared__ int last_flag;
     const u32 tid = threadIdx.x;
     const EvalTable t = a.tables[blockIdx.y];
-    const PointSplit s = split_point(t.n);
-    small_eq_tables(a.p, s, part0, part1);
-    __syncthreads();
-    const u64 n_rows = 1ull << (t.n - s.lo);
+    const u64 n_rows = t.n > EVAL_LO_BITS ? 1ull << (t.n - EVAL_LO_BITS) : 1;
+    const u64 count = blockIdx.x < n_rows ? (n_rows - blockIdx.x + gridDim.x - 1) / gridDim.x : 0;
     E2 acc[1];
-    acc[0] = t.t1 ? eval_rows<1>(t, s, a.p, blockIdx.x, n_rows, gridDim.x, part0, part1) : eval_rows<0>(t, s, a.p, blockIdx.x, n_rows, gridDim.x, part0, part1);
+    acc[0] = t.t1 ? eval_rows<1>(t.t0, t.t1, a.p, t.n, blockIdx.x, gridDim.x, count, groups, rw, hw0, hw1)
+                  : eval_rows<0>(t.t0, nullptr, a.p, t.n, blockIdx.x, gridDim.x, count, groups, rw, hw0, hw1);
     block_reduce<1>(acc, lds);
     if (tid == 0) {
         u64 *o = a.partial + 2 * ((u64)blockIdx.y * a.shares + blockIdx.x);
@@ -3101,16 +3156,23 @@ __global__ void __launch_bounds__(BLOCK) eval_tables_kernel(EvalTablesArgs a)
         st_agent(o + 1, acc[0].c1);
     }
     if (!take_ticket(a.counter, a.shares * a.n_tables, &last_flag)) return;
+    // adjacent lanes share a table's shares (one thread a table waited for 256 loads one behind the other)
+    const u32 lanes = a.shares < (u32)WAVE ? a.shares : WAVE;  // (a power of two)
     u64 x = 0;
-    for (u32 k = tid; k < a.n_tables; k += BLOCK) {
+    for (u32 k0 = 0; k0 < a.n_tables; k0 += BLOCK / lanes) {
+        const u32 k = k0 + tid / lanes, first = tid % lanes;
         E2 v = gl::e2_zero();
-        for (u32 q = 0; q < a.shares; q++) {
+        for (u32 q = first; q < a.shares && k < a.n_tables; q += lanes) {
             const u64 *o = a.partial + 2 * ((u64)k * a.shares + q);
             v = gl::add(v, gl::e2(ld_agent(o), ld_agent(o + 1)));
         }
-        st_sys(a.fin_out + 2 * k, v.c0);
-        st_sys(a.fin_out + 2 * k + 1, v.c1);
-        x ^= sl_fin_mix(v.c0, 2 * k) ^ sl_fin_mix(v.c1, 2 * k + 1);
+        for (u32 off = 1; off < lanes; off <<= 1)
+            v = gl::add(v, gl::e2(__shfl_xor((unsigned long long)v.c0, off, WAVE), __shfl_xor((unsigned long long)v.c1, off, WAVE)));
+        if (first == 0 && k < a.n_tables) {
+            st_sys(a.fin_out + 2 * k, v.c0);
+            st_sys(a.fin_out + 2 * k + 1, v.c1);
+            x ^= sl_fin_mix(v.c0, 2 * k) ^ sl_fin_mix(v.c1, 2 * k + 1);
+        }
     }
 #pragma unroll
     for (int off = WAVE / 2; off >= 1; off >>= 1) x ^= __shfl_xor(x, off, WAVE);

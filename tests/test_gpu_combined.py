@@ -142,3 +142,14 @@ def test_session_given_up_and_errors(dp, ctx, orc):
         assert (se.round(chal) == oproof[j]).all()
         chal = opoint[j]
     assert (se.finish(chal) == ofinals).all()
+
+
+# rows of 512 and of 1024 entries on either side of 2^18; descriptors beyond what the kernel arguments hold, read from the host's
+# memory (up to 256 workgroups) and from a copy (2^19); more than 64 items of one table
+@pytest.mark.parametrize("n,k", [(8, 3), (9, 4), (10, 70), (13, 66), (18, 20), (19, 14)])
+def test_many_claims_on_one_table(dp, ctx, orc, n, k):
+    s = Sum(ctx, orc, n, 6000 + 10 * n + k)
+    x = s.table(base=True)
+    for e in s.eqs([n] * k):
+        s.term(x, e)
+    s.check(dp)
