@@ -152,7 +152,11 @@ size_t round_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 // Behind the Lagrange weights: the ticket counter (and at +128 the words through which a launch's first workgroup
 // passes the mail on), then the sum counters of a resident launch of several workgroups and their ticket.
 constexpr size_t SLICE_CTR_WORDS = (size_t)dpk::SL_MAX_GROUPS * dpk::SL_GROUP_WORDS * dpk::SL_CTR_STRIDE;  // counters of a resident launch, each apart
-constexpr size_t COUNTER_BYTES = 256 + SLICE_CTR_WORDS * 8 + 256 + (size_t)dpk::MAIL_RELAY_WORDS * 8;
+// Behind the mail's copies: a ticket counter for each tile of outputs that several workgroups of a partial evaluation share.
+constexpr size_t AXIS_CTR_OFF = 256 + SLICE_CTR_WORDS * 8 + 256 + (size_t)dpk::MAIL_RELAY_WORDS * 8;
+constexpr u32 AXIS_TILES = 256;
+constexpr size_t COUNTER_BYTES = AXIS_CTR_OFF + AXIS_TILES * 4;
+static_assert(AXIS_CTR_OFF % 8 == 0, "words and counters stay aligned");
 
 // Address of `scratch` on a device, asked for once per device with that device current (every GPU has its own copy).
 constexpr int WS_MAX_DEVICES = 64;
@@ -1189,82 +1193,101 @@ extern "C" int32_t dps_eq_build_many(dps_ctx *ctx, const uint64_t *const *points
 // ---------------------------------------------------------------------------
 namespace {
 
-struct AxisJob {
+// One axis contracted with the eq table of `point`, or (`axis` < 0) nothing: a plain copy with the embedding.  `out`: rows of
+// `row_len` outputs, `padded_len` apart.
+struct AxisPointJob {
     const u64 *in0 = nullptr, *in1 = nullptr;
     int in_int = 0;  // bytes per raw integer entry, 0 for field elements
-    const u64 *b0 = nullptr, *b1 = nullptr;
-    u64 K = 1, stride_k = 1;
-    std::vector<u64> pre_dims, pre_strides, post_dims, post_strides;
+    const u64 *point = nullptr;
+    u32 m = 0;
+    std::vector<u64> dims, strides;
+    int axis = -1;
+    u64 row_len = 1, padded_len = 1, rows = 1;
     u64 *o0 = nullptr, *o1 = nullptr;
 };
 
-int32_t axis_dot(dps_ctx *ctx, const AxisJob &j)
+int32_t axis_point(dps_ctx *ctx, const AxisPointJob &j)
 {
-    dpk::AxisArgs a;
+    dpk::AxisPointArgs a;
     memset(&a, 0, sizeof a);
-    if (j.pre_dims.size() > dpk::AX_MAX_DIMS || j.post_dims.size() > dpk::AX_MAX_DIMS)
-        return fail(ctx, DPS_ERR_UNSUPPORTED, "tensor rank above %d", dpk::AX_MAX_DIMS);
     a.in0 = j.in0;
     a.in1 = j.in1;
-    a.in_int = j.in_int;
-    a.b0 = j.b0;
-    a.b1 = j.b1;
-    a.K = j.K;
-    a.stride_k = j.stride_k;
-    a.n_pre = (u32)j.pre_dims.size();
-    a.n_post = (u32)j.post_dims.size();
-    a.P = a.C = 1;
-    for (u32 d = 0; d < a.n_pre; d++) {
-        a.pre_dims[d] = j.pre_dims[d];
-        a.pre_strides[d] = j.pre_strides[d];
-        a.P *= j.pre_dims[d];
+    a.m = j.m;
+    a.K = a.P = a.C = 1;
+    for (int d = 0; d < (int)j.dims.size(); d++) {
+        if (d == j.axis) {
+            a.K = j.dims[d];
+            a.stride_k = j.strides[d];
+            continue;
+        }
+        const bool pre = d < j.axis;
+        (pre ? a.pre_dims[a.n_pre] : a.post_dims[a.n_post]) = j.dims[d];
+        (pre ? a.pre_strides[a.n_pre++] : a.post_strides[a.n_post++]) = j.strides[d];
+        (pre ? a.P : a.C) *= j.dims[d];
     }
-    for (u32 d = 0; d < a.n_post; d++) {
-        a.post_dims[d] = j.post_dims[d];
-        a.post_strides[d] = j.post_strides[d];
-        a.C *= j.post_dims[d];
-    }
+    if (j.m) memcpy(a.p, j.point, 16 * (size_t)j.m);
+    a.row_len = j.row_len;
+    a.padded_len = j.padded_len;
+    a.n_pads = j.rows * (j.padded_len - j.row_len);
+    a.o0 = j.o0;
+    a.o1 = j.o1;
     const u64 outputs = a.P * a.C;
-    if (outputs == 0 || a.K == 0) return fail(ctx, DPS_ERR_INVALID, "empty axis contraction");
+    // lanes over the outputs from half a wavefront of adjacent ones on, over k below
     const bool col = a.C >= 32;
-    // split k over workgroups when there are too few outputs to fill the chip
-    const u64 out_blocks = col ? a.P * ((a.C + dpk::WAVE - 1) / dpk::WAVE) : outputs;
-    // k values one workgroup should at least own (two trips of four per wavefront, or one per lane); a few thousand workgroups
-    // keep enough loads in flight to hide the latency of a launch that is a few megabytes in all
-    const u64 k_unit = col ? 32 : 1024;
-    u32 n_slices = 1;
-    if (out_blocks < 2048 && a.K > k_unit) n_slices = (u32)std::min<u64>((a.K + k_unit - 1) / k_unit, std::max<u64>(1, 4096 / out_blocks));
-    if (n_slices > 65535) n_slices = 65535;
-    a.k_per_slice = (a.K + n_slices - 1) / n_slices;
-    n_slices = (u32)((a.K + a.k_per_slice - 1) / a.k_per_slice);
-    a.n_slices = n_slices;
-    if (out_blocks > 0x7fffffffull) return fail(ctx, DPS_ERR_UNSUPPORTED, "axis contraction too large");
-    void *tmp = nullptr;
-    if (n_slices > 1) {
-        CHK(pool_alloc(ctx, (size_t)n_slices * outputs * 16, &tmp));
-        a.o0 = (u64 *)tmp;
-        a.o1 = a.o0 + (size_t)n_slices * outputs;
+    u64 grid_x;
+    a.waves_per_out = 1;
+    if (col) {
+        grid_x = a.P * ((a.C + dpk::WAVE - 1) / dpk::WAVE);
+        // A tile's k is shared out where the tiles alone leave compute units idle: 32 values a workgroup at least (eight a
+        // wavefront, all in flight together), about four workgroups a compute unit at most
+        u64 n_slices = 1;
+        if (grid_x <= AXIS_TILES) n_slices = std::min<u64>((a.K + 31) / 32, std::max<u64>(1, 4 * COMPUTE_UNITS / grid_x));
+        a.k_per_slice = (a.K + n_slices - 1) / n_slices;
+        a.n_slices = (u32)((a.K + a.k_per_slice - 1) / a.k_per_slice);
     } else {
-        a.o0 = j.o0;
-        a.o1 = j.o1;
+        // the four wavefronts of a workgroup share an output of several steps while there are few outputs, and several
+        // workgroups one of many steps: four at least for each, about four workgroups a compute unit
+        const u64 steps = (a.K + (1u << dpk::AXP_ROW_BITS) - 1) >> dpk::AXP_ROW_BITS;
+        if (steps > 0xffffffffull) return fail(ctx, DPS_ERR_UNSUPPORTED, "axis contraction too large");
+        if (steps > 1 && outputs < 4096) a.waves_per_out = dpk::BLOCK / dpk::WAVE;
+        u64 n_slices = 1;
+        if (a.waves_per_out > 1 && outputs <= AXIS_TILES)
+            n_slices = std::min<u64>({(steps + 3) / 4, std::max<u64>(1, 4 * COMPUTE_UNITS / outputs), (u64)dpk::BLOCK});
+        a.k_per_slice = (steps + n_slices - 1) / n_slices;
+        a.n_slices = (u32)((steps + a.k_per_slice - 1) / a.k_per_slice);
+        grid_x = a.waves_per_out == 1 ? (outputs + dpk::BLOCK / dpk::WAVE - 1) / (dpk::BLOCK / dpk::WAVE) : outputs;
     }
-    const double elem = j.in1 ? 16.0 : 8.0;
+    if (grid_x > 0x7fffffffull) return fail(ctx, DPS_ERR_UNSUPPORTED, "axis contraction too large");
+    void *tmp = nullptr;
+    if (a.n_slices > 1) {
+        CHK(pool_alloc(ctx, (size_t)a.n_slices * outputs * 16, &tmp));
+        a.part0 = (u64 *)tmp;
+        a.part1 = a.part0 + (size_t)a.n_slices * outputs;
+        a.counters = reinterpret_cast<u32 *>(reinterpret_cast<char *>(ctx->d_counter) + AXIS_CTR_OFF);
+    }
+    const dim3 grid((u32)grid_x, a.n_slices);
     hipError_t e;
     {
-        ProfScope ps(ctx, DPS_K_AXIS_DOT, (double)outputs * (double)a.K * elem + (double)outputs * 16.0);
-        if (col)
-            dpk::axis_dot_col_kernel<<<dim3((u32)out_blocks, n_slices), dpk::BLOCK, 0, ctx->stream>>>(a);
+        ProfScope ps(ctx, DPS_K_AXIS_DOT, (double)outputs * (double)a.K * (j.in1 ? 16.0 : j.in_int ? (double)j.in_int : 8.0) + (double)outputs * 16.0);
+        auto launch = [&](auto kind) {
+            constexpr int KIND = decltype(kind)::value;
+            if (col)
+                dpk::axis_point_col_kernel<KIND><<<grid, dpk::BLOCK, 0, ctx->stream>>>(a);
+            else
+                dpk::axis_point_row_kernel<KIND><<<grid, dpk::BLOCK, 0, ctx->stream>>>(a);
+        };
+        if (j.in_int == 8)
+            launch(std::integral_constant<int, 8>());
+        else if (j.in_int == 2)
+            launch(std::integral_constant<int, 2>());
+        else if (j.in1)
+            launch(std::integral_constant<int, 1>());
         else
-            dpk::axis_dot_row_kernel<<<dim3((u32)out_blocks, n_slices), dpk::BLOCK, 0, ctx->stream>>>(a);
+            launch(std::integral_constant<int, 0>());
         e = hipGetLastError();
     }
-    if (e == hipSuccess && n_slices > 1) {
-        dpk::slice_sum_kernel<<<(u32)((outputs + dpk::BLOCK - 1) / dpk::BLOCK), dpk::BLOCK, 0, ctx->stream>>>(
-            a.o0, a.o1, outputs, n_slices, j.o0, j.o1);
-        e = hipGetLastError();
-    }
-    pool_free(ctx, tmp);
-    if (e != hipSuccess) return fail(ctx, DPS_ERR_HIP, "axis_dot launch: %s", hipGetErrorString(e));
+    pool_free(ctx, tmp);  // (reused in stream order)
+    if (e != hipSuccess) return fail(ctx, DPS_ERR_HIP, "axis_point launch: %s", hipGetErrorString(e));
     return DPS_OK;
 }
 
@@ -1336,35 +1359,30 @@ extern "C" int32_t dps_mle_fix_high(dps_ctx *ctx, const dps_mle *mle, const uint
     if (!ctx || !mle || !out || (k && !point)) return fail(ctx, DPS_ERR_INVALID, "dps_mle_fix_high: bad argument");
     if (mle->pad_vars) return fail(ctx, DPS_ERR_UNSUPPORTED, "dps_mle_fix_high: the table is a zero-padded view");
     if (!is_pow2(mle->len) || (1ull << k) > mle->len) return fail(ctx, DPS_ERR_INVALID, "dps_mle_fix_high: too many variables");
+    if (k > dpk::EQ_MAX_VARS) return fail(ctx, DPS_ERR_INVALID, "dps_mle_fix_high: bad argument");
+    if (!canonical(point, 2 * (size_t)k)) return fail(ctx, DPS_ERR_INVALID, "dps_mle_fix_high: point not canonical");
     DeviceGuard g(ctx->device);
     tail_abort(ctx);
     CHK(plain_ready(mle));
-    dps_mle *eq = nullptr;
-    CHK(dps_eq_build(ctx, point, k, &eq));
-    if (int32_t rc_ = plain_ready(eq); rc_ != DPS_OK) {
-        delete eq;
-        return rc_;
-    }
     u64 rest = mle->len >> k;
     dps_mle *res = nullptr;
     int32_t rc = new_table(ctx, DPS_EXT2, rest, &res);
     if (rc == DPS_OK) {
-        AxisJob j;
+        AxisPointJob j;
         j.in0 = mle->p0();
         j.in1 = mle->p1();
         j.in_int = raw_bytes(mle->kind);
-        j.b0 = eq->p0();
-        j.b1 = eq->p1();
-        j.K = 1ull << k;
-        j.stride_k = rest;
-        j.post_dims = {rest};
-        j.post_strides = {1};
+        j.point = point;
+        j.m = k;
+        j.dims = {1ull << k, rest};
+        j.strides = {rest, 1};
+        j.axis = 0;
+        j.row_len = j.padded_len = rest;
         j.o0 = res->st->c0;
         j.o1 = res->st->c1;
-        rc = axis_dot(ctx, j);
+        rc = axis_point(ctx, j);
     }
     hipError_t e = hipStreamSynchronize(ctx->stream);
-    delete eq;
     if (rc == DPS_OK && e != hipSuccess) rc = fail(ctx, DPS_ERR_HIP, "fix_high: %s", hipGetErrorString(e));
     if (rc != DPS_OK) {
         delete res;
@@ -1423,87 +1441,6 @@ extern "C" int32_t dps_mle_fix_low(dps_ctx *ctx, const dps_mle *mle, const uint6
     return DPS_OK;
 }
 
-namespace {
-
-// The last step of a partial evaluation: what is left of the tensor is indexed by the stacked and contracted axes in
-// their original order; like the reference (axis.rs:1222-1233) the flat result is cut into chunks of `contraction`
-// entries, one table per chunk, each padded to a power of two.  `cur`: the result of the contractions so far (owned
-// here), or nullptr when no outer axis was fixed (the source is then read through `dims` / `strides`).
-int32_t rows_as_tables(dps_ctx *ctx, dps_mle *cur, const u64 *in0, const u64 *in1, int in_int, const std::vector<u64> &dims,
-                       const std::vector<u64> &strides, u64 stacked, u64 contraction, dps_mle **out)
-{
-    int32_t rc = DPS_OK;
-    u32 nv = log2u(contraction);
-    u64 tl = 1ull << nv;
-    dps_mle *all = nullptr;
-    // rows that are a power of two long already: the result is the table as it stands
-    const bool as_it_stands = cur && contraction == tl && cur->kind == DPS_EXT2 && cur->offset == 0 && cur->len == stacked * tl;
-    if (as_it_stands) {
-        all = cur;
-        cur = nullptr;
-    } else {
-        rc = new_table(ctx, DPS_EXT2, stacked * tl, &all);
-    }
-    if (rc == DPS_OK && !as_it_stands) {
-        if (cur) {
-            dpk::pad_rows_kernel<<<grid_for(stacked * tl), dpk::BLOCK, 0, ctx->stream>>>(cur->st->c0, cur->st->c1, stacked, contraction, tl,
-                                                                                    all->st->c0, all->st->c1);
-            hipError_t e = hipGetLastError();
-            if (e != hipSuccess) rc = fail(ctx, DPS_ERR_HIP, "pad launch: %s", hipGetErrorString(e));
-        } else {
-            // no outer axis: contract a unit axis with the table {1} to copy the unpadded region
-            u64 one[2] = {0, 0};
-            dps_mle *unit = nullptr;
-            rc = dps_eq_build(ctx, one, 0, &unit);
-            if (rc == DPS_OK) rc = plain_ready(unit);
-            dps_mle *flat = nullptr;
-            if (rc == DPS_OK) rc = new_table(ctx, DPS_EXT2, stacked * contraction, &flat);
-            if (rc == DPS_OK) {
-                AxisJob j;
-                j.in0 = in0;
-                j.in1 = in1;
-                j.in_int = in_int;
-                j.b0 = unit->p0();
-                j.b1 = unit->p1();
-                j.K = 1;
-                j.stride_k = 0;
-                j.post_dims = dims;
-                j.post_strides = strides;
-                j.o0 = flat->st->c0;
-                j.o1 = flat->st->c1;
-                rc = axis_dot(ctx, j);
-            }
-            if (rc == DPS_OK) {
-                dpk::pad_rows_kernel<<<grid_for(stacked * tl), dpk::BLOCK, 0, ctx->stream>>>(flat->st->c0, flat->st->c1, stacked, contraction,
-                                                                                        tl, all->st->c0, all->st->c1);
-                hipError_t e = hipGetLastError();
-                if (e != hipSuccess) rc = fail(ctx, DPS_ERR_HIP, "pad launch: %s", hipGetErrorString(e));
-            }
-            (void)hipStreamSynchronize(ctx->stream);
-            delete unit;
-            delete flat;
-        }
-    }
-    // (no wait for the stream: the blocks given back are reused in stream order, and whoever consumes the result waits)
-    delete cur;
-    if (rc != DPS_OK) {
-        delete all;
-        return rc;
-    }
-    for (u64 s = 0; s < stacked; s++) {
-        rc = dps_mle_view(all, s * tl, nv, &out[s]);
-        if (rc != DPS_OK) {
-            for (u64 q = 0; q < s; q++) delete out[q];
-            delete all;
-            return rc;
-        }
-    }
-    delete all;  // the views keep the storage alive
-    return DPS_OK;
-}
-
-}  // namespace
-
 extern "C" int32_t dps_partial_eval(dps_ctx *ctx, const dps_mle *tensor, const uint64_t *padded_dims,
                                     const uint64_t *unpadded_dims, uint32_t n_dims, const int32_t *kinds,
                                     const uint64_t *const *points, dps_mle **out, uint32_t out_cap, uint32_t *n_out)
@@ -1543,63 +1480,79 @@ extern "C" int32_t dps_partial_eval(dps_ctx *ctx, const dps_mle *tensor, const u
             orig[a] = a;
         }
     }
-    const u64 *in0 = tensor->p0(), *in1 = tensor->p1();
-    int in_int = raw_bytes(tensor->kind);
-    dps_mle *cur = nullptr;  // owns the intermediate
-    int32_t rc = DPS_OK;
-    // the reference walks the axes from the last to the first (axis.rs:1152)
-    for (int a = (int)dims.size() - 1; a >= 0 && rc == DPS_OK; a--) {
-        if (kd[a] != DPS_AXIS_OUTER) continue;
-        u32 oa = orig[a];
-        u32 m = log2u(padded_dims[oa]);
-        dps_mle *beta = nullptr;
-        rc = dps_eq_build(ctx, points[oa], m, &beta);
-        if (rc == DPS_OK) rc = plain_ready(beta);
-        if (rc != DPS_OK) {
-            delete beta;
-            break;
-        }
-        AxisJob j;
-        j.in0 = in0;
-        j.in1 = in1;
-        j.in_int = in_int;
-        j.b0 = beta->p0();
-        j.b1 = beta->p1();
-        j.K = dims[a];  // evals(point)[..size]
-        j.stride_k = strides[a];
-        u64 outputs = 1;
-        for (int d = 0; d < (int)dims.size(); d++) {
-            if (d == a) continue;
-            (d < a ? j.pre_dims : j.post_dims).push_back(dims[d]);
-            (d < a ? j.pre_strides : j.post_strides).push_back(strides[d]);
-            outputs *= dims[d];
+    for (u32 a = 0; a < n_dims; a++) {
+        if (kinds[a] != DPS_AXIS_OUTER) continue;
+        const u32 m = log2u(padded_dims[a]);
+        if (m > dpk::EQ_MAX_VARS) return fail(ctx, DPS_ERR_INVALID, "dps_partial_eval: outer axis %u too long", a);
+        if (!canonical(points[a], 2 * (size_t)m)) return fail(ctx, DPS_ERR_INVALID, "dps_partial_eval: point of axis %u not canonical", a);
+    }
+    AxisPointJob j;
+    j.in0 = tensor->p0();
+    j.in1 = tensor->p1();
+    j.in_int = raw_bytes(tensor->kind);
+    u32 left = 0;  // axes still to contract
+    for (int32_t k : kd) left += k == DPS_AXIS_OUTER;
+    // What is left at the end is indexed by the stacked and contracted axes in their original order; like the reference
+    // (axis.rs:1222-1233) the flat result is cut into chunks of `contraction` entries, one table per chunk, each padded to a
+    // power of two: the last launch writes it that way.  (No wait for the stream: the blocks given back are reused in stream
+    // order, and whoever consumes the result waits.)
+    const u32 nv = log2u(contraction);
+    dps_mle *cur = nullptr, *all = nullptr;  // cur: owns the intermediate
+    int32_t rc = new_table(ctx, DPS_EXT2, stacked << nv, &all);
+    do {
+        if (rc != DPS_OK) break;
+        // the reference walks the axes from the last to the first (axis.rs:1152)
+        j.axis = -1;
+        for (int a = 0; a < (int)dims.size(); a++)
+            if (kd[a] == DPS_AXIS_OUTER) j.axis = a;
+        j.dims = dims;
+        j.strides = strides;
+        j.m = 0;
+        if (j.axis >= 0) {
+            j.point = points[orig[j.axis]];
+            j.m = log2u(padded_dims[orig[j.axis]]);  // evals(point)[..size]
+            left--;
         }
         dps_mle *next = nullptr;
-        rc = new_table(ctx, DPS_EXT2, outputs, &next);
-        if (rc == DPS_OK) {
+        if (left == 0) {
+            j.rows = stacked;
+            j.row_len = contraction;
+            j.padded_len = 1ull << nv;
+            j.o0 = all->st->c0;
+            j.o1 = all->st->c1;
+        } else {
+            u64 outputs = 1;
+            for (int d = 0; d < (int)dims.size(); d++)
+                if (d != j.axis) outputs *= dims[d];
+            j.rows = 1;
+            j.row_len = j.padded_len = outputs;
+            rc = new_table(ctx, DPS_EXT2, outputs, &next);
+            if (rc != DPS_OK) break;
             j.o0 = next->st->c0;
             j.o1 = next->st->c1;
-            rc = axis_dot(ctx, j);
         }
-        delete beta;
+        rc = axis_point(ctx, j);
         delete cur;
         cur = next;
-        if (rc != DPS_OK) break;
+        if (rc != DPS_OK || left == 0) break;
         // the result is compact over the remaining axes
-        dims.erase(dims.begin() + a);
-        kd.erase(kd.begin() + a);
-        orig.erase(orig.begin() + a);
+        dims.erase(dims.begin() + j.axis);
+        kd.erase(kd.begin() + j.axis);
+        orig.erase(orig.begin() + j.axis);
         strides.assign(dims.size(), 1);
         for (int d = (int)dims.size() - 2; d >= 0; d--) strides[d] = strides[d + 1] * dims[d + 1];
-        in0 = cur->st->c0;
-        in1 = cur->st->c1;
-        in_int = 0;
+        j.in0 = cur->st->c0;
+        j.in1 = cur->st->c1;
+        j.in_int = 0;
+    } while (true);
+    delete cur;
+    for (u64 q = 0; q < stacked && rc == DPS_OK; q++) {
+        rc = dps_mle_view(all, q << nv, nv, &out[q]);
+        if (rc != DPS_OK)
+            for (u64 u = 0; u < q; u++) delete out[u];
     }
-    if (rc != DPS_OK) {
-        delete cur;
-        return rc;
-    }
-    CHK(rows_as_tables(ctx, cur, in0, in1, in_int, dims, strides, stacked, contraction, out));
+    delete all;  // the views keep the storage alive
+    if (rc != DPS_OK) return rc;
     *n_out = (u32)stacked;
     return DPS_OK;
 }

@@ -2663,30 +2663,8 @@ __global__ void __launch_bounds__(BLOCK) pad_tensor_kernel(PadTensorArgs a)
     }
 }
 
-// ---------------------------------------------------------------------------
-// contraction of one tensor axis with a table beta (partial evaluation):
-//   out[pre][i] = sum_k in[off_pre(pre) + k * stride_k + off_post(i)] * beta[k]
-// The input is addressed through per-dimension strides so that the unpadded
-// region of a padded tensor is read in place.
-// ---------------------------------------------------------------------------
-constexpr int AX_MAX_DIMS = 6;
-struct AxisArgs {
-    const u64 *in0;
-    const u64 *in1;  // nullptr: base field or raw integers
-    int in_int;      // 0: field elements; 8: raw int64; 2: raw int16 (embedded on load)
-    const u64 *b0;
-    const u64 *b1;
-    u64 K, stride_k;
-    u32 n_pre, n_post;
-    u64 pre_dims[AX_MAX_DIMS], pre_strides[AX_MAX_DIMS];
-    u64 post_dims[AX_MAX_DIMS], post_strides[AX_MAX_DIMS];
-    u64 P, C;  // products of pre_dims / post_dims
-    u64 k_per_slice;
-    u32 n_slices;
-    u64 *o0;
-    u64 *o1;  // [slice][pre][i] when n_slices > 1, else [pre][i]
-};
-
+constexpr int AX_MAX_DIMS = 6;  // rank of a tensor
+// sum of coordinate times stride, `flat` counting the last dimension fastest
 __device__ __forceinline__ u64 ax_offset(u64 flat, u32 n, const u64 *dims, const u64 *strides)
 {
     u64 off = 0;
@@ -2696,85 +2674,6 @@ __device__ __forceinline__ u64 ax_offset(u64 flat, u32 n, const u64 *dims, const
         flat = q;
     }
     return off;
-}
-
-__device__ __forceinline__ E2 ax_load(const AxisArgs &a, u64 off)
-{
-    if (a.in_int == 8) return gl::e2(gl::from_i64(((const int64_t *)a.in0)[off]), 0);
-    if (a.in_int == 2) return gl::e2(gl::from_i64(((const int16_t *)a.in0)[off]), 0);
-    return gl::e2(a.in0[off], a.in1 ? a.in1[off] : 0);
-}
-
-// lanes over the kept trailing index i (coalesced when the last kept dimension is contiguous)
-__global__ void __launch_bounds__(BLOCK) axis_dot_col_kernel(AxisArgs a)
-{
-    __shared__ u64 lds[BLOCK * 2];
-    const u32 lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
-    const u64 tiles = (a.C + WAVE - 1) / WAVE;
-    const u64 pre = blockIdx.x / tiles;
-    const u64 i = (blockIdx.x - pre * tiles) * WAVE + lane;
-    const u32 slice = blockIdx.y;
-    E2 acc = gl::e2_zero();
-    if (i < a.C) {
-        const u64 base = ax_offset(pre, a.n_pre, a.pre_dims, a.pre_strides) + ax_offset(i, a.n_post, a.post_dims, a.post_strides);
-        u64 k0 = (u64)slice * a.k_per_slice, k1 = k0 + a.k_per_slice;
-        if (k1 > a.K) k1 = a.K;
-        // four rows in flight per wavefront: the loop is a chain of loads otherwise (a row is 512 B per wavefront)
-        constexpr u64 STEP = BLOCK / WAVE;
-        auto term = [&](E2 v, E2 b) { return a.in1 ? gl::mul(v, b) : gl::mul_base(b, v.c0); };
-        u64 k = k0 + wave;
-        for (; k + 3 * STEP < k1; k += 4 * STEP) {
-            const E2 v0 = ax_load(a, base + k * a.stride_k), v1 = ax_load(a, base + (k + STEP) * a.stride_k);
-            const E2 v2 = ax_load(a, base + (k + 2 * STEP) * a.stride_k), v3 = ax_load(a, base + (k + 3 * STEP) * a.stride_k);
-            const E2 b0 = gl::e2(a.b0[k], a.b1[k]), b1 = gl::e2(a.b0[k + STEP], a.b1[k + STEP]);
-            const E2 b2 = gl::e2(a.b0[k + 2 * STEP], a.b1[k + 2 * STEP]), b3 = gl::e2(a.b0[k + 3 * STEP], a.b1[k + 3 * STEP]);
-            acc = gl::add(acc, gl::add(gl::add(term(v0, b0), term(v1, b1)), gl::add(term(v2, b2), term(v3, b3))));
-        }
-        for (; k < k1; k += STEP) acc = gl::add(acc, term(ax_load(a, base + k * a.stride_k), gl::e2(a.b0[k], a.b1[k])));
-    }
-    lds[threadIdx.x * 2] = acc.c0;
-    lds[threadIdx.x * 2 + 1] = acc.c1;
-    __syncthreads();
-    if (wave == 0 && i < a.C) {
-#pragma unroll
-        for (int w = 1; w < BLOCK / WAVE; w++) {
-            acc.c0 = gl::add(acc.c0, lds[(w * WAVE + lane) * 2]);
-            acc.c1 = gl::add(acc.c1, lds[(w * WAVE + lane) * 2 + 1]);
-        }
-        u64 o = ((u64)slice * a.P + pre) * a.C + i;
-        a.o0[o] = acc.c0;
-        a.o1[o] = acc.c1;
-    }
-}
-
-// one workgroup per output, lanes over k (for C < 64, e.g. a row dot product)
-__global__ void __launch_bounds__(BLOCK) axis_dot_row_kernel(AxisArgs a)
-{
-    __shared__ u32 lds[(BLOCK / WAVE) * 6];
-    const u64 pre = blockIdx.x / a.C;
-    const u64 i = blockIdx.x - pre * a.C;
-    const u32 slice = blockIdx.y;
-    const u64 base = ax_offset(pre, a.n_pre, a.pre_dims, a.pre_strides) + ax_offset(i, a.n_post, a.post_dims, a.post_strides);
-    u64 k0 = (u64)slice * a.k_per_slice, k1 = k0 + a.k_per_slice;
-    if (k1 > a.K) k1 = a.K;
-    E2 acc[1] = {gl::e2_zero()};
-    // four elements in flight per lane
-    auto term = [&](E2 v, E2 b) { return a.in1 ? gl::mul(v, b) : gl::mul_base(b, v.c0); };
-    u64 k = k0 + threadIdx.x;
-    for (; k + 3 * BLOCK < k1; k += 4 * BLOCK) {
-        const E2 v0 = ax_load(a, base + k * a.stride_k), v1 = ax_load(a, base + (k + BLOCK) * a.stride_k);
-        const E2 v2 = ax_load(a, base + (k + 2 * BLOCK) * a.stride_k), v3 = ax_load(a, base + (k + 3 * BLOCK) * a.stride_k);
-        const E2 b0 = gl::e2(a.b0[k], a.b1[k]), b1 = gl::e2(a.b0[k + BLOCK], a.b1[k + BLOCK]);
-        const E2 b2 = gl::e2(a.b0[k + 2 * BLOCK], a.b1[k + 2 * BLOCK]), b3 = gl::e2(a.b0[k + 3 * BLOCK], a.b1[k + 3 * BLOCK]);
-        acc[0] = gl::add(acc[0], gl::add(gl::add(term(v0, b0), term(v1, b1)), gl::add(term(v2, b2), term(v3, b3))));
-    }
-    for (; k < k1; k += BLOCK) acc[0] = gl::add(acc[0], term(ax_load(a, base + k * a.stride_k), gl::e2(a.b0[k], a.b1[k])));
-    block_reduce<1>(acc, lds);
-    if (threadIdx.x == 0) {
-        u64 o = ((u64)slice * a.P + pre) * a.C + i;
-        a.o0[o] = acc[0].c0;
-        a.o1[o] = acc[0].c1;
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -2958,6 +2857,282 @@ __global__ void __launch_bounds__(BLOCK) eval_point_kernel(EvalArgs a, FastFin f
         E2 q[1];
         gather_partials<1>(ff, lds, q);
         publish_sums<1>(ff.out_host, ff.seq, ff.counter, q);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Partial evaluation: one axis of a tensor contracted with the eq table of a point, in one launch,
+//   out[pre][post] = sum_k in[pre][k][post] * eq(point, k),
+// written where the sumcheck reads it: the outputs in their order cut into rows of `row_len`, each row filled up with zeros to
+// `padded_len`.  No eq table is in memory: the point travels in the kernel arguments, every workgroup makes the tables of
+// its coordinates, three at a time, and from them the weights it uses.  The input is addressed through strides, so the
+// unpadded region of a padded tensor is read in place.
+//   axis_point_col_kernel  lanes over the outputs (32 and more adjacent ones), a share of k a wavefront; where that leaves the
+//                          chip idle several workgroups share a tile of 64 outputs and the last one adds the partial sums.
+//   axis_point_row_kernel  a wavefront, or the four of a workgroup, per output, lanes over k 512 at a time: an entry costs its
+//                          product with one of eight weights that all lanes share.  Several workgroups share a long row of
+//                          few outputs, as above.
+// Bound: the latency of a launch and of about ten field products at the sizes of a layer (3 to 19 MB), HBM above.  Through the
+// eq table, a contraction, a sum over its shares and a launch for the padding, each started when the one before had
+// ended, a tensor took about 22 us of kernels and as much of gaps and launch calls.  [512 x 768] int64 14.6 us and [768 x 3072]
+// int64 12.5 us (kernel trace); proofs of that product 114 -> 91 us, of one row of it 159 -> 102 us, of both products of an
+// attention layer of 12 heads over 197 tokens 237 -> 203 us.
+// ---------------------------------------------------------------------------
+constexpr u32 AXP_GROUPS = (EQ_MAX_VARS + 2) / 3;
+constexpr u32 AXP_ROW_BITS = 9, AXP_ROW_STEPS = 64;  // columns a step of a row (log2), steps whose weights are made together
+struct AxisPointArgs {
+    const void *in0;
+    const u64 *in1;
+    u32 m, n_slices;  // coordinates; workgroups that share a tile's (an output's) k
+    u64 K, stride_k;
+    u32 n_pre, n_post;
+    u64 pre_dims[AX_MAX_DIMS], pre_strides[AX_MAX_DIMS];
+    u64 post_dims[AX_MAX_DIMS], post_strides[AX_MAX_DIMS];
+    u64 P, C;         // products of pre_dims / post_dims
+    u64 k_per_slice;  // (steps of 512 values in the row kernel)
+    u64 row_len, padded_len, n_pads;
+    u32 waves_per_out, pad;
+    u64 *o0, *o1;
+    u64 *part0, *part1;  // [slice][pre][post] when n_slices > 1
+    u32 *counters;       // one per tile, zero between launches
+    u64 p[2 * EQ_MAX_VARS];
+};
+struct AxisGroups {
+    u64 c0[AXP_GROUPS][8], c1[AXP_GROUPS][8];
+    __device__ __forceinline__ E2 at(u32 g, u32 e) const { return gl::e2(c0[g][e], c1[g][e]); }
+};
+// tables of three coordinates each, in order; coordinates beyond the point's count as zero (at least `least` tables)
+__device__ __forceinline__ u32 axis_groups(const AxisPointArgs &a, u32 least, AxisGroups &out)
+{
+    const u32 have = (a.m + 2) / 3, n_groups = have < least ? least : have, g = threadIdx.x / 8, e = threadIdx.x % 8;
+    static_assert(8 * AXP_GROUPS <= BLOCK, "an entry a thread");
+    if (g < n_groups) {
+        E2 v = gl::e2_one();
+#pragma unroll
+        for (u32 b = 0; b < 3; b++) {
+            const u32 c = 3 * g + b;
+            const E2 r = c < a.m ? gl::e2(a.p[2 * c], a.p[2 * c + 1]) : gl::e2_zero();
+            const E2 x = ((e >> b) & 1) ? r : gl::sub(gl::e2_one(), r);
+            v = b == 0 ? x : gl::mul(v, x);
+        }
+        out.c0[g][e] = v.c0;
+        out.c1[g][e] = v.c1;
+    }
+    return n_groups;
+}
+// product of the entries that the bits of k choose, from table `first` on
+__device__ __forceinline__ E2 axis_weight(const AxisGroups &t, u32 first, u32 n_groups, u64 k)
+{
+    if (first >= n_groups) return gl::e2_one();
+    E2 v = t.at(first, (u32)k & 7);
+    for (u32 g = first + 1; g < n_groups; g++) v = gl::mul(v, t.at(g, (u32)(k >> (3 * (g - first))) & 7));
+    return v;
+}
+template <int KIND>
+__device__ __forceinline__ E2 axis_entry(const AxisPointArgs &a, u64 off)
+{
+    if (KIND == 8) return gl::e2(gl::from_i64(reinterpret_cast<const int64_t *>(a.in0)[off]), 0);
+    if (KIND == 2) return gl::e2(gl::from_i64(reinterpret_cast<const int16_t *>(a.in0)[off]), 0);
+    return gl::e2(reinterpret_cast<const u64 *>(a.in0)[off], KIND == 1 ? a.in1[off] : 0);
+}
+template <int KIND>
+__device__ __forceinline__ void axis_acc(gl::E2Acc &s, E2 v, const gl::E2P &w)
+{
+    if (KIND == 1)
+        gl::acc_mul(s, v, w);
+    else
+        gl::acc_mul_base(s, gl::e2(w.c0, w.c1), v.c0);
+}
+__device__ __forceinline__ void axis_store(const AxisPointArgs &a, u64 o, E2 v)
+{
+    if (a.row_len != a.padded_len) {
+        const u64 row = o / a.row_len;
+        o = row * a.padded_len + (o - row * a.row_len);
+    }
+    a.o0[o] = v.c0;
+    a.o1[o] = v.c1;
+}
+// the zeros behind the rows, shared out over the whole launch
+__device__ __forceinline__ void axis_pads(const AxisPointArgs &a)
+{
+    const u64 width = a.padded_len - a.row_len, stride = (u64)gridDim.x * gridDim.y * BLOCK;
+    for (u64 j = ((u64)blockIdx.y * gridDim.x + blockIdx.x) * BLOCK + threadIdx.x; j < a.n_pads; j += stride) {
+        const u64 row = j / width, o = row * a.padded_len + a.row_len + (j - row * width);
+        a.o0[o] = 0;
+        a.o1[o] = 0;
+    }
+}
+
+template <int KIND>
+__global__ void __launch_bounds__(BLOCK) axis_point_col_kernel(AxisPointArgs a)
+{
+    __shared__ AxisGroups groups;
+    __shared__ u64 w0[BLOCK], w1[BLOCK];  // weights of up to BLOCK values of k
+    __shared__ u64 lds[BLOCK * 2];
+    __shared__ int last_flag;
+    const u32 tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
+    const u64 tiles = (a.C + WAVE - 1) / WAVE;
+    const u64 pre = blockIdx.x / tiles;
+    const u64 i = (blockIdx.x - pre * tiles) * WAVE + lane;
+    const u64 o = pre * a.C + i;
+    const bool mine = i < a.C;
+    const u64 base = ax_offset(pre, a.n_pre, a.pre_dims, a.pre_strides) + (mine ? ax_offset(i, a.n_post, a.post_dims, a.post_strides) : 0);
+    const u32 n_groups = axis_groups(a, 0, groups);
+    axis_pads(a);
+    const u64 k0 = (u64)blockIdx.y * a.k_per_slice, k1 = k0 + a.k_per_slice < a.K ? k0 + a.k_per_slice : a.K;
+    gl::E2Acc s = gl::e2acc_zero();
+    for (u64 at = k0; at < k1; at += BLOCK) {
+        const u32 here = k1 - at < BLOCK ? (u32)(k1 - at) : BLOCK;
+        __syncthreads();  // the tables are there; the weights before have been read
+        if (tid < here) {
+            const E2 v = axis_weight(groups, 0, n_groups, at + tid);
+            w0[tid] = v.c0;
+            w1[tid] = v.c1;
+        }
+        __syncthreads();
+        if (!mine) continue;
+        // eight rows in flight per wavefront
+        constexpr u32 STEP = BLOCK / WAVE, AHEAD = 8;
+        for (u32 k = wave; k < here; k += AHEAD * STEP) {
+            E2 v[AHEAD];
+#pragma unroll
+            for (u32 u = 0; u < AHEAD; u++) v[u] = k + u * STEP < here ? axis_entry<KIND>(a, base + (at + k + u * STEP) * a.stride_k) : gl::e2_zero();
+#pragma unroll
+            for (u32 u = 0; u < AHEAD; u++) {
+                const u32 q = k + u * STEP < here ? k + u * STEP : wave;  // (an entry of zero beyond the end)
+                const E2 w = gl::e2(w0[q], w1[q]);
+                axis_acc<KIND>(s, v[u], KIND == 1 ? gl::prep(w) : gl::E2P{w.c0, w.c1, 0});
+            }
+        }
+    }
+    // the sum of the four wavefronts' values, valid in the first
+    auto sum_waves = [&](E2 v) {
+        lds[tid * 2] = v.c0;
+        lds[tid * 2 + 1] = v.c1;
+        __syncthreads();
+        if (wave == 0) {
+#pragma unroll
+            for (u32 w = 1; w < BLOCK / WAVE; w++) v = gl::add(v, gl::e2(lds[(w * WAVE + lane) * 2], lds[(w * WAVE + lane) * 2 + 1]));
+        }
+        return v;
+    };
+    E2 v = sum_waves(gl::acc_reduce(s));
+    if (a.n_slices == 1) {
+        if (wave == 0 && mine) axis_store(a, o, v);
+        return;
+    }
+    const u64 outputs = a.P * a.C;
+    if (wave == 0 && mine) {
+        st_agent(a.part0 + (u64)blockIdx.y * outputs + o, v.c0);
+        st_agent(a.part1 + (u64)blockIdx.y * outputs + o, v.c1);
+    }
+    // (the partial sums are the first wavefront's stores, and its thread 0 takes the ticket when they have been acknowledged)
+    if (!take_ticket(a.counters + blockIdx.x, a.n_slices, &last_flag)) return;
+    v = gl::e2_zero();
+    if (mine) {
+        constexpr u32 STEP = BLOCK / WAVE, AHEAD = 4;
+        for (u32 q = wave; q < a.n_slices; q += AHEAD * STEP) {
+            E2 x[AHEAD];
+#pragma unroll
+            for (u32 u = 0; u < AHEAD; u++) {
+                const u64 at = (u64)(q + u * STEP) * outputs + o;
+                x[u] = q + u * STEP < a.n_slices ? gl::e2(ld_agent(a.part0 + at), ld_agent(a.part1 + at)) : gl::e2_zero();
+            }
+#pragma unroll
+            for (u32 u = 0; u < AHEAD; u++) v = gl::add(v, x[u]);
+        }
+    }
+    v = sum_waves(v);  // (take_ticket's barrier is behind the last reads of the area)
+    if (wave == 0 && mine) axis_store(a, o, v);
+    if (tid == 0) a.counters[blockIdx.x] = 0;
+}
+
+template <int KIND>
+__global__ void __launch_bounds__(BLOCK) axis_point_row_kernel(AxisPointArgs a)
+{
+    __shared__ AxisGroups groups;
+    __shared__ u64 sw0[AXP_ROW_STEPS], sw1[AXP_ROW_STEPS];
+    __shared__ u64 lds[2 * (BLOCK / WAVE)];
+    __shared__ int last_flag;
+    const u32 tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
+    const u32 S = a.waves_per_out, sub = wave % S;  // 1 or 4
+    const u64 outputs = a.P * a.C, o = (u64)blockIdx.x * (BLOCK / WAVE / S) + wave / S;
+    const bool mine = o < outputs;
+    const u64 pre = (mine ? o : 0) / a.C, i = (mine ? o : 0) - pre * a.C;
+    const u64 base = ax_offset(pre, a.n_pre, a.pre_dims, a.pre_strides) + ax_offset(i, a.n_post, a.post_dims, a.post_strides);
+    const u32 steps = (u32)((a.K + (1u << AXP_ROW_BITS) - 1) >> AXP_ROW_BITS);
+    auto load = [&](u32 step, E2 (&v)[8]) {
+#pragma unroll
+        for (u32 j = 0; j < 8; j++) {
+            const u64 k = ((u64)step << AXP_ROW_BITS) + WAVE * j + lane;
+            v[j] = mine && k < a.K ? axis_entry<KIND>(a, base + k * a.stride_k) : gl::e2_zero();
+        }
+    };
+    // (a workgroup's share of the steps: all of them unless several share an output)
+    const u32 s0 = blockIdx.y * (u32)a.k_per_slice, s1 = s0 + (u32)a.k_per_slice < steps ? s0 + (u32)a.k_per_slice : steps;
+    E2 v[8];
+    load(s0 + sub, v);  // asked for before the weights are made
+    const u32 n_groups = axis_groups(a, AXP_ROW_BITS / 3, groups);
+    axis_pads(a);
+    gl::E2P w[8];
+    gl::E2Acc total = gl::e2acc_zero();
+    for (u32 at = s0; at < s1; at += AXP_ROW_STEPS) {
+        const u32 end = at + AXP_ROW_STEPS < s1 ? at + AXP_ROW_STEPS : s1;
+        __syncthreads();  // the tables are there; the weights before have been read
+        if (tid < end - at) {
+            const E2 h = axis_weight(groups, AXP_ROW_BITS / 3, n_groups, at + tid);
+            sw0[tid] = h.c0;
+            sw1[tid] = h.c1;
+        }
+        __syncthreads();
+#pragma unroll
+        for (u32 j = 0; j < 8; j++) w[j] = KIND == 1 ? gl::prep(groups.at(2, j)) : gl::E2P{groups.c0[2][j], groups.c1[2][j], 0};
+        for (u32 step = at + sub; step < end; step += S) {
+            gl::E2Acc s = gl::e2acc_zero();
+#pragma unroll
+            for (u32 j = 0; j < 8; j++) axis_acc<KIND>(s, v[j], w[j]);
+            if (step + S < s1) load(step + S, v);
+            gl::acc_mul(total, gl::acc_reduce(s), gl::prep(gl::e2(sw0[step - at], sw1[step - at])));
+        }
+    }
+    auto sum_lanes = [&](E2 x) {
+#pragma unroll
+        for (int off = 1; off < WAVE; off <<= 1)
+            x = gl::add(x, gl::e2(__shfl_xor((unsigned long long)x.c0, off, WAVE), __shfl_xor((unsigned long long)x.c1, off, WAVE)));
+        return x;
+    };
+    E2 x = sum_lanes(gl::mul(gl::acc_reduce(total), gl::mul(groups.at(0, lane & 7), groups.at(1, lane >> 3))));
+    if (S == 1) {
+        if (mine && lane == 0) axis_store(a, o, x);
+        return;
+    }
+    // the sum of the four wavefronts' values, valid in thread 0
+    auto sum_waves = [&](E2 y) {
+        if (lane == 0) {
+            lds[2 * wave] = y.c0;
+            lds[2 * wave + 1] = y.c1;
+        }
+        __syncthreads();
+        if (tid == 0)
+            for (u32 q = 1; q < BLOCK / WAVE; q++) y = gl::add(y, gl::e2(lds[2 * q], lds[2 * q + 1]));
+        return y;
+    };
+    x = sum_waves(x);
+    if (a.n_slices == 1) {
+        if (tid == 0) axis_store(a, o, x);
+        return;
+    }
+    if (tid == 0) {
+        st_agent(a.part0 + (u64)blockIdx.y * outputs + o, x.c0);
+        st_agent(a.part1 + (u64)blockIdx.y * outputs + o, x.c1);
+    }
+    if (!take_ticket(a.counters + blockIdx.x, a.n_slices, &last_flag)) return;
+    // (at most a share a thread)
+    x = tid < a.n_slices ? gl::e2(ld_agent(a.part0 + (u64)tid * outputs + o), ld_agent(a.part1 + (u64)tid * outputs + o)) : gl::e2_zero();
+    x = sum_waves(sum_lanes(x));
+    if (tid == 0) {
+        axis_store(a, o, x);
+        a.counters[blockIdx.x] = 0;
     }
 }
 
@@ -3183,36 +3358,6 @@ __global__ void __launch_bounds__(BLOCK) eval_tables_kernel(EvalTablesArgs a)
         *a.counter = 0;
         st_sys(a.fin_out + SL_FIN_CHK_SLOT, x ^ a.seq);
         st_sys(a.fin_out + SL_FIN_SEQ_SLOT, a.seq);
-    }
-}
-
-// sum the k-slices: out[j] = sum_s in[s * n + j]
-__global__ void __launch_bounds__(BLOCK)
-slice_sum_kernel(const u64 *__restrict__ i0, const u64 *__restrict__ i1, u64 n, u32 n_slices, u64 *__restrict__ o0,
-                 u64 *__restrict__ o1)
-{
-    u64 j = (u64)blockIdx.x * BLOCK + threadIdx.x;
-    if (j >= n) return;
-    u64 a0 = 0, a1 = 0;
-    for (u32 s = 0; s < n_slices; s++) {
-        a0 = gl::add(a0, i0[(u64)s * n + j]);
-        a1 = gl::add(a1, i1[(u64)s * n + j]);
-    }
-    o0[j] = a0;
-    o1[j] = a1;
-}
-
-// copy `rows` rows of `row_len` entries into rows of `padded_len`, zero filling
-__global__ void __launch_bounds__(BLOCK)
-pad_rows_kernel(const u64 *__restrict__ i0, const u64 *__restrict__ i1, u64 rows, u64 row_len, u64 padded_len,
-                u64 *__restrict__ o0, u64 *__restrict__ o1)
-{
-    u64 total = rows * padded_len;
-    for (u64 j = (u64)blockIdx.x * BLOCK + threadIdx.x; j < total; j += (u64)gridDim.x * BLOCK) {
-        u64 r = j / padded_len, c = j - r * padded_len;
-        bool in = c < row_len;
-        o0[j] = in ? i0[r * row_len + c] : 0;
-        o1[j] = in ? (i1 ? i1[r * row_len + c] : 0) : 0;
     }
 }
 
