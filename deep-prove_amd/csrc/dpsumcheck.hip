@@ -156,6 +156,7 @@ constexpr size_t SLICE_CTR_WORDS = (size_t)dpk::SL_MAX_GROUPS * dpk::SL_GROUP_WO
 constexpr size_t AXIS_CTR_OFF = 256 + SLICE_CTR_WORDS * 8 + 256 + (size_t)dpk::MAIL_RELAY_WORDS * 8;
 constexpr u32 AXIS_TILES = 256;
 constexpr size_t COUNTER_BYTES = AXIS_CTR_OFF + AXIS_TILES * 4;
+static_assert(dpk::LOGUP_BATCH <= LOGUP_OUT_AREAS, "the trees of a launch leave their outputs apart");
 static_assert(AXIS_CTR_OFF % 8 == 0, "words and counters stay aligned");
 
 // Address of `scratch` on a device, asked for once per device with that device current (every GPU has its own copy).
@@ -4893,20 +4894,21 @@ struct dps_logup {
 
 static_assert(LOGUP_SHADOW_STRIDE >= dpk::LOGUP_SHADOW_WORDS, "a tree's small levels fit their area");
 
-extern "C" int32_t dps_logup_build(dps_ctx *ctx, const dps_mle *const *cols, uint32_t n_cols, const dps_mle *numer,
-                                   const uint64_t c[2], const uint64_t beta[2], dps_logup **out)
+namespace {
+
+// A tree's description checked, its layers' memory allocated; the launches are dps_logup_build_many's
+int32_t logup_prepare(dps_ctx *ctx, const dps_logup_input &in, std::unique_ptr<dps_logup> *out)
 {
-    if (!ctx || !cols || !out || !c || !beta || n_cols == 0) return fail(ctx, DPS_ERR_INVALID, "dps_logup_build: bad argument");
+    const u32 n_cols = in.n_cols;
+    if (!in.cols || n_cols == 0) return fail(ctx, DPS_ERR_INVALID, "dps_logup_build: bad argument");
     if (n_cols > dpk::LOGUP_MAX_COLS) return fail(ctx, DPS_ERR_UNSUPPORTED, "dps_logup_build: more than %d columns", dpk::LOGUP_MAX_COLS);
-    if (!canonical(c, 2) || !canonical(beta, 2)) return fail(ctx, DPS_ERR_INVALID, "dps_logup_build: challenge not canonical");
-    DeviceGuard g(ctx->device);
-    tail_abort(ctx);
-    u64 len = cols[0] ? cols[0]->len : 0;
+    if (!canonical(in.c, 2) || !canonical(in.beta, 2)) return fail(ctx, DPS_ERR_INVALID, "dps_logup_build: challenge not canonical");
+    u64 len = in.cols[0] ? in.cols[0]->len : 0;
     if (!is_pow2(len) || len < 2) return fail(ctx, DPS_ERR_INVALID, "dps_logup_build: column length must be a power of two >= 2");
     for (u32 k = 0; k < n_cols; k++)
-        if (!cols[k] || cols[k]->kind != DPS_BASE || cols[k]->len != len || cols[k]->ctx != ctx || cols[k]->pad_vars)
+        if (!in.cols[k] || in.cols[k]->kind != DPS_BASE || in.cols[k]->len != len || in.cols[k]->ctx != ctx || in.cols[k]->pad_vars)
             return fail(ctx, DPS_ERR_INVALID, "dps_logup_build: column %u is not a base table of %llu entries", k, (unsigned long long)len);
-    if (numer && (numer->kind != DPS_BASE || numer->len != len)) return fail(ctx, DPS_ERR_INVALID, "dps_logup_build: multiplicity table mismatch");
+    if (in.numer && (in.numer->kind != DPS_BASE || in.numer->len != len)) return fail(ctx, DPS_ERR_INVALID, "dps_logup_build: multiplicity table mismatch");
     std::unique_ptr<dps_logup> lg(new (std::nothrow) dps_logup());
     if (!lg) return fail(ctx, DPS_ERR_OOM, "host allocation failed");
     lg->ctx = ctx;
@@ -4927,64 +4929,129 @@ extern "C" int32_t dps_logup_build(dps_ctx *ctx, const dps_mle *const *cols, uin
     CHK(pool_alloc(ctx, std::max<u64>(words, 4) * 8, &p1));
     st->c1 = (u64 *)p1;
     lg->arena = st;
-    if (top >= 2) {
-        dpk::LogupFirstArgs a;
+    *out = std::move(lg);
+    return DPS_OK;
+}
+
+// The level from which a tree's levels are one launch of one workgroup; the larger ones behind the first are a launch each
+u32 logup_tail_first(const dps_logup &lg)
+{
+    u32 k = 2;
+    while (k < lg.n_layers && (lg.len >> k) > (1ull << dpk::LOGUP_TAIL_BITS)) k++;
+    return k;
+}
+
+}  // namespace
+
+extern "C" int32_t dps_logup_build_many(dps_ctx *ctx, const dps_logup_input *in, uint32_t count, dps_logup **out)
+{
+    if (!ctx || !out || (count && !in)) return fail(ctx, DPS_ERR_INVALID, "dps_logup_build: bad argument");
+    DeviceGuard g(ctx->device);
+    tail_abort(ctx);
+    for (u32 i = 0; i < count; i++) out[i] = nullptr;
+    std::vector<std::unique_ptr<dps_logup>> trees(count);
+    for (u32 i = 0; i < count; i++) CHK(logup_prepare(ctx, in[i], &trees[i]));
+    // the first levels
+    dpk::LogupFirstBatch fb;
+    u32 n_first = 0;
+    u64 most = 0;
+    double bytes = 0;
+    auto launch_first = [&]() -> int32_t {
+        if (!n_first) return DPS_OK;
+        ProfScope ps(ctx, DPS_K_LOGUP, bytes);
+        dpk::logup_first_kernel<<<dim3(grid_for(most), n_first), dpk::BLOCK, 0, ctx->stream>>>(fb);
+        n_first = 0, most = 0, bytes = 0;
+        HIPCHK(ctx, hipGetLastError());
+        return DPS_OK;
+    };
+    for (u32 i = 0; i < count; i++) {
+        dps_logup &lg = *trees[i];
+        if (lg.n_layers < 2) continue;
+        dpk::LogupFirstArgs &a = fb.tree[n_first++];
         memset(&a, 0, sizeof a);
-        for (u32 k = 0; k < n_cols; k++) a.cols[k] = cols[k]->p0();
-        a.n_cols = n_cols;
-        a.numer = numer ? numer->p0() : nullptr;
-        a.c0 = c[0];
-        a.c1 = c[1];
-        E2 pw = gl::e2_one(), b = gl::e2(beta[0], beta[1]);
-        for (u32 k = 0; k < n_cols; k++) {
+        for (u32 k = 0; k < in[i].n_cols; k++) a.cols[k] = in[i].cols[k]->p0();
+        a.n_cols = in[i].n_cols;
+        a.numer = in[i].numer ? in[i].numer->p0() : nullptr;
+        a.c0 = in[i].c[0];
+        a.c1 = in[i].c[1];
+        E2 pw = gl::e2_one(), b = gl::e2(in[i].beta[0], in[i].beta[1]);
+        for (u32 k = 0; k < in[i].n_cols; k++) {
             a.pw[2 * k] = pw.c0;
             a.pw[2 * k + 1] = pw.c1;
             pw = gl::mul(pw, b);
         }
-        u64 half = len >> 1;
+        const u64 half = lg.len >> 1;
         a.half = half;
-        a.n0 = st->c0 + lg->layer_off[1];
-        a.n1 = st->c1 + lg->layer_off[1];
+        a.n0 = lg.arena->c0 + lg.layer_off[1];
+        a.n1 = lg.arena->c1 + lg.layer_off[1];
         a.d0 = a.n0 + half;
         a.d1 = a.n1 + half;
-        {
-            ProfScope ps(ctx, DPS_K_LOGUP, (double)len * 8.0 * (n_cols + (numer ? 1 : 0)) + (double)half * 32.0);
-            dpk::logup_first_kernel<<<grid_for(half), dpk::BLOCK, 0, ctx->stream>>>(a);
-            HIPCHK(ctx, hipGetLastError());
-        }
-        // levels of more than 2^LOGUP_TAIL_BITS entries: a launch each; the others in one launch of one workgroup
-        u32 k = 2;
-        for (; k < top && (len >> k) > (1ull << dpk::LOGUP_TAIL_BITS); k++) {
-            u64 prev = len >> (k - 1), cur = len >> k;
-            const u64 *pn0 = st->c0 + lg->layer_off[k - 1], *pn1 = st->c1 + lg->layer_off[k - 1];
-            u64 *n0 = st->c0 + lg->layer_off[k], *n1 = st->c1 + lg->layer_off[k];
+        most = std::max(most, half);
+        bytes += (double)lg.len * 8.0 * (in[i].n_cols + (in[i].numer ? 1 : 0)) + (double)half * 32.0;
+        if (n_first == (u32)dpk::LOGUP_BATCH) CHK(launch_first());
+    }
+    CHK(launch_first());
+    // levels of more than 2^LOGUP_TAIL_BITS entries
+    for (u32 i = 0; i < count; i++) {
+        const dps_logup &lg = *trees[i];
+        const Storage &st = *lg.arena;
+        for (u32 k = 2; k < logup_tail_first(lg); k++) {
+            u64 prev = lg.len >> (k - 1), cur = lg.len >> k;
+            const u64 *pn0 = st.c0 + lg.layer_off[k - 1], *pn1 = st.c1 + lg.layer_off[k - 1];
+            u64 *n0 = st.c0 + lg.layer_off[k], *n1 = st.c1 + lg.layer_off[k];
             ProfScope ps(ctx, DPS_K_LOGUP, (double)prev * 32.0 + (double)cur * 32.0);
             dpk::logup_next_kernel<<<grid_for(cur), dpk::BLOCK, 0, ctx->stream>>>(pn0, pn1, pn0 + prev, pn1 + prev, cur, n0, n1, n0 + cur, n1 + cur);
             HIPCHK(ctx, hipGetLastError());
         }
-        if (k < top) {
-            dpk::LogupTailArgs ta;
-            memset(&ta, 0, sizeof ta);
-            ta.c0 = st->c0;
-            ta.c1 = st->c1;
-            ta.n_levels = top - k;
-            ta.first_cur = len >> k;
-            for (u32 l = 0; l <= ta.n_levels; l++) ta.off[l] = lg->layer_off[k - 1 + l];
-            lg->out_slot = (u32)(ctx->logup_builds++ % LOGUP_OUT_AREAS);
-            lg->out_build = ctx->logup_builds;
-            lg->out_seq = ++ctx->seq;
-            ta.out_host = ctx->d_pinned + logup_out_off(ctx, lg->out_slot);
-            ta.seq = lg->out_seq;
-            if (ctx->d_shadow) {
-                ta.shadow = ctx->d_shadow + (size_t)lg->out_slot * LOGUP_SHADOW_STRIDE;
-                lg->shadow_first = k;
-            }
-            ProfScope ps(ctx, DPS_K_LOGUP, (double)ta.first_cur * 4 * 32.0);
-            dpk::logup_tail_kernel<<<1, dpk::LOGUP_TAIL_BLOCK, 0, ctx->stream>>>(ta);
-            HIPCHK(ctx, hipGetLastError());
-        }
     }
-    *out = lg.release();
+    // the others
+    dpk::LogupTailBatch tb;
+    u32 n_tail = 0;
+    bytes = 0;
+    auto launch_tails = [&]() -> int32_t {
+        if (!n_tail) return DPS_OK;
+        ProfScope ps(ctx, DPS_K_LOGUP, bytes);
+        dpk::logup_tail_kernel<<<n_tail, dpk::LOGUP_TAIL_BLOCK, 0, ctx->stream>>>(tb);
+        n_tail = 0, bytes = 0;
+        HIPCHK(ctx, hipGetLastError());
+        return DPS_OK;
+    };
+    for (u32 i = 0; i < count; i++) {
+        dps_logup &lg = *trees[i];
+        const u32 k = logup_tail_first(lg);
+        if (k >= lg.n_layers) continue;
+        dpk::LogupTailArgs &ta = tb.tree[n_tail++];
+        memset(&ta, 0, sizeof ta);
+        ta.c0 = lg.arena->c0;
+        ta.c1 = lg.arena->c1;
+        ta.n_levels = lg.n_layers - k;
+        ta.first_cur = lg.len >> k;
+        for (u32 l = 0; l <= ta.n_levels; l++) ta.off[l] = lg.layer_off[k - 1 + l];
+        lg.out_slot = (u32)(ctx->logup_builds++ % LOGUP_OUT_AREAS);
+        lg.out_build = ctx->logup_builds;
+        lg.out_seq = ++ctx->seq;
+        ta.out_host = ctx->d_pinned + logup_out_off(ctx, lg.out_slot);
+        ta.seq = lg.out_seq;
+        if (ctx->d_shadow) {
+            ta.shadow = ctx->d_shadow + (size_t)lg.out_slot * LOGUP_SHADOW_STRIDE;
+            lg.shadow_first = k;
+        }
+        bytes += (double)ta.first_cur * 4 * 32.0;
+        if (n_tail == (u32)dpk::LOGUP_BATCH) CHK(launch_tails());
+    }
+    CHK(launch_tails());
+    for (u32 i = 0; i < count; i++) out[i] = trees[i].release();
+    return DPS_OK;
+}
+
+extern "C" int32_t dps_logup_build(dps_ctx *ctx, const dps_mle *const *cols, uint32_t n_cols, const dps_mle *numer,
+                                   const uint64_t c[2], const uint64_t beta[2], dps_logup **out)
+{
+    if (!ctx || !cols || !out || !c || !beta || n_cols == 0) return fail(ctx, DPS_ERR_INVALID, "dps_logup_build: bad argument");
+    const dps_logup_input in{cols, n_cols, numer, {c[0], c[1]}, {beta[0], beta[1]}};
+    dps_logup *lg = nullptr;
+    CHK(dps_logup_build_many(ctx, &in, 1, &lg));
+    *out = lg;
     return DPS_OK;
 }
 

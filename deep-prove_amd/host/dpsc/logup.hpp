@@ -56,21 +56,34 @@ struct LogUpInput {
 };
 
 // LogUpCircuit (circuit.rs:503-590): layer 0 is the caller's columns, the layers
-// above live in one GPU arena built by dps_logup_build.
+// above live in one GPU arena built by dps_logup_build_many.
 class LogUpCircuit {
 public:
     LogUpCircuit(const Context &ctx, std::vector<const DensePolynomial *> cols, const DensePolynomial *mult, const F &c, const F &beta)
         : ctx_(&ctx), cols_(std::move(cols)), mult_(mult), c_(c), beta_(beta)
     {
-        std::vector<const dps_mle *> hs;
-        for (auto *p : cols_) hs.push_back(p->raw());
-        uint64_t cc[2] = {c.c0, c.c1}, bb[2] = {beta.c0, beta.c1};
-        dps_logup *h = nullptr;
-        ctx.check(dps_logup_build(ctx.raw(), hs.data(), (uint32_t)hs.size(), mult ? mult->raw() : nullptr, cc, bb, &h), "dps_logup_build");
-        h_.reset(h, &dps_logup_free);
-        uint32_t nl = 0;
-        dps_logup_num_layers(h, &nl);
-        n_layers_ = nl;
+    }
+    // the fraction trees of all circuits of a batch
+    static void build(const Context &ctx, std::vector<LogUpCircuit> &circuits)
+    {
+        std::vector<std::vector<const dps_mle *>> cols;
+        std::vector<dps_logup_input> in;
+        for (auto &q : circuits) {
+            cols.emplace_back();
+            for (auto *p : q.cols_) cols.back().push_back(p->raw());
+        }
+        for (size_t i = 0; i < circuits.size(); i++) {
+            const LogUpCircuit &q = circuits[i];
+            in.push_back(dps_logup_input{cols[i].data(), (uint32_t)cols[i].size(), q.mult_ ? q.mult_->raw() : nullptr, {q.c_.c0, q.c_.c1}, {q.beta_.c0, q.beta_.c1}});
+        }
+        std::vector<dps_logup *> h(in.size(), nullptr);
+        ctx.check(dps_logup_build_many(ctx.raw(), in.data(), (uint32_t)in.size(), h.data()), "dps_logup_build");
+        for (size_t i = 0; i < circuits.size(); i++) {
+            circuits[i].h_.reset(h[i], &dps_logup_free);
+            uint32_t nl = 0;
+            dps_logup_num_layers(h[i], &nl);
+            circuits[i].n_layers_ = nl;
+        }
     }
     // variables of the sumcheck over the input layer (circuit.rs:67-80,564-566)
     size_t num_vars() const { return n_layers_ - 1; }
@@ -205,6 +218,7 @@ inline LogUpBatchProof new_batch_multiple_sizes_prove(const Context &ctx, const 
             }
         }
     }
+    LogUpCircuit::build(ctx, circuits);
     const size_t num_instances = circuits.size();
     size_t total_layers = circuits[0].num_vars();
     for (size_t i = 1; i < circuits.size(); i++) {

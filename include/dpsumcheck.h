@@ -210,6 +210,14 @@ int32_t dps_sc_prove(dps_sc *sc, dps_round_fn fn, void *user, uint64_t *proof_ou
  * table (table instance) or NULL (lookup instance, numerators -1). */
 int32_t dps_logup_build(dps_ctx *ctx, const dps_mle *const *cols, uint32_t n_cols, const dps_mle *numer,
                         const uint64_t c[2], const uint64_t beta[2], dps_logup **out);
+/* The trees of a batch, their small levels in launches they share; none is returned unless all are. */
+typedef struct dps_logup_input {
+    const dps_mle *const *cols;
+    uint32_t n_cols;
+    const dps_mle *numer;
+    uint64_t c[2], beta[2];
+} dps_logup_input;
+int32_t dps_logup_build_many(dps_ctx *ctx, const dps_logup_input *in, uint32_t count, dps_logup **out);
 /* number of layers including the input layer 0 */
 int32_t dps_logup_num_layers(const dps_logup *lg, uint32_t *n_layers);
 /* numerator and denominator tables of layer k >= 1 (views; free them with dps_mle_free).  The layers of at most 256

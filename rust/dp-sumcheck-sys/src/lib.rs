@@ -77,6 +77,17 @@ pub struct dps_term {
     pub factors: [u32; DPS_MAX_FACTORS],
 }
 
+/// One fraction tree of a batch (dps_logup_build_many).
+#[repr(C)]
+#[derive(Clone, Copy, Debug)]
+pub struct dps_logup_input {
+    pub cols: *const *const dps_mle,
+    pub n_cols: u32,
+    pub numer: *const dps_mle,
+    pub c: [u64; 2],
+    pub beta: [u64; 2],
+}
+
 /// Transcript hook: absorb `n_evals` extension elements of round `round` (1-based), write the
 /// squeezed challenge (two limbs).  Non-zero aborts the proof.
 pub type dps_round_fn = Option<
@@ -173,6 +184,7 @@ extern "C" {
         beta: *const u64,
         out: *mut *mut dps_logup,
     ) -> i32;
+    pub fn dps_logup_build_many(ctx: *mut dps_ctx, input: *const dps_logup_input, count: u32, out: *mut *mut dps_logup) -> i32;
     pub fn dps_logup_num_layers(lg: *const dps_logup, n_layers: *mut u32) -> i32;
     pub fn dps_logup_layer(lg: *const dps_logup, k: u32, num: *mut *mut dps_mle, den: *mut *mut dps_mle) -> i32;
     pub fn dps_logup_outputs(lg: *const dps_logup, out: *mut u64) -> i32;
