@@ -216,8 +216,45 @@ __global__ void __launch_bounds__(BLOCK) eq_define_kernel(EqJobs js)
     }
 }
 
+// The tables of a point's coordinates, three at a time in their order; an entry of the eq table is a product of one entry of
+// each.  A workgroup makes them with two field products one behind the other.
+constexpr u32 POINT_GROUPS = (EQ_MAX_VARS + 2) / 3;
+struct PointGroups {
+    u64 c0[POINT_GROUPS][8], c1[POINT_GROUPS][8];
+    __device__ __forceinline__ E2 at(u32 g, u32 e) const { return gl::e2(c0[g][e], c1[g][e]); }
+};
+// (visible after a barrier; coordinates beyond the point's `m` count as zero, at least `least` tables; the number of tables)
+__device__ __forceinline__ u32 point_groups(const u64 *p, u32 m, u32 least, PointGroups &out)
+{
+    const u32 have = (m + 2) / 3, n_groups = have < least ? least : have, g = threadIdx.x / 8, e = threadIdx.x % 8;
+    static_assert(8 * POINT_GROUPS <= BLOCK, "an entry a thread");
+    if (g < n_groups) {
+        E2 v = gl::e2_one();
+#pragma unroll
+        for (u32 b = 0; b < 3; b++) {
+            const u32 c = 3 * g + b;
+            const E2 r = c < m ? gl::e2(p[2 * c], p[2 * c + 1]) : gl::e2_zero();
+            const E2 x = ((e >> b) & 1) ? r : gl::sub(gl::e2_one(), r);
+            v = b == 0 ? x : gl::mul(v, x);
+        }
+        out.c0[g][e] = v.c0;
+        out.c1[g][e] = v.c1;
+    }
+    return n_groups;
+}
+// product of the entries that the bits of k choose, from table `first` on
+__device__ __forceinline__ E2 point_weight(const PointGroups &t, u32 first, u32 n_groups, u64 k)
+{
+    if (first >= n_groups) return gl::e2_one();
+    E2 v = t.at(first, (u32)k & 7);
+    for (u32 g = first + 1; g < n_groups; g++) v = gl::mul(v, t.at(g, (u32)(k >> (3 * (g - first))) & 7));
+    return v;
+}
+
 // The same for jobs of several tables at once (many small eq tables, each with its own point): descriptors and
-// points lie in host-visible memory, written just before the launch.
+// points lie in host-visible memory, written just before the launch, and a coordinate is read once a workgroup.  Bound: the
+// chain of products, a third of the coordinates long and two (one per coordinate and a load from the host's memory with each
+// before: an opening's 12 tables of up to 2^11 entries 12.7 -> 8.1 us, two tables of a small lookup layer 8.3 -> 6.7 us).
 struct EqJobM {
     u64 *o0, *o1;     // where the job's entries go
     u32 first, n_bits;
@@ -226,15 +263,14 @@ struct EqJobM {
 };
 __global__ void __launch_bounds__(BLOCK) eq_define_many_kernel(const EqJobM *__restrict__ jobs, const u64 *__restrict__ points)
 {
+    __shared__ PointGroups groups;
     const EqJobM j = jobs[blockIdx.y];
     const u64 i = (u64)blockIdx.x * BLOCK + threadIdx.x;
+    if ((u64)blockIdx.x * BLOCK >= ((u64)1 << j.n_bits)) return;  // (the whole workgroup)
+    const u32 n_groups = point_groups(points + j.point_off + 2 * j.first, j.n_bits, 0, groups);
+    __syncthreads();
     if (i >= ((u64)1 << j.n_bits)) return;
-    const u64 *pt = points + j.point_off;
-    E2 acc = gl::e2_one();
-    for (u32 b = 0; b < j.n_bits; b++) {
-        E2 r = gl::e2(pt[2 * (j.first + b)], pt[2 * (j.first + b) + 1]);
-        acc = gl::mul(acc, ((i >> b) & 1) ? r : gl::sub(gl::e2_one(), r));
-    }
+    const E2 acc = point_weight(groups, 0, n_groups, i);
     j.o0[i] = acc.c0;
     j.o1[i] = acc.c1;
 }
@@ -2878,7 +2914,6 @@ __global__ void __launch_bounds__(BLOCK) eval_point_kernel(EvalArgs a, FastFin f
 // int64 12.5 us (kernel trace); proofs of that product 114 -> 91 us, of one row of it 159 -> 102 us, of both products of an
 // attention layer of 12 heads over 197 tokens 237 -> 203 us.
 // ---------------------------------------------------------------------------
-constexpr u32 AXP_GROUPS = (EQ_MAX_VARS + 2) / 3;
 constexpr u32 AXP_ROW_BITS = 9, AXP_ROW_STEPS = 64;  // columns a step of a row (log2), steps whose weights are made together
 struct AxisPointArgs {
     const void *in0;
@@ -2897,37 +2932,6 @@ struct AxisPointArgs {
     u32 *counters;       // one per tile, zero between launches
     u64 p[2 * EQ_MAX_VARS];
 };
-struct AxisGroups {
-    u64 c0[AXP_GROUPS][8], c1[AXP_GROUPS][8];
-    __device__ __forceinline__ E2 at(u32 g, u32 e) const { return gl::e2(c0[g][e], c1[g][e]); }
-};
-// tables of three coordinates each, in order; coordinates beyond the point's count as zero (at least `least` tables)
-__device__ __forceinline__ u32 axis_groups(const AxisPointArgs &a, u32 least, AxisGroups &out)
-{
-    const u32 have = (a.m + 2) / 3, n_groups = have < least ? least : have, g = threadIdx.x / 8, e = threadIdx.x % 8;
-    static_assert(8 * AXP_GROUPS <= BLOCK, "an entry a thread");
-    if (g < n_groups) {
-        E2 v = gl::e2_one();
-#pragma unroll
-        for (u32 b = 0; b < 3; b++) {
-            const u32 c = 3 * g + b;
-            const E2 r = c < a.m ? gl::e2(a.p[2 * c], a.p[2 * c + 1]) : gl::e2_zero();
-            const E2 x = ((e >> b) & 1) ? r : gl::sub(gl::e2_one(), r);
-            v = b == 0 ? x : gl::mul(v, x);
-        }
-        out.c0[g][e] = v.c0;
-        out.c1[g][e] = v.c1;
-    }
-    return n_groups;
-}
-// product of the entries that the bits of k choose, from table `first` on
-__device__ __forceinline__ E2 axis_weight(const AxisGroups &t, u32 first, u32 n_groups, u64 k)
-{
-    if (first >= n_groups) return gl::e2_one();
-    E2 v = t.at(first, (u32)k & 7);
-    for (u32 g = first + 1; g < n_groups; g++) v = gl::mul(v, t.at(g, (u32)(k >> (3 * (g - first))) & 7));
-    return v;
-}
 template <int KIND>
 __device__ __forceinline__ E2 axis_entry(const AxisPointArgs &a, u64 off)
 {
@@ -2966,7 +2970,7 @@ __device__ __forceinline__ void axis_pads(const AxisPointArgs &a)
 template <int KIND>
 __global__ void __launch_bounds__(BLOCK) axis_point_col_kernel(AxisPointArgs a)
 {
-    __shared__ AxisGroups groups;
+    __shared__ PointGroups groups;
     __shared__ u64 w0[BLOCK], w1[BLOCK];  // weights of up to BLOCK values of k
     __shared__ u64 lds[BLOCK * 2];
     __shared__ int last_flag;
@@ -2977,7 +2981,7 @@ __global__ void __launch_bounds__(BLOCK) axis_point_col_kernel(AxisPointArgs a)
     const u64 o = pre * a.C + i;
     const bool mine = i < a.C;
     const u64 base = ax_offset(pre, a.n_pre, a.pre_dims, a.pre_strides) + (mine ? ax_offset(i, a.n_post, a.post_dims, a.post_strides) : 0);
-    const u32 n_groups = axis_groups(a, 0, groups);
+    const u32 n_groups = point_groups(a.p, a.m, 0, groups);
     axis_pads(a);
     const u64 k0 = (u64)blockIdx.y * a.k_per_slice, k1 = k0 + a.k_per_slice < a.K ? k0 + a.k_per_slice : a.K;
     gl::E2Acc s = gl::e2acc_zero();
@@ -2985,7 +2989,7 @@ __global__ void __launch_bounds__(BLOCK) axis_point_col_kernel(AxisPointArgs a)
         const u32 here = k1 - at < BLOCK ? (u32)(k1 - at) : BLOCK;
         __syncthreads();  // the tables are there; the weights before have been read
         if (tid < here) {
-            const E2 v = axis_weight(groups, 0, n_groups, at + tid);
+            const E2 v = point_weight(groups, 0, n_groups, at + tid);
             w0[tid] = v.c0;
             w1[tid] = v.c1;
         }
@@ -3050,7 +3054,7 @@ __global__ void __launch_bounds__(BLOCK) axis_point_col_kernel(AxisPointArgs a)
 template <int KIND>
 __global__ void __launch_bounds__(BLOCK) axis_point_row_kernel(AxisPointArgs a)
 {
-    __shared__ AxisGroups groups;
+    __shared__ PointGroups groups;
     __shared__ u64 sw0[AXP_ROW_STEPS], sw1[AXP_ROW_STEPS];
     __shared__ u64 lds[2 * (BLOCK / WAVE)];
     __shared__ int last_flag;
@@ -3072,7 +3076,7 @@ __global__ void __launch_bounds__(BLOCK) axis_point_row_kernel(AxisPointArgs a)
     const u32 s0 = blockIdx.y * (u32)a.k_per_slice, s1 = s0 + (u32)a.k_per_slice < steps ? s0 + (u32)a.k_per_slice : steps;
     E2 v[8];
     load(s0 + sub, v);  // asked for before the weights are made
-    const u32 n_groups = axis_groups(a, AXP_ROW_BITS / 3, groups);
+    const u32 n_groups = point_groups(a.p, a.m, AXP_ROW_BITS / 3, groups);
     axis_pads(a);
     gl::E2P w[8];
     gl::E2Acc total = gl::e2acc_zero();
@@ -3080,7 +3084,7 @@ __global__ void __launch_bounds__(BLOCK) axis_point_row_kernel(AxisPointArgs a)
         const u32 end = at + AXP_ROW_STEPS < s1 ? at + AXP_ROW_STEPS : s1;
         __syncthreads();  // the tables are there; the weights before have been read
         if (tid < end - at) {
-            const E2 h = axis_weight(groups, AXP_ROW_BITS / 3, n_groups, at + tid);
+            const E2 h = point_weight(groups, AXP_ROW_BITS / 3, n_groups, at + tid);
             sw0[tid] = h.c0;
             sw1[tid] = h.c1;
         }
