@@ -3117,7 +3117,8 @@ namespace {
 //     (2^17 entries; merging four claims on 2^20 entries: 450 -> 250 us), and wherever a sum has more tables than
 //     the resident launches take or zero-padded ones, which only the general launches read (a launch for every fold and 430 us a
 //     round for 67 tables);
-//   - by eq tables only in that last case, when it leaves fewer tables or the sum has zero-padded ones.
+//   - by eq tables only in that last case: with zero-padded tables always, otherwise where it leaves at most eight products of
+//     fewer tables, or the tables are large, or their groups would not be resident side by side.
 struct CombinedTable {
     u32 factor;                                // X, or the eq table E_g
     std::vector<std::pair<u32, E2>> items;     // tables and coefficients
@@ -3160,7 +3161,25 @@ bool plan_combination(const dps_sc *sc, const dps_mle *const *mles, const std::v
         if (is_new) plan->push_back(CombinedTable{t.factors[f], {}});
         (*plan)[it->second].items.emplace_back(t.factors[f ^ 1], coeff_of(t));
     }
-    return any_zpad || 2 * plan->size() < n_mles;
+    if (any_zpad) return true;
+    if (2 * plan->size() >= n_mles) return false;
+    if (n_vars >= 17 || 4 * plan->size() <= (size_t)dpk::SL_MAX_TABS) return true;
+    // More products than that are no faster in the resident launches than groups of tables resident side by side, which is how
+    // the sum as it stands runs while it has no more groups than fit (132 tables at 16 points: 0.40 ms as it stands,
+    // 0.43 combined; 60 tables at 8 points: 0.30 and 0.19).
+    size_t groups = 1;  // (as SessionSetup::group_terms cuts them)
+    std::vector<u32> cur;
+    for (const dps_term &t : sc->terms) {
+        std::vector<u32> merged = cur;
+        for (u32 f = 0; f < 2; f++)
+            if (std::find(merged.begin(), merged.end(), t.factors[f]) == merged.end()) merged.push_back(t.factors[f]);
+        if (merged.size() > (size_t)dpk::POLY_MAXT) {
+            groups++;
+            merged.assign(t.factors, t.factors + 2);
+        }
+        cur = merged;
+    }
+    return groups > POLY_RAW_MAX_GROUPS;
 }
 
 // Carries the plan out: the tables M (and eq tables with their padding), and the session over them.

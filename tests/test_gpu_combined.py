@@ -153,3 +153,15 @@ def test_many_claims_on_one_table(dp, ctx, orc, n, k):
     for e in s.eqs([n] * k):
         s.term(x, e)
     s.check(dp)
+
+
+# full-size tables at several points: combined up to eight points, as they stand beyond that while their groups of tables fit side by
+# side, combined again where they do not (34 points) and for large tables
+@pytest.mark.parametrize("n,polys,points", [(9, 40, 8), (9, 40, 9), (11, 60, 17), (8, 80, 34), (17, 40, 17)])
+def test_claims_at_many_points(dp, ctx, orc, n, polys, points):
+    s = Sum(ctx, orc, n, 8000 + n + points)
+    tables = [s.table(base=i % 2 == 0) for i in range(polys)]
+    eqs = s.eqs([n] * points)
+    for i, t in enumerate(tables):
+        s.term(t, eqs[i % points])
+    s.check(dp)
