@@ -25,11 +25,6 @@ using gl::E2;
 using gl::u32;
 using gl::u64;
 
-// Work area of dps_mle_evaluate_noalloc, the one entry point that allocates nothing: per-workgroup partial sums and a
-// ticket counter (dpk::WS_WORDS words, 16 KiB), zero between calls.  File-scope device memory: every GPU the library runs on holds its own copy, at its own address, until the process ends.  In host
-// code the name below is only a handle for hipGetSymbolAddress; kernels are given the address that call returns.
-static __device__ __align__(256) uint64_t scratch[dpk::WS_WORDS];
-
 namespace {
 
 // 3 workgroups per CU on 256 CUs: measured best for the streaming kernels (each workgroup pays a fixed
@@ -92,8 +87,9 @@ struct dps_ctx {
     u64 seq = 0;                // last sequence number handed to a launch
     struct dps_sc *tail_owner = nullptr;  // session whose tail kernel is resident on the stream
     u32 units_held = 0;         // compute units of the device's ledger that launch holds (admit_waiting_launch)
-    u64 *d_eval = nullptr;      // work area of dps_mle_evaluate (dpk::WS_WORDS words)
-    u64 *ws = nullptr;          // this device's copy of the allocation-free entry point's work area
+    // Work area of the evaluations (dpk::WS_WORDS words): partial sums and a ticket counter that the launch which used it leaves
+    // at zero.  A context's own: its launches follow one another on its stream, so each finds the counter as the one before left it.
+    u64 *d_eval = nullptr;
     bool profiling = false;
     std::vector<ProfRec> recs;
     std::vector<hipEvent_t> ev_pool;
@@ -159,25 +155,7 @@ constexpr size_t COUNTER_BYTES = AXIS_CTR_OFF + AXIS_TILES * 4;
 static_assert(dpk::LOGUP_BATCH <= LOGUP_OUT_AREAS, "the trees of a launch leave their outputs apart");
 static_assert(AXIS_CTR_OFF % 8 == 0, "words and counters stay aligned");
 
-// Address of `scratch` on a device, asked for once per device with that device current (every GPU has its own copy).
-constexpr int WS_MAX_DEVICES = 64;
-int32_t work_area_of_device(int device, u64 **out)
-{
-    static std::mutex mu;
-    static u64 *ptr_of[WS_MAX_DEVICES] = {};
-    if (device < 0 || device >= WS_MAX_DEVICES) return DPS_ERR_UNSUPPORTED;
-    std::lock_guard<std::mutex> lock(mu);
-    if (!ptr_of[device]) {
-        void *p = nullptr;
-        if (hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)) != hipSuccess || !p) {
-            (void)hipGetLastError();
-            return DPS_ERR_HIP;
-        }
-        ptr_of[device] = static_cast<u64 *>(p);
-    }
-    *out = ptr_of[device];
-    return DPS_OK;
-}
+constexpr int MAX_DEVICES = 64;
 
 // ---------------------------------------------------------------------------
 // Admission of launches that wait on the GPU.
@@ -203,7 +181,7 @@ struct DeviceLedger {
 };
 DeviceLedger &ledger_of(int device)
 {
-    static DeviceLedger ledgers[WS_MAX_DEVICES];
+    static DeviceLedger ledgers[MAX_DEVICES];
     return ledgers[device];
 }
 
@@ -522,9 +500,8 @@ extern "C" int32_t dps_ctx_create(int32_t device, dps_ctx **out)
         delete ctx;
         return rc;
     };
+    if (device >= MAX_DEVICES) return bail(DPS_ERR_UNSUPPORTED);
     if (hipStreamCreate(&ctx->stream) != hipSuccess) return bail(DPS_ERR_HIP);
-    // (the context's device is current here)
-    if (int32_t rc = work_area_of_device(device, &ctx->ws); rc != DPS_OK) return bail(rc);
     {
         int cus = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cus <= 0) return bail(DPS_ERR_HIP);
@@ -619,7 +596,7 @@ extern "C" int32_t dps_ctx_destroy(dps_ctx *ctx)
 
 extern "C" int32_t dps_device_set_resident_budget(int32_t device, int32_t compute_units)
 {
-    if (device < 0 || device >= WS_MAX_DEVICES || compute_units < -1) return DPS_ERR_INVALID;
+    if (device < 0 || device >= MAX_DEVICES || compute_units < -1) return DPS_ERR_INVALID;
     DeviceLedger &l = ledger_of(device);
     std::lock_guard<std::mutex> lock(l.mu);
     l.limit = compute_units;
@@ -628,7 +605,7 @@ extern "C" int32_t dps_device_set_resident_budget(int32_t device, int32_t comput
 
 extern "C" int32_t dps_device_resident_budget(int32_t device, int32_t *in_use, int32_t *budget)
 {
-    if (device < 0 || device >= WS_MAX_DEVICES) return DPS_ERR_INVALID;
+    if (device < 0 || device >= MAX_DEVICES) return DPS_ERR_INVALID;
     DeviceLedger &l = ledger_of(device);
     std::lock_guard<std::mutex> lock(l.mu);
     if (in_use) *in_use = l.used;
@@ -1298,9 +1275,9 @@ namespace {
 
 int32_t wait_result(dps_ctx *ctx, u64 seq, u32 slot0, u32 n, u64 *out);
 
-// The value of a table at a point: one launch, whose last workgroup hands it to the host (`area`: the words the launch
-// keeps its partial sums and its ticket counter in, WS_WORDS of them, one such launch at a time).
-int32_t evaluate_at(dps_ctx *ctx, const dps_mle *mle, const uint64_t *point, u32 n, u64 *area, uint64_t out[2])
+// The value of a table at a point: one launch, whose last workgroup hands it to the host (`timed`: between two events when the
+// context measures its launches)
+int32_t evaluate_at(dps_ctx *ctx, const dps_mle *mle, const uint64_t *point, u32 n, bool timed, uint64_t out[2])
 {
     if (mle->eq && !(mle->eq->built & 1)) {
         // An eq table whose entries nobody has read yet is not in memory, and need not be: the multilinear extension of
@@ -1324,13 +1301,12 @@ int32_t evaluate_at(dps_ctx *ctx, const dps_mle *mle, const uint64_t *point, u32
     if (n) memcpy(a.p, point, 16 * (size_t)n);
     dpk::FastFin ff;
     memset(&ff, 0, sizeof ff);
-    ff.partial = area + dpk::WS_OFF_PARTIAL;
+    ff.partial = ctx->d_eval + dpk::WS_OFF_PARTIAL;
     ff.n_blocks = blocks;
     ff.out_host = ctx->d_pinned + ctx->res_off;
     ff.seq = ++ctx->seq;
-    ff.counter = reinterpret_cast<u32 *>(area + dpk::WS_OFF_COUNTER);
-    // (no timing events in the entry point that allocates nothing: creating one is an allocation of the runtime's)
-    ProfScope ps(ctx, DPS_K_AXIS_DOT, (double)mle->len * (mle->p1() ? 16.0 : mle->kind == DPS_I16 ? 2.0 : 8.0), area != ctx->ws);
+    ff.counter = reinterpret_cast<u32 *>(ctx->d_eval + dpk::WS_OFF_COUNTER);
+    ProfScope ps(ctx, DPS_K_AXIS_DOT, (double)mle->len * (mle->p1() ? 16.0 : mle->kind == DPS_I16 ? 2.0 : 8.0), timed);
     switch (mle->kind) {
     case DPS_BASE: dpk::eval_point_kernel<0><<<blocks, dpk::BLOCK, 0, ctx->stream>>>(a, ff); break;
     case DPS_EXT2: dpk::eval_point_kernel<1><<<blocks, dpk::BLOCK, 0, ctx->stream>>>(a, ff); break;
@@ -1352,7 +1328,7 @@ extern "C" int32_t dps_mle_evaluate(dps_ctx *ctx, const dps_mle *mle, const uint
     if (!canonical(point, 2 * (size_t)n)) return fail(ctx, DPS_ERR_INVALID, "dps_mle_evaluate: point not canonical");
     DeviceGuard g(ctx->device);
     tail_abort(ctx);
-    return evaluate_at(ctx, mle, point, n, ctx->d_eval, out);
+    return evaluate_at(ctx, mle, point, n, true, out);
 }
 
 extern "C" int32_t dps_mle_fix_high(dps_ctx *ctx, const dps_mle *mle, const uint64_t *point, uint32_t k, dps_mle **out)
@@ -4869,7 +4845,7 @@ extern "C" int32_t dps_sc_prove(dps_sc *sc, dps_round_fn fn, void *user, uint64_
 
 // ---------------------------------------------------------------------------
 // DensePolynomial::evaluate for callers that must not allocate (tight serving loops, harnesses that forbid hipMalloc):
-// the same value as dps_mle_evaluate, with everything beyond the table and the result kept in `scratch`.
+// the same value as dps_mle_evaluate, with everything beyond the table and the result kept in the context's work area.
 // No hipMalloc, hipFree, stream wait or host allocation on the way; the result crosses through the context's
 // pinned result area like a round message, and the call returns when it is there (the host polls for it, so this is
 // not a call to make under stream capture).
@@ -4885,15 +4861,11 @@ extern "C" int32_t dps_mle_evaluate_noalloc(dps_ctx *ctx, const dps_mle *mle, co
         return fail(ctx, DPS_ERR_UNSUPPORTED, "dps_mle_evaluate_noalloc: a table of %u variables is beyond the work area's limit of %u (use dps_mle_evaluate)", n,
                     dpk::WS_MAX_VARS);
     if (!canonical(point, 2 * (size_t)n)) return fail(ctx, DPS_ERR_INVALID, "dps_mle_evaluate_noalloc: point not canonical");
-    if (!ctx->ws) return fail(ctx, DPS_ERR_STATE, "dps_mle_evaluate_noalloc: the context has no work area");
     // (ending a launch that waits on the GPU for a session of this context would mean a stream wait and a memset)
     if (ctx->tail_owner) return fail(ctx, DPS_ERR_STATE, "dps_mle_evaluate_noalloc: a session of this context has a launch waiting on the GPU");
     DeviceGuard g(ctx->device);
-    // every context on a GPU shares that GPU's work area: one call at a time per device, from the first launch until the
-    // result is here
-    static std::mutex area_in_use[WS_MAX_DEVICES];
-    std::lock_guard<std::mutex> lock(area_in_use[ctx->device]);
-    return evaluate_at(ctx, mle, point, n, ctx->ws, out);
+    // (no timing events: creating one is an allocation of the runtime's)
+    return evaluate_at(ctx, mle, point, n, false, out);
 }
 
 // ---------------------------------------------------------------------------

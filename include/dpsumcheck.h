@@ -136,9 +136,8 @@ int32_t dps_mle_evaluate(dps_ctx *ctx, const dps_mle *mle, const uint64_t *point
 /* The same evaluation for callers that cannot allocate.  No counterpart in the reference: it is for tight serving
  * loops and harnesses that forbid hipMalloc.  The call makes no hipMalloc, hipFree or host allocation and waits for
  * no stream (it returns when the value has crossed to the host, which it polls for: not a call to record under stream
- * capture); its partial sums and ticket counter live in a file-scope device array of the library (16 KiB
- * per GPU, held until the process ends).  At most 24 variables (DPS_ERR_UNSUPPORTED beyond).  Every context on one
- * GPU shares that GPU's array: the library lets one such call at a time use it, others wait their turn.  An eq table
+ * capture); its partial sums and ticket counter live in 16,640 bytes of device memory that the context has held
+ * since it was created.  At most 24 variables (DPS_ERR_UNSUPPORTED beyond).  An eq table
  * whose entries have not been read yet (dps_eq_build keeps a large one unmaterialised) is evaluated in closed form on
  * the host.  DPS_ERR_STATE while a session of the context has a launch waiting on the GPU (between its rounds):
  * ending that launch would take a stream wait. */

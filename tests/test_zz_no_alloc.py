@@ -1,5 +1,5 @@
 """The entry point that allocates nothing (dps_mle_evaluate_noalloc) against the existing dps_mle_evaluate: same bits,
-on calls in a row that share the library's one work area per GPU, the later ones with smaller inputs."""
+on calls in a row that share a context's work area, the later ones with smaller inputs, and from contexts side by side."""
 import importlib
 
 import numpy as np
@@ -24,7 +24,7 @@ def ctx(dp):
 
 def test_evaluate_noalloc_matches_evaluate(dp, ctx, orc):
     # two calls in a row through the C ABI, the second with a smaller input: the work area keeps the first call's
-    # contents (longer eq tables, more partial sums) and the second must not be disturbed by them
+    # contents (more partial sums) and the second must not be disturbed by them
     big, small = 16, 9
     tb, ts = rand_e2(1 << big, 31001), rand_base(1 << small, 31002)
     pb, ps = rand_e2(big, 31003), rand_e2(small, 31004)
@@ -154,7 +154,7 @@ def test_evaluate_noalloc_refuses_while_a_launch_waits(dp, ctx, orc):
 
 
 def test_evaluate_noalloc_from_two_threads(dp, orc):
-    # two contexts on two threads share the GPU's one work area: the library lets one call at a time use it
+    # two contexts on two threads, each with a work area of its own
     import threading
 
     errors = []
@@ -182,3 +182,36 @@ def test_evaluate_noalloc_from_two_threads(dp, orc):
         t.join(120)
     assert not any(t.is_alive() for t in ts), "a thread did not finish"
     assert not errors, errors
+
+
+def test_evaluate_noalloc_contexts_in_turn(dp, orc):
+    # contexts on one GPU launch on streams of their own, so a call may start while the launch of another context's call
+    # is still ending; every table here has several workgroups (2^12 entries and more), whose last one a counter tells
+    import threading
+
+    sizes, errors = (12, 13, 16), []
+    tabs = {k: (rand_e2(1 << k, 37000 + k), rand_e2(k, 37100 + k)) for k in sizes}
+    want = {k: orc.mle_evaluate(*tabs[k]) for k in sizes}
+    contexts = [dp.Context(0) for _ in range(3)]
+    mles = [{k: c.mle_from_ext2(tabs[k][0]) for k in sizes} for c in contexts]
+
+    def calls(which, count):
+        for it in range(count):
+            i, k = which[it % len(which)], sizes[it % 3]
+            got = mles[i][k].evaluate_noalloc(tabs[k][1])
+            if not (got == want[k]).all():
+                errors.append("context %d, 2^%d entries, call %d: %r != %r" % (i, k, it, got, want[k]))
+                return
+
+    calls([0, 1, 2], 300)
+    assert not errors, errors
+    ts = [threading.Thread(target=calls, args=([i], 300)) for i in range(3)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join(120)
+    assert not any(t.is_alive() for t in ts), "a thread did not finish"
+    assert not errors, errors
+    del mles
+    for c in contexts:
+        c.close()
