@@ -1581,6 +1581,7 @@ struct dps_sc {
     std::vector<Stage> stages;
     std::vector<u32> slice_ids;                // the tables of the resident launches (session indices), in slot order
     std::vector<dpk::SliceTerm> slice_terms;   // sums of several terms: the terms, their tables as slots of slice_ids
+    bool slice_shorter = false;                // ... some of the tables have fewer variables than the sum
     std::vector<uint8_t> round_kind;  // per round (1-based): 0 a launch of its own, 1 starts a trip, 2 starts a trip of two rounds, 3 second round of a trip,
                                       // 4 worked out on the host
     std::vector<uint8_t> round_wide;  // per round: its trip is made by several workgroups (whose counters run on from trip to trip): the sets of counters they add into
@@ -1726,17 +1727,35 @@ void tail_abort(dps_ctx *ctx)
 // result area of the resident product launches (dpk::SL_AREA_WORDS words of the pinned buffer, behind the areas of resident groups)
 size_t slice_area_off(const dps_ctx *ctx) { return ctx->pinned_words / 2 + 64 + 64 * 32; }
 
+// The sizes of a resident launch's arguments: a product's, and by its tables and terms a sum's (`shorter`: some table has fewer
+// variables than the sum)
+enum SliceSize { SLICE_PRODUCT, SLICE_FEW, SLICE_MANY };
+SliceSize slice_size(bool sum, size_t n_tabs, size_t n_terms, bool shorter)
+{
+    if (!sum) return SLICE_PRODUCT;
+    return n_tabs <= (size_t)dpk::SL_FEW_TABS && n_terms <= (size_t)dpk::SL_FEW_TERMS && !shorter ? SLICE_FEW : SLICE_MANY;
+}
+template <SliceSize SIZE>
+using SliceArgsFor = std::conditional_t<SIZE == SLICE_PRODUCT, dpk::SliceArgsProduct, std::conditional_t<SIZE == SLICE_FEW, dpk::SliceArgsFew, dpk::SliceArgs>>;
+template <int NF, bool EQ, SliceSize SIZE>
+constexpr auto slice_variant = &dpk::slice_kernel<NF, EQ, SIZE != SLICE_PRODUCT, dpk::SL_BLOCK, SliceArgsFor<SIZE>>;
+template <SliceSize SIZE>
+size_t slice_lds_bytes(u32 n_tabs, u32 cap, bool eq)
+{
+    return (size_t)dpk::slice_lds_words(n_tabs, cap, dpk::SL_BLOCK, eq, SliceArgsFor<SIZE>::TERMS) * 8;
+}
+
 // A workgroup of a resident launch may take most of a compute unit's LDS (it is alone there: 1024 threads); more than
 // 64 KB has to be asked for, once per kernel and device.  What a launch of this kernel can have, in bytes.
 constexpr u32 SLICE_LDS_DEFAULT = 64 * 1024, SLICE_LDS_LARGE = 160 * 1024;
-template <int NF, bool EQ, bool TERMS>
+template <int NF, bool EQ, SliceSize SIZE>
 u32 slice_lds_granted(dps_ctx *ctx)
 {
     static std::atomic<int> granted[64];  // 0 not asked, 1 granted, 2 refused
     std::atomic<int> &gr = granted[ctx->device & 63];
     int v = gr.load();
     if (v == 0) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&dpk::slice_kernel<NF, EQ, TERMS>), hipFuncAttributeMaxDynamicSharedMemorySize,
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(slice_variant<NF, EQ, SIZE>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                            (int)SLICE_LDS_LARGE);
         if (e != hipSuccess) (void)hipGetLastError();
         v = e == hipSuccess ? 1 : 2;
@@ -1745,62 +1764,68 @@ u32 slice_lds_granted(dps_ctx *ctx)
     return v == 1 ? SLICE_LDS_LARGE : SLICE_LDS_DEFAULT;
 }
 
-template <int NF, bool EQ, bool TERMS>
-void launch_slice(dps_ctx *ctx, u32 workgroups, u32 n_tabs, u32 cap, const dpk::SliceArgs &a)
-{
-    dpk::slice_kernel<NF, EQ, TERMS><<<workgroups, dpk::SL_BLOCK, dpk::slice_lds_words(n_tabs, cap, dpk::SL_BLOCK, EQ) * 8, ctx->stream>>>(a);
-}
-
 // the compiled variants: a product of 1 or 2 tables times eq, of 2 or 3 without; sums of several terms up to degree 4
-#define SLICE_VARIANTS(SK)                                                              \
-    SK(1, true, false) SK(2, true, false) SK(2, false, false) SK(3, false, false)       \
-    SK(1, true, true) SK(2, true, true) SK(3, true, true) SK(4, true, true)             \
-    SK(1, false, true) SK(2, false, true) SK(3, false, true) SK(4, false, true)
-int32_t launch_slice_dispatch(dps_ctx *ctx, bool terms, u32 nf, bool eq, u32 workgroups, u32 n_tabs, u32 cap, const dpk::SliceArgs &a)
+#define SLICE_SUM_VARIANTS(SK, SIZE_)                                                       \
+    SK(1, true, SIZE_) SK(2, true, SIZE_) SK(3, true, SIZE_) SK(4, true, SIZE_)             \
+    SK(1, false, SIZE_) SK(2, false, SIZE_) SK(3, false, SIZE_) SK(4, false, SIZE_)
+#define SLICE_VARIANTS(SK)                                                                                              \
+    SK(1, true, SLICE_PRODUCT) SK(2, true, SLICE_PRODUCT) SK(2, false, SLICE_PRODUCT) SK(3, false, SLICE_PRODUCT)       \
+    SLICE_SUM_VARIANTS(SK, SLICE_FEW) SLICE_SUM_VARIANTS(SK, SLICE_MANY)
+template <SliceSize SIZE>
+int32_t launch_slice(dps_ctx *ctx, u32 nf, bool eq, u32 workgroups, u32 n_tabs, u32 cap, const SliceArgsFor<SIZE> &a)
 {
-#define SK(NF_, EQ_, T_)                                                  \
-    if (terms == T_ && nf == NF_ && eq == EQ_) {                          \
-        launch_slice<NF_, EQ_, T_>(ctx, workgroups, n_tabs, cap, a);      \
-        return DPS_OK;                                                    \
-    }
+#define SK(NF_, EQ_, SIZE_)                                                                                                                     \
+    if constexpr (SIZE == SIZE_)                                                                                                                \
+        if (nf == NF_ && eq == EQ_) {                                                                                                           \
+            slice_variant<NF_, EQ_, SIZE_><<<workgroups, dpk::SL_BLOCK, slice_lds_bytes<SIZE_>(n_tabs, cap, EQ_), ctx->stream>>>(a);            \
+            return DPS_OK;                                                                                                                      \
+        }
     SLICE_VARIANTS(SK)
 #undef SK
-    return fail(ctx, DPS_ERR_UNSUPPORTED, "no resident kernel for degree %u, eq %d, several terms %d", nf, (int)eq, (int)terms);
+    return fail(ctx, DPS_ERR_UNSUPPORTED, "no resident kernel for degree %u, eq %d, several terms %d", nf, (int)eq, (int)(SIZE != SLICE_PRODUCT));
 }
 // Workgroups of a resident launch of the variant that one compute unit holds at once, with the LDS it is launched with
 // (the runtime's occupancy calculation; 0: such a workgroup does not fit, or no such variant).  Asked once per
 // variant, device and LDS size.
-template <int NF, bool EQ, bool TERMS>
+template <int NF, bool EQ, SliceSize SIZE>
 int slice_occupancy(dps_ctx *ctx, u32 n_tabs, u32 cap)
 {
     static std::mutex mu;
     static std::map<std::pair<int, size_t>, int> known;
-    const size_t lds = dpk::slice_lds_words(n_tabs, cap, dpk::SL_BLOCK, EQ) * 8;
+    const size_t lds = slice_lds_bytes<SIZE>(n_tabs, cap, EQ);
     std::lock_guard<std::mutex> lock(mu);
     auto it = known.find({ctx->device, lds});
     if (it != known.end()) return it->second;
     int n = 0;
-    if (lds > slice_lds_granted<NF, EQ, TERMS>(ctx) ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void *>(&dpk::slice_kernel<NF, EQ, TERMS>), (int)dpk::SL_BLOCK, lds) != hipSuccess) {
+    if (lds > slice_lds_granted<NF, EQ, SIZE>(ctx) ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void *>(slice_variant<NF, EQ, SIZE>), (int)dpk::SL_BLOCK, lds) != hipSuccess) {
         (void)hipGetLastError();
         n = 0;
     }
     known[{ctx->device, lds}] = n;
     return n;
 }
-int slice_workgroups_per_cu(dps_ctx *ctx, bool terms, u32 nf, bool eq, u32 n_tabs, u32 cap)
+int slice_workgroups_per_cu(dps_ctx *ctx, SliceSize size, u32 nf, bool eq, u32 n_tabs, u32 cap)
 {
-#define SK(NF_, EQ_, T_) \
-    if (terms == T_ && nf == NF_ && eq == EQ_) return slice_occupancy<NF_, EQ_, T_>(ctx, n_tabs, cap);
+#define SK(NF_, EQ_, SIZE_) \
+    if (size == SIZE_ && nf == NF_ && eq == EQ_) return slice_occupancy<NF_, EQ_, SIZE_>(ctx, n_tabs, cap);
     SLICE_VARIANTS(SK)
 #undef SK
     return 0;
 }
-// LDS a launch of the variant can have; 0: no such variant
-u32 slice_lds_limit(dps_ctx *ctx, bool terms, u32 nf, bool eq)
+// Most pairs a workgroup of the variant can take in its first round: its LDS holds twice as many entries per table and half
+// of that again.  0: no such variant
+template <int NF, bool EQ, SliceSize SIZE>
+u32 slice_pairs(dps_ctx *ctx, u32 n_tabs)
 {
-#define SK(NF_, EQ_, T_) \
-    if (terms == T_ && nf == NF_ && eq == EQ_) return slice_lds_granted<NF_, EQ_, T_>(ctx);
+    u32 cap = 4096;
+    while (cap > 2 && slice_lds_bytes<SIZE>(n_tabs, cap, EQ) > slice_lds_granted<NF, EQ, SIZE>(ctx)) cap >>= 1;
+    return cap / 2;
+}
+u32 slice_pairs_per_workgroup(dps_ctx *ctx, SliceSize size, u32 nf, bool eq, u32 n_tabs)
+{
+#define SK(NF_, EQ_, SIZE_) \
+    if (size == SIZE_ && nf == NF_ && eq == EQ_) return slice_pairs<NF_, EQ_, SIZE_>(ctx, n_tabs);
     SLICE_VARIANTS(SK)
 #undef SK
     return 0;
@@ -2117,15 +2142,7 @@ int32_t ensure_descs(dps_sc *sc)
 
 namespace {
 
-// Most pairs a workgroup of a resident launch can take in its first round: its LDS holds twice as many entries per table
-// and half of that again.
-u32 slice_pairs_per_workgroup(u32 n_tabs, bool eq, u32 lds_bytes)
-{
-    u32 cap = 4096;
-    while (cap > 2 && dpk::slice_lds_words(n_tabs, cap, dpk::SL_BLOCK, eq) * 8 > lds_bytes) cap >>= 1;
-    return cap / 2;
-}
-// ... and the fewest it is given when the sum is small enough for that: shorter chains of work per lane, more workgroups
+// The fewest pairs a workgroup of a resident launch is given when the sum is small enough for that: shorter chains of work per lane, more workgroups
 // (measured with 128, 64, 32, 16: 8 products over 16 tables 0.130, 0.119, 0.114, 0.111 ms; the fraction-tree proof 3.37, 3.30,
 // 3.28, 3.38 ms -- more workgroups cost little since their sums go into several sets of counters)
 constexpr u32 SLICE_MIN_PAIRS = 32;
@@ -2222,11 +2239,11 @@ void plan_resident_rounds(dps_sc *sc, u32 n_tabs, u32 n_mles)
         const E2 rho = sc->eq_info->point[round - 1];
         return !(rho.c0 == 0 && rho.c1 == 0);
     };
-    const u32 lds_bytes = slice_lds_limit(sc->ctx, sc->poly, sc->fast_nf, has_eq);
-    if (lds_bytes == 0) return;
+    const u32 pairs_fit = slice_pairs_per_workgroup(sc->ctx, slice_size(sc->poly, n_tabs, sc->slice_terms.size(), sc->slice_shorter), sc->fast_nf, has_eq, n_tabs);
+    if (pairs_fit == 0) return;
     // (more pairs per workgroup would make more rounds resident, but a trip's arithmetic is a workgroup's alone: with 512
     // pairs of a 3-term sum the first trip took 75 us where a launch for the round and a trip of 128 pairs take 66)
-    const u32 per_wg_max = std::min<u32>(slice_pairs_per_workgroup(n_tabs, has_eq, lds_bytes), sc->poly ? 128 : 512);
+    const u32 per_wg_max = std::min<u32>(pairs_fit, sc->poly ? 128 : 512);
     auto pairs_of = [&](u32 round) { return (u64)1 << (n - round); };
     u32 j = first_ok;
     while (pairs_of(j) > (u64)per_wg_max * SLICE_MAX_WORKGROUPS) j++;
@@ -2637,6 +2654,7 @@ int32_t SessionSetup::plan_and_ready_tables()
         for (u32 k : ids) ok = ok && !mles[k]->pad_vars;
         if (ok) {
             sc->slice_ids = ids;
+            for (u32 k : ids) sc->slice_shorter = sc->slice_shorter || nv0[k] != n_vars;
             for (const dps_term &t : sc->terms) {
                 dpk::SliceTerm tm;
                 memset(&tm, 0, sizeof tm);
@@ -2706,11 +2724,11 @@ int32_t SessionSetup::plan_and_ready_tables()
             }
             const u64 need = ((2ull << n_vars) - 1) & ~((1ull << first_level) - 1);
             CHK(eq_ensure(ctx, *sc->eq_info, const_cast<u64 *>(sc->eq_c0), const_cast<u64 *>(sc->eq_c1), need, sc->fast));
-        } else {
+        } else if (mles[k]->eq) {
             plain.push_back(mles[k]);
         }
     }
-    return eq_ready_many(ctx, plain);
+    return plain.empty() ? DPS_OK : eq_ready_many(ctx, plain);
 }
 
 int32_t SessionSetup::layout_scratch()
@@ -3734,6 +3752,8 @@ struct FusedRound {
     int32_t end_waiting_launch();
     bool admit_stages();
     int32_t launch_stages_at(u64 seq0, u32 first_go = 0);
+    template <SliceSize SIZE>
+    int32_t launch_stages_of(u64 seq0, u32 first_go);
     int32_t resident_round();
     Plan plan_round(u32 jj, bool skip1_jj) const;
     int32_t launch_round(u32 jj, const Plan &p, bool skip1_jj, bool ahead, u64 seq_jj);
@@ -3935,9 +3955,10 @@ int32_t FusedRound::end_waiting_launch()
 bool FusedRound::admit_stages()
 {
         u32 widest = 1;
+        const SliceSize size = slice_size(sc->poly, sc->slice_ids.size(), sc->slice_terms.size(), sc->slice_shorter);
         for (const dps_sc::Stage &st : sc->stages) {
             widest = std::max(widest, st.W);
-            if (slice_workgroups_per_cu(ctx, sc->poly, sc->fast_nf, sc->fast_eq >= 0, (u32)sc->slice_ids.size(), st.cap) < 1) return false;
+            if (slice_workgroups_per_cu(ctx, size, sc->fast_nf, sc->fast_eq >= 0, (u32)sc->slice_ids.size(), st.cap) < 1) return false;
         }
         return admit_waiting_launch(ctx, widest, true);
 }
@@ -3945,6 +3966,16 @@ bool FusedRound::admit_stages()
 // The launches of the resident rounds, queued one behind the other: the trip that starts at the first resident
 // round has the sequence number seq0 (a round's call takes one number whether or not it makes a trip).
 int32_t FusedRound::launch_stages_at(u64 seq0, u32 first_go)
+{
+        switch (slice_size(sc->poly, sc->slice_ids.size(), sc->slice_terms.size(), sc->slice_shorter)) {
+        case SLICE_PRODUCT: return launch_stages_of<SLICE_PRODUCT>(seq0, first_go);
+        case SLICE_FEW: return launch_stages_of<SLICE_FEW>(seq0, first_go);
+        default: return launch_stages_of<SLICE_MANY>(seq0, first_go);
+        }
+}
+
+template <SliceSize SIZE>
+int32_t FusedRound::launch_stages_of(u64 seq0, u32 first_go)
 {
         const u32 first = sc->tail_j0;
         // No resident launch of this context is running now: whatever an abandoned one left in the result area goes -- before
@@ -3957,7 +3988,7 @@ int32_t FusedRound::launch_stages_at(u64 seq0, u32 first_go)
             // the first workgroup takes the others' entries up and goes on alone
             const bool merged = st.W > 1 && si + 2 == sc->stages.size() && sc->stages[si + 1].W == 1 && sc->stages[si + 1].cap <= st.cap;
             const size_t last_si = merged ? si + 1 : si;
-            dpk::SliceArgs sa;
+            SliceArgsFor<SIZE> sa;
             memset(&sa, 0, sizeof sa);
             const u32 n_tabs = (u32)sc->slice_ids.size();
             for (u32 f = 0; f < n_tabs; f++) {
@@ -3973,7 +4004,7 @@ int32_t FusedRound::launch_stages_at(u64 seq0, u32 first_go)
                     const dpk::PolyTab &tb = sc->h_poly_groups[(size_t)(first - 1) * sc->poly_tabs.size() + g].tab[slot];
                     sa.s0[f] = tb.s0;
                     sa.s1[f] = tb.s1;
-                    if (tb.mode == dpk::POLY_BCAST || (tb.mode == dpk::POLY_PAIR && first > 1)) {
+                    if (SliceArgsFor<SIZE>::LACKS && (tb.mode == dpk::POLY_BCAST || (tb.mode == dpk::POLY_PAIR && first > 1))) {
                         // fewer variables than the round (POLY_BCAST: a pair's value is entry pair >> shift), or as many, not folded
                         sa.lacks[f] = (uint8_t)(tb.mode == dpk::POLY_BCAST ? tb.shift + 2 : 1);
                         sa.any_lacks = 1;
@@ -3993,7 +4024,7 @@ int32_t FusedRound::launch_stages_at(u64 seq0, u32 first_go)
             sa.hw0 = st.h0[n_tabs];
             sa.hw1 = st.h1[n_tabs];
             sa.n_tabs = n_tabs;
-            if (sc->poly) {
+            if (SIZE != SLICE_PRODUCT) {
                 sa.n_terms = (u32)sc->slice_terms.size();
                 std::copy(sc->slice_terms.begin(), sc->slice_terms.end(), sa.terms);
             }
@@ -4023,7 +4054,7 @@ int32_t FusedRound::launch_stages_at(u64 seq0, u32 first_go)
             sa.gate = reinterpret_cast<u32 *>(ctx->d_slice_ctr + SLICE_CTR_WORDS);
             sa.groups_log = slice_counter_sets_log(st.W);
             ProfScope ps(ctx, DPS_K_TAIL, 0.0);
-            CHK(launch_slice_dispatch(ctx, sc->poly, nf, has_eq, st.W, n_tabs, st.cap, sa));
+            CHK(launch_slice<SIZE>(ctx, nf, has_eq, st.W, n_tabs, st.cap, sa));
             HIPCHK(ctx, hipGetLastError());
             si = last_si;
         }

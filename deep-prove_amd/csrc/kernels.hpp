@@ -1522,10 +1522,14 @@ constexpr int SL_AREA_WORDS = SL_GROUP_WORDS * (int)SL_MAX_GROUPS + 32;
 constexpr int SL_WAITING_SLOT = SL_GROUP_WORDS * (int)SL_MAX_GROUPS, SL_HAD_SLOT = SL_WAITING_SLOT + 1;
 constexpr int SL_FIN_MAX_WORDS = 2048, SL_FIN_SEQ_SLOT = SL_FIN_MAX_WORDS, SL_FIN_CHK_SLOT = SL_FIN_MAX_WORDS + 1, SL_FIN_AREA_WORDS = SL_FIN_MAX_WORDS + 2;
 constexpr int SL_MAX_TRIPS = 32;
-// Tables and terms of a sum of several terms (a product has at most 3 tables).  What they cost a launch that does not use
-// them is the kernel arguments' copy; 32 tables of 64 pairs still fit a workgroup's LDS.
+// Tables and terms of a sum of several terms: 32 tables of 64 pairs still fit a workgroup's LDS.  They travel in the kernel
+// arguments, which the host clears and the runtime copies whatever of them is used, so there are three sizes of them: a
+// product's, and two for sums, of which only the larger one knows tables of fewer variables.  With one size for all (3.8 KB where
+// the smaller one has 1.6) a proof of 2^22 lookups of two columns, 24 such launches, took 3302 us; now 3265 (means of 16 processes).
 constexpr int SL_MAX_TABS = 32;
 constexpr int SL_MAX_TERMS = 64;
+constexpr int SL_FEW_TABS = 16;
+constexpr int SL_FEW_TERMS = 24;
 static_assert(2 * 4 * SL_MAX_TABS <= SL_FIN_MAX_WORDS, "the last entries of every table fit their area");
 // the check word's share of word i of that area
 __host__ __device__ __forceinline__ u64 sl_fin_mix(u64 word, u32 i) { return rotl64(word, (i & 31) + 1); }
@@ -1536,9 +1540,12 @@ struct SliceTerm {
     uint8_t slot[DPS_MAX_FACTORS];
     u32 pad;
 };
-struct SliceArgs {
-    const u64 *s0[SL_MAX_TABS];
-    const u64 *s1[SL_MAX_TABS];  // the tables before the folds that are pending when the launch starts: src_len entries each
+template <int TABS_, int TERMS_, bool LACKS_>
+struct SliceArgsOf {
+    static constexpr int TABS = TABS_, TERMS = TERMS_;
+    static constexpr bool LACKS = LACKS_;  // tables of fewer variables are among them
+    const u64 *s0[TABS];
+    const u64 *s1[TABS];         // the tables before the folds that are pending when the launch starts: src_len entries each
                                  // (nullptr: base-field entries; only tables nothing has folded yet are)
     u64 src_len;
     u32 pend0;         // folds pending at the first trip: 0 (the launch starts with round 1), 1, or 2
@@ -1564,33 +1571,36 @@ struct SliceArgs {
     u64 seq0;          // sequence number of the trip that starts at round j0; the one that starts at round j has seq0 + (j - j0)
     u64 *ctr;          // several workgroups: SL_MAX_GROUPS * 4 * SL_MAX_SUMS counters in device memory, SL_CTR_STRIDE words apart, zero when the launch starts
     u32 *gate;         // ... and the count of workgroups that have left their tables in h0 / h1 (zero when the launch starts)
-    u64 *h0[SL_MAX_TABS];  // where each workgroup leaves its last state (workgroup-major): for the first workgroup to go on with,
-    u64 *h1[SL_MAX_TABS];  // or (a launch that ends before the last round) for the launch queued behind this one
+    u64 *h0[TABS];         // where each workgroup leaves its last state (workgroup-major): for the first workgroup to go on with,
+    u64 *h1[TABS];         // or (a launch that ends before the last round) for the launch queued behind this one
     u64 *hw0, *hw1;        // ... and its eq weights (eq factor only; half as many entries), for the first workgroup to go on with
     // a sum of several terms (TERMS): the tables are those of all terms, the polynomial summed is sum_k coeff_k prod table
     u32 n_tabs, n_terms;
-    SliceTerm terms[SL_MAX_TERMS];
     // Tables of fewer variables than the round the launch starts with (they depend on the highest ones): 1 + the number of low
     // variables they lack.  No fold is pending on them; their entries are repeated as they are taken into LDS, and from then on
     // they are tables like the others (a fold of two equal entries is that entry).  0: a table that folds with the rest.
-    uint8_t lacks[SL_MAX_TABS];
     u32 any_lacks;
+    uint8_t lacks[TABS];
+    SliceTerm terms[TERMS];
 };
+using SliceArgs = SliceArgsOf<SL_MAX_TABS, SL_MAX_TERMS, true>;
+using SliceArgsFew = SliceArgsOf<SL_FEW_TABS, SL_FEW_TERMS, false>;
+using SliceArgsProduct = SliceArgsOf<4, 1, false>;  // (at most 3 tables, no terms)
 static_assert(sizeof(SliceArgs) <= 4096, "kernel arguments");
 
 // dynamic LDS of slice_kernel, in 64-bit words: counters per wavefront, mailbox copy, flags, the terms, then the two table buffers
-// (`blk`: threads of a workgroup)
+// (`blk`: threads of a workgroup, `terms`: room for them in the arguments)
 constexpr u32 SL_LDS_CTR = 0;
 __host__ __device__ constexpr u32 sl_lds_box(u32 blk) { return (blk / WAVE) * 4 * SL_MAX_SUMS; }
 __host__ __device__ constexpr u32 sl_lds_flags(u32 blk) { return sl_lds_box(blk) + 8; }
 __host__ __device__ constexpr u32 sl_lds_terms(u32 blk) { return sl_lds_flags(blk) + 2; }
-__host__ __device__ constexpr u32 sl_lds_tables(u32 blk) { return sl_lds_terms(blk) + SL_MAX_TERMS * (sizeof(SliceTerm) / 8); }
+__host__ __device__ constexpr u32 sl_lds_tables(u32 blk, u32 terms) { return sl_lds_terms(blk) + terms * (u32)(sizeof(SliceTerm) / 8); }
 static_assert(sizeof(SliceTerm) % 8 == 0, "terms are copied as 64-bit words");
 // (`eq`: the weights of the eq factor, one per pair of a table's entries, are kept like a table of half the size)
 __host__ __device__ constexpr u32 sl_weights_cap(u32 cap) { return cap / 2 > 0 ? cap / 2 : 1; }
-__host__ __device__ constexpr u32 slice_lds_words(u32 n_tabs, u32 cap, u32 blk, bool eq)
+__host__ __device__ constexpr u32 slice_lds_words(u32 n_tabs, u32 cap, u32 blk, bool eq, u32 terms = SL_MAX_TERMS)
 {
-    return sl_lds_tables(blk) + n_tabs * 2 * (cap + cap / 2) + (eq ? 2 * (sl_weights_cap(cap) + sl_weights_cap(cap / 2)) : 0);
+    return sl_lds_tables(blk, terms) + n_tabs * 2 * (cap + cap / 2) + (eq ? 2 * (sl_weights_cap(cap) + sl_weights_cap(cap / 2)) : 0);
 }
 // A workgroup of these launches is 1024 threads: what a round costs here is the longest chain of dependent field
 // multiplications in any one lane, and with more lanes each has fewer units of work behind one another.
@@ -1599,11 +1609,12 @@ constexpr int SL_PRE = 2;  // items (table, entry) a thread of a launch made ahe
 
 // NF: tables of the product, or with TERMS the largest number of factors of a term (the degree of the polynomial summed)
 // BLK: threads of a workgroup (SL_BLOCK in the library; the kernel's CPU test runs smaller ones)
-template <int NF, bool EQ, bool TERMS, int BLK = SL_BLOCK>
-__global__ void __launch_bounds__(BLK) slice_kernel(SliceArgs a)
+// ARGS: the size of the arguments
+template <int NF, bool EQ, bool TERMS, int BLK = SL_BLOCK, class ARGS = SliceArgs>
+__global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
 {
     constexpr int BLOCK = BLK;
-    constexpr u32 SL_LDS_BOX = sl_lds_box(BLK), SL_LDS_FLAGS = sl_lds_flags(BLK), SL_LDS_TERMS = sl_lds_terms(BLK), SL_LDS_TABLES = sl_lds_tables(BLK);
+    constexpr u32 SL_LDS_BOX = sl_lds_box(BLK), SL_LDS_FLAGS = sl_lds_flags(BLK), SL_LDS_TERMS = sl_lds_terms(BLK), SL_LDS_TABLES = sl_lds_tables(BLK, ARGS::TERMS);
     constexpr int NP = NF + 1;          // sums of the trip's first round: q(0..NF), q(1) left zero when it comes from the claim
     constexpr int NPT = NF;             // points of its second round: t = 0, 2, .., NF
     constexpr int NSMP = NF + 1;        // samples of that round's sums as a polynomial in the challenge: 0..NF-1, leading coefficient
@@ -1698,7 +1709,7 @@ __global__ void __launch_bounds__(BLK) slice_kernel(SliceArgs a)
         // but not yet its challenges: the entries this thread will fold are asked for before it waits for the mail, so
         // that they cross from device memory during the wait (up to SL_PRE items a thread; more are loaded after the mail).
         U64x2 pre[SL_PRE][4];
-        const bool have_pre = k == 0 && !a.first_go && pend >= 1 && (nt << len_log) <= (u32)(SL_PRE * BLOCK) && !(TERMS && a.any_lacks);
+        const bool have_pre = k == 0 && !a.first_go && pend >= 1 && (nt << len_log) <= (u32)(SL_PRE * BLOCK) && !(ARGS::LACKS && a.any_lacks);
         if (have_pre) {
             const u64 base = (u64)wg * src_each;
 #pragma unroll
@@ -1760,7 +1771,7 @@ __global__ void __launch_bounds__(BLK) slice_kernel(SliceArgs a)
                 const u32 f = u >> len_log, i = u & (len - 1);
                 const u64 *p0 = regroup ? a.h0[f] : a.s0[f], *p1 = regroup ? a.h1[f] : a.s1[f];
                 E2 v;
-                if (TERMS && k == 0 && a.any_lacks && a.lacks[f]) {
+                if (ARGS::LACKS && k == 0 && a.any_lacks && a.lacks[f]) {
                     const u64 e = ((base >> pend) + i) >> (a.lacks[f] - 1);
                     v = gl::e2(p0[e], p1 ? p1[e] : 0);
                 } else if (pend == 0) {

@@ -87,3 +87,21 @@ def test_many_tables_without_resident_launches(dp, ctx, orc, case):
         _check(dp, ctx, orc, n, gpu, host, terms)
     finally:
         dp.set_resident_budget(0, -1)
+
+
+@pytest.mark.parametrize("tables,n_terms,eq,short", [(16, 24, False, False), (17, 24, False, False), (16, 25, False, False), (16, 24, True, False),
+                                                     (17, 25, True, False), (4, 3, True, True), (16, 24, False, True)])
+def test_sizes_of_the_arguments(dp, ctx, orc, tables, n_terms, eq, short):
+    """A launch's arguments have room for 16 tables and 24 terms or for 32 and 64, and only the larger ones take tables of fewer
+    variables: sums on both sides, in one workgroup and in several."""
+    for n, deg in ((5, 2), (12, 2 if eq else 3)):
+        table_vars = [n] * tables
+        if short:
+            table_vars[1] = n - 2
+        gpu, host, terms = _instance(ctx, orc, 900 + tables + n_terms + n, table_vars, [0], n_terms, deg)
+        if eq:
+            rho = rand_e2(n, 950 + n)
+            gpu.append(ctx.eq_build(rho))
+            host.append(orc.eq_evals(rho))
+            terms = [(c, fs + [tables]) for c, fs in terms]
+        _check(dp, ctx, orc, n, gpu, host, terms)
