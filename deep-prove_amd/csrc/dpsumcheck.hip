@@ -4974,14 +4974,17 @@ extern "C" int32_t dps_logup_build_many(dps_ctx *ctx, const dps_logup_input *in,
     std::vector<std::unique_ptr<dps_logup>> trees(count);
     for (u32 i = 0; i < count; i++) CHK(logup_prepare(ctx, in[i], &trees[i]));
     // the first levels
-    dpk::LogupFirstBatch fb;
+    dpk::LogupFirstBatch<dpk::LOGUP_BATCH> fb;
     u32 n_first = 0;
     u64 most = 0;
     double bytes = 0;
     auto launch_first = [&]() -> int32_t {
         if (!n_first) return DPS_OK;
         ProfScope ps(ctx, DPS_K_LOGUP, bytes);
-        dpk::logup_first_kernel<<<dim3(grid_for(most), n_first), dpk::BLOCK, 0, ctx->stream>>>(fb);
+        if (n_first == 1)
+            dpk::logup_first_kernel<1><<<grid_for(most), dpk::BLOCK, 0, ctx->stream>>>(dpk::LogupFirstBatch<1>{{fb.tree[0]}});
+        else
+            dpk::logup_first_kernel<dpk::LOGUP_BATCH><<<dim3(grid_for(most), n_first), dpk::BLOCK, 0, ctx->stream>>>(fb);
         n_first = 0, most = 0, bytes = 0;
         HIPCHK(ctx, hipGetLastError());
         return DPS_OK;
@@ -5027,13 +5030,16 @@ extern "C" int32_t dps_logup_build_many(dps_ctx *ctx, const dps_logup_input *in,
         }
     }
     // the others
-    dpk::LogupTailBatch tb;
+    dpk::LogupTailBatch<dpk::LOGUP_BATCH> tb;
     u32 n_tail = 0;
     bytes = 0;
     auto launch_tails = [&]() -> int32_t {
         if (!n_tail) return DPS_OK;
         ProfScope ps(ctx, DPS_K_LOGUP, bytes);
-        dpk::logup_tail_kernel<<<n_tail, dpk::LOGUP_TAIL_BLOCK, 0, ctx->stream>>>(tb);
+        if (n_tail == 1)
+            dpk::logup_tail_kernel<1><<<1, dpk::LOGUP_TAIL_BLOCK, 0, ctx->stream>>>(dpk::LogupTailBatch<1>{{tb.tree[0]}});
+        else
+            dpk::logup_tail_kernel<dpk::LOGUP_BATCH><<<n_tail, dpk::LOGUP_TAIL_BLOCK, 0, ctx->stream>>>(tb);
         n_tail = 0, bytes = 0;
         HIPCHK(ctx, hipGetLastError());
         return DPS_OK;

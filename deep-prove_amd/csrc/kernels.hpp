@@ -3393,14 +3393,17 @@ struct LogupFirstArgs {
 
 // Several trees built together share the launch of their first levels and the launch of their last ones (a grid row, a
 // workgroup each): the last one is a chain of up to ten levels in one workgroup, 15 us by itself, and five trees of 2^7 .. 2^11
-// entries took five of them one behind the other (these batches with their table, proved and verified: 1621 -> 1568 us).
+// entries took five of them one behind the other (these batches with their table, proved and verified: 1621 -> 1568 us).  A tree by
+// itself has launches of its own size: with the arguments of eight a tree of 2^22 entries took 116.0 us instead of 114.6
 constexpr int LOGUP_BATCH = 8;
+template <int TREES>
 struct LogupFirstBatch {
-    LogupFirstArgs tree[LOGUP_BATCH];
+    LogupFirstArgs tree[TREES];
 };
-__global__ void __launch_bounds__(BLOCK) logup_first_kernel(LogupFirstBatch trees)
+template <int TREES>
+__global__ void __launch_bounds__(BLOCK) logup_first_kernel(LogupFirstBatch<TREES> trees)
 {
-    const LogupFirstArgs &a = trees.tree[blockIdx.y];
+    const LogupFirstArgs &a = trees.tree[TREES == 1 ? 0 : blockIdx.y];
     for (u64 i = (u64)blockIdx.x * BLOCK + threadIdx.x; i < a.half; i += (u64)gridDim.x * BLOCK) {
         // (the first column's power of the column challenge is 1: no product)
         E2 dlo = gl::e2(gl::add(a.c0, a.cols[0][i]), a.c1), dhi = gl::e2(gl::add(a.c0, a.cols[0][i + a.half]), a.c1);
@@ -3462,13 +3465,15 @@ struct LogupTailArgs {
     u64 seq;
     u64 *shadow;                        // host memory for the small levels (LOGUP_SHADOW_WORDS words), or nullptr
 };
+template <int TREES>
 struct LogupTailBatch {
-    LogupTailArgs tree[LOGUP_BATCH];
+    LogupTailArgs tree[TREES];
 };
-static_assert(sizeof(LogupFirstBatch) <= 4096 && sizeof(LogupTailBatch) <= 4096, "kernel arguments");
-__global__ void __launch_bounds__(LOGUP_TAIL_BLOCK) logup_tail_kernel(LogupTailBatch trees)
+static_assert(sizeof(LogupFirstBatch<LOGUP_BATCH>) <= 4096 && sizeof(LogupTailBatch<LOGUP_BATCH>) <= 4096, "kernel arguments");
+template <int TREES>
+__global__ void __launch_bounds__(LOGUP_TAIL_BLOCK) logup_tail_kernel(LogupTailBatch<TREES> trees)
 {
-    const LogupTailArgs &a = trees.tree[blockIdx.x];
+    const LogupTailArgs &a = trees.tree[TREES == 1 ? 0 : blockIdx.x];
     constexpr u32 CAP = 1u << LOGUP_TAIL_BITS;
     // numerators (two limb arrays) and denominators (two) of a level: CAP entries each in `big`, half of that in `small`
     __shared__ u64 big[4 * CAP], small_[2 * CAP];
