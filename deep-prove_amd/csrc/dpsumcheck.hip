@@ -150,10 +150,10 @@ size_t round_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 constexpr size_t SLICE_CTR_WORDS = (size_t)dpk::SL_MAX_GROUPS * dpk::SL_GROUP_WORDS * dpk::SL_CTR_STRIDE;  // counters of a resident launch, each apart
 // Behind the mail's copies: a ticket counter for each tile of outputs that several workgroups of a partial evaluation share.
 constexpr size_t AXIS_CTR_OFF = 256 + SLICE_CTR_WORDS * 8 + 256 + (size_t)dpk::MAIL_RELAY_WORDS * 8;
-constexpr u32 AXIS_TILES = 256;
+constexpr u32 AXIS_TILES = 1024;
 constexpr size_t COUNTER_BYTES = AXIS_CTR_OFF + AXIS_TILES * 4;
 static_assert(dpk::LOGUP_BATCH <= LOGUP_OUT_AREAS, "the trees of a launch leave their outputs apart");
-static_assert(AXIS_CTR_OFF % 8 == 0, "words and counters stay aligned");
+static_assert(AXIS_CTR_OFF % 8 == 0 && AXIS_TILES % 2 == 0, "words and counters stay aligned");
 
 constexpr int MAX_DEVICES = 64;
 
@@ -1216,10 +1216,16 @@ int32_t axis_point(dps_ctx *ctx, const AxisPointJob &j)
     a.waves_per_out = 1;
     if (col) {
         grid_x = a.P * ((a.C + dpk::WAVE - 1) / dpk::WAVE);
-        // A tile's k is shared out where the tiles alone leave compute units idle: 32 values a workgroup at least (eight a
-        // wavefront, all in flight together), about four workgroups a compute unit at most
+        // A tile's k is shared out where the tiles alone are fewer than four workgroups a compute unit, so that they become
+        // four: down to 32 values a workgroup (eight a wavefront, all in flight together) while there are fewer tiles than compute
+        // units, to 256 from there on, where the shares' way through memory counts.  Not shared, [1024 x 17000], [3072 x 16400] and
+        // [4096 x 20000] int64 (266, 257 and 313 tiles) took 111, 376 and 531 us with the call, shared 58, 144 and 194; [300 x
+        // 30000] (469 tiles) 47, and 57 when cut into shares of 100.
         u64 n_slices = 1;
-        if (grid_x <= AXIS_TILES) n_slices = std::min<u64>((a.K + 31) / 32, std::max<u64>(1, 4 * COMPUTE_UNITS / grid_x));
+        if (grid_x <= COMPUTE_UNITS)
+            n_slices = std::min<u64>((a.K + 31) / 32, 4 * COMPUTE_UNITS / grid_x);
+        else if (grid_x < AXIS_TILES)
+            n_slices = std::min<u64>(std::max<u64>(1, a.K / 256), (4 * COMPUTE_UNITS + grid_x - 1) / grid_x);
         a.k_per_slice = (a.K + n_slices - 1) / n_slices;
         a.n_slices = (u32)((a.K + a.k_per_slice - 1) / a.k_per_slice);
     } else {

@@ -44,6 +44,8 @@ CASES = (
     [((1, 70000), [C_, O_]), ((70000,), [O_]), ((2, 300000), [S_, O_]), ((4100, 600), [C_, O_]), ((4097, 33), [C_, O_]), ((70000, 31), [O_, C_])] +
     # more tiles than are shared, stacked rows with padding, several axes
     [((3, 40, 20000), [S_, O_, C_]), ((12, 197, 197), [S_, O_, C_]), ((12, 197, 64), [S_, C_, O_]), ((3, 5, 7, 9), [O_, S_, O_, C_]), ((33, 2, 40), [O_, C_, O_])] +
+    # tiles that are shared between workgroups, more than one a compute unit of them (257, 266), and that are not (few values; 1025)
+    [((512, 16448), [O_, C_]), ((520, 17000), [O_, C_]), ((300, 30000), [O_, C_]), ((40, 65600), [O_, C_])] +
     # nothing to contract
     [((1,), [C_]), ((768,), [C_]), ((3, 5, 100), [S_, C_, C_])]
 )
