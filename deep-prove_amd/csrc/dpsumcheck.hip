@@ -1212,9 +1212,15 @@ int32_t axis_point(dps_ctx *ctx, const AxisPointJob &j)
     const u64 outputs = a.P * a.C;
     // lanes over the outputs from half a wavefront of adjacent ones on, over k below
     const bool col = a.C >= 32;
+    // ... a thread an output for few values of many outputs, 4096 outputs for every value at least (int64 and extension entries, with
+    // the call, a thread an output and a tile of 64: 32 values of 131072 outputs 26.7 and 28.9 us, 28.4 and 34.0; 64 of 131072
+    // 43.2 and 37.9, 36.3 and 46.2; 64 of 262144 47.7 and 57.6, 56.1 and 69.8; 256 values are slower whatever the outputs)
+    const bool wide = col && a.K <= dpk::AXP_WIDE_MAX_K && outputs >= 4096 * a.K;
     u64 grid_x;
-    a.waves_per_out = 1;
-    if (col) {
+    a.waves_per_out = a.n_slices = 1;
+    if (wide) {
+        grid_x = std::min<u64>((outputs + dpk::BLOCK - 1) / dpk::BLOCK, 8 * COMPUTE_UNITS);
+    } else if (col) {
         grid_x = a.P * ((a.C + dpk::WAVE - 1) / dpk::WAVE);
         // A tile's k is shared out where the tiles alone are fewer than four workgroups a compute unit, so that they become
         // four: down to 32 values a workgroup (eight a wavefront, all in flight together) while there are fewer tiles than compute
@@ -1255,7 +1261,9 @@ int32_t axis_point(dps_ctx *ctx, const AxisPointJob &j)
         ProfScope ps(ctx, DPS_K_AXIS_DOT, (double)outputs * (double)a.K * (j.in1 ? 16.0 : j.in_int ? (double)j.in_int : 8.0) + (double)outputs * 16.0);
         auto launch = [&](auto kind) {
             constexpr int KIND = decltype(kind)::value;
-            if (col)
+            if (wide)
+                dpk::axis_point_wide_kernel<KIND><<<grid, dpk::BLOCK, 0, ctx->stream>>>(a);
+            else if (col)
                 dpk::axis_point_col_kernel<KIND><<<grid, dpk::BLOCK, 0, ctx->stream>>>(a);
             else
                 dpk::axis_point_row_kernel<KIND><<<grid, dpk::BLOCK, 0, ctx->stream>>>(a);

@@ -2711,16 +2711,16 @@ __global__ void __launch_bounds__(BLOCK) pad_tensor_kernel(PadTensorArgs a)
 }
 
 constexpr int AX_MAX_DIMS = 6;  // rank of a tensor
-// sum of coordinate times stride, `flat` counting the last dimension fastest
+// sum of coordinate times stride, `flat` (below the product of the dimensions) counting the last dimension fastest
 __device__ __forceinline__ u64 ax_offset(u64 flat, u32 n, const u64 *dims, const u64 *strides)
 {
     u64 off = 0;
-    for (int d = (int)n - 1; d >= 0; d--) {
-        u64 q = flat / dims[d];
+    for (int d = (int)n - 1; d >= 1; d--) {
+        const u64 q = flat / dims[d];
         off += (flat - q * dims[d]) * strides[d];
         flat = q;
     }
-    return off;
+    return n ? off + flat * strides[0] : 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -2916,6 +2916,7 @@ __global__ void __launch_bounds__(BLOCK) eval_point_kernel(EvalArgs a, FastFin f
 // unpadded region of a padded tensor is read in place.
 //   axis_point_col_kernel  lanes over the outputs (32 and more adjacent ones), a share of k a wavefront; where that leaves the
 //                          chip idle several workgroups share a tile of 64 outputs and the last one adds the partial sums.
+//   axis_point_wide_kernel a thread an output, for many outputs of few values each.
 //   axis_point_row_kernel  a wavefront, or the four of a workgroup, per output, lanes over k 512 at a time: an entry costs its
 //                          product with one of eight weights that all lanes share.  Several workgroups share a long row of
 //                          few outputs, as above.
@@ -3060,6 +3061,47 @@ __global__ void __launch_bounds__(BLOCK) axis_point_col_kernel(AxisPointArgs a)
     v = sum_waves(v);  // (take_ticket's barrier is behind the last reads of the area)
     if (wave == 0 && mine) axis_store(a, o, v);
     if (tid == 0) a.counters[blockIdx.x] = 0;
+}
+
+// Many outputs of few values: a thread sums an output's values by itself and the workgroup goes on to the next 256 outputs with the
+// weights it has made once.  (A tile of 64 outputs a workgroup makes the weights anew for each, and wavefronts without a
+// value of k idle.)  The highest variable of 2^24 base entries fixed: 415 -> 60 us with the call, of 2^20 extension entries
+// 62 -> 21; the highest four of 2^24 base entries 79 -> 44.  Bound: HBM (268 MB in the first of them, 54 us at the rate of a copy).
+constexpr u32 AXP_WIDE_MAX_K = 128;
+static_assert(AXP_WIDE_MAX_K <= BLOCK, "a weight a thread");
+template <int KIND>
+__global__ void __launch_bounds__(BLOCK) axis_point_wide_kernel(AxisPointArgs a)
+{
+    __shared__ PointGroups groups;
+    __shared__ u64 w0[AXP_WIDE_MAX_K], w1[AXP_WIDE_MAX_K], w2[KIND == 1 ? AXP_WIDE_MAX_K : 1];  // (prepared for extension entries)
+    const u32 tid = threadIdx.x, K = (u32)a.K;
+    const u64 outputs = a.P * a.C;
+    const u32 n_groups = point_groups(a.p, a.m, 0, groups);
+    axis_pads(a);
+    __syncthreads();
+    if (tid < K) {
+        const E2 v = point_weight(groups, 0, n_groups, tid);
+        w0[tid] = v.c0;
+        w1[tid] = v.c1;
+        if (KIND == 1) w2[tid] = gl::mul_small(v.c1, (u32)gl::W);
+    }
+    __syncthreads();
+    for (u64 o = (u64)blockIdx.x * BLOCK + tid; o < outputs; o += (u64)gridDim.x * BLOCK) {
+        const u64 pre = a.P == 1 ? 0 : o / a.C, i = o - pre * a.C;
+        const u64 base = ax_offset(pre, a.n_pre, a.pre_dims, a.pre_strides) + ax_offset(i, a.n_post, a.post_dims, a.post_strides);
+        gl::E2Acc s = gl::e2acc_zero();
+        constexpr u32 AHEAD = 8;  // entries in flight a thread
+        for (u32 k = 0; k < K; k += AHEAD) {
+            E2 v[AHEAD];
+#pragma unroll
+            for (u32 u = 0; u < AHEAD; u++)
+                if (k + u < K) v[u] = axis_entry<KIND>(a, base + (k + u) * a.stride_k);
+#pragma unroll
+            for (u32 u = 0; u < AHEAD; u++)
+                if (k + u < K) axis_acc<KIND>(s, v[u], gl::E2P{w0[k + u], w1[k + u], KIND == 1 ? w2[k + u] : 0});
+        }
+        axis_store(a, o, gl::acc_reduce(s));
+    }
 }
 
 template <int KIND>

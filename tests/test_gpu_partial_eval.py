@@ -46,8 +46,11 @@ CASES = (
     [((3, 40, 20000), [S_, O_, C_]), ((12, 197, 197), [S_, O_, C_]), ((12, 197, 64), [S_, C_, O_]), ((3, 5, 7, 9), [O_, S_, O_, C_]), ((33, 2, 40), [O_, C_, O_])] +
     # tiles that are shared between workgroups, more than one a compute unit of them (257, 266), and that are not (few values; 1025)
     [((512, 16448), [O_, C_]), ((520, 17000), [O_, C_]), ((300, 30000), [O_, C_]), ((40, 65600), [O_, C_])] +
+    # a thread an output: on both sides of 4096 outputs a value, with rows to pad, several axes, more outputs than a pass
+    [((1, 4095), [O_, C_]), ((1, 4096), [O_, C_]), ((2, 8191), [O_, C_]), ((2, 8193), [O_, C_]), ((9, 36865), [O_, C_]), ((30, 131000), [O_, C_]),
+     ((33, 135300), [O_, C_]), ((3, 600007), [O_, C_]), ((600, 4, 40), [C_, O_, C_]), ((300, 2, 33), [S_, O_, C_])] +
     # nothing to contract
-    [((1,), [C_]), ((768,), [C_]), ((3, 5, 100), [S_, C_, C_])]
+    [((3, 5, 5000), [S_, C_, C_]), ((1,), [C_]), ((768,), [C_]), ((3, 5, 100), [S_, C_, C_])]
 )
 
 
@@ -65,7 +68,7 @@ def test_shapes(ctx, orc, case):
                 assert (g.download() == w).all()
 
 
-@pytest.mark.parametrize("rows,cols", [(4, 8), (64, 32), (2, 1024), (512, 64)])
+@pytest.mark.parametrize("rows,cols", [(4, 8), (64, 32), (2, 1024), (512, 64), (4, 16384)])
 @pytest.mark.parametrize("first", [True, False])
 def test_field_tables(ctx, orc, rows, cols, first):
     """tables of either field, against the definition: sum_k in[k] eq(point, k)"""
