@@ -1216,10 +1216,16 @@ int32_t axis_point(dps_ctx *ctx, const AxisPointJob &j)
     // the call, a thread an output and a tile of 64: 32 values of 131072 outputs 26.7 and 28.9 us, 28.4 and 34.0; 64 of 131072
     // 43.2 and 37.9, 36.3 and 46.2; 64 of 262144 47.7 and 57.6, 56.1 and 69.8; 256 values are slower whatever the outputs)
     const bool wide = col && a.K <= dpk::AXP_WIDE_MAX_K && outputs >= 4096 * a.K;
+    // ... several outputs a wavefront where there are many of few values (rows of 64, 100 and 128 values, 2000, 5000 and 8000 of
+    // them, with the call: 24.7, 22.9 and 23.2 us, a wavefront an output 21.0, 26.5 and 30.4)
+    const u32 parts = !col && outputs >= 4096 ? (a.K <= 64 ? 1 : a.K <= 128 ? 2 : a.K <= 256 ? 4 : 0) : 0;
     u64 grid_x;
     a.waves_per_out = a.n_slices = 1;
     if (wide) {
         grid_x = std::min<u64>((outputs + dpk::BLOCK - 1) / dpk::BLOCK, 8 * COMPUTE_UNITS);
+    } else if (parts) {
+        const u64 per_block = (dpk::BLOCK / dpk::WAVE) * (8 / parts);
+        grid_x = std::min<u64>((outputs + per_block - 1) / per_block, 8 * COMPUTE_UNITS);
     } else if (col) {
         grid_x = a.P * ((a.C + dpk::WAVE - 1) / dpk::WAVE);
         // A tile's k is shared out where the tiles alone are fewer than four workgroups a compute unit, so that they become
@@ -1235,17 +1241,20 @@ int32_t axis_point(dps_ctx *ctx, const AxisPointJob &j)
         a.k_per_slice = (a.K + n_slices - 1) / n_slices;
         a.n_slices = (u32)((a.K + a.k_per_slice - 1) / a.k_per_slice);
     } else {
-        // the four wavefronts of a workgroup share an output of several steps while there are few outputs, and several
-        // workgroups one of many steps: four at least for each, about four workgroups a compute unit
+        // Wavefronts share an output of several steps, at most the four of a workgroup and at most a step each, while the
+        // workgroups of all outputs fit the chip together, eight a compute unit ([3000 x 3072] and [2500 x 1024] int64 with four
+        // wavefronts an output 56.2 and 35.8 us with the call, with two 47.8 and 28.5).  Several workgroups share one of
+        // many steps: four at least for each, about four workgroups a compute unit.
         const u64 steps = (a.K + (1u << dpk::AXP_ROW_BITS) - 1) >> dpk::AXP_ROW_BITS;
         if (steps > 0xffffffffull) return fail(ctx, DPS_ERR_UNSUPPORTED, "axis contraction too large");
-        if (steps > 1 && outputs < 4096) a.waves_per_out = dpk::BLOCK / dpk::WAVE;
+        constexpr u32 WAVES = dpk::BLOCK / dpk::WAVE;
+        while (a.waves_per_out < WAVES && 2 * a.waves_per_out <= steps && 2 * a.waves_per_out * outputs <= 8 * COMPUTE_UNITS * WAVES) a.waves_per_out *= 2;
         u64 n_slices = 1;
-        if (a.waves_per_out > 1 && outputs <= AXIS_TILES)
+        if (a.waves_per_out == WAVES && outputs <= AXIS_TILES)
             n_slices = std::min<u64>({(steps + 3) / 4, std::max<u64>(1, 4 * COMPUTE_UNITS / outputs), (u64)dpk::BLOCK});
         a.k_per_slice = (steps + n_slices - 1) / n_slices;
         a.n_slices = (u32)((steps + a.k_per_slice - 1) / a.k_per_slice);
-        grid_x = a.waves_per_out == 1 ? (outputs + dpk::BLOCK / dpk::WAVE - 1) / (dpk::BLOCK / dpk::WAVE) : outputs;
+        grid_x = (outputs + WAVES / a.waves_per_out - 1) / (WAVES / a.waves_per_out);
     }
     if (grid_x > 0x7fffffffull) return fail(ctx, DPS_ERR_UNSUPPORTED, "axis contraction too large");
     void *tmp = nullptr;
@@ -1263,6 +1272,12 @@ int32_t axis_point(dps_ctx *ctx, const AxisPointJob &j)
             constexpr int KIND = decltype(kind)::value;
             if (wide)
                 dpk::axis_point_wide_kernel<KIND><<<grid, dpk::BLOCK, 0, ctx->stream>>>(a);
+            else if (parts == 1)
+                dpk::axis_point_short_kernel<KIND, 1><<<grid, dpk::BLOCK, 0, ctx->stream>>>(a);
+            else if (parts == 2)
+                dpk::axis_point_short_kernel<KIND, 2><<<grid, dpk::BLOCK, 0, ctx->stream>>>(a);
+            else if (parts == 4)
+                dpk::axis_point_short_kernel<KIND, 4><<<grid, dpk::BLOCK, 0, ctx->stream>>>(a);
             else if (col)
                 dpk::axis_point_col_kernel<KIND><<<grid, dpk::BLOCK, 0, ctx->stream>>>(a);
             else

@@ -2917,7 +2917,8 @@ __global__ void __launch_bounds__(BLOCK) eval_point_kernel(EvalArgs a, FastFin f
 //   axis_point_col_kernel  lanes over the outputs (32 and more adjacent ones), a share of k a wavefront; where that leaves the
 //                          chip idle several workgroups share a tile of 64 outputs and the last one adds the partial sums.
 //   axis_point_wide_kernel a thread an output, for many outputs of few values each.
-//   axis_point_row_kernel  a wavefront, or the four of a workgroup, per output, lanes over k 512 at a time: an entry costs its
+//   axis_point_short_kernel several outputs a wavefront, for many outputs of few values that are not adjacent.
+//   axis_point_row_kernel  a wavefront, or two or the four of a workgroup, per output, lanes over k 512 at a time: an entry costs its
 //                          product with one of eight weights that all lanes share.  Several workgroups share a long row of
 //                          few outputs, as above.
 // Bound: the latency of a launch and of about ten field products at the sizes of a layer (3 to 19 MB), HBM above.  Through the
@@ -3112,7 +3113,7 @@ __global__ void __launch_bounds__(BLOCK) axis_point_row_kernel(AxisPointArgs a)
     __shared__ u64 lds[2 * (BLOCK / WAVE)];
     __shared__ int last_flag;
     const u32 tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
-    const u32 S = a.waves_per_out, sub = wave % S;  // 1 or 4
+    const u32 S = a.waves_per_out, sub = wave % S;  // 1, 2 or 4 (4 where several workgroups share an output)
     const u64 outputs = a.P * a.C, o = (u64)blockIdx.x * (BLOCK / WAVE / S) + wave / S;
     const bool mine = o < outputs;
     const u64 pre = (mine ? o : 0) / a.C, i = (mine ? o : 0) - pre * a.C;
@@ -3163,20 +3164,20 @@ __global__ void __launch_bounds__(BLOCK) axis_point_row_kernel(AxisPointArgs a)
         if (mine && lane == 0) axis_store(a, o, x);
         return;
     }
-    // the sum of the four wavefronts' values, valid in thread 0
-    auto sum_waves = [&](E2 y) {
+    // the sum of `count` wavefronts' values, valid in the first lane of the first of them
+    auto sum_waves = [&](E2 y, u32 count) {
         if (lane == 0) {
             lds[2 * wave] = y.c0;
             lds[2 * wave + 1] = y.c1;
         }
         __syncthreads();
-        if (tid == 0)
-            for (u32 q = 1; q < BLOCK / WAVE; q++) y = gl::add(y, gl::e2(lds[2 * q], lds[2 * q + 1]));
+        if (lane == 0 && wave % count == 0)
+            for (u32 q = wave + 1; q < wave + count; q++) y = gl::add(y, gl::e2(lds[2 * q], lds[2 * q + 1]));
         return y;
     };
-    x = sum_waves(x);
+    x = sum_waves(x, S);
     if (a.n_slices == 1) {
-        if (tid == 0) axis_store(a, o, x);
+        if (lane == 0 && sub == 0 && mine) axis_store(a, o, x);
         return;
     }
     if (tid == 0) {
@@ -3186,10 +3187,61 @@ __global__ void __launch_bounds__(BLOCK) axis_point_row_kernel(AxisPointArgs a)
     if (!take_ticket(a.counters + blockIdx.x, a.n_slices, &last_flag)) return;
     // (at most a share a thread)
     x = tid < a.n_slices ? gl::e2(ld_agent(a.part0 + (u64)tid * outputs + o), ld_agent(a.part1 + (u64)tid * outputs + o)) : gl::e2_zero();
-    x = sum_waves(sum_lanes(x));
+    x = sum_waves(sum_lanes(x), BLOCK / WAVE);
     if (tid == 0) {
         axis_store(a, o, x);
         a.counters[blockIdx.x] = 0;
+    }
+}
+
+// Many short rows: a wavefront sums 8 / PARTS outputs of up to 64 PARTS values at a time, their loads in flight together, and goes
+// on to its next ones with the weights it has made once; a lane's weights carry every coordinate, so an output is its products, one
+// reduction and its share of a sum over lanes that serves all of them.  (A step of 512 values an output was mostly work on zeros, and
+// every workgroup made the weights for four outputs.)  Rows of 64 int64 values, 100000 of them: 180 -> 54 us with the call, 20000
+// of 200: 55 -> 37.  Bound: HBM at the largest (51 MB, 10 us), the launch and the call at the others.
+template <int KIND, int PARTS>
+__global__ void __launch_bounds__(BLOCK) axis_point_short_kernel(AxisPointArgs a)
+{
+    constexpr u32 OUTS = 8 / PARTS;  // outputs a wavefront works on together
+    __shared__ PointGroups groups;
+    const u32 lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const u64 outputs = a.P * a.C;
+    const u32 n_groups = point_groups(a.p, a.m, AXP_ROW_BITS / 3, groups);
+    axis_pads(a);
+    __syncthreads();
+    gl::E2P w[PARTS];
+    {
+        const E2 of_lane = gl::mul(gl::mul(groups.at(0, lane & 7), groups.at(1, lane >> 3)), point_weight(groups, AXP_ROW_BITS / 3, n_groups, 0));
+#pragma unroll
+        for (u32 j = 0; j < (u32)PARTS; j++) w[j] = gl::prep(gl::mul(of_lane, groups.at(2, j)));
+    }
+    for (u64 first = ((u64)blockIdx.x * (BLOCK / WAVE) + wave) * OUTS; first < outputs; first += (u64)gridDim.x * (BLOCK / WAVE) * OUTS) {
+        E2 v[OUTS][PARTS];
+#pragma unroll
+        for (u32 q = 0; q < OUTS; q++) {
+            const u64 o = first + q < outputs ? first + q : first;
+            const u64 pre = a.C == 1 ? o : o / a.C, i = o - pre * a.C;
+            const u64 base = ax_offset(pre, a.n_pre, a.pre_dims, a.pre_strides) + ax_offset(i, a.n_post, a.post_dims, a.post_strides);
+#pragma unroll
+            for (u32 j = 0; j < (u32)PARTS; j++) {
+                const u64 k = WAVE * j + lane;
+                v[q][j] = k < a.K ? axis_entry<KIND>(a, base + k * a.stride_k) : gl::e2_zero();
+            }
+        }
+        u64 sums[2 * OUTS];
+#pragma unroll
+        for (u32 q = 0; q < OUTS; q++) {
+            gl::E2Acc s = gl::e2acc_zero();
+#pragma unroll
+            for (u32 j = 0; j < (u32)PARTS; j++) axis_acc<KIND>(s, v[q][j], w[j]);
+            const E2 x = gl::acc_reduce(s);
+            sums[2 * q] = x.c0, sums[2 * q + 1] = x.c1;
+        }
+        wave_sum_field<2 * OUTS>(sums);
+        if (lane == WAVE - 1)
+#pragma unroll
+            for (u32 q = 0; q < OUTS; q++)
+                if (first + q < outputs) axis_store(a, first + q, gl::e2(sums[2 * q], sums[2 * q + 1]));
     }
 }
 

@@ -49,6 +49,11 @@ CASES = (
     # a thread an output: on both sides of 4096 outputs a value, with rows to pad, several axes, more outputs than a pass
     [((1, 4095), [O_, C_]), ((1, 4096), [O_, C_]), ((2, 8191), [O_, C_]), ((2, 8193), [O_, C_]), ((9, 36865), [O_, C_]), ((30, 131000), [O_, C_]),
      ((33, 135300), [O_, C_]), ((3, 600007), [O_, C_]), ((600, 4, 40), [C_, O_, C_]), ((300, 2, 33), [S_, O_, C_])] +
+    # several outputs a wavefront: on both sides of 4096 outputs, of 64, 128 and 256 values, and adjacent outputs
+    [((c, k), [C_, O_]) for c, k in ((4095, 64), (4096, 64), (4097, 1), (70001, 64), (4099, 65), (4096, 128), (5000, 129), (4097, 256), (4096, 257))] +
+    [((2050, 100, 2), [S_, O_, C_]), ((137, 60, 31), [C_, O_, C_])] +
+    # one, two and four wavefronts an output of several steps
+    [((c, k), [C_, O_]) for c, k in ((300, 513), (2049, 2049), (2048, 2049), (3001, 1100), (4097, 513), (4095, 513))] +
     # nothing to contract
     [((3, 5, 5000), [S_, C_, C_]), ((1,), [C_]), ((768,), [C_]), ((3, 5, 100), [S_, C_, C_])]
 )
@@ -68,7 +73,7 @@ def test_shapes(ctx, orc, case):
                 assert (g.download() == w).all()
 
 
-@pytest.mark.parametrize("rows,cols", [(4, 8), (64, 32), (2, 1024), (512, 64), (4, 16384)])
+@pytest.mark.parametrize("rows,cols", [(4, 8), (64, 32), (2, 1024), (512, 64), (4, 16384), (4096, 8), (8192, 64), (4096, 256)])
 @pytest.mark.parametrize("first", [True, False])
 def test_field_tables(ctx, orc, rows, cols, first):
     """tables of either field, against the definition: sum_k in[k] eq(point, k)"""
