@@ -2680,7 +2680,7 @@ int32_t SessionSetup::plan_and_ready_tables()
             for (u32 k : g)
                 if (std::find(ids.begin(), ids.end(), k) == ids.end()) ids.push_back(k);
         bool ok = n_mles == ids.size() + (sc->fast_eq >= 0 ? 1 : 0) && ids.size() <= (size_t)dpk::SL_MAX_TABS;
-        for (u32 k : ids) ok = ok && !mles[k]->pad_vars;
+        for (u32 k : ids) ok = ok && !zpad_of(k);  // (a full-size table that is marked as padded is one like the others)
         if (ok) {
             sc->slice_ids = ids;
             for (u32 k : ids) sc->slice_shorter = sc->slice_shorter || nv0[k] != n_vars;
@@ -3140,12 +3140,16 @@ namespace {
 //     (2^17 entries; merging four claims on 2^20 entries: 450 -> 250 us), and wherever a sum has more tables than
 //     the resident launches take or zero-padded ones, which only the general launches read (a launch for every fold and 430 us a
 //     round for 67 tables);
-//   - by eq tables only in that last case: with zero-padded tables always, otherwise where it leaves at most eight products of
-//     fewer tables, or the tables are large, or their groups would not be resident side by side.
+//   - by eq tables only in that last case: with zero-padded tables always; otherwise where the products left, of fewer tables, fit a
+//     resident launch (up to 16 of them, and 60 and 132 tables of 2^7 .. 2^14 entries: 158 .. 428 us where the sum as it stands takes
+//     213 .. 964), or the tables are large (20 products of 60 and 132 tables, combined and as they stand: of 2^10 entries 395 and 358,
+//     481 and 491, of 2^12 429 and 468, 513 and 630), or their groups would not be resident side by side.
 struct CombinedTable {
     u32 factor;                                // X, or the eq table E_g
     std::vector<std::pair<u32, E2>> items;     // tables and coefficients
 };
+
+constexpr u32 COMBINE_MANY_MIN_VARS = 12;
 
 bool plan_combination(const dps_sc *sc, const dps_mle *const *mles, const std::vector<u32> &nv0, std::vector<CombinedTable> *plan)
 {
@@ -3186,10 +3190,7 @@ bool plan_combination(const dps_sc *sc, const dps_mle *const *mles, const std::v
     }
     if (any_zpad) return true;
     if (2 * plan->size() >= n_mles) return false;
-    if (n_vars >= 17 || 4 * plan->size() <= (size_t)dpk::SL_MAX_TABS) return true;
-    // More products than that are no faster in the resident launches than groups of tables resident side by side, which is how
-    // the sum as it stands runs while it has no more groups than fit (132 tables at 16 points: 0.40 ms as it stands,
-    // 0.43 combined; 60 tables at 8 points: 0.30 and 0.19).
+    if (n_vars >= COMBINE_MANY_MIN_VARS || 2 * plan->size() <= (size_t)dpk::SL_MAX_TABS) return true;
     size_t groups = 1;  // (as SessionSetup::group_terms cuts them)
     std::vector<u32> cur;
     for (const dps_term &t : sc->terms) {

@@ -25,13 +25,15 @@ def ctx(dp):
 
 
 class Sum:
-    def __init__(self, ctx, orc, n, seed):
-        self.ctx, self.orc, self.n, self.seed, self.rng = ctx, orc, n, seed, py_rng(seed)
+    def __init__(self, ctx, orc, n, seed, marked=False):
+        # (marked: full-size tables are zero-padded to their own size, as the opening of committed polynomials passes all of its tables)
+        self.ctx, self.orc, self.n, self.seed, self.rng, self.marked = ctx, orc, n, seed, py_rng(seed), marked
         self.gpu, self.host, self.terms, self.k = [], [], [], 0
 
     def _pad(self, v, h, m):
-        if m < self.n:
+        if m < self.n or self.marked:
             h = h.zero_pad(self.n)
+        if m < self.n:
             v = np.concatenate([v, np.zeros(((1 << self.n) - (1 << m), 2), dtype=np.uint64)])
         self.gpu.append(h)
         self.host.append(v)
@@ -164,4 +166,33 @@ def test_claims_at_many_points(dp, ctx, orc, n, polys, points):
     eqs = s.eqs([n] * points)
     for i, t in enumerate(tables):
         s.term(t, eqs[i % points])
+    s.check(dp)
+
+
+# full-size tables that carry the mark of padding run like the others: resident launches for the products that are left (up to 16
+# points; 17 as they stand, and from 2^12 entries on combined), and for a small sum as it stands
+@pytest.mark.parametrize("n,polys,points", [(6, 40, 4), (10, 40, 8), (10, 60, 15), (10, 60, 16), (10, 60, 17), (11, 60, 17), (12, 60, 17), (7, 60, 16), (9, 12, 4)])
+def test_marked_claims_at_several_points(dp, ctx, orc, n, polys, points):
+    s = Sum(ctx, orc, n, 9000 + n + points, marked=True)
+    tables = [s.table(base=i % 2 == 0) for i in range(polys)]
+    eqs = s.eqs([n] * points)
+    for i, t in enumerate(tables):
+        s.term(t, eqs[i * points // polys])
+    s.check(dp)
+    ctx.profile(True)
+    try:
+        ctx.profile_reset()
+        s.ctx.sumcheck_prove(s.n, s.gpu, s.terms, dp.Transcript(b"c"))
+        resident = ctx.profile_read()["tail"]["launches"]
+    finally:
+        ctx.profile(False)
+    assert (resident > 0) == (points <= 16), resident
+
+
+def test_marked_products_of_one_table(dp, ctx, orc):
+    s = Sum(ctx, orc, 13, 9500, marked=True)
+    x, y = s.table(base=True), s.table()
+    for e in s.eqs([13] * 2):
+        s.term(x, e)
+    s.term(x, y)
     s.check(dp)
