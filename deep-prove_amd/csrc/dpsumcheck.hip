@@ -3151,6 +3151,25 @@ struct CombinedTable {
 
 constexpr u32 COMBINE_MANY_MIN_VARS = 12;
 
+// Groups of tables a sum of products of two is cut into (as SessionSetup::group_terms cuts them)
+size_t groups_of_pairs(const dps_sc *sc)
+{
+    size_t groups = 1;
+    u32 cur[dpk::POLY_MAXT], n = 0;
+    for (const dps_term &t : sc->terms) {
+        u32 missing[2], m = 0;
+        for (u32 f = 0; f < 2; f++)
+            if (std::find(cur, cur + n, t.factors[f]) == cur + n) missing[m++] = t.factors[f];
+        if (n + m > (u32)dpk::POLY_MAXT) {
+            groups++;
+            n = 0, m = 2;
+            missing[0] = t.factors[0], missing[1] = t.factors[1];
+        }
+        for (u32 i = 0; i < m; i++) cur[n++] = missing[i];
+    }
+    return groups;
+}
+
 bool plan_combination(const dps_sc *sc, const dps_mle *const *mles, const std::vector<u32> &nv0, std::vector<CombinedTable> *plan)
 {
     const u32 n_vars = sc->n_vars, n_mles = sc->n_mles;
@@ -3179,31 +3198,28 @@ bool plan_combination(const dps_sc *sc, const dps_mle *const *mles, const std::v
         return true;
     }
     if (!too_many && !any_zpad) return false;
-    plan->clear();
-    std::map<u32, u32> at;
+    // by eq tables: whether to, from a count of them, before anything is written down
+    constexpr u32 NONE = ~0u;
+    std::vector<u32> place(n_mles, NONE);  // of the table among the eq tables of the terms
+    u32 n_eq = 0;
+    auto eq_factor = [&](const dps_term &t) { return is_eq(t.factors[1]) ? 1u : 0u; };
     for (const dps_term &t : sc->terms) {
-        const u32 f = is_eq(t.factors[1]) ? 1 : 0;
-        if (!is_eq(t.factors[f])) return false;
-        auto [it, is_new] = at.emplace(t.factors[f], (u32)plan->size());
-        if (is_new) plan->push_back(CombinedTable{t.factors[f], {}});
-        (*plan)[it->second].items.emplace_back(t.factors[f ^ 1], coeff_of(t));
+        const u32 k = t.factors[eq_factor(t)];
+        if (!is_eq(k)) return false;
+        if (place[k] == NONE) place[k] = n_eq++;
     }
-    if (any_zpad) return true;
-    if (2 * plan->size() >= n_mles) return false;
-    if (n_vars >= COMBINE_MANY_MIN_VARS || 2 * plan->size() <= (size_t)dpk::SL_MAX_TABS) return true;
-    size_t groups = 1;  // (as SessionSetup::group_terms cuts them)
-    std::vector<u32> cur;
+    if (!any_zpad) {
+        if (2 * n_eq >= n_mles) return false;
+        if (2 * n_eq > (u32)dpk::SL_MAX_TABS && n_vars < COMBINE_MANY_MIN_VARS && groups_of_pairs(sc) <= POLY_RAW_MAX_GROUPS) return false;
+    }
+    plan->assign(n_eq, CombinedTable{0, {}});
     for (const dps_term &t : sc->terms) {
-        std::vector<u32> merged = cur;
-        for (u32 f = 0; f < 2; f++)
-            if (std::find(merged.begin(), merged.end(), t.factors[f]) == merged.end()) merged.push_back(t.factors[f]);
-        if (merged.size() > (size_t)dpk::POLY_MAXT) {
-            groups++;
-            merged.assign(t.factors, t.factors + 2);
-        }
-        cur = merged;
+        const u32 f = eq_factor(t);
+        CombinedTable &c = (*plan)[place[t.factors[f]]];
+        c.factor = t.factors[f];
+        c.items.emplace_back(t.factors[f ^ 1], coeff_of(t));
     }
-    return groups > POLY_RAW_MAX_GROUPS;
+    return true;
 }
 
 // Carries the plan out: the tables M (and eq tables with their padding), and the session over them.
