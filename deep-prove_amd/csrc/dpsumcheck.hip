@@ -3473,15 +3473,14 @@ extern "C" int32_t dps_sc_begin(dps_ctx *ctx, uint32_t n_vars, const dps_mle *co
 
     if (std::vector<CombinedTable> plan; plan_combination(sc.get(), mles, nv0, &plan)) {
         bool fits = false;
-        if (const int32_t rc = combine_terms(ctx, sc.get(), mles, nv0, plan, &fits); rc != DPS_OK) {
-            drop_combined(sc.get());
-            return rc;
-        }
-        if (fits) {
+        const int32_t rc = combine_terms(ctx, sc.get(), mles, nv0, plan, &fits);
+        if (rc == DPS_OK && fits) {
             *out = sc.release();
             return DPS_OK;
         }
         drop_combined(sc.get());
+        // (where the tables made on the way do not fit beside the others the sum as it stands may)
+        if (rc != DPS_OK && rc != DPS_ERR_OOM) return rc;
     }
     if (const int32_t rc = su.run(); rc != DPS_OK) {
         pool_free(ctx, sc->scratch);

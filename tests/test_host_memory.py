@@ -1,0 +1,69 @@
+"""The library's host code without a device (tests/cpp/no_device.c): what a call does when an allocation fails."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    """runs statements in a process of their own in which `dp` is the package and `dev` the runtime without a device"""
+    cc = shutil.which("gcc") or shutil.which("cc")
+    if cc is None:
+        pytest.skip("no C compiler")
+    lib = tmp_path_factory.mktemp("no_device") / "no_device.so"
+    subprocess.check_call([cc, "-O1", "-Wall", "-Wextra", "-Werror", "-shared", "-fPIC", "-o", str(lib), os.path.join(ROOT, "tests", "cpp", "no_device.c")])
+
+    def go(body):
+        text = "import ctypes, importlib, sys\nimport numpy as np\n"
+        text += "dev = ctypes.CDLL(%r, ctypes.RTLD_GLOBAL)\n" % str(lib)  # (before the library: its calls are found here)
+        text += "for f in ('no_device_in_use', 'no_device_most'): getattr(dev, f).restype = ctypes.c_int64\n"
+        text += "dev.no_device_budget.argtypes = [ctypes.c_int64]\n"
+        text += "sys.path.insert(0, %r)\ndp = importlib.import_module('deep-prove_amd')\n" % ROOT + body
+        res = subprocess.run([sys.executable, "-c", text], stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True, timeout=300)
+        assert res.returncode == 0, res.stdout[-2000:] + res.stderr[-2000:]
+        assert "done" in res.stdout
+
+    return go
+
+
+def test_a_sum_that_is_rewritten_falls_back_when_the_new_tables_do_not_fit(run):
+    # X Y + X Z over 2^18 entries runs as X (Y + Z): more memory than the sum as it stands, which is taken where only it fits
+    run("""
+n = 18
+one = np.array([1, 0], dtype=np.uint64)
+def tables(ctx):
+    z = np.zeros((1 << n, 2), dtype=np.uint64)
+    return [ctx.mle_from_ext2(z) for _ in range(3)]
+terms = [(one, [0, 1]), (one, [0, 2])]
+ctx = dp.Context(0)
+tabs = tables(ctx)
+before = dev.no_device_in_use()
+dev.no_device_most_from_now()
+s = ctx.session(n, tabs, terms)
+rewritten = dev.no_device_most() - before
+assert rewritten > 0
+del s, tabs
+ctx.close()
+ctx = dp.Context(0)
+tabs = tables(ctx)
+before = dev.no_device_in_use()
+dev.no_device_budget(before + rewritten - 1)
+s = ctx.session(n, tabs, terms)
+as_it_stands = dev.no_device_most() - before
+assert s.degree == 2
+del s
+dev.no_device_budget(before)  # nothing fits beside the tables
+try:
+    s = ctx.session(n, tabs, terms)
+    raise SystemExit("a session without memory")
+except dp.DpsError as e:
+    assert e.status == 3, e  # out of memory
+dev.no_device_budget(1 << 60)
+s = ctx.session(n, tabs, terms)
+print("done")
+""")
