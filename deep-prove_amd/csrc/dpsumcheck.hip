@@ -3340,18 +3340,18 @@ int32_t combine_terms(dps_ctx *ctx, dps_sc *sc, const dps_mle *const *mles, cons
     return dps_sc_begin(ctx, n_vars, in_mles.data(), (u32)in_mles.size(), in_terms.data(), (u32)in_terms.size(), &sc->inner);
 }
 
-// The final evaluations of a sum whose rounds were another session's (combine_terms)
+// The final evaluations of a sum whose rounds were another session's (combine_terms): that session's end first, then a launch for
+// the tables other than eq tables, which runs while the host works out the eq tables.
 int32_t finish_combined(dps_sc *sc, const u64 *challenge, u64 *final_evals_out)
 {
     dps_ctx *ctx = sc->ctx;
-    sc->point.insert(sc->point.end(), challenge, challenge + 2);
     std::vector<u64> inner(2 * (size_t)std::max<u32>(sc->inner->n_mles, 1));
-    // Tables other than eq tables are evaluated on the GPU: the launch is queued before the inner session's end is looked
-    // at, unless that session still has a launch of its own to make
+    CHK(dps_sc_finish(sc->inner, challenge, inner.data()));
+    // (once: a session that has ended refuses to end again)
+    sc->point.insert(sc->point.end(), challenge, challenge + 2);
     std::vector<const dps_sc::Outside *> dev;
     for (const dps_sc::Outside &o : sc->outside)
         if (!o.eq) dev.push_back(&o);
-    CHK(dps_sc_finish(sc->inner, challenge, inner.data()));
     u64 seq = 0;
     if (!dev.empty()) {
         u32 most = 0;
