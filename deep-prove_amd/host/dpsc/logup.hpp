@@ -59,31 +59,34 @@ struct LogUpInput {
 // above live in one GPU arena built by dps_logup_build_many.
 class LogUpCircuit {
 public:
+    // what a circuit is built from: columns, multiplicities (a table's) and the two challenges
+    struct Instance {
+        std::vector<const DensePolynomial *> cols;
+        const DensePolynomial *mult;
+        F c, beta;
+    };
     LogUpCircuit(const Context &ctx, std::vector<const DensePolynomial *> cols, const DensePolynomial *mult, const F &c, const F &beta)
-        : ctx_(&ctx), cols_(std::move(cols)), mult_(mult), c_(c), beta_(beta)
+        : LogUpCircuit(std::move(build(ctx, {Instance{std::move(cols), mult, c, beta}})[0]))
     {
     }
-    // the fraction trees of all circuits of a batch
-    static void build(const Context &ctx, std::vector<LogUpCircuit> &circuits)
+    // the circuits of a batch, their fraction trees built together
+    static std::vector<LogUpCircuit> build(const Context &ctx, std::vector<Instance> instances)
     {
         std::vector<std::vector<const dps_mle *>> cols;
         std::vector<dps_logup_input> in;
-        for (auto &q : circuits) {
+        for (auto &q : instances) {
             cols.emplace_back();
-            for (auto *p : q.cols_) cols.back().push_back(p->raw());
+            for (auto *p : q.cols) cols.back().push_back(p->raw());
         }
-        for (size_t i = 0; i < circuits.size(); i++) {
-            const LogUpCircuit &q = circuits[i];
-            in.push_back(dps_logup_input{cols[i].data(), (uint32_t)cols[i].size(), q.mult_ ? q.mult_->raw() : nullptr, {q.c_.c0, q.c_.c1}, {q.beta_.c0, q.beta_.c1}});
+        for (size_t i = 0; i < instances.size(); i++) {
+            const Instance &q = instances[i];
+            in.push_back(dps_logup_input{cols[i].data(), (uint32_t)cols[i].size(), q.mult ? q.mult->raw() : nullptr, {q.c.c0, q.c.c1}, {q.beta.c0, q.beta.c1}});
         }
         std::vector<dps_logup *> h(in.size(), nullptr);
         ctx.check(dps_logup_build_many(ctx.raw(), in.data(), (uint32_t)in.size(), h.data()), "dps_logup_build");
-        for (size_t i = 0; i < circuits.size(); i++) {
-            circuits[i].h_.reset(h[i], &dps_logup_free);
-            uint32_t nl = 0;
-            dps_logup_num_layers(h[i], &nl);
-            circuits[i].n_layers_ = nl;
-        }
+        std::vector<LogUpCircuit> circuits;
+        for (size_t i = 0; i < instances.size(); i++) circuits.push_back(LogUpCircuit(ctx, std::move(instances[i]), h[i]));
+        return circuits;
     }
     // variables of the sumcheck over the input layer (circuit.rs:67-80,564-566)
     size_t num_vars() const { return n_layers_ - 1; }
@@ -171,6 +174,13 @@ public:
     }
 
 private:
+    LogUpCircuit(const Context &ctx, Instance in, dps_logup *tree)
+        : ctx_(&ctx), cols_(std::move(in.cols)), mult_(in.mult), c_(in.c), beta_(in.beta), h_(tree, &dps_logup_free)
+    {
+        uint32_t nl = 0;
+        ctx.check(dps_logup_num_layers(tree, &nl), "dps_logup_num_layers");
+        n_layers_ = nl;
+    }
     const Context *ctx_;
     std::vector<const DensePolynomial *> cols_;
     const DensePolynomial *mult_;
@@ -206,19 +216,19 @@ inline LogUpBatchProof new_batch_multiple_sizes_prove(const Context &ctx, const 
 {
     if (input.empty()) throw Error(DPS_ERR_INVALID, "No inputs provided for LogUp");
     const ProofType proof_type = input[0].type;
-    std::vector<LogUpCircuit> circuits;
+    std::vector<LogUpCircuit::Instance> instances;
     for (auto &in : input) {
         if (in.type != proof_type) throw Error(DPS_ERR_INVALID, "Not all proof types matched");
         if (in.type == ProofType::Table) {
-            circuits.emplace_back(ctx, in.column_evals, in.multiplicities, in.constant_challenge, in.column_separation_challenge);
+            instances.push_back({in.column_evals, in.multiplicities, in.constant_challenge, in.column_separation_challenge});
         } else {
             for (size_t i = 0; i < in.column_evals.size(); i += in.columns_per_instance) {
                 std::vector<const DensePolynomial *> cols(in.column_evals.begin() + i, in.column_evals.begin() + i + in.columns_per_instance);
-                circuits.emplace_back(ctx, cols, nullptr, in.constant_challenge, in.column_separation_challenge);
+                instances.push_back({cols, nullptr, in.constant_challenge, in.column_separation_challenge});
             }
         }
     }
-    LogUpCircuit::build(ctx, circuits);
+    std::vector<LogUpCircuit> circuits = LogUpCircuit::build(ctx, std::move(instances));
     const size_t num_instances = circuits.size();
     size_t total_layers = circuits[0].num_vars();
     for (size_t i = 1; i < circuits.size(); i++) {

@@ -1,4 +1,5 @@
-"""The library's host code without a device (tests/cpp/no_device.c): what a call does when an allocation fails."""
+"""The library's host code without a device (tests/cpp/no_device.c): what a call does when an allocation fails, and objects of the
+host mirror that need a context but no result."""
 import os
 import shutil
 import subprocess
@@ -10,17 +11,22 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 @pytest.fixture(scope="module")
-def run(tmp_path_factory):
-    """runs statements in a process of their own in which `dp` is the package and `dev` the runtime without a device"""
+def no_device(tmp_path_factory):
     cc = shutil.which("gcc") or shutil.which("cc")
     if cc is None:
         pytest.skip("no C compiler")
-    lib = tmp_path_factory.mktemp("no_device") / "no_device.so"
+    lib = tmp_path_factory.mktemp("no_device") / "libno_device.so"
     subprocess.check_call([cc, "-O1", "-Wall", "-Wextra", "-Werror", "-shared", "-fPIC", "-o", str(lib), os.path.join(ROOT, "tests", "cpp", "no_device.c")])
+    return lib
+
+
+@pytest.fixture(scope="module")
+def run(no_device):
+    """runs statements in a process of their own in which `dp` is the package and `dev` the runtime without a device"""
 
     def go(body):
         text = "import ctypes, importlib, sys\nimport numpy as np\n"
-        text += "dev = ctypes.CDLL(%r, ctypes.RTLD_GLOBAL)\n" % str(lib)  # (before the library: its calls are found here)
+        text += "dev = ctypes.CDLL(%r, ctypes.RTLD_GLOBAL)\n" % str(no_device)  # (before the library: its calls are found here)
         text += "for f in ('no_device_in_use', 'no_device_most'): getattr(dev, f).restype = ctypes.c_int64\n"
         text += "dev.no_device_budget.argtypes = [ctypes.c_int64]\n"
         text += "sys.path.insert(0, %r)\ndp = importlib.import_module('deep-prove_amd')\n" % ROOT + body
@@ -67,3 +73,12 @@ dev.no_device_budget(1 << 60)
 s = ctx.session(n, tabs, terms)
 print("done")
 """)
+
+
+def test_a_logup_circuit_is_complete_as_its_constructor_leaves_it(no_device, tmp_path):
+    exe, lib = tmp_path / "test_logup_circuit", os.path.join(ROOT, "deep-prove_amd", "lib")
+    # (linked before the library: its calls are found in the runtime without a device)
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-o", str(exe), os.path.join(ROOT, "tests", "cpp", "test_logup_circuit.cpp"), "-Wl,--no-as-needed",
+                           "-L" + str(no_device.parent), "-lno_device", "-L" + lib, "-ldpsumcheck", "-Wl,-rpath," + str(no_device.parent) + ":" + lib])
+    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert out.returncode == 0 and "ok" in out.stdout, out.stdout + out.stderr
