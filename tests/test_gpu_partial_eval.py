@@ -52,6 +52,8 @@ CASES = (
     # several outputs a wavefront: on both sides of 4096 outputs, of 64, 128 and 256 values, and adjacent outputs
     [((c, k), [C_, O_]) for c, k in ((4095, 64), (4096, 64), (4097, 1), (70001, 64), (4099, 65), (4096, 128), (5000, 129), (4097, 256), (4096, 257))] +
     [((2050, 100, 2), [S_, O_, C_]), ((137, 60, 31), [C_, O_, C_])] +
+    # a second contraction, of the first one's extension entries, over rows that several workgroups share and over tiles that they share
+    [((2, 3000, 5), [C_, O_, O_]), ((1, 70000, 3), [C_, O_, O_]), ((3, 700, 40), [O_, O_, C_]), ((300, 40, 3), [O_, C_, O_])] +
     # one, two and four wavefronts an output of several steps
     [((c, k), [C_, O_]) for c, k in ((300, 513), (2049, 2049), (2048, 2049), (3001, 1100), (4097, 513), (4095, 513))] +
     # nothing to contract
@@ -92,6 +94,28 @@ def test_field_tables(ctx, orc, rows, cols, first):
             for a, b in zip(line, eq):
                 want = orc.e2_add(want, orc.e2_mul(a, b))
             assert (got[i] == want).all()
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 4096), (2, 65536), (8, 8192), (1, 1 << 18)])
+@pytest.mark.parametrize("ext", [False, True])
+def test_long_rows_of_field_tables(ctx, orc, rows, cols, ext):
+    """rows that several workgroups share, of base and extension entries: a row's value is its evaluation at the point"""
+    point = rand_e2(cols.bit_length() - 1, 81)
+    v = rand_e2(rows * cols, 82 + rows) if ext else orc.embed_base(rand_base(rows * cols, 83 + rows))
+    table = ctx.mle_from_ext2(v) if ext else ctx.mle_from_base(v[:, 0].copy())
+    got = ctx.partial_eval(table, [rows, cols], [rows, cols], [C_, O_], [None, point])[0].download()
+    for r in range(rows):
+        assert (got[r] == orc.mle_evaluate(v[r * cols:(r + 1) * cols], point)).all()
+
+
+@pytest.mark.parametrize("n,rest", [(12, 0), (14, 2), (17, 4), (18, 1), (13, 5), (16, 15), (18, 13)])
+@pytest.mark.parametrize("ext", [False, True])
+def test_fix_high_down_to_a_few_entries(ctx, orc, n, rest, ext):
+    v = rand_e2(1 << n, 91 + n) if ext else orc.embed_base(rand_base(1 << n, 92 + n))
+    point = rand_e2(n - rest, 93 + rest)
+    table = ctx.mle_from_ext2(v) if ext else ctx.mle_from_base(v[:, 0].copy())
+    got = table.fix_high(point).download()
+    assert (got == orc.mle_fix_high(v, point)).all()
 
 
 def test_points_are_checked(dp, ctx):
