@@ -102,6 +102,7 @@ struct Term {
 // library works them out on the host): its last trip ends before them and hands over that many more entries.
 static bool g_two_behind = false;  // the first launch's sources are two folds behind its first round (as behind a launch that covered two rounds)
 static bool g_first_go = false;  // launches that start with round 1 are told at once whether t = 1 is evaluated, and get no first mail
+static std::vector<u32> g_lacks;  // per table, tables of fewer variables: 1 + how many low ones they lack at the first round (0: none of this)
 template <int NF, bool EQ, bool TERMS = false>
 static void run_case(const char *name, u32 n_vars, u32 j0, u32 wide, u32 n_tabs_in, std::vector<u32> single_rounds = {}, std::vector<Term> terms = {},
                      u32 base_tabs = 0, bool separate = false, u32 host_rounds = 0)
@@ -124,6 +125,17 @@ static void run_case(const char *name, u32 n_vars, u32 j0, u32 wide, u32 n_tabs_
     std::vector<Table> ref(NT, Table((size_t)1 << (n_vars - j0 + 1 + first_pend)));
     for (u32 f = 0; f < NT; f++)
         for (auto &x : ref[f]) x = f < base_tabs ? gl::e2(felt(), 0) : felt2();
+    // a table of fewer variables: what the launch reads, and in the reference the same entries repeated
+    std::vector<std::vector<u64>> short0(NT), short1(NT);
+    for (u32 f = 0; f < NT && !g_lacks.empty(); f++) {
+        if (!g_lacks[f]) continue;
+        const u32 shift = first_pend + g_lacks[f] - 1;
+        for (size_t i = 0; i < ref[f].size() >> shift; i++) {
+            const E2 x = f < base_tabs ? gl::e2(felt(), 0) : felt2();
+            short0[f].push_back(x.c0), short1[f].push_back(x.c1);
+        }
+        for (size_t i = 0; i < ref[f].size(); i++) ref[f][i] = gl::e2(short0[f][i >> shift], short1[f][i >> shift]);
+    }
     std::vector<E2> chal(n_vars + 1);
     for (auto &c : chal) c = felt2();
     // eq storage: level l at (2 << n) - (2 << (n - l)), eq(rho_{l..n-1}, .)
@@ -216,6 +228,12 @@ static void run_case(const char *name, u32 n_vars, u32 j0, u32 wide, u32 n_tabs_
             a.s0[f] = d0[f].data();
             // a table nothing has folded yet may be a base-field one (no second limb array)
             a.s1[f] = (si == 0 && f < base_tabs) ? nullptr : d1[f].data();
+            if (si == 0 && !short0[f].empty()) {
+                a.s0[f] = short0[f].data();
+                a.s1[f] = f < base_tabs ? nullptr : short1[f].data();
+                a.lacks[f] = (uint8_t)g_lacks[f];
+                a.any_lacks = 1;
+            }
             h0[f].assign(st.src_len, 0);
             h1[f].assign(st.src_len, 0);
             a.h0[f] = h0[f].data();
@@ -495,6 +513,17 @@ int main()
     run_case<2, false>("two tables from round 1, t = 1 evaluated in round 1, first trip without mail", 8, 1, 1, 0, {1, 4});
     run_case<2, false, true>("16 tables, 8 products, from round 1, first trip without mail", 8, 1, 1, 16, {}, stacked, 0, false, 2);
     g_first_go = false;
+    // tables of fewer variables, one short of them down to a single entry, base-field ones among them
+    g_lacks = {0, 1, 3, 0, 8};
+    run_case<3, false, true>("tables of fewer variables, from round 1", 7, 1, 1, 5, {}, {Term{felt2(), {0, 1, 2}}, Term{felt2(), {3, 4}}, Term{felt2(), {2}}}, 2);
+    g_lacks = {2, 0, 1, 4, 0};
+    run_case<2, true, true>("the same with eq over 4 workgroups, from round 2", 10, 2, 4, 5, {}, {Term{felt2(), {0, 1}}, Term{felt2(), {2, 3}}, Term{felt2(), {4, 4}}}, 1);
+    g_lacks.assign(32, 0);
+    for (u32 f = 0; f < 32; f += 3) g_lacks[f] = 1 + f % 4;
+    std::vector<Term> wide_sum;
+    for (u32 i = 0; i < 64; i++) wide_sum.push_back(Term{felt2(), {i % 32, (7 * i + 5) % 32}});
+    run_case<2, false, true>("32 tables, 64 terms, some of fewer variables, the last round left out", 5, 1, 1, 32, {}, wide_sum, 0, false, 1);
+    g_lacks.clear();
     printf("%s\n", failures ? "FAILED" : "all cases ok");
     return failures ? 1 : 0;
 }

@@ -1,5 +1,5 @@
 """The hot kernels' bodies on the CPU under the host sanitizers (tests/cpp/emu_prod_kernel.cpp, tests/cpp/emu_slice_kernel.cpp,
-tests/cpp/emu_poly_kernel.cpp): no GPU involved.  The three programs are built and run side by side (a build under the
+tests/cpp/emu_poly_kernel.cpp, tests/cpp/emu_point_kernels.cpp): no GPU involved.  The programs are built and run side by side (a build under the
 sanitizers takes over a minute), once per test session; each test then reads its program's outcome."""
 import os
 import shutil
@@ -11,7 +11,8 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CLANG = "/opt/rocm/llvm/bin/clang++"
 needs_clang = pytest.mark.skipif(not os.path.exists(CLANG), reason="needs clang (ext_vector_type, -ftrivial-auto-var-init)")
 
-PROGRAMS = {"prod": ("emu_prod_kernel.cpp", ["quick"]), "slice": ("emu_slice_kernel.cpp", []), "poly": ("emu_poly_kernel.cpp", [])}
+PROGRAMS = {"prod": ("emu_prod_kernel.cpp", ["quick"]), "slice": ("emu_slice_kernel.cpp", []), "poly": ("emu_poly_kernel.cpp", []),
+            "point": ("emu_point_kernels.cpp", [])}
 
 
 @pytest.fixture(scope="module")
@@ -29,7 +30,7 @@ def outcomes(tmp_path_factory):
         build = " ".join([CLANG, "-std=c++17", "-O1", "-g", "-fsanitize=address,undefined", "-fno-sanitize-recover=undefined",
                           "-ftrivial-auto-var-init=pattern", "-I", str(tmp_path), "-I", os.path.join(ROOT, "tests", "cpp", "emu"),
                           "-I", os.path.join(ROOT, "include"), "-pthread", "-o", str(exe), os.path.join(ROOT, "tests", "cpp", source)])
-        # build, then run, in one shell per program: the three go on side by side
+        # build, then run, in one shell per program: they go on side by side
         procs[name] = subprocess.Popen(["bash", "-c", build + " && exec " + " ".join([str(exe)] + args)], stdout=subprocess.PIPE,
                                        stderr=subprocess.PIPE, text=True)
     out = {}
@@ -67,3 +68,9 @@ def test_poly_kernel_body_under_host_sanitizers(outcomes):
     # sums of several terms over shared tables: term by term and as a nested program, a pair's work over 1, 4 and 16 lanes,
     # many groups, launches made ahead, factored eq weights, a launch that stays for every remaining round
     _check(outcomes["poly"])
+
+
+@needs_clang
+def test_point_kernel_bodies_under_host_sanitizers(outcomes):
+    # partial evaluations, evaluations at a point, combined tables: every kernel that takes its weights from a point
+    _check(outcomes["point"])
