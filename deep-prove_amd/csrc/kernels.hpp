@@ -2923,8 +2923,8 @@ __global__ void __launch_bounds__(BLOCK) eval_point_kernel(EvalArgs a, FastFin f
 //                          few outputs, as above.
 // Bound: the latency of a launch and of about ten field products at the sizes of a layer (3 to 19 MB), HBM above.  Through the
 // eq table, a contraction, a sum over its shares and a launch for the padding, each started when the one before had
-// ended, a tensor took about 22 us of kernels and as much of gaps and launch calls.  [512 x 768] int64 14.6 us and [768 x 3072]
-// int64 12.5 us (kernel trace); proofs of that product 114 -> 91 us, of one row of it 159 -> 102 us, of both products of an
+// ended, a tensor took about 22 us of kernels and as much of gaps and launch calls.  [512 x 768] int64 13.9 us and [768 x 3072]
+// int64 12.6 us (kernel trace); proofs of that product 114 -> 91 us, of one row of it 159 -> 102 us, of both products of an
 // attention layer of 12 heads over 197 tokens 237 -> 203 us.
 // ---------------------------------------------------------------------------
 constexpr u32 AXP_ROW_BITS = 9, AXP_ROW_STEPS = 64;  // columns a step of a row (log2), steps whose weights are made together
@@ -3257,7 +3257,7 @@ __global__ void __launch_bounds__(BLOCK) axis_point_short_kernel(AxisPointArgs a
 // in flight) where rows of 1024 (STEPS = 2) would not make a workgroup a compute unit (four eq tables of 2^16 entries 13.0
 // and 13.7 us, of 2^19 27 and 18 us; rows of 2048 take 256 registers: 17 and 19 us).
 // Bound: each table once in, M once out; for eq tables one extension product an entry and table.  Four eq tables of 2^20
-// entries: 77 -> 33 us; 34 tables of 2^11 entries from about 100 others: 41 -> 19 us (kernel trace).  (Before, descriptors were read one item after
+// entries: 77 -> 33 us; 19 tables of 2^11 entries from 78 others: 41 -> 19 us (kernel trace).  (Before, descriptors were read one item after
 // the other and every item cost the workgroup a chain of about 20 field products and a weight per entry.)
 //
 // eval_tables_kernel evaluates the tables that are in no product any more at the sum's final point (grid: a workgroup per
