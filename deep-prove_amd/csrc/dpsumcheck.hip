@@ -403,6 +403,11 @@ struct EqInfo {
     bool fact_built = false;  // ... and the low tables are there (built when a product session first wants them)
     u64 built = 0;        // bit l: level l is materialised
     std::vector<E2> point;
+    std::shared_ptr<struct EqBatch> batch;  // the tables it was asked for with, of at most 2^16 entries: none of them built yet
+};
+// Tables that dps_eq_build_many described together: the first reader of one of them builds them all, in one launch
+struct EqBatch {
+    std::vector<std::pair<std::weak_ptr<EqInfo>, std::weak_ptr<Storage>>> members;
 };
 
 struct dps_mle {
@@ -946,6 +951,84 @@ u32 eq_first_direct(u32 m) { return m > dpk::EQ_DIRECT_BITS ? m - dpk::EQ_DIRECT
 u64 eq_low_off(u32 m, u32 l) { return (2ull << m) + ((u64)(l - 1) << dpk::EQ_LO_BITS); }
 u64 eq_storage_entries(u32 m) { return (2ull << m) + ((u64)eq_fact_levels(m) << dpk::EQ_LO_BITS); }
 
+// The staging region of the pinned buffer (descriptors of launches that read them from there), h_pinned[STAGE_LO ..
+// pinned_words / 2): the previous launch that read it must be done with it.
+constexpr size_t STAGE_LO = 1024;
+int32_t stage_region(dps_ctx *ctx)
+{
+    if (ctx->stage_pending) {
+        HIPCHK(ctx, hipEventSynchronize(ctx->stage_event));
+        ctx->stage_pending = false;
+    }
+    return DPS_OK;
+}
+int32_t stage_region_read(dps_ctx *ctx)
+{
+    HIPCHK(ctx, hipEventRecord(ctx->stage_event, ctx->stream));
+    ctx->stage_pending = true;
+    return DPS_OK;
+}
+
+// Levels of eq tables of at most 2^16 entries straight from the definition, in as few launches as the staging region allows
+struct EqWant {
+    EqInfo *info;
+    const Storage *st;
+    u64 levels;  // bit l: level l
+};
+int32_t eq_define(dps_ctx *ctx, const std::vector<EqWant> &wants)
+{
+    for (size_t at = 0; at < wants.size();) {
+        std::vector<dpk::EqJobM> jobs;
+        std::vector<u64> pts;
+        u32 max_bits = 0;
+        const size_t first = at;
+        for (; at < wants.size(); at++) {
+            const EqInfo &e = *wants[at].info;
+            const size_t more = (size_t)__builtin_popcountll(wants[at].levels);
+            if (at > first && (jobs.size() + more > 65535 ||
+                               STAGE_LO + ((jobs.size() + more) * sizeof(dpk::EqJobM)) / 8 + pts.size() + 2 * (size_t)e.m > ctx->pinned_words / 2))
+                break;
+            for (u32 l = 0; l <= e.m; l++)
+                if ((wants[at].levels >> l) & 1) {
+                    jobs.push_back(dpk::EqJobM{wants[at].st->c0 + eq_level_off(e.m, l), wants[at].st->c1 + eq_level_off(e.m, l), l, e.m - l, (u32)pts.size(), 0});
+                    max_bits = std::max(max_bits, e.m - l);
+                }
+            for (const E2 &r : e.point) pts.push_back(r.c0), pts.push_back(r.c1);
+        }
+        if (!jobs.empty()) {
+            CHK(stage_region(ctx));
+            const size_t job_words = jobs.size() * sizeof(dpk::EqJobM) / 8;
+            memcpy(ctx->h_pinned + STAGE_LO, jobs.data(), job_words * 8);
+            if (!pts.empty()) memcpy(ctx->h_pinned + STAGE_LO + job_words, pts.data(), pts.size() * 8);
+            {
+                ProfScope ps(ctx, DPS_K_EQ, 0.0);
+                dpk::eq_define_many_kernel<<<dim3((u32)(((1ull << max_bits) + dpk::BLOCK - 1) / dpk::BLOCK), (u32)jobs.size()), dpk::BLOCK, 0, ctx->stream>>>(
+                    reinterpret_cast<const dpk::EqJobM *>(ctx->d_pinned + STAGE_LO), ctx->d_pinned + STAGE_LO + job_words);
+                HIPCHK(ctx, hipGetLastError());
+            }
+            CHK(stage_region_read(ctx));
+        }
+        for (size_t i = first; i < at; i++) wants[i].info->built |= wants[i].levels;
+    }
+    return DPS_OK;
+}
+
+// Every level of the tables of a batch that are still there
+int32_t eq_build_batch(dps_ctx *ctx, std::shared_ptr<EqBatch> batch)
+{
+    std::vector<std::pair<std::shared_ptr<EqInfo>, std::shared_ptr<Storage>>> there;
+    std::vector<EqWant> wants;
+    for (auto &m : batch->members) {
+        auto info = m.first.lock();
+        auto st = m.second.lock();
+        if (!info || !st) continue;
+        info->batch.reset();
+        wants.push_back(EqWant{info.get(), st.get(), ((2ull << info->m) - 1) & ~info->built});
+        there.emplace_back(std::move(info), std::move(st));
+    }
+    return eq_define(ctx, wants);
+}
+
 // Materialises the levels in `need` (bit l: level l = eq(rho_{l..m-1}, .), 2^(m-l) entries at eq_level_off) that are not
 // there yet, and with `need_low` the low tables.  Levels of at most 2^16 entries come straight from the definition, in
 // one launch together with the low tables and the 2^8-entry seeds eq(rho_{l..l+7}, .) the larger levels need; a larger
@@ -955,6 +1038,7 @@ int32_t eq_ensure(dps_ctx *ctx, EqInfo &info, u64 *o0, u64 *o1, u64 need, bool n
     const u32 m = info.m;
     const u32 first_small = eq_first_direct(m);  // levels first_small..m come straight from the definition
     need &= (2ull << m) - 1;
+    if ((need & ~info.built) && info.batch) CHK(eq_build_batch(ctx, info.batch));
     u64 todo = need & ~info.built;
     // a large level needs level l + 8
     for (u32 l = 0; l < first_small; l++)
@@ -1042,24 +1126,6 @@ int32_t plain_ready(const dps_mle *t)
     return eq_ensure(t->ctx, *t->eq, t->st->c0, t->st->c1, 1, false);
 }
 
-// The staging region of the pinned buffer (descriptors of launches that read them from there), h_pinned[STAGE_LO ..
-// pinned_words / 2): the previous launch that read it must be done with it.
-constexpr size_t STAGE_LO = 1024;
-int32_t stage_region(dps_ctx *ctx)
-{
-    if (ctx->stage_pending) {
-        HIPCHK(ctx, hipEventSynchronize(ctx->stage_event));
-        ctx->stage_pending = false;
-    }
-    return DPS_OK;
-}
-int32_t stage_region_read(dps_ctx *ctx)
-{
-    HIPCHK(ctx, hipEventRecord(ctx->stage_event, ctx->stream));
-    ctx->stage_pending = true;
-    return DPS_OK;
-}
-
 // The same for several tables, those of at most 2^16 entries in one launch (a launch each is 10 us of the host's and the
 // GPU's time, whatever is in it)
 int32_t eq_ready_many(dps_ctx *ctx, const std::vector<const dps_mle *> &tables)
@@ -1075,33 +1141,10 @@ int32_t eq_ready_many(dps_ctx *ctx, const std::vector<const dps_mle *> &tables)
         else
             CHK(plain_ready(t));
     }
-    if (small.size() == 1) return plain_ready(small[0]);
-    for (size_t at = 0; at < small.size();) {
-        std::vector<dpk::EqJobM> jobs;
-        std::vector<u64> pts;
-        u32 max_bits = 0;
-        const size_t first = at;
-        for (; at < small.size() && jobs.size() < 65535; at++) {
-            const EqInfo &e = *small[at]->eq;
-            if (STAGE_LO + ((jobs.size() + 1) * sizeof(dpk::EqJobM)) / 8 + pts.size() + 2 * (size_t)e.m > ctx->pinned_words / 2) break;
-            jobs.push_back(dpk::EqJobM{small[at]->st->c0, small[at]->st->c1, 0, e.m, (u32)pts.size(), 0});
-            for (const E2 &r : e.point) pts.push_back(r.c0), pts.push_back(r.c1);
-            max_bits = std::max(max_bits, e.m);
-        }
-        CHK(stage_region(ctx));
-        const size_t job_words = jobs.size() * sizeof(dpk::EqJobM) / 8;
-        memcpy(ctx->h_pinned + STAGE_LO, jobs.data(), job_words * 8);
-        if (!pts.empty()) memcpy(ctx->h_pinned + STAGE_LO + job_words, pts.data(), pts.size() * 8);
-        {
-            ProfScope ps(ctx, DPS_K_EQ, 0.0);
-            dpk::eq_define_many_kernel<<<dim3((u32)(((1ull << max_bits) + dpk::BLOCK - 1) / dpk::BLOCK), (u32)jobs.size()), dpk::BLOCK, 0, ctx->stream>>>(
-                reinterpret_cast<const dpk::EqJobM *>(ctx->d_pinned + STAGE_LO), ctx->d_pinned + STAGE_LO + job_words);
-            HIPCHK(ctx, hipGetLastError());
-        }
-        CHK(stage_region_read(ctx));
-        for (size_t i = first; i < at; i++) small[i]->eq->built |= 1;
-    }
-    return DPS_OK;
+    if (small.size() == 1 && !small[0]->eq->batch) return plain_ready(small[0]);
+    std::vector<EqWant> wants;
+    for (const dps_mle *t : small) wants.push_back(EqWant{t->eq.get(), t->st.get(), 1});
+    return eq_define(ctx, wants);
 }
 
 }  // namespace
@@ -1151,8 +1194,10 @@ extern "C" int32_t dps_eq_build_many(dps_ctx *ctx, const uint64_t *const *points
         }
         return rc;
     };
-    // nothing is built here: a session that reads several of them builds them together (eq_ready_many), one that takes them in
-    // closed form never reads entries
+    // Nothing is built here: a session may take them in closed form and read no entries, one that reads entries of several builds
+    // those together (eq_ready_many), and whoever else is the first to read one builds them all in one launch (16 products with one of 16
+    // tables each, of 2^8 and 2^12 entries: 780 and 1205 us, 860 and 1260 with a launch for every table).
+    auto batch = std::make_shared<EqBatch>();
     for (u32 i = 0; i < count; i++) {
         dps_mle *t = nullptr;
         if (const int32_t rc = new_table(ctx, DPS_EXT2, eq_storage_entries(m[i]), &t); rc != DPS_OK) return undo(rc);
@@ -1162,6 +1207,10 @@ extern "C" int32_t dps_eq_build_many(dps_ctx *ctx, const uint64_t *const *points
         t->eq->m = m[i];
         t->eq->fact_levels = eq_fact_levels(m[i]);
         for (u32 k = 0; k < m[i]; k++) t->eq->point.push_back(gl::e2(points[i][2 * k], points[i][2 * k + 1]));
+        if (m[i] <= 16) {
+            t->eq->batch = batch;
+            batch->members.emplace_back(t->eq, t->st);
+        }
     }
     return DPS_OK;
 }
