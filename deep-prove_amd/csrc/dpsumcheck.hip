@@ -1033,12 +1033,12 @@ int32_t eq_build_batch(dps_ctx *ctx, std::shared_ptr<EqBatch> batch)
 // there yet, and with `need_low` the low tables.  Levels of at most 2^16 entries come straight from the definition, in
 // one launch together with the low tables and the 2^8-entry seeds eq(rho_{l..l+7}, .) the larger levels need; a larger
 // level l is level l + 8 expanded by seed l (so asking for level 0 of a 24-variable table builds levels 0, 8, 16 only).
-int32_t eq_ensure(dps_ctx *ctx, EqInfo &info, u64 *o0, u64 *o1, u64 need, bool need_low)
+// (This table alone, whatever it was described with.)
+int32_t eq_ensure_alone(dps_ctx *ctx, EqInfo &info, u64 *o0, u64 *o1, u64 need, bool need_low)
 {
     const u32 m = info.m;
     const u32 first_small = eq_first_direct(m);  // levels first_small..m come straight from the definition
     need &= (2ull << m) - 1;
-    if ((need & ~info.built) && info.batch) CHK(eq_build_batch(ctx, info.batch));
     u64 todo = need & ~info.built;
     // a large level needs level l + 8
     for (u32 l = 0; l < first_small; l++)
@@ -1119,6 +1119,13 @@ int32_t eq_ensure(dps_ctx *ctx, EqInfo &info, u64 *o0, u64 *o1, u64 need, bool n
     return rc;
 }
 
+// The same, and the tables of its batch with it
+int32_t eq_ensure(dps_ctx *ctx, EqInfo &info, u64 *o0, u64 *o1, u64 need, bool need_low)
+{
+    if ((need & ((2ull << info.m) - 1) & ~info.built) && info.batch) CHK(eq_build_batch(ctx, info.batch));
+    return eq_ensure_alone(ctx, info, o0, o1, need, need_low);
+}
+
 // a table about to be read as ordinary entries: if it is an eq table, its level 0 has to be there
 int32_t plain_ready(const dps_mle *t)
 {
@@ -1141,7 +1148,7 @@ int32_t eq_ready_many(dps_ctx *ctx, const std::vector<const dps_mle *> &tables)
         else
             CHK(plain_ready(t));
     }
-    if (small.size() == 1 && !small[0]->eq->batch) return plain_ready(small[0]);
+    if (small.size() == 1) return eq_ensure_alone(ctx, *small[0]->eq, small[0]->st->c0, small[0]->st->c1, 1, false);
     std::vector<EqWant> wants;
     for (const dps_mle *t : small) wants.push_back(EqWant{t->eq.get(), t->st.get(), 1});
     return eq_define(ctx, wants);
