@@ -3192,7 +3192,9 @@ namespace {
 // What it saves: M costs one read of every Y_k and one write of M, and no Y_k is folded from round to round; eq tables among
 // the Y_k are never in memory at all.  What it costs: the launch that makes M and, for tables other than eq tables, a launch
 // that evaluates them at the final point, about 15 us.  Taken
-//   - for a common X always when every Y_k is an eq table, otherwise from the sizes on whose rounds are not all resident
+//   - for a common X when every Y_k is an eq table, from six variables on, or three where there are at most three claims (2, 3, 6, 12
+//     claims, combined and as they stand: on 2 variables 63, 67, 82, 109 and 40, 43, 50, 66 us, on 4 41, 45, 61, 90 and 43, 46, 56,
+//     73, on 6 46, 50, 66, 94 and 50, 53, 68, 92, on 9 58, 62, 78, 109 and 69, 72, 90, 112), otherwise from the sizes on whose rounds are not all resident
 //     (2^17 entries; merging four claims on 2^20 entries: 450 -> 250 us), and wherever a sum has more tables than
 //     the resident launches take or zero-padded ones, which only the general launches read (a launch for every fold and 430 us a
 //     round for 67 tables);
@@ -3248,7 +3250,8 @@ bool plan_combination(const dps_sc *sc, const dps_mle *const *mles, const std::v
             all = all && (t.factors[0] == x || t.factors[1] == x);
             others_eq = others_eq && is_eq(t.factors[0] == x ? t.factors[1] : t.factors[0]);
         }
-        if (!all || !(others_eq || too_many || any_zpad || n_vars >= 17)) continue;
+        const bool few_rounds = n_vars < 6 && (n_vars < 3 || sc->n_terms > 3);
+        if (!all || !((others_eq && !few_rounds) || too_many || any_zpad || n_vars >= 17)) continue;
         plan->assign(1, CombinedTable{x, {}});
         for (const dps_term &t : sc->terms) plan->back().items.emplace_back(t.factors[0] == x ? t.factors[1] : t.factors[0], coeff_of(t));
         return true;

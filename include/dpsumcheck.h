@@ -128,7 +128,7 @@ int32_t dps_eq_build(dps_ctx *ctx, const uint64_t *point /* 2*m */, uint32_t m, 
 /* `count` eq tables, table i at points[i] of m[i] coordinates (zkml/src/poly_commit/prover.rs:176-181 and
  * zkml/src/iop/same_poly.rs:88-91 build one per claim).  Nothing is launched here: whoever is the first to read one of
  * them builds all of at most 2^16 entries in one launch (a sum that reads entries of several: those alone), and a claim
- * merge never has them in memory. */
+ * merge of six variables and more never has them in memory. */
 int32_t dps_eq_build_many(dps_ctx *ctx, const uint64_t *const *points, const uint32_t *m, uint32_t count, dps_mle **out);
 
 /* ---- DensePolynomial::{evaluate, fix_low_variables, fix_high_variables}

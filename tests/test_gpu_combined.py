@@ -69,7 +69,7 @@ class Sum:
             assert tr.state() == otr.state()
 
 
-@pytest.mark.parametrize("n,k,base", [(1, 2, False), (3, 3, True), (7, 2, False), (10, 5, True), (11, 2, False), (12, 4, True), (16, 3, True),
+@pytest.mark.parametrize("n,k,base", [(1, 2, False), (2, 6, True), (3, 3, True), (3, 4, False), (5, 4, False), (5, 3, True), (6, 4, False), (7, 2, False), (10, 5, True), (11, 2, False), (12, 4, True), (16, 3, True),
                                       (17, 2, False), (18, 9, True), (20, 4, True)])
 def test_claims_on_one_table(dp, ctx, orc, n, k, base):
     s = Sum(ctx, orc, n, 1000 + 10 * n + k)
