@@ -1652,6 +1652,27 @@ struct dps_sc {
     const u64 *eq_c0, *eq_c1;  // its storage (level 0 at entry 0)
     E2 fast_coeff;
     E2 eq_scalar;       // product of eq1(rho_i, r_{i+1}) over the bound variables
+    // A sum over several eq factors (wsum_kernel): every term has one of them, all in closed form.  In order of their polynomials' degrees, highest first;
+    // p(1) of a round gives the first one's sum at 1
+    struct WeightedEq {
+        u32 k;                        // the eq table as registered
+        std::shared_ptr<EqInfo> info;
+        const u64 *c0, *c1;           // its storage (level 0 at entry 0)
+        u32 degree;                   // of the polynomial it weights
+        E2 scalar;                    // product of eq1(rho_i, r_{i+1}) over the bound variables
+        u32 op_begin, op_end;         // the polynomial's program in h_poly_ops
+        bool base_program;            // ... all of whose coefficients are in the base field
+        u32 off_q, off_d;             // where a resident trip's sums lie (dpk::SliceArgsEqs)
+    };
+    std::vector<WeightedEq> weq;
+    u32 weq_sums1 = 0, weq_sums2 = 0; // of a trip of one round, of two
+    bool closed_eq(u32 k) const
+    {
+        if ((int)k == fast_eq) return true;
+        for (const WeightedEq &w : weq)
+            if (w.k == k) return true;
+        return false;
+    }
     E2 claim;           // p(0) + p(1) expected from the next message (valid from round 2; from round 1 with dps_sc_set_claim)
     bool have_claim;    // the caller said what the whole sum is
     std::vector<E2> last_msg;
@@ -1814,20 +1835,23 @@ size_t slice_area_off(const dps_ctx *ctx) { return ctx->pinned_words / 2 + 64 + 
 
 // The sizes of a resident launch's arguments: a product's, and by its tables and terms a sum's (`shorter`: some table has fewer
 // variables than the sum)
-enum SliceSize { SLICE_PRODUCT, SLICE_FEW, SLICE_MANY };
-SliceSize slice_size(bool sum, size_t n_tabs, size_t n_terms, bool shorter)
+enum SliceSize { SLICE_PRODUCT, SLICE_FEW, SLICE_MANY, SLICE_EQS };
+SliceSize slice_size(bool sum, size_t n_tabs, size_t n_terms, bool shorter, size_t n_eqs)
 {
+    if (n_eqs) return SLICE_EQS;
     if (!sum) return SLICE_PRODUCT;
     return n_tabs <= (size_t)dpk::SL_FEW_TABS && n_terms <= (size_t)dpk::SL_FEW_TERMS && !shorter ? SLICE_FEW : SLICE_MANY;
 }
 template <SliceSize SIZE>
-using SliceArgsFor = std::conditional_t<SIZE == SLICE_PRODUCT, dpk::SliceArgsProduct, std::conditional_t<SIZE == SLICE_FEW, dpk::SliceArgsFew, dpk::SliceArgs>>;
+using SliceArgsFor = std::conditional_t<SIZE == SLICE_PRODUCT, dpk::SliceArgsProduct,
+                                        std::conditional_t<SIZE == SLICE_FEW, dpk::SliceArgsFew, std::conditional_t<SIZE == SLICE_EQS, dpk::SliceArgsEqs, dpk::SliceArgs>>>;
 template <int NF, bool EQ, SliceSize SIZE>
 constexpr auto slice_variant = &dpk::slice_kernel<NF, EQ, SIZE != SLICE_PRODUCT, dpk::SL_BLOCK, SliceArgsFor<SIZE>>;
 template <SliceSize SIZE>
 size_t slice_lds_bytes(u32 n_tabs, u32 cap, bool eq)
 {
-    return (size_t)dpk::slice_lds_words(n_tabs, cap, dpk::SL_BLOCK, eq, SliceArgsFor<SIZE>::TERMS) * 8;
+    // (several eq factors: sized for as many as there can be)
+    return (size_t)dpk::slice_lds_words(n_tabs, cap, dpk::SL_BLOCK, SIZE == SLICE_EQS ? dpk::SL_MAX_EQS : eq, SliceArgsFor<SIZE>::TERMS) * 8;
 }
 
 // A workgroup of a resident launch may take most of a compute unit's LDS (it is alone there: 1024 threads); more than
@@ -1855,7 +1879,8 @@ u32 slice_lds_granted(dps_ctx *ctx)
     SK(1, false, SIZE_) SK(2, false, SIZE_) SK(3, false, SIZE_) SK(4, false, SIZE_)
 #define SLICE_VARIANTS(SK)                                                                                              \
     SK(1, true, SLICE_PRODUCT) SK(2, true, SLICE_PRODUCT) SK(2, false, SLICE_PRODUCT) SK(3, false, SLICE_PRODUCT)       \
-    SLICE_SUM_VARIANTS(SK, SLICE_FEW) SLICE_SUM_VARIANTS(SK, SLICE_MANY)
+    SLICE_SUM_VARIANTS(SK, SLICE_FEW) SLICE_SUM_VARIANTS(SK, SLICE_MANY)                                                \
+    SK(2, true, SLICE_EQS) SK(3, true, SLICE_EQS) SK(4, true, SLICE_EQS)
 template <SliceSize SIZE>
 int32_t launch_slice(dps_ctx *ctx, u32 nf, bool eq, u32 workgroups, u32 n_tabs, u32 cap, const SliceArgsFor<SIZE> &a)
 {
@@ -1993,6 +2018,30 @@ int32_t launch_poly_dispatch(dps_ctx *ctx, u32 nf, bool eq, bool skip1, const dp
     case 5: launch_poly<5>(ctx, eq, skip1, a, grid, lds, partial, ff); break;
     case 6: launch_poly<6>(ctx, eq, skip1, a, grid, lds, partial, ff); break;
     default: return fail(ctx, DPS_ERR_UNSUPPORTED, "no fused kernel for degree %u", nf);
+    }
+    return DPS_OK;
+}
+
+// (the compiled variants over base-field tables are those of two factors)
+bool wsum_general(u32 n_eqs, u32 second_degree) { return n_eqs > 2 || second_degree > 1; }
+template <int NF, bool SKIP1>
+void launch_wsum_degree(dps_ctx *ctx, bool base, const dpk::WsumArgs &a, u32 blocks, u64 *partial, const dpk::FastFin &ff)
+{
+    const size_t table = (size_t)dpk::BLOCK * 8;  // a limb of the values or slopes of a table
+    if (wsum_general(a.n_eqs, a.degree[1]))
+        dpk::wsum_kernel<NF, SKIP1, false, true><<<blocks, dpk::BLOCK, a.n_tabs * 4 * table, ctx->stream>>>(a, partial, ff);
+    else if (base)
+        dpk::wsum_kernel<NF, SKIP1, true, false><<<blocks, dpk::BLOCK, a.n_tabs * 2 * table, ctx->stream>>>(a, partial, ff);
+    else
+        dpk::wsum_kernel<NF, SKIP1, false, false><<<blocks, dpk::BLOCK, a.n_tabs * 4 * table, ctx->stream>>>(a, partial, ff);
+}
+int32_t launch_wsum(dps_ctx *ctx, bool skip1, bool base, const dpk::WsumArgs &a, u32 blocks, u64 *partial, const dpk::FastFin &ff)
+{
+    switch (a.degree[0]) {
+    case 2: skip1 ? launch_wsum_degree<2, true>(ctx, base, a, blocks, partial, ff) : launch_wsum_degree<2, false>(ctx, base, a, blocks, partial, ff); break;
+    case 3: skip1 ? launch_wsum_degree<3, true>(ctx, base, a, blocks, partial, ff) : launch_wsum_degree<3, false>(ctx, base, a, blocks, partial, ff); break;
+    case 4: skip1 ? launch_wsum_degree<4, true>(ctx, base, a, blocks, partial, ff) : launch_wsum_degree<4, false>(ctx, base, a, blocks, partial, ff); break;
+    default: return fail(ctx, DPS_ERR_UNSUPPORTED, "no kernel for several eq factors, degree %u", a.degree[0]);
     }
     return DPS_OK;
 }
@@ -2145,7 +2194,8 @@ u32 horner_build(std::vector<HornerTerm> ts, u32 depth, std::vector<dpk::PolyOp>
         op.c0 = c.c0;
         op.c1 = c.c1;
         op.w = gl::mul_small(c.c1, (u32)gl::W);
-        op.code = kind | d << 2 | slot << 8;
+        const u32 cls = c.c1 ? dpk::POLY_COEFF_ANY : c.c0 == 1 ? dpk::POLY_COEFF_ONE : c.c0 == gl::P - 1 ? dpk::POLY_COEFF_MINUS_ONE : dpk::POLY_COEFF_BASE;
+        op.code = kind | d << 2 | (kind == dpk::POLY_OP_LEAF ? cls : 0) << 6 | slot << 8;
         return op;
     };
     u32 products = 0;
@@ -2281,9 +2331,11 @@ u32 quad_launches_fit(const dps_sc *sc, u32 n_mles, u32 first_resident)
 // A round of a sum of several terms with a common eq factor whose launch (poly_kernel, a thread per pair) takes the eq
 // weights from the low table of its level and from the level 16 rounds later instead of streaming its own level: the
 // rounds of more than 2^16 pairs, whose grid stride is a multiple of 2^16, of a table that has its low tables.
-bool poly_round_weights_factored(const dps_sc *sc, u32 jj)
+// (`low_tables`: they are there, or about to be)
+bool poly_round_weights_factored(const dps_sc *sc, u32 jj, bool low_tables = false)
 {
-    if (!sc->poly || sc->fast_eq < 0 || !sc->eq_info || !sc->eq_info->fact_built || jj > sc->eq_info->fact_levels) return false;
+    const EqInfo *eq = !sc->weq.empty() ? sc->weq[0].info.get() : sc->fast_eq >= 0 ? sc->eq_info.get() : nullptr;
+    if (!sc->poly || !eq || !(eq->fact_built || low_tables) || jj > eq->fact_levels) return false;
     const u64 n_pairs = 1ull << (sc->n_vars - jj);
     if (n_pairs <= POLY_SPLIT_MAX_PAIRS) return false;  // (those rounds spread a pair over lanes: poly_split_kernel)
     return ((u64)blocks_for_pairs(n_pairs) * dpk::BLOCK) % (1ull << dpk::EQ_LO_BITS) == 0;
@@ -2302,6 +2354,13 @@ u32 slice_counter_sets_log(u32 W)
 // point for some of the terms (slice_kernel's q_split), the lanes of a pass cover BLOCK / (q_split NF (NF + 1)) quads
 u32 slice_second_round_passes(const dps_sc *sc, u32 n_quads)
 {
+    if (!sc->weq.empty()) {
+        // (every factor has its own lanes; a lane takes a quad at one challenge)
+        const u32 per = ((u32)dpk::SL_BLOCK / (u32)sc->weq.size()) & ~63u;
+        u32 most = 0;
+        for (const dps_sc::WeightedEq &w : sc->weq) most = std::max(most, (n_quads * (w.degree + 1) + per - 1) / per);
+        return most;
+    }
     const u32 nf = sc->fast_nf, per_quad_pts = nf * (nf + 1);
     const u32 n_terms = sc->poly ? (u32)sc->slice_terms.size() : 1;
     const u32 q_split = n_terms * per_quad_pts <= (u32)dpk::SL_BLOCK ? n_terms : 1;
@@ -2316,15 +2375,15 @@ constexpr u32 SLICE_SECOND_ROUND_BUDGET = 10;
 void plan_resident_rounds(dps_sc *sc, u32 n_tabs, u32 n_mles)
 {
     const u32 n = sc->n_vars;
-    const bool has_eq = sc->fast_eq >= 0;
+    const bool has_eq = sc->fast_eq >= 0 || !sc->weq.empty();
     const u32 first_ok = 1;
     auto claim_gives_p1 = [&](u32 round) {
         if (sc->fast_coeff.c0 == 0 && sc->fast_coeff.c1 == 0) return false;
         if (!has_eq) return true;
-        const E2 rho = sc->eq_info->point[round - 1];
+        const E2 rho = (sc->weq.empty() ? sc->eq_info : sc->weq[0].info)->point[round - 1];
         return !(rho.c0 == 0 && rho.c1 == 0);
     };
-    const u32 pairs_fit = slice_pairs_per_workgroup(sc->ctx, slice_size(sc->poly, n_tabs, sc->slice_terms.size(), sc->slice_shorter), sc->fast_nf, has_eq, n_tabs);
+    const u32 pairs_fit = slice_pairs_per_workgroup(sc->ctx, slice_size(sc->poly, n_tabs, sc->slice_terms.size(), sc->slice_shorter, sc->weq.size()), sc->fast_nf, has_eq, n_tabs);
     if (pairs_fit == 0) return;
     // (more pairs per workgroup would make more rounds resident, but a trip's arithmetic is a workgroup's alone: with 512
     // pairs of a 3-term sum the first trip took 75 us where a launch for the round and a trip of 128 pairs take 66)
@@ -2383,6 +2442,7 @@ void plan_resident_rounds(dps_sc *sc, u32 n_tabs, u32 n_mles)
             // trips from 32 entries a workgroup on, 0.83 -> 0.72 ms) and on 8 products over 16 tables (0.145 -> 0.135 ms).
             if (dbl && slice_second_round_passes(sc, (u32)(len >> 2)) * (sc->fast_nf + 1) > SLICE_SECOND_ROUND_BUDGET) dbl = false;
             if (W > 1 && j + 1 == n_gpu) dbl = false;  // the last trip is the single workgroup's
+            if (!sc->weq.empty() && sc->weq_sums2 > (u32)dpk::SL_MAX_SUMS) dbl = false;
             if (dbl) st.dbl_mask |= 1u << st.n_trips;
             st.n_trips++;
             sc->round_kind[j] = dbl ? 2 : 1;
@@ -2452,12 +2512,15 @@ struct SessionSetup {
 
     // a zero-padded table keeps folding after it is down to one entry: both of its buffers hold at least that entry
     bool zpad_of(u32 k) const { return mles[k]->pad_vars != 0 && nv0[k] < n_vars; }
-    u64 len_a(u32 k) const { return nv0[k] >= 1 ? (1ull << (nv0[k] - 1)) : (zpad_of(k) ? 1ull : 0ull); }
-    u64 len_b(u32 k) const { return nv0[k] >= 2 ? (1ull << (nv0[k] - 2)) : (zpad_of(k) ? 1ull : 0ull); }
+    // (eq tables of a sum over several of them are never folded: no buffers)
+    u64 len_a(u32 k) const { return weighted(k) ? 0ull : nv0[k] >= 1 ? (1ull << (nv0[k] - 1)) : (zpad_of(k) ? 1ull : 0ull); }
+    u64 len_b(u32 k) const { return weighted(k) ? 0ull : nv0[k] >= 2 ? (1ull << (nv0[k] - 2)) : (zpad_of(k) ? 1ull : 0ull); }
     bool in_fast(u32 k) const;
+    bool weighted(u32 k) const { return !sc->weq.empty() && sc->closed_eq(k); }
 
     void detect_product();
     bool closed_form_eq_factor();
+    bool several_eq_factors();
     bool group_terms();
     void adopt_groups();
     void nested_programs();
@@ -2566,6 +2629,86 @@ bool SessionSetup::closed_form_eq_factor()
     return ok;
 }
 
+// A sum each of whose terms has one eq table, two or three of them in all, times polynomials of degree 4 at most over up to POLY_MAXT
+// other tables, all of full size: the eq factors in closed form, a nested program each for the polynomials (wsum_kernel).  What
+// does not fit (degrees, numbers of operations and sums) runs as before, with the eq tables as tables.
+bool SessionSetup::several_eq_factors()
+{
+    std::vector<dps_sc::WeightedEq> eqs;
+    std::vector<u32> tabs, eq_of_term;
+    for (const dps_term &t : sc->terms) {
+        int e = -1;
+        for (u32 f = 0; f < t.n_factors; f++) {
+            const u32 k = t.factors[f];
+            const dps_mle *h = mles[k];
+            if (nv0[k] != n_vars) return false;
+            if (h->eq && h->eq->m == n_vars && h->kind == DPS_EXT2) {
+                if (e >= 0) return false;
+                e = (int)k;
+            } else if (std::find(tabs.begin(), tabs.end(), k) == tabs.end()) {
+                tabs.push_back(k);
+            }
+        }
+        if (e < 0) return false;
+        size_t g = 0;
+        while (g < eqs.size() && eqs[g].k != (u32)e) g++;
+        if (g == eqs.size()) {
+            if (eqs.size() == dpk::WSUM_MAX_EQS) return false;
+            eqs.push_back(dps_sc::WeightedEq{(u32)e, mles[e]->eq, mles[e]->p0(), mles[e]->p1(), 0, gl::e2_one(), 0, 0, true, 0, 0});
+        }
+        eqs[g].degree = std::max(eqs[g].degree, t.n_factors - 1);
+        eq_of_term.push_back((u32)e);
+    }
+    if (eqs.size() < 2 || tabs.empty() || tabs.size() > (size_t)dpk::POLY_MAXT || n_mles != tabs.size() + eqs.size()) return false;
+    std::stable_sort(eqs.begin(), eqs.end(), [](const auto &x, const auto &y) { return x.degree > y.degree; });
+    if (eqs[0].degree < 2 || eqs[0].degree > 4 || eqs.back().degree < 1) return false;
+    std::vector<dpk::PolyOp> ops;
+    for (dps_sc::WeightedEq &w : eqs) {
+        std::vector<HornerTerm> ts;
+        dpk::PolyOp enter;
+        memset(&enter, 0, sizeof enter);
+        enter.code = dpk::POLY_OP_ENTER;
+        for (u32 ti = 0; ti < sc->n_terms; ti++) {
+            if (eq_of_term[ti] != w.k) continue;
+            const dps_term &t = sc->terms[ti];
+            HornerTerm ht;
+            ht.coeff = gl::e2(t.coeff[0], t.coeff[1]);
+            w.base_program = w.base_program && t.coeff[1] == 0;
+            for (u32 f = 0; f < t.n_factors; f++)
+                if (t.factors[f] != w.k) ht.slots.push_back((uint8_t)(std::find(tabs.begin(), tabs.end(), t.factors[f]) - tabs.begin()));
+            if (ht.slots.empty()) {
+                const E2 c = gl::add(gl::e2(enter.c0, enter.c1), ht.coeff);
+                enter.c0 = c.c0, enter.c1 = c.c1;
+            }
+            ts.push_back(std::move(ht));
+        }
+        w.op_begin = (u32)ops.size();
+        ops.push_back(enter);
+        horner_build(std::move(ts), 0, ops);
+        w.op_end = (u32)ops.size();
+    }
+    if (ops.size() > (size_t)dpk::SL_EQS_OPS) return false;
+    // the places of a trip's sums
+    u32 sums = 0;
+    for (dps_sc::WeightedEq &w : eqs) w.off_q = sums, sums += w.degree + 1;
+    sc->weq_sums1 = sums;
+    for (size_t g = 0; g < eqs.size(); g++) {
+        eqs[g].off_d = sums;
+        sums += (g == 0 ? eqs[g].degree : eqs[g].degree + 1) * (eqs[g].degree + 1);
+    }
+    sc->weq_sums2 = sums;
+    if (sc->weq_sums1 > (u32)dpk::SL_MAX_SUMS) return false;
+    sc->weq = std::move(eqs);
+    sc->h_poly_ops = std::move(ops);
+    nf = sc->weq[0].degree;
+    groups.assign(1, tabs);
+    tb.assign(1, 0);
+    te.assign(1, sc->n_terms);
+    sc->poly_op_begin.assign(1, 0);
+    sc->poly_op_end.assign(1, 0);
+    return true;
+}
+
 // The terms in order, a new group whenever the tables no longer fit one (POLY_MAXT).  False: a term has too many tables.
 bool SessionSetup::group_terms()
 {
@@ -2639,7 +2782,7 @@ void SessionSetup::adopt_groups()
             pt.c1 = t.coeff[1];
             pt.w = gl::mul_small(t.coeff[1], (u32)gl::W);
             for (u32 f = 0; f < t.n_factors; f++) {
-                if ((int)t.factors[f] == eq) continue;
+                if ((int)t.factors[f] == eq || weighted(t.factors[f])) continue;
                 const auto &gt = groups[g];
                 pt.slot[pt.n_factors++] = (uint8_t)(std::find(gt.begin(), gt.end(), t.factors[f]) - gt.begin());
             }
@@ -2696,7 +2839,12 @@ void SessionSetup::detect_multi_term()
     sc->d_poly_groups = nullptr;
     sc->d_poly_terms = nullptr;
     if (sc->fast || sc->n_terms < 1 || n_vars < 1) return;
-    if (!closed_form_eq_factor() || !group_terms()) return;
+    if (!closed_form_eq_factor()) return;
+    if (eq < 0 && several_eq_factors()) {
+        adopt_groups();
+        return;
+    }
+    if (!group_terms()) return;
     adopt_groups();
     nested_programs();
 }
@@ -2735,7 +2883,7 @@ int32_t SessionSetup::plan_and_ready_tables()
         for (const auto &g : sc->poly_tabs)
             for (u32 k : g)
                 if (std::find(ids.begin(), ids.end(), k) == ids.end()) ids.push_back(k);
-        bool ok = n_mles == ids.size() + (sc->fast_eq >= 0 ? 1 : 0) && ids.size() <= (size_t)dpk::SL_MAX_TABS;
+        bool ok = n_mles == ids.size() + (sc->fast_eq >= 0 ? 1 : 0) + sc->weq.size() && ids.size() <= (size_t)dpk::SL_MAX_TABS;
         for (u32 k : ids) ok = ok && !zpad_of(k);  // (a full-size table that is marked as padded is one like the others)
         if (ok) {
             sc->slice_ids = ids;
@@ -2744,8 +2892,11 @@ int32_t SessionSetup::plan_and_ready_tables()
                 dpk::SliceTerm tm;
                 memset(&tm, 0, sizeof tm);
                 tm.c0 = t.coeff[0], tm.c1 = t.coeff[1], tm.w = gl::mul_small(t.coeff[1], (u32)gl::W);
+                for (size_t g = 0; g < sc->weq.size(); g++)
+                    for (u32 f = 0; f < t.n_factors; f++)
+                        if (t.factors[f] == sc->weq[g].k) tm.eq = (u32)g;
                 for (u32 f = 0; f < t.n_factors; f++)
-                    if ((int)t.factors[f] != sc->fast_eq) tm.slot[tm.n_factors++] = (uint8_t)(std::find(ids.begin(), ids.end(), t.factors[f]) - ids.begin());
+                    if (!sc->closed_eq(t.factors[f])) tm.slot[tm.n_factors++] = (uint8_t)(std::find(ids.begin(), ids.end(), t.factors[f]) - ids.begin());
                 sc->slice_terms.push_back(tm);
             }
             plan_resident_rounds(sc, (u32)ids.size(), n_mles);
@@ -2792,6 +2943,12 @@ int32_t SessionSetup::plan_and_ready_tables()
             return DPS_OK;      // nothing of any table is read on the device
         }
     }
+    // (several eq factors: as one common to all terms, each)
+    for (const dps_sc::WeightedEq &w : sc->weq) {
+        u32 first_level = 1;
+        while (first_level <= n_vars && poly_round_weights_factored(sc, first_level, sc->tail_j0 != 1)) first_level++;
+        CHK(eq_ensure(ctx, *w.info, const_cast<u64 *>(w.c0), const_cast<u64 *>(w.c1), ((2ull << n_vars) - 1) & ~((1ull << first_level) - 1), sc->tail_j0 != 1));
+    }
     // What this session reads of its tables: an eq table taken in closed form is read level by level -- level j in round j,
     // except in the large rounds of a product, which take the low table of level j and level j + 16 instead -- and
     // anything else as ordinary entries.  Whatever of that an eq table has not built yet is built now, on the stream.
@@ -2809,7 +2966,7 @@ int32_t SessionSetup::plan_and_ready_tables()
             }
             const u64 need = ((2ull << n_vars) - 1) & ~((1ull << first_level) - 1);
             CHK(eq_ensure(ctx, *sc->eq_info, const_cast<u64 *>(sc->eq_c0), const_cast<u64 *>(sc->eq_c1), need, sc->fast));
-        } else if (mles[k]->eq) {
+        } else if (mles[k]->eq && !sc->closed_eq(k)) {
             plain.push_back(mles[k]);
         }
     }
@@ -2874,7 +3031,7 @@ void SessionSetup::fold_step(u32 j)
         }
         for (u32 k = 0; k < n_mles; k++) {
             SessMle &s = sim[k];
-            if ((int)k == sc->fast_eq) continue;
+            if (sc->closed_eq(k)) continue;
             if (s.zpad) {
                 // depends on the low variables: folds in every step, and keeps folding against 0 once it is one entry
                 const bool single = s.nv == 0;
@@ -3017,6 +3174,7 @@ void SessionSetup::launch_limits()
     // (the launch of the first two rounds: 18 words a workgroup where the others have at most 16)
     if (sc->pair12) sc->max_blocks = std::max<u32>(sc->max_blocks, (PAIR12_BLOCKS * 2 * dpk::PAIR12_SUMS + 2 * dpk::MAX_PTS - 1) / (2 * dpk::MAX_PTS));
     for (const dps_sc::QuadStep &q : sc->quads) sc->max_blocks = std::max<u32>(sc->max_blocks, q.blocks);
+    if (!sc->weq.empty()) sc->max_blocks *= (2 * dpk::WSUM_MAX_SUMS + 2 * dpk::MAX_PTS - 1) / (2 * dpk::MAX_PTS);
     sc->poly_split_cap = 0;
     sc->poly_finish_in_kernel = false;
     if (sc->poly) {
@@ -3055,7 +3213,7 @@ int32_t SessionSetup::allocate_device_block()
     // what a resident stage that does not run to the last round leaves for the next: two limb arrays per table
     size_t bytes_hand = 0;
     const u32 slice_tabs = (u32)sc->slice_ids.size();
-    for (size_t i = 0; i + 1 < sc->stages.size(); i++) bytes_hand += round_up((size_t)sc->stages[i + 1].src_len * 8, 256) * 2 * (slice_tabs + 1);
+    for (size_t i = 0; i + 1 < sc->stages.size(); i++) bytes_hand += round_up((size_t)sc->stages[i + 1].src_len * 8, 256) * 2 * (slice_tabs + std::max<size_t>(1, sc->weq.size()));
     size_t total = bytes_fold + bytes_fold_x + bytes_terms + bytes_fin + bytes_gath + bytes_pg + bytes_pt + bytes_po + bytes_partial + bytes_result + bytes_hand;
     CHK(pool_alloc(ctx, total, &sc->dev_block));
     char *p = (char *)sc->dev_block;
@@ -3082,10 +3240,12 @@ int32_t SessionSetup::allocate_device_block()
     for (size_t i = 0; i + 1 < sc->stages.size(); i++) {
         const size_t limb = round_up((size_t)sc->stages[i + 1].src_len * 8, 256);
         for (u32 f = 0; f <= slice_tabs; f++) {
+            // (behind the tables the eq weights, one factor's behind the other's)
+            const size_t n = f < slice_tabs ? 1 : std::max<size_t>(1, sc->weq.size());
             sc->stages[i].h0[f] = (u64 *)p;
-            p += limb;
+            p += n * limb;
             sc->stages[i].h1[f] = (u64 *)p;
-            p += limb;
+            p += n * limb;
         }
     }
     sc->d_counter = ctx->d_counter;
@@ -3756,6 +3916,54 @@ void host_tail_advance(dps_sc *sc, E2 r)
     fold_all(r);
 }
 
+// eq(rho_{j+1..n}, x) over the pairs of round j: variable j + 1 is the lowest bit of the pair's index
+std::vector<E2> host_pair_weights(const EqInfo &eq, u32 j, u32 n_vars, u32 n_pairs)
+{
+    std::vector<E2> weight(n_pairs, gl::e2_one());
+    u32 have = 1;
+    for (u32 i = j + 1; i <= n_vars; i++) {
+        const E2 rho = eq.point[i - 1], one_minus = gl::sub(gl::e2_one(), rho);
+        for (u32 x = 0; x < have; x++) {
+            weight[x + have] = gl::mul(weight[x], rho);
+            weight[x] = gl::mul(weight[x], one_minus);
+        }
+        have *= 2;
+    }
+    return weight;
+}
+
+// The sums q_g(t), t = 0 .. degree of factor g, of a round of a sum over several eq factors on the tables the host holds (q_0(1) left
+// out when it comes from the claim), factor g's from q[g * MAX_PTS] on
+void host_tail_weighted_sums(dps_sc *sc, u32 j, bool skip1, E2 *q)
+{
+    const u32 n_tabs = (u32)sc->slice_ids.size(), len = sc->host_len, n_pairs = len / 2;
+    std::vector<E2> weight[dpk::WSUM_MAX_EQS];
+    for (size_t g = 0; g < sc->weq.size(); g++) {
+        weight[g] = host_pair_weights(*sc->weq[g].info, j, sc->n_vars, n_pairs);
+        for (u32 t = 0; t <= sc->weq[g].degree; t++) q[g * dpk::MAX_PTS + t] = gl::e2_zero();
+    }
+    E2 val[dpk::POLY_MAXT], d[dpk::POLY_MAXT];
+    for (u32 p = 0; p < n_pairs; p++) {
+        for (u32 f = 0; f < n_tabs; f++) {
+            val[f] = sc->host_state[(size_t)f * len + 2 * p];
+            d[f] = gl::sub(sc->host_state[(size_t)f * len + 2 * p + 1], val[f]);
+        }
+        for (u32 t = 0; t <= sc->fast_nf; t++) {
+            if (t > 0)
+                for (u32 f = 0; f < n_tabs; f++) val[f] = gl::add(val[f], d[f]);
+            E2 poly[dpk::WSUM_MAX_EQS] = {};
+            for (const dpk::SliceTerm &tm : sc->slice_terms) {
+                if (t > sc->weq[tm.eq].degree || (tm.eq == 0 && t == 1 && skip1)) continue;
+                E2 prod = gl::e2(tm.c0, tm.c1);
+                for (u32 k = 0; k < tm.n_factors; k++) prod = gl::mul(prod, val[tm.slot[k]]);
+                poly[tm.eq] = gl::add(poly[tm.eq], prod);
+            }
+            for (size_t g = 0; g < sc->weq.size(); g++)
+                if (t <= sc->weq[g].degree) q[g * dpk::MAX_PTS + t] = gl::add(q[g * dpk::MAX_PTS + t], gl::mul(poly[g], weight[g][p]));
+        }
+    }
+}
+
 // The sums q(t), t = 0 .. nf, of a round on the tables the host holds (q(1) left out when it comes from the claim):
 // what slice_kernel adds up, by the definition.
 void host_tail_sums(dps_sc *sc, u32 j, u32 nf, bool skip1, E2 *q)
@@ -3763,19 +3971,7 @@ void host_tail_sums(dps_sc *sc, u32 j, u32 nf, bool skip1, E2 *q)
     const u32 n_tabs = (u32)sc->slice_ids.size();
     const u32 len = sc->host_len, n_pairs = len / 2;
     const bool has_eq = sc->fast_eq >= 0;
-    // eq(rho_{j+1..n}, x) over the pairs: variable j + 1 is the lowest bit of the pair's index
-    std::vector<E2> weight(n_pairs, gl::e2_one());
-    if (has_eq) {
-        u32 have = 1;
-        for (u32 i = j + 1; i <= sc->n_vars; i++) {
-            const E2 rho = sc->eq_info->point[i - 1], one_minus = gl::sub(gl::e2_one(), rho);
-            for (u32 x = 0; x < have; x++) {
-                weight[x + have] = gl::mul(weight[x], rho);
-                weight[x] = gl::mul(weight[x], one_minus);
-            }
-            have *= 2;
-        }
-    }
+    const std::vector<E2> weight = has_eq ? host_pair_weights(*sc->eq_info, j, sc->n_vars, n_pairs) : std::vector<E2>(n_pairs, gl::e2_one());
     for (u32 t = 0; t <= nf; t++) q[t] = gl::e2_zero();
     E2 val[dpk::SL_MAX_TABS];
     for (u32 p = 0; p < n_pairs; p++) {
@@ -3859,9 +4055,13 @@ struct FusedRound {
     template <SliceSize SIZE>
     int32_t launch_stages_of(u64 seq0, u32 first_go);
     int32_t resident_round();
+    void form_weighted_message(E2 *q);
+    int32_t take_weighted_sums();
+    int32_t launch_weighted(u32 jj, bool skip1_jj, bool ahead, u64 seq_jj);
+    bool weighted() const { return !sc->weq.empty(); }
     Plan plan_round(u32 jj, bool skip1_jj) const;
     int32_t launch_round(u32 jj, const Plan &p, bool skip1_jj, bool ahead, u64 seq_jj);
-    u32 slots_of(const Plan &p) const { return p.reside ? (n_groups > 1 ? n_groups : 0) : slots_for(p.blocks * n_groups); }
+    u32 slots_of(const Plan &p) const { return weighted() ? 0 : p.reside ? (n_groups > 1 ? n_groups : 0) : slots_for(p.blocks * n_groups); }
     int32_t multi_term_round();
     int32_t product_launch_ahead(u32 ahead = 1);
     int32_t product_round();
@@ -3893,12 +4093,14 @@ int32_t FusedRound::begin()
         a.ra1 = sc->prev_chal.c1;
         CHK(launch_folds(sc, j, true, challenge));
         if (has_eq) sc->eq_scalar = gl::mul(sc->eq_scalar, h_eq1(sc->eq_info->point[j - 2], r));
+        for (dps_sc::WeightedEq &w : sc->weq) w.scalar = gl::mul(w.scalar, h_eq1(w.info->point[j - 2], r));
     }
     // scale(t) = coeff * S * eq1(rho_{j-1}, t).  Only whether scale(1) vanishes matters to the kernel (it then has to
     // evaluate t = 1); everything else about the message is worked out while the kernel runs (prepare_message).
     base_scale = sc->fast_coeff;
     if (has_eq) base_scale = gl::mul(base_scale, sc->eq_scalar);
     s1 = has_eq ? gl::mul(base_scale, h_eq1(sc->eq_info->point[j - 1], gl::e2_one())) : base_scale;
+    if (weighted()) s1 = gl::mul(sc->weq[0].scalar, sc->weq[0].info->point[j - 1]);  // (eq1(rho, 1) = rho)
     skip1 = (j >= 2 || sc->have_claim) && !(s1.c0 == 0 && s1.c1 == 0);
     a.skip1 = skip1 ? 1 : 0;
     if (has_eq) set_eq_weights(a, j, blocks);
@@ -4006,6 +4208,60 @@ void FusedRound::form_message(const E2 *q)
         }
 }
 
+// The message of a sum over several eq factors from their sums q_g(t), t = 0 .. degree[g] (factor g's from q[g * MAX_PTS] on; prepare_message
+// has run): p(t) = sum_g S_g eq1(rho_g, t) q_g(t) + const.  q_0(1) is missing when p(1) comes from the claim: it is
+// solved for, since the points beyond the degrees are extrapolated.
+void FusedRound::form_weighted_message(E2 *q)
+{
+        const size_t G = sc->weq.size();
+        auto scale = [&](size_t g, u32 t) { return gl::mul(sc->weq[g].scalar, h_eq1(sc->weq[g].info->point[j - 1], gl::e2(t, 0))); };
+        auto beyond = [&](size_t g, u32 t) {
+            const u32 d = sc->weq[g].degree;
+            E2 v = gl::e2_zero();
+            for (u32 i = 0; i <= d; i++) v = gl::add(v, gl::mul_base(q[g * dpk::MAX_PTS + i], ctx->h_lagrange[(d * 9 + t) * 9 + i]));
+            return v;
+        };
+        E2 msg[dpk::MAX_PTS + 1];
+        for (u32 t = 0; t <= sc->degree; t++) {
+            E2 v = cst;
+            for (size_t g = 0; g < G; g++) {
+                if (g == 0 && t == 1 && a.skip1) continue;
+                if (t > sc->weq[g].degree) q[g * dpk::MAX_PTS + t] = beyond(g, t);
+                v = gl::add(v, gl::mul(scale(g, t), q[g * dpk::MAX_PTS + t]));
+            }
+            if (t == 1 && a.skip1) {
+                const E2 p1 = gl::sub(sc->claim, msg[0]);
+                q[1] = gl::mul(gl::sub(p1, v), h_e2_inv(s1));
+                v = p1;
+            }
+            msg[t] = v;
+        }
+        sc->last_msg.assign(msg, msg + sc->degree + 1);
+        for (u32 t = 0; t <= sc->degree; t++) {
+            evals_out[2 * t] = msg[t].c0;
+            evals_out[2 * t + 1] = msg[t].c1;
+        }
+}
+
+// Waits for those sums of a launch of its own (wsum_kernel)
+int32_t FusedRound::take_weighted_sums()
+{
+        prepare_message();
+        const int n0 = (int)nf + (a.skip1 ? 0 : 1);
+        const bool general = wsum_general((u32)sc->weq.size(), sc->weq[1].degree);
+        u64 w[2 * dpk::WSUM_MAX_SUMS];
+        CHK(wait_result_at(ctx, ctx->res_off, fa.seq, 0, 2 * (u32)dpk::wsum_sums((int)nf, a.skip1 != 0, general), w, dpk::WSUM_SEQ_SLOT, dpk::WSUM_CHK_SLOT));
+        E2 q[dpk::WSUM_MAX_EQS * dpk::MAX_PTS];
+        for (int i = 0; i < n0; i++) q[a.skip1 && i > 0 ? i + 1 : i] = gl::e2(w[2 * i], w[2 * i + 1]);
+        for (size_t g = 1; g < sc->weq.size(); g++)
+            for (u32 t = 0; t <= sc->weq[g].degree; t++) {
+                const int i = n0 + (int)(g - 1) * dpk::wsum_rest((int)nf, general) + (int)t;
+                q[g * dpk::MAX_PTS + t] = gl::e2(w[2 * i], w[2 * i + 1]);
+            }
+        form_weighted_message(q);
+        return DPS_OK;
+}
+
 // Waits for the sums q(t), t = 0..nf, of this round (one set in the main result area, or n_slots sets in areas of their own --
 // resident groups, or the workgroups of a small launch -- which are added) and forms the message.
 int32_t FusedRound::take_sums(u32 n_slots)
@@ -4059,10 +4315,10 @@ int32_t FusedRound::end_waiting_launch()
 bool FusedRound::admit_stages()
 {
         u32 widest = 1;
-        const SliceSize size = slice_size(sc->poly, sc->slice_ids.size(), sc->slice_terms.size(), sc->slice_shorter);
+        const SliceSize size = slice_size(sc->poly, sc->slice_ids.size(), sc->slice_terms.size(), sc->slice_shorter, sc->weq.size());
         for (const dps_sc::Stage &st : sc->stages) {
             widest = std::max(widest, st.W);
-            if (slice_workgroups_per_cu(ctx, size, sc->fast_nf, sc->fast_eq >= 0, (u32)sc->slice_ids.size(), st.cap) < 1) return false;
+            if (slice_workgroups_per_cu(ctx, size, sc->fast_nf, sc->fast_eq >= 0 || weighted(), (u32)sc->slice_ids.size(), st.cap) < 1) return false;
         }
         return admit_waiting_launch(ctx, widest, true);
 }
@@ -4071,7 +4327,8 @@ bool FusedRound::admit_stages()
 // round has the sequence number seq0 (a round's call takes one number whether or not it makes a trip).
 int32_t FusedRound::launch_stages_at(u64 seq0, u32 first_go)
 {
-        switch (slice_size(sc->poly, sc->slice_ids.size(), sc->slice_terms.size(), sc->slice_shorter)) {
+        switch (slice_size(sc->poly, sc->slice_ids.size(), sc->slice_terms.size(), sc->slice_shorter, sc->weq.size())) {
+        case SLICE_EQS: return launch_stages_of<SLICE_EQS>(seq0, first_go);
         case SLICE_PRODUCT: return launch_stages_of<SLICE_PRODUCT>(seq0, first_go);
         case SLICE_FEW: return launch_stages_of<SLICE_FEW>(seq0, first_go);
         default: return launch_stages_of<SLICE_MANY>(seq0, first_go);
@@ -4128,7 +4385,19 @@ int32_t FusedRound::launch_stages_of(u64 seq0, u32 first_go)
             sa.hw0 = st.h0[n_tabs];
             sa.hw1 = st.h1[n_tabs];
             sa.n_tabs = n_tabs;
-            if (SIZE != SLICE_PRODUCT) {
+            if constexpr (SIZE == SLICE_EQS) {
+                // (the programs in the terms' place)
+                memcpy(static_cast<void *>(sa.terms), sc->h_poly_ops.data(), sc->h_poly_ops.size() * sizeof(dpk::PolyOp));
+                sa.n_eqs = (u32)sc->weq.size();
+                sa.hw_stride = si + 1 < sc->stages.size() ? (u32)(round_up((size_t)sc->stages[si + 1].src_len * 8, 256) / 8) : 0;
+                for (u32 g = 0; g < sa.n_eqs; g++) {
+                    const dps_sc::WeightedEq &w = sc->weq[g];
+                    sa.geq0[g] = w.c0, sa.geq1[g] = w.c1;
+                    sa.degree[g] = w.degree, sa.off_q[g] = w.off_q, sa.off_d[g] = w.off_d;
+                    sa.op_begin[g] = w.op_begin, sa.op_end[g] = w.op_end;
+                }
+                sa.n_sums1 = sc->weq_sums1, sa.n_sums2 = sc->weq_sums2;
+            } else if (SIZE != SLICE_PRODUCT) {
                 sa.n_terms = (u32)sc->slice_terms.size();
                 std::copy(sc->slice_terms.begin(), sc->slice_terms.end(), sa.terms);
             }
@@ -4158,7 +4427,7 @@ int32_t FusedRound::launch_stages_of(u64 seq0, u32 first_go)
             sa.gate = reinterpret_cast<u32 *>(ctx->d_slice_ctr + SLICE_CTR_WORDS);
             sa.groups_log = slice_counter_sets_log(st.W);
             ProfScope ps(ctx, DPS_K_TAIL, 0.0);
-            CHK(launch_slice<SIZE>(ctx, nf, has_eq, st.W, n_tabs, st.cap, sa));
+            CHK(launch_slice<SIZE>(ctx, nf, has_eq || weighted(), st.W, n_tabs, st.cap, sa));
             HIPCHK(ctx, hipGetLastError());
             si = last_si;
         }
@@ -4175,16 +4444,42 @@ int32_t FusedRound::resident_round()
 {
     const u32 kind = sc->round_kind[j];
     const u32 np = nf + 1;
-    E2 q[dpk::MAX_PTS];
+    E2 q[dpk::MAX_PTS], wq[dpk::WSUM_MAX_EQS * dpk::MAX_PTS];
     int32_t rc = DPS_OK;
     if (kind == 4) {
         // A round of the few pairs that are left once the launch has gone: worked out here.
         if (sc->host_len < (j == 1 ? 2u : 4u)) return fail(ctx, DPS_ERR_STATE, "dps_sc_round: the tables of the last rounds are not here");
         // (round 1 of a sum that is the host's from the start has nothing to fold)
         if (j >= 2) host_tail_advance(sc, gl::e2(challenge[0], challenge[1]));
-        host_tail_sums(sc, j, nf, a.skip1 != 0, q);
+        if (weighted())
+            host_tail_weighted_sums(sc, j, a.skip1 != 0, wq);
+        else
+            host_tail_sums(sc, j, nf, a.skip1 != 0, q);
         prepare_message();
-        form_message(q);
+        if (weighted())
+            form_weighted_message(wq);
+        else
+            form_message(q);
+    } else if (kind == 3 && weighted()) {
+        // Second round of a trip: every sum of this round is a polynomial of its factor's degree in the challenge that has now
+        // been drawn, known at 0 .. degree (point 1 of the first factor comes from the claim)
+        const E2 r = gl::e2(challenge[0], challenge[1]);
+        for (size_t g = 0; g < sc->weq.size(); g++) {
+            const dps_sc::WeightedEq &w = sc->weq[g];
+            const u32 d = w.degree, npt = g == 0 ? d : d + 1;
+            for (u32 ti = 0; ti < npt; ti++) wq[g * dpk::MAX_PTS + (g == 0 && ti > 0 ? ti + 1 : ti)] = gl::e2_zero();
+            for (u32 k = 0; k <= d; k++) {
+                E2 basis = gl::e2(ctx->h_inv_den[d][k], 0);
+                for (u32 m = 0; m <= d; m++)
+                    if (m != k) basis = gl::mul(basis, gl::sub(r, gl::e2(m, 0)));
+                for (u32 ti = 0; ti < npt; ti++) {
+                    E2 &v = wq[g * dpk::MAX_PTS + (g == 0 && ti > 0 ? ti + 1 : ti)];
+                    v = gl::add(v, gl::mul(basis, sc->stash[w.off_d - sc->weq_sums1 + k * npt + ti]));
+                }
+            }
+        }
+        prepare_message();
+        form_weighted_message(wq);
     } else if (kind == 3) {
         // Second round of a trip: the kernel handed over this round's sums as a polynomial in the challenge that has
         // now been drawn (values at 0..nf-1 and the leading coefficient, per point t = 0, 2, .., nf); p(1) comes
@@ -4216,7 +4511,7 @@ int32_t FusedRound::resident_round()
         sc->wait_fresh = false;
         prepare_message();
         // sums of this round, and with a trip of two rounds those of the next
-        const u32 ns = kind == 2 ? np + np * nf : np;
+        const u32 ns = weighted() ? (kind == 2 ? sc->weq_sums2 : sc->weq_sums1) : kind == 2 ? np + np * nf : np;
         u64 cnt[dpk::SL_MAX_GROUPS * dpk::SL_GROUP_WORDS];
         const u32 n_sets = sc->round_wide[j] ? sc->round_wide[j] : 1;
         rc = wait_slice_sums(ctx, fa.seq, ns, a.skip1 != 0, n_sets, cnt);
@@ -4239,9 +4534,19 @@ int32_t FusedRound::resident_round()
                 const unsigned __int128 t = (unsigned __int128)cnt[2 * i] + ((unsigned __int128)cnt[2 * i + 1] << 32);
                 w[i] = gl::reduce128((u64)t, (u64)(t >> 64));
             }
-            for (u32 t = 0; t < np; t++) q[t] = gl::e2(w[2 * t], w[2 * t + 1]);
-            for (u32 i = np; i < ns; i++) sc->stash[i - np] = gl::e2(w[2 * i], w[2 * i + 1]);
-            form_message(q);
+            if (weighted()) {
+                for (size_t g = 0; g < sc->weq.size(); g++)
+                    for (u32 t = 0; t <= sc->weq[g].degree; t++) {
+                        const u32 i = sc->weq[g].off_q + t;
+                        wq[g * dpk::MAX_PTS + t] = gl::e2(w[2 * i], w[2 * i + 1]);
+                    }
+                for (u32 i = sc->weq_sums1; i < ns; i++) sc->stash[i - sc->weq_sums1] = gl::e2(w[2 * i], w[2 * i + 1]);
+                form_weighted_message(wq);
+            } else {
+                for (u32 t = 0; t < np; t++) q[t] = gl::e2(w[2 * t], w[2 * t + 1]);
+                for (u32 i = np; i < ns; i++) sc->stash[i - np] = gl::e2(w[2 * i], w[2 * i + 1]);
+                form_message(q);
+            }
             sc->last_trip_seq = fa.seq;
             // the last trip: what is left of the tables has come with it
             if (j + (kind == 2 ? 1 : 0) == sc->n_vars - sc->host_rounds) rc = host_tail_load(sc, fa.seq);
@@ -4270,7 +4575,7 @@ FusedRound::Plan FusedRound::plan_round(u32 jj, bool skip1_jj) const
 {
         Plan p;
         p.n_pairs = 1ull << (sc->n_vars - jj);
-        p.split = p.n_pairs <= POLY_SPLIT_MAX_PAIRS;
+        p.split = p.n_pairs <= POLY_SPLIT_MAX_PAIRS && !weighted();
         p.split_log = 0;
         p.blocks = blocks_for_pairs(p.n_pairs);
         if (p.split) poly_split_plan(p.n_pairs, sc->poly_split_cap, n_groups <= POLY_RAW_MAX_GROUPS, &p.split_log, &p.blocks);
@@ -4285,6 +4590,7 @@ FusedRound::Plan FusedRound::plan_round(u32 jj, bool skip1_jj) const
 // waits for the mail of sequence number `seq_jj` and takes the challenge and the message's scalars from it.
 int32_t FusedRound::launch_round(u32 jj, const Plan &p, bool skip1_jj, bool ahead, u64 seq_jj)
 {
+        if (weighted()) return launch_weighted(jj, skip1_jj, ahead, seq_jj);
         dpk::PolyArgs pa;
         pa.groups = sc->d_poly_groups + (size_t)(jj - 1) * n_groups;
         pa.terms = sc->d_poly_terms;
@@ -4372,6 +4678,47 @@ int32_t FusedRound::launch_round(u32 jj, const Plan &p, bool skip1_jj, bool ahea
         return DPS_OK;
 }
 
+// The launch of round jj of a sum over several eq factors (wsum_kernel); `ahead`, seq_jj: as above
+int32_t FusedRound::launch_weighted(u32 jj, bool skip1_jj, bool ahead, u64 seq_jj)
+{
+        dpk::WsumArgs wa;
+        memset(&wa, 0, sizeof wa);
+        const dpk::PolyGroup &pg = sc->h_poly_groups[jj - 1];
+        bool base = true;
+        for (u32 k = 0; k < pg.n_tabs; k++) {
+            wa.tab[k] = pg.tab[k];
+            base = base && pg.tab[k].mode == dpk::POLY_PAIR && !pg.tab[k].s1;
+        }
+        wa.n_tabs = pg.n_tabs;
+        wa.n_eqs = (u32)sc->weq.size();
+        const bool fact = poly_round_weights_factored(sc, jj);
+        const u64 off = eq_level_off(sc->n_vars, jj), lo = fact ? eq_low_off(sc->n_vars, jj) : 0, hi = fact ? eq_level_off(sc->n_vars, jj + dpk::EQ_LO_BITS) : 0;
+        for (u32 g = 0; g < wa.n_eqs; g++) {
+            const dps_sc::WeightedEq &w = sc->weq[g];
+            wa.op_begin[g] = w.op_begin, wa.op_end[g] = w.op_end, wa.degree[g] = w.degree;
+            if (w.base_program) wa.base_program |= 1u << g;
+            wa.q0[g] = w.c0 + off, wa.q1[g] = w.c1 + off;
+            if (fact) wa.lq0[g] = w.c0 + lo, wa.lq1[g] = w.c1 + lo, wa.hq0[g] = w.c0 + hi, wa.hq1[g] = w.c1 + hi;
+        }
+        std::copy(sc->h_poly_ops.begin(), sc->h_poly_ops.end(), wa.ops);
+        wa.n_pairs = 1ull << (sc->n_vars - jj);
+        wa.r0 = ahead ? 0 : a.r0;
+        wa.r1 = ahead ? 0 : a.r1;
+        const u32 n_blocks = blocks_for_pairs(wa.n_pairs);
+        wa.wait_first = ahead ? 1 : 0;
+        wa.spin_limit = wait_units(ctx, AHEAD_SPIN_LIMIT);
+        wa.mail = ctx->d_pinned + (ctx->res_off - 64);
+        wa.relay = ahead && n_blocks > POLY_AHEAD_MAX_WORKGROUPS ? mail_relay(ctx) : nullptr;
+        dpk::FastFin fl = ff;
+        fl.seq = seq_jj;
+        fl.n_blocks = n_blocks;
+        fl.slots = nullptr;
+        ProfScope ps(ctx, DPS_K_EVAL_TERMS, (double)wa.n_pairs * pg.n_tabs * (jj >= 2 ? 4 * 16.0 + 2 * 16.0 : 2 * 16.0));
+        CHK(launch_wsum(ctx, skip1_jj, base, wa, n_blocks, sc->d_partial, fl));
+        HIPCHK(ctx, hipGetLastError());
+        return DPS_OK;
+}
+
 // A round of sums of several terms over shared tables (poly_kernel / poly_split_kernel): this round's launch, or the mail for
 // one that waits on the GPU; then the next round's launch behind it.
 int32_t FusedRound::multi_term_round()
@@ -4415,8 +4762,8 @@ int32_t FusedRound::multi_term_round()
         if (j < sc->n_vars && !ctx->profiling && !sc->no_ahead) {
             // p(1) comes from the claim unless the scale vanishes at 1, i.e. unless the eq point is 0 there
             bool skip1_next = true;
-            if (has_eq) {
-                const E2 rho = sc->eq_info->point[j];
+            if (has_eq || weighted()) {
+                const E2 rho = (weighted() ? sc->weq[0].info : sc->eq_info)->point[j];
                 skip1_next = !(rho.c0 == 0 && rho.c1 == 0);
             }
             const Plan pn = plan_round(j + 1, skip1_next);
@@ -4442,7 +4789,7 @@ int32_t FusedRound::multi_term_round()
             }
         }
     }
-    int32_t rc = take_sums(slots_now);
+    int32_t rc = weighted() ? take_weighted_sums() : take_sums(slots_now);
     if (rc != DPS_OK) {
         // a launch that left without publishing may have taken some of its tickets and written some of its tables
         sc->broken = true;
@@ -4852,6 +5199,20 @@ extern "C" int32_t dps_sc_round(dps_sc *sc, const uint64_t *challenge, uint64_t 
     return DPS_OK;
 }
 
+namespace {
+
+// The final evaluations of the eq tables of a sum over several of them; `r`: the last challenge
+void weighted_eq_finals(const dps_sc *sc, E2 r, uint64_t *final_evals_out)
+{
+    for (const dps_sc::WeightedEq &w : sc->weq) {
+        const E2 v = gl::mul(w.scalar, h_eq1(w.info->point[sc->n_vars - 1], r));
+        final_evals_out[2 * w.k] = v.c0;
+        final_evals_out[2 * w.k + 1] = v.c1;
+    }
+}
+
+}  // namespace
+
 extern "C" int32_t dps_sc_finish(dps_sc *sc, const uint64_t *challenge, uint64_t *final_evals_out)
 {
     if (!sc || (sc->n_mles && !final_evals_out)) return DPS_ERR_INVALID;
@@ -4901,6 +5262,7 @@ extern "C" int32_t dps_sc_finish(dps_sc *sc, const uint64_t *challenge, uint64_t
             final_evals_out[2 * sc->fast_eq] = v.c0;
             final_evals_out[2 * sc->fast_eq + 1] = v.c1;
         }
+        weighted_eq_finals(sc, r, final_evals_out);
         sc->finished = true;
         return DPS_OK;
     }
@@ -4919,6 +5281,7 @@ extern "C" int32_t dps_sc_finish(dps_sc *sc, const uint64_t *challenge, uint64_t
         final_evals_out[2 * sc->fast_eq] = v.c0;
         final_evals_out[2 * sc->fast_eq + 1] = v.c1;
     }
+    if (sc->n_vars >= 1) weighted_eq_finals(sc, gl::e2(challenge[0], challenge[1]), final_evals_out);
     sc->finished = true;
     return DPS_OK;
 }

@@ -1471,6 +1471,161 @@ __global__ void __launch_bounds__(PAIR12_BLOCK) pair12_kernel(Pair12Args a, u64 
 }
 
 // ---------------------------------------------------------------------------
+// nested programs of sums of several terms
+// ---------------------------------------------------------------------------
+// The terms of a group in nested form: factoring the most frequent table out of the terms that contain it, again
+// and again, turns sum_k c_k prod table into a tree whose every edge is one product,
+//     G = c + sum_children table_child * G_child.
+// The tree is walked depth first with one running value per depth:
+//     ENTER d, c      acc[d] = c                          (a node with children; c = coefficient of the term ending here, or 0)
+//     LEAF  d, s, c   acc[d] += table_s * c               (a child without children)
+//     LEAVE d, s      acc[d - 1] += table_s * acc[d]      (back to the parent)
+// and G = acc[0].  One product per edge instead of one per factor and coefficient of every term.
+constexpr u32 POLY_OP_ENTER = 0, POLY_OP_LEAF = 1, POLY_OP_LEAVE = 2;
+struct PolyOp {
+    u64 c0, c1, w;  // coefficient, prepared (ENTER, LEAF)
+    u32 code;       // kind | depth << 2 | class of the coefficient << 6 | slot << 8
+    u32 pad;
+};
+// What a LEAF's coefficient is (told by the program's builder; wsum_walk saves the product or half of it)
+constexpr u32 POLY_COEFF_ANY = 0, POLY_COEFF_ONE = 1, POLY_COEFF_MINUS_ONE = 2, POLY_COEFF_BASE = 3;
+
+// A node of the nested program at depth D: starts from its constant, adds table * c for every LEAF, table * (child's
+// value) for every child (ENTER D + 1 ... LEAVE D + 1, walked by the next depth's function), and ends at the LEAVE of its
+// own depth, which it leaves for its parent to read the table from (or at the end of the program: the root).
+// `op(o)`: operation o; `table(slot)`: the slot's table at the evaluation point in hand.
+template <int D, int MAXD, typename OpAt, typename TableAt>
+__device__ __forceinline__ E2 poly_walk(u32 &pc, u32 n_ops, E2 acc, OpAt &&op, TableAt &&table)
+{
+    while (pc < n_ops) {
+        const PolyOp &o = op(pc);
+        const u32 code = __builtin_amdgcn_readfirstlane(o.code);
+        const u32 kind = code & 3, sl = code >> 8;
+        if (kind == POLY_OP_LEAF) {
+            gl::E2P cp;
+            cp.c0 = o.c0;
+            cp.c1 = o.c1;
+            cp.w = o.w;
+            acc = gl::fma(table(sl), cp, acc);
+            pc++;
+        } else if (kind == POLY_OP_ENTER) {
+            pc++;
+            if constexpr (D < MAXD) {
+                const E2 child = poly_walk<D + 1, MAXD>(pc, n_ops, gl::e2(o.c0, o.c1), op, table);
+                // (the child stopped at its LEAVE, which names the table on the edge to it)
+                const u32 edge = __builtin_amdgcn_readfirstlane(op(pc).code) >> 8;
+                acc = gl::fma(child, gl::prep(table(edge)), acc);
+                pc++;
+            }
+        } else {
+            break;
+        }
+    }
+    return acc;
+}
+
+// The walk of a program at N points at once: an operation is fetched and decoded once, a table's value and slope are read
+// once, and the points' products do not depend on one another.  (With a walk per point the round of 2^19 pairs of the sum that links an
+// activation to its lookups took 64 us, the fetches one behind the other.)  The coefficients' classes are used, and tables of
+// base-field entries (T = u64) where that is what a round reads: a product is then two base products, or one where the running
+// value is in the base field as well (V = u64, programs all of whose coefficients are).
+__device__ __forceinline__ E2 wsum_add(E2 acc, E2 t) { return gl::add(acc, t); }
+__device__ __forceinline__ E2 wsum_add(E2 acc, u64 t) { return gl::e2(gl::add(acc.c0, t), acc.c1); }
+__device__ __forceinline__ u64 wsum_add(u64 acc, u64 t) { return gl::add(acc, t); }
+__device__ __forceinline__ E2 wsum_sub(E2 acc, E2 t) { return gl::sub(acc, t); }
+__device__ __forceinline__ E2 wsum_sub(E2 acc, u64 t) { return gl::e2(gl::sub(acc.c0, t), acc.c1); }
+__device__ __forceinline__ u64 wsum_sub(u64 acc, u64 t) { return gl::sub(acc, t); }
+__device__ __forceinline__ E2 wsum_base(E2 acc, E2 t, u64 c) { return gl::e2(gl::muladd(t.c0, c, acc.c0), gl::muladd(t.c1, c, acc.c1)); }
+__device__ __forceinline__ E2 wsum_base(E2 acc, u64 t, u64 c) { return gl::e2(gl::muladd(t, c, acc.c0), acc.c1); }
+__device__ __forceinline__ u64 wsum_base(u64 acc, u64 t, u64 c) { return gl::muladd(t, c, acc); }
+__device__ __forceinline__ E2 wsum_any(E2 acc, E2 t, gl::E2P c) { return gl::fma(t, c, acc); }
+__device__ __forceinline__ E2 wsum_any(E2 acc, u64 t, gl::E2P c) { return gl::e2(gl::muladd(c.c0, t, acc.c0), gl::muladd(c.c1, t, acc.c1)); }
+__device__ __forceinline__ u64 wsum_any(u64 acc, u64 t, gl::E2P c) { return gl::muladd(c.c0, t, acc); }
+// acc + child * table
+__device__ __forceinline__ E2 wsum_edge(E2 acc, E2 child, E2 t) { return gl::fma(child, gl::prep(t), acc); }
+__device__ __forceinline__ E2 wsum_edge(E2 acc, E2 child, u64 t) { return gl::e2(gl::muladd(child.c0, t, acc.c0), gl::muladd(child.c1, t, acc.c1)); }
+__device__ __forceinline__ u64 wsum_edge(u64 acc, u64 child, u64 t) { return gl::muladd(child, t, acc); }
+template <class V>
+__device__ __forceinline__ V wsum_const(const PolyOp &o)
+{
+    if constexpr (std::is_same_v<V, u64>)
+        return o.c0;
+    else
+        return gl::e2(o.c0, o.c1);
+}
+template <class T, int N>
+struct WsumPoints {
+    T v[N];
+};
+// a table's values at the points 0, 1, 2, .. or (SKIP) 0, 2, 3, .. from its value at 0 and its slope
+template <int N, bool SKIP, class T>
+__device__ __forceinline__ WsumPoints<T, N> wsum_points(T lo, T d)
+{
+    WsumPoints<T, N> p;
+    p.v[0] = lo;
+    T x = SKIP ? gl::add(lo, d) : lo;
+#pragma unroll
+    for (int i = 1; i < N; i++) p.v[i] = x = gl::add(x, d);
+    return p;
+}
+// `table(slot)`: the table's values at the points
+template <int D, int MAXD, int N, class V, typename OpAt, typename TableAt>
+__device__ __forceinline__ void wsum_walk(u32 &pc, u32 n_ops, V (&acc)[N], OpAt &&op, TableAt &&table)
+{
+    while (pc < n_ops) {
+        const PolyOp &o = op(pc);
+        const u32 code = __builtin_amdgcn_readfirstlane(o.code);
+        const u32 kind = code & 3, cls = (code >> 6) & 3, sl = code >> 8;
+        if (kind == POLY_OP_LEAF) {
+            const auto t = table(sl);
+            if (cls == POLY_COEFF_ONE) {
+#pragma unroll
+                for (int i = 0; i < N; i++) acc[i] = wsum_add(acc[i], t.v[i]);
+            } else if (cls == POLY_COEFF_MINUS_ONE) {
+#pragma unroll
+                for (int i = 0; i < N; i++) acc[i] = wsum_sub(acc[i], t.v[i]);
+            } else if (cls == POLY_COEFF_BASE) {
+#pragma unroll
+                for (int i = 0; i < N; i++) acc[i] = wsum_base(acc[i], t.v[i], o.c0);
+            } else {
+                gl::E2P cp;
+                cp.c0 = o.c0;
+                cp.c1 = o.c1;
+                cp.w = o.w;
+#pragma unroll
+                for (int i = 0; i < N; i++) acc[i] = wsum_any(acc[i], t.v[i], cp);
+            }
+            pc++;
+        } else if (kind == POLY_OP_ENTER) {
+            pc++;
+            if constexpr (D < MAXD) {
+                V child[N];
+#pragma unroll
+                for (int i = 0; i < N; i++) child[i] = wsum_const<V>(o);
+                wsum_walk<D + 1, MAXD, N, V>(pc, n_ops, child, op, table);
+                const u32 edge = __builtin_amdgcn_readfirstlane(op(pc).code) >> 8;
+                const auto t = table(edge);
+#pragma unroll
+                for (int i = 0; i < N; i++) acc[i] = wsum_edge(acc[i], child[i], t.v[i]);
+                pc++;
+            }
+        } else {
+            break;
+        }
+    }
+}
+// a whole program; its first operation enters the root with the constant
+template <int DEGREE, int N, class V, typename OpAt, typename TableAt>
+__device__ __forceinline__ void wsum_program(u32 begin, u32 end, V (&out)[N], OpAt &&op, TableAt &&table)
+{
+    const PolyOp &root = op(begin);
+#pragma unroll
+    for (int i = 0; i < N; i++) out[i] = wsum_const<V>(root);
+    u32 pc = begin + 1;
+    wsum_walk<0, DEGREE - 1, N, V>(pc, end, out, op, table);
+}
+
+// ---------------------------------------------------------------------------
 // slice kernel: the rounds of a product sumcheck that are latency, not bytes
 //
 // Once a round moves a few megabytes a launch per round is pure latency (dispatch, a wavefront's instruction stream,
@@ -1538,11 +1693,12 @@ struct SliceTerm {
     u64 c0, c1, w;
     u32 n_factors;
     uint8_t slot[DPS_MAX_FACTORS];
-    u32 pad;
+    u32 eq;  // (host: the eq factor it belongs to, in a sum over several)
 };
 template <int TABS_, int TERMS_, bool LACKS_>
 struct SliceArgsOf {
     static constexpr int TABS = TABS_, TERMS = TERMS_;
+    static constexpr u32 EQS = 0;  // (SliceArgsEqs: several eq factors)
     static constexpr bool LACKS = LACKS_;  // tables of fewer variables are among them
     const u64 *s0[TABS];
     const u64 *s1[TABS];         // the tables before the folds that are pending when the launch starts: src_len entries each
@@ -1586,6 +1742,21 @@ struct SliceArgsOf {
 using SliceArgs = SliceArgsOf<SL_MAX_TABS, SL_MAX_TERMS, true>;
 using SliceArgsFew = SliceArgsOf<SL_FEW_TABS, SL_FEW_TERMS, false>;
 using SliceArgsProduct = SliceArgsOf<4, 1, false>;  // (at most 3 tables, no terms)
+// A sum over several eq factors, sum_g eq(rho_g, x) P_g(x) with polynomials P_g over shared tables (wsum_kernel says why they are kept
+// apart).  The weights of every factor live in LDS; P_g is a nested program in the terms' place, walked by lanes of its own, whole
+// wavefronts of them, so that a wavefront runs one program.  Sums: P_g's q_g(t), t = 0 .. degree[g], from off_q[g] on; with a trip of two
+// rounds, from off_d[g] on, those of the second round at its points (t = 0, 2, .. for the first factor, whose t = 1 comes from
+// the claim, t = 0, 1, 2, .. for the others), each at the challenges 0 .. degree[g] (a polynomial of that degree in the challenge).
+constexpr u32 SL_MAX_EQS = 3;
+constexpr int SL_EQS_OPS = 64;
+struct SliceArgsEqs : SliceArgsOf<8, SL_EQS_OPS * (int)sizeof(PolyOp) / (int)sizeof(SliceTerm) + 1, false> {
+    static constexpr u32 EQS = SL_MAX_EQS;
+    u32 n_eqs, hw_stride;               // hw0, hw1: hw_stride words for every factor
+    const u64 *geq0[SL_MAX_EQS], *geq1[SL_MAX_EQS];
+    u32 degree[SL_MAX_EQS], off_q[SL_MAX_EQS], off_d[SL_MAX_EQS], op_begin[SL_MAX_EQS], op_end[SL_MAX_EQS];
+    u32 n_sums1, n_sums2;               // of a trip of one round, of two
+};
+static_assert(sizeof(SliceArgsEqs) <= 4096 && sizeof(SliceArgsEqs::terms) >= SL_EQS_OPS * sizeof(PolyOp), "kernel arguments");
 static_assert(sizeof(SliceArgs) <= 4096, "kernel arguments");
 
 // dynamic LDS of slice_kernel, in 64-bit words: counters per wavefront, mailbox copy, flags, the terms, then the two table buffers
@@ -1598,9 +1769,10 @@ __host__ __device__ constexpr u32 sl_lds_tables(u32 blk, u32 terms) { return sl_
 static_assert(sizeof(SliceTerm) % 8 == 0, "terms are copied as 64-bit words");
 // (`eq`: the weights of the eq factor, one per pair of a table's entries, are kept like a table of half the size)
 __host__ __device__ constexpr u32 sl_weights_cap(u32 cap) { return cap / 2 > 0 ? cap / 2 : 1; }
-__host__ __device__ constexpr u32 slice_lds_words(u32 n_tabs, u32 cap, u32 blk, bool eq, u32 terms = SL_MAX_TERMS)
+// (`eq`: how many eq factors there are)
+__host__ __device__ constexpr u32 slice_lds_words(u32 n_tabs, u32 cap, u32 blk, u32 eq, u32 terms = SL_MAX_TERMS)
 {
-    return sl_lds_tables(blk, terms) + n_tabs * 2 * (cap + cap / 2) + (eq ? 2 * (sl_weights_cap(cap) + sl_weights_cap(cap / 2)) : 0);
+    return sl_lds_tables(blk, terms) + n_tabs * 2 * (cap + cap / 2) + eq * 2 * (sl_weights_cap(cap) + sl_weights_cap(cap / 2));
 }
 // A workgroup of these launches is 1024 threads: what a round costs here is the longest chain of dependent field
 // multiplications in any one lane, and with more lanes each has fewer units of work behind one another.
@@ -1639,10 +1811,21 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
     // The weights of the eq factor, R_j(p) = eq(rho_{j+1..}, p) for the pairs p of round j, live beside the tables in the
     // same two buffers: read once when the launch starts, and from round to round the weight of a pair is the sum of the
     // weights of the two pairs it is made of (R_{j+1}(p) = R_j(2p) + R_j(2p + 1)), so a fold of the tables is an add here.
-    u64 *const wts_big = buf_small + (size_t)nt * 2 * (cap / 2), *const wts_small = wts_big + 2 * sl_weights_cap(cap);
-    auto wts = [&](bool big, int limb) -> u64 * { return big ? wts_big + (size_t)limb * sl_weights_cap(cap) : wts_small + (size_t)limb * sl_weights_cap(cap / 2); };
-    auto weight = [&](bool big, u32 p) { return gl::e2(wts(big, 0)[p], wts(big, 1)[p]); };
-    if (TERMS) {
+    // (several eq factors: `g` is the factor, their weights follow one another)
+    static_assert(ARGS::EQS == 0 || (EQ && TERMS), "several eq factors belong to a sum of several terms");
+    u32 n_eqs = 1;
+    if constexpr (ARGS::EQS > 0) n_eqs = a.n_eqs;
+    u64 *const wts_big = buf_small + (size_t)nt * 2 * (cap / 2), *const wts_small = wts_big + n_eqs * 2 * sl_weights_cap(cap);
+    auto wts = [&](bool big, int limb, u32 g = 0) -> u64 * {
+        return big ? wts_big + (size_t)(2 * g + limb) * sl_weights_cap(cap) : wts_small + (size_t)(2 * g + limb) * sl_weights_cap(cap / 2);
+    };
+    auto weight = [&](bool big, u32 p, u32 g = 0) { return gl::e2(wts(big, 0, g)[p], wts(big, 1, g)[p]); };
+    if constexpr (ARGS::EQS > 0) {
+        // the programs, in the terms' place
+        const u64 *src = reinterpret_cast<const u64 *>(a.terms);
+        u64 *dst = dyn + SL_LDS_TERMS;
+        for (u32 w = tid; w < a.op_end[a.n_eqs - 1] * (u32)(sizeof(PolyOp) / 8); w += BLOCK) dst[w] = src[w];
+    } else if (TERMS) {
         // the terms are read per pair and point: staged in LDS once (visible after the first wait's barrier)
         const u64 *src = reinterpret_cast<const u64 *>(a.terms);
         u64 *dst = dyn + SL_LDS_TERMS;
@@ -1668,7 +1851,13 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
                 st_agent(a.h0[f] + (u64)wg * len + i, tab(in_big, f, 0)[i]);
                 st_agent(a.h1[f] + (u64)wg * len + i, tab(in_big, f, 1)[i]);
             }
-            if (EQ)
+            if constexpr (ARGS::EQS > 0) {
+                for (u32 g = 0; g < n_eqs; g++)
+                    for (u32 i = tid; i < (len >> 1); i += BLOCK) {
+                        st_agent(a.hw0 + (u64)g * a.hw_stride + (u64)wg * (len >> 1) + i, wts(in_big, 0, g)[i]);
+                        st_agent(a.hw1 + (u64)g * a.hw_stride + (u64)wg * (len >> 1) + i, wts(in_big, 1, g)[i]);
+                    }
+            } else if (EQ)
                 for (u32 i = tid; i < (len >> 1); i += BLOCK) {
                     st_agent(a.hw0 + (u64)wg * (len >> 1) + i, wts(in_big, 0)[i]);
                     st_agent(a.hw1 + (u64)wg * (len >> 1) + i, wts(in_big, 1)[i]);
@@ -1808,15 +1997,33 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
                 tab(!in_big, f, 1)[i] = v.c1;
             }
             if (EQ)
-                for (u32 i = tid; i < (len >> 1); i += BLOCK) {
-                    E2 v = weight(in_big, i << pend);
-                    for (u32 q = 1; q < (1u << pend); q++) v = gl::add(v, weight(in_big, (i << pend) + q));
-                    wts(!in_big, 0)[i] = v.c0;
-                    wts(!in_big, 1)[i] = v.c1;
-                }
+                for (u32 g = 0; g < n_eqs; g++)
+                    for (u32 i = tid; i < (len >> 1); i += BLOCK) {
+                        E2 v = weight(in_big, i << pend, g);
+                        for (u32 q = 1; q < (1u << pend); q++) v = gl::add(v, weight(in_big, (i << pend) + q, g));
+                        wts(!in_big, 0, g)[i] = v.c0;
+                        wts(!in_big, 1, g)[i] = v.c1;
+                    }
             in_big = !in_big;
         }
-        if (EQ && k == 0) {
+        if constexpr (ARGS::EQS > 0) {
+            if (k == 0 || regroup)
+                for (u32 g = 0; g < n_eqs; g++) {
+                    const u64 e0 = ((2ull << a.n_vars) - (2ull << (a.n_vars - j))) + (u64)wg * (len >> 1);
+                    for (u32 i = tid; i < (len >> 1); i += BLOCK) {
+                        E2 v;
+                        if (k == 0) {
+                            v = gl::e2(a.geq0[g][e0 + i], a.geq1[g][e0 + i]);
+                        } else {
+                            const u64 e = (u64)g * a.hw_stride + ((u64)i << pend);
+                            v = gl::e2(a.hw0[e], a.hw1[e]);
+                            for (u32 q = 1; q < (1u << pend); q++) v = gl::add(v, gl::e2(a.hw0[e + q], a.hw1[e + q]));
+                        }
+                        wts(true, 0, g)[i] = v.c0;
+                        wts(true, 1, g)[i] = v.c1;
+                    }
+                }
+        } else if (EQ && k == 0) {
             // the weights of round j's pairs, from the eq table's level of that round
             const u64 e0 = ((2ull << a.n_vars) - (2ull << (a.n_vars - j))) + (u64)wg * (len >> 1);
             for (u32 i = tid; i < (len >> 1); i += BLOCK) {
@@ -1834,7 +2041,9 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
             }
         }
         // this wavefront's counters start the trip at zero
-        for (u32 c = lane; c < 4 * (u32)NS; c += WAVE) ctr[wave * 4 * SL_MAX_SUMS + c] = 0;
+        u32 ns = NS;  // sums of this trip
+        if constexpr (ARGS::EQS > 0) ns = dbl ? a.n_sums2 : a.n_sums1;
+        for (u32 c = lane; c < 4 * ns; c += WAVE) ctr[wave * 4 * SL_MAX_SUMS + c] = 0;
         __syncthreads();
         const bool big = in_big;
         // adds a lane's canonical sum into the counters of extension sum `idx`
@@ -1844,6 +2053,23 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
             atomicAdd(reinterpret_cast<unsigned long long *>(c + 1), (unsigned long long)(v.c0 >> 32));
             atomicAdd(reinterpret_cast<unsigned long long *>(c + 2), (unsigned long long)(u32)v.c1);
             atomicAdd(reinterpret_cast<unsigned long long *>(c + 3), (unsigned long long)(v.c1 >> 32));
+        };
+        // the same for a wavefront all of whose lanes have a share of one sum (`wanted`: the same in all of them): added up first
+        auto flush_wave = [&](u32 idx, E2 v, bool wanted) {
+            if (!wanted) return;
+            u64 *c = ctr + wave * 4 * SL_MAX_SUMS + 4 * idx;
+#pragma unroll
+            for (int limb = 0; limb < 2; limb++) {
+                const u64 x = limb ? v.c1 : v.c0;
+                const u32 lo = (u32)x, hi = (u32)(x >> 32);
+                const u64 c0 = wave_sum_u32(lo & 0x3FFFFFu), c1 = wave_sum_u32((lo >> 22) | ((hi & 0xFFFu) << 10)), c2 = wave_sum_u32(hi >> 12);
+                // c0 + c1 2^22 + c2 2^44, as low 32 bits and the rest
+                const u64 low = c0 + (c1 << 22);
+                if (lane == WAVE - 1) {
+                    c[2 * limb] += (u32)low;
+                    c[2 * limb + 1] += (low >> 32) + (c2 << 12);
+                }
+            }
         };
         // entry e of table f of the state
         auto ent = [&](u32 f, u32 e) { return gl::e2(tab(big, f, 0)[e], tab(big, f, 1)[e]); };
@@ -1888,7 +2114,68 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
         // dependent instructions, so the work of a pair is cut into units of one evaluation point (and one term) each
         // and spread over the lanes; every unit's value goes into the point's counters, where the pieces add up.
         // ---- round j: pairs of the state; units taken from the last thread down, those of the quads from the first up ----
-        {
+        if constexpr (ARGS::EQS > 0) {
+            // This wavefront's factor, and this lane's place among the lanes of that factor.  A unit of work is a pair, or with a trip of two
+            // rounds a quad at one challenge (first the pairs, then the quads challenge by challenge): a lane walks the program at
+            // all of its factor's points, and where a wavefront's units are of one kind it adds its sums up before they go into the
+            // counters (a counter that every lane adds to serves them one after the other).
+            const u32 per = (BLOCK / n_eqs) & ~(u32)(WAVE - 1);
+            const u32 g = __builtin_amdgcn_readfirstlane(tid / per), l = tid - g * per;
+            auto units = [&](auto n_points, auto skips, auto program_degree) {
+                constexpr int N = decltype(n_points)::value, DEG = decltype(program_degree)::value;
+                constexpr bool SKIP = decltype(skips)::value;
+                const PolyOp *ops = reinterpret_cast<const PolyOp *>(lterms);
+                const u32 d = a.degree[g], npt = g == 0 ? d : d + 1;  // (points of a round that takes p(1) from its claim)
+                const u32 n_pairs = len >> 1, n_quads = len >> 2, n_units = n_pairs + (dbl ? n_quads * (d + 1) : 0);
+                const u32 quads_log = len_log >= 2 ? len_log - 2 : 0;
+                for (u32 base = 0; base < n_units; base += per) {
+                    const u32 u = base + l;
+                    const bool mine = u < n_units, pair = u < n_pairs;
+                    const u32 v = pair || !mine ? 0 : u - n_pairs, smp = v >> quads_log, at = !mine ? 0 : pair ? u : v & (n_quads - 1);
+                    auto table = [&](u32 f) {
+                        E2 lo, hi;
+                        if (pair || !mine) {
+                            lo = ent(f, 2 * at), hi = ent(f, 2 * at + 1);
+                        } else {
+                            lo = line_at(ent(f, 4 * at), ent(f, 4 * at + 1), smp), hi = line_at(ent(f, 4 * at + 2), ent(f, 4 * at + 3), smp);
+                        }
+                        return wsum_points<N, SKIP>(lo, gl::sub(hi, lo));
+                    };
+                    E2 out[N];
+                    wsum_program<DEG>(a.op_begin[g], a.op_end[g], out, [&](u32 o) -> const PolyOp & { return ops[o]; }, table);
+                    E2 w = gl::e2_zero();
+                    if (mine) w = pair ? weight(big, at, g) : gl::add(weight(big, 2 * at, g), weight(big, 2 * at + 1, g));
+                    const gl::E2P wp = gl::prep(w);
+                    // where the sums of point i go: those of pairs from off_q on, those of quads from off_d on
+                    const u32 kind = !mine ? ~0u : pair ? 0 : 1 + smp;
+                    const bool alike = __shfl(kind, 0, WAVE) == __shfl(kind, WAVE - 1, WAVE);
+#pragma unroll
+                    for (int i = 0; i < N; i++) {
+                        const u32 t = SKIP && i > 0 ? (u32)i + 1 : (u32)i;
+                        const u32 ti = g == 0 && t > 1 ? t - 1 : t;
+                        const bool wanted = mine && t <= d && (pair ? !(g == 0 && t == 1 && skip1) : !(g == 0 && t == 1));
+                        const u32 idx = pair ? a.off_q[g] + t : a.off_d[g] + smp * npt + ti;
+                        const E2 x = gl::mulp(out[i], wp);
+                        if (alike)
+                            flush_wave(idx, x, wanted);
+                        else if (wanted)
+                            flush(idx, x);
+                    }
+                }
+            };
+            // (the first factor's polynomial is of the highest degree, NF)
+            if (g == 0) {
+                if (skip1)
+                    units(std::integral_constant<int, NF>{}, std::true_type{}, std::integral_constant<int, NF>{});
+                else
+                    units(std::integral_constant<int, NF + 1>{}, std::false_type{}, std::integral_constant<int, NF>{});
+            } else if (g < n_eqs) {
+                if (a.degree[g] == 1)
+                    units(std::integral_constant<int, 2>{}, std::false_type{}, std::integral_constant<int, 1>{});
+                else
+                    units(std::integral_constant<int, NF + 1>{}, std::false_type{}, std::integral_constant<int, NF>{});
+            }
+        } else {
             const u32 n_pairs = len >> 1;
             const u32 rt = BLOCK - 1 - tid;
             const u32 m0 = rt % p_split, t = (rt / p_split) % (u32)NP, slot = rt / (p_split * (u32)NP), n_slots = BLOCK / (p_split * (u32)NP);
@@ -1904,7 +2191,7 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
             if (any) flush(t, acc);
         }
         // ---- round j + 1 as a polynomial in the challenge of round j: quads of the state ----
-        if (dbl) {
+        if (ARGS::EQS == 0 && dbl) {
             const u32 n_quads = len >> 2;
             // a lane keeps one sample at one point (of some of the terms)
             const u32 m0 = tid % q_split, ti = (tid / q_split) % (u32)NPT, smp = (tid / (q_split * (u32)NPT)) % (u32)NSMP;
@@ -1931,7 +2218,7 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
         }
         __syncthreads();
         // ---- hand the sums over: one counter per lane ----
-        if (tid < 4 * (u32)NS && !(skip1 && tid >= 4 && tid < 8)) {
+        if (tid < 4 * ns && !(skip1 && tid >= 4 && tid < 8)) {
             const u32 c = tid;
             u64 v = 0;
 #pragma unroll
@@ -2050,20 +2337,6 @@ struct PolyTerm {
     uint8_t slot[DPS_MAX_FACTORS];  // table slots within the group
     u32 pad;
 };
-// The terms of a group in nested form: factoring the most frequent table out of the terms that contain it, again
-// and again, turns sum_k c_k prod table into a tree whose every edge is one product,
-//     G = c + sum_children table_child * G_child.
-// The tree is walked depth first with one running value per depth:
-//     ENTER d, c      acc[d] = c                          (a node with children; c = coefficient of the term ending here, or 0)
-//     LEAF  d, s, c   acc[d] += table_s * c               (a child without children)
-//     LEAVE d, s      acc[d - 1] += table_s * acc[d]      (back to the parent)
-// and G = acc[0].  One product per edge instead of one per factor and coefficient of every term.
-constexpr u32 POLY_OP_ENTER = 0, POLY_OP_LEAF = 1, POLY_OP_LEAVE = 2;
-struct PolyOp {
-    u64 c0, c1, w;  // coefficient, prepared (ENTER, LEAF)
-    u32 code;       // kind | depth << 2 | slot << 8
-    u32 pad;
-};
 constexpr int POLY_LDS_OPS = POLY_LDS_TERMS * 40 / 32;  // a program shares the terms' place in LDS and in the kernel arguments
 static_assert(sizeof(PolyTerm) == 40 && sizeof(PolyOp) == 32, "terms and operations share storage");
 static_assert(HOST_FINALS_SLOT + 4 * POLY_MAXT <= HOST_PAIRS_SEQ_SLOT && 4 * POLY_MAXT <= 6 * MAX_PTS, "last pairs of a group fit its result area");
@@ -2123,40 +2396,6 @@ template <int N, typename F>
 __device__ __forceinline__ void static_for(F &&f)
 {
     static_for_each(f, std::make_integer_sequence<int, N>{});
-}
-
-// A node of the nested program at depth D: starts from its constant, adds table * c for every LEAF, table * (child's
-// value) for every child (ENTER D + 1 ... LEAVE D + 1, walked by the next depth's function), and ends at the LEAVE of its
-// own depth, which it leaves for its parent to read the table from (or at the end of the program: the root).
-// `op(o)`: operation o; `table(slot)`: the slot's table at the evaluation point in hand.
-template <int D, int MAXD, typename OpAt, typename TableAt>
-__device__ __forceinline__ E2 poly_walk(u32 &pc, u32 n_ops, E2 acc, OpAt &&op, TableAt &&table)
-{
-    while (pc < n_ops) {
-        const PolyOp &o = op(pc);
-        const u32 code = __builtin_amdgcn_readfirstlane(o.code);
-        const u32 kind = code & 3, sl = code >> 8;
-        if (kind == POLY_OP_LEAF) {
-            gl::E2P cp;
-            cp.c0 = o.c0;
-            cp.c1 = o.c1;
-            cp.w = o.w;
-            acc = gl::fma(table(sl), cp, acc);
-            pc++;
-        } else if (kind == POLY_OP_ENTER) {
-            pc++;
-            if constexpr (D < MAXD) {
-                const E2 child = poly_walk<D + 1, MAXD>(pc, n_ops, gl::e2(o.c0, o.c1), op, table);
-                // (the child stopped at its LEAVE, which names the table on the edge to it)
-                const u32 edge = __builtin_amdgcn_readfirstlane(op(pc).code) >> 8;
-                acc = gl::fma(child, gl::prep(table(edge)), acc);
-                pc++;
-            }
-        } else {
-            break;
-        }
-    }
-    return acc;
 }
 
 template <int NF, bool EQ, bool SKIP1>
@@ -2358,7 +2597,197 @@ __global__ void __launch_bounds__(BLOCK) poly_kernel(PolyArgs a, u64 *__restrict
     }
 }
 
-// The same sum for rounds of few pairs, where a launch is one serial chain per thread: the work of a pair is
+// ---------------------------------------------------------------------------
+// sums over several eq factors: sum_g eq(rho_g, x) P_g(x), P_g polynomials over a few shared tables
+//
+// Every factor is taken in closed form as prod_kernel takes its one: bound below v it is S_g eq1(rho_g,v, x_v) R_g(x'), the launch sums
+//     q_g(t) = sum_x' R_g(x') P_g(t, x'),   t = 0 .. deg P_g,
+// for every factor apart, and the host forms p(t) = sum_g S_g eq1(rho_g,v, t) q_g(t).  No eq table is read at a round's size, folded or
+// written, the programs are of a degree less, and a factor of low degree is evaluated at its own few points.  (With the eq tables as
+// tables among the others -- poly_kernel -- the sum that links an activation to its lookups, eq (v - b^2 v + c b^2 + d b) + eq' (s v + s^2 b)
+// over 2^21 entries, was four tables and forty extension products a pair.)
+// Per pair a lane folds the tables and leaves value and slope in LDS (as in poly_kernel, the programs pick them by index), then
+// walks every factor's program once, at all of its points (wsum_walk).  Bound: vector ALU.
+// NF: degree of the first factor's polynomial, the highest.  GENERAL: up to two more factors of any degree up to NF; otherwise one, of degree
+// 1.  BASE: base-field tables read unfolded.  SKIP1: the first factor is not evaluated at t = 1.
+// Sums, in order: the first factor's at its points, then NF + 1 (GENERAL; a factor of degree 1: two of them) or 2 of every other.
+// ---------------------------------------------------------------------------
+constexpr u32 WSUM_MAX_EQS = SL_MAX_EQS;
+__host__ __device__ constexpr int wsum_rest(int nf, bool general) { return general ? nf + 1 : 2; }
+__host__ __device__ constexpr int wsum_sums(int nf, bool skip1, bool general) { return (skip1 ? nf : nf + 1) + wsum_rest(nf, general) * (general ? (int)WSUM_MAX_EQS - 1 : 1); }
+constexpr int WSUM_MAX_SUMS = wsum_sums(4, false, true);
+constexpr int WSUM_SEQ_SLOT = 62, WSUM_CHK_SLOT = 63;
+static_assert(2 * WSUM_MAX_SUMS <= WSUM_SEQ_SLOT, "the sums fit the result area");
+struct WsumArgs {
+    PolyTab tab[POLY_MAXT];
+    u32 n_tabs, n_eqs;
+    u32 op_begin[WSUM_MAX_EQS], op_end[WSUM_MAX_EQS], degree[WSUM_MAX_EQS];
+    u32 base_program;              // bit g: all coefficients of program g are in the base field
+    // weights of this round's pairs: streamed (q), or factored as in prod_kernel (lq, hq; lq[0] == nullptr: streamed)
+    const u64 *q0[WSUM_MAX_EQS], *q1[WSUM_MAX_EQS], *lq0[WSUM_MAX_EQS], *lq1[WSUM_MAX_EQS], *hq0[WSUM_MAX_EQS], *hq1[WSUM_MAX_EQS];
+    u64 n_pairs, r0, r1;
+    u32 wait_first, spin_limit;
+    const u64 *mail;
+    u64 *relay;
+    PolyOp ops[SL_EQS_OPS];
+};
+static_assert(sizeof(WsumArgs) <= 4000, "kernel arguments");
+template <int NF, bool SKIP1, bool BASE, bool GENERAL>
+__global__ void __launch_bounds__(BLOCK) wsum_kernel(WsumArgs a, u64 *__restrict__ partial, FastFin ff)
+{
+    constexpr int N0 = SKIP1 ? NF : NF + 1, NR = wsum_rest(NF, GENERAL), NS = wsum_sums(NF, SKIP1, GENERAL);
+    extern __shared__ u64 dyn[];  // [n_tabs][4 (BASE: 2)][BLOCK]: value, slope
+    __shared__ u32 lds[(BLOCK / WAVE) * 6 * NS];
+    __shared__ u64 res[2 * NS];
+    __shared__ int last_flag;
+    __shared__ u64 box[MAIL_WORDS];
+    __shared__ int ok_flag;
+    const u32 tid = threadIdx.x;
+    constexpr u32 W = BASE ? 2 : 4;
+    auto at = [&](u32 k, u32 c) -> u64 & { return dyn[(k * W + c) * BLOCK + tid]; };
+    E2 r = gl::e2(a.r0, a.r1);
+    if (a.wait_first) {
+        if (!wait_first_mail(a.mail, a.relay, blockIdx.x == 0, a.spin_limit, ff.seq, SKIP1 ? 0 : 1, box, &ok_flag)) return;
+        if ((box[MAIL_SKIP1] != 0) != SKIP1) return;
+        r = gl::e2(uniform64(box[MAIL_R]), uniform64(box[MAIL_R + 1]));
+    }
+    const gl::E2P rp = gl::prep(r);
+    const bool fact = a.lq0[0] != nullptr;
+    E2 lz[NS];
+#pragma unroll
+    for (int k = 0; k < NS; k++) lz[k] = gl::e2_zero();
+    for (u64 i = (u64)blockIdx.x * BLOCK + tid; i < a.n_pairs; i += (u64)gridDim.x * BLOCK) {
+        for (u32 k = 0; k < a.n_tabs; k++) {
+            const PolyTab &tb = a.tab[k];
+            if (BASE) {
+                const U64x2 x = ld2(tb.s0 + 2 * i);
+                at(k, 0) = x.x;
+                at(k, 1) = gl::sub(x.y, x.x);
+                continue;
+            }
+            E2 lo, hi;
+            if (tb.mode == POLY_PAIR_FOLD) {
+                const U64x2 x0 = ld2(tb.s0 + 4 * i), y0 = ld2(tb.s0 + 4 * i + 2);
+                if (tb.s1) {
+                    const U64x2 x1 = ld2(tb.s1 + 4 * i), y1 = ld2(tb.s1 + 4 * i + 2);
+                    lo = fold1p(gl::e2(x0.x, x1.x), gl::e2(x0.y, x1.y), rp);
+                    hi = fold1p(gl::e2(y0.x, y1.x), gl::e2(y0.y, y1.y), rp);
+                } else {
+                    lo = fold1_base(x0.x, x0.y, r);
+                    hi = fold1_base(y0.x, y0.y, r);
+                }
+                st2_stream(tb.d0 + 2 * i, lo.c0, hi.c0);
+                st2_stream(tb.d1 + 2 * i, lo.c1, hi.c1);
+            } else {
+                const U64x2 x0 = ld2(tb.s0 + 2 * i);
+                U64x2 x1 = U64x2{0, 0};
+                if (tb.s1) x1 = ld2(tb.s1 + 2 * i);
+                lo = gl::e2(x0.x, x1.x);
+                hi = gl::e2(x0.y, x1.y);
+            }
+            const E2 d = gl::sub(hi, lo);
+            at(k, 0) = lo.c0;
+            at(k, 1) = lo.c1;
+            at(k, W - 2) = d.c0;
+            at(k, W - 1) = d.c1;
+        }
+        // (the factored weight is the same for the whole workgroup: its pairs lie within one run of 2^EQ_LO_BITS)
+        const u32 hi = __builtin_amdgcn_readfirstlane((u32)(i >> EQ_LO_BITS));
+        auto rest_of = [&](u32 g) { return fact ? gl::e2(a.hq0[g][hi], a.hq1[g][hi]) : gl::e2(a.q0[g][i], a.q1[g][i]); };
+        auto op = [&](u32 o) -> const PolyOp & { return a.ops[o]; };
+        // factor g's sums at N points into lz[first ..]
+        auto factor = [&](auto n_points, auto skips, auto program_degree, auto first, u32 g) {
+            constexpr int N = decltype(n_points)::value, DEG = decltype(program_degree)::value, FIRST = decltype(first)::value;
+            constexpr bool SKIP = decltype(skips)::value;
+            const E2 rest = rest_of(g);
+            const gl::E2P restp = gl::prep(rest);
+            if constexpr (BASE) {
+                auto table = [&](u32 sl) { return wsum_points<N, SKIP>(at(sl, 0), at(sl, 1)); };
+                if ((a.base_program >> g) & 1) {
+                    u64 v[N];
+                    wsum_program<DEG>(a.op_begin[g], a.op_end[g], v, op, table);
+#pragma unroll
+                    for (int k = 0; k < N; k++) lz[FIRST + k] = gl::e2(gl::muladd(rest.c0, v[k], lz[FIRST + k].c0), gl::muladd(rest.c1, v[k], lz[FIRST + k].c1));
+                    return;
+                }
+                E2 v[N];
+                wsum_program<DEG>(a.op_begin[g], a.op_end[g], v, op, table);
+#pragma unroll
+                for (int k = 0; k < N; k++) lz[FIRST + k] = gl::fma(v[k], restp, lz[FIRST + k]);
+            } else {
+                auto table = [&](u32 sl) { return wsum_points<N, SKIP>(gl::e2(at(sl, 0), at(sl, 1)), gl::e2(at(sl, W - 2), at(sl, W - 1))); };
+                E2 v[N];
+                wsum_program<DEG>(a.op_begin[g], a.op_end[g], v, op, table);
+#pragma unroll
+                for (int k = 0; k < N; k++) lz[FIRST + k] = gl::fma(v[k], restp, lz[FIRST + k]);
+            }
+        };
+        using std::integral_constant;
+        factor(integral_constant<int, N0>{}, integral_constant<bool, SKIP1>{}, integral_constant<int, NF>{}, integral_constant<int, 0>{}, 0);
+        auto other = [&](auto first, u32 g) {
+            if (!GENERAL || a.degree[g] == 1)
+                factor(integral_constant<int, 2>{}, std::false_type{}, integral_constant<int, 1>{}, first, g);
+            else
+                factor(integral_constant<int, NR>{}, std::false_type{}, integral_constant<int, NF>{}, first, g);
+        };
+        other(integral_constant<int, N0>{}, 1);
+        if constexpr (GENERAL)
+            if (a.n_eqs > 2) other(integral_constant<int, N0 + NR>{}, 2);
+    }
+    if (fact) {
+        // the low part of the weights: the same for all of a thread's pairs (the grid's stride is a multiple of 2^EQ_LO_BITS)
+        const u32 lo = (blockIdx.x * BLOCK + tid) & ((1u << EQ_LO_BITS) - 1);
+#pragma unroll
+        for (int k = 0; k < NS; k++) {
+            const u32 g = k < N0 ? 0 : 1 + (k - N0) / NR;
+            if (g < a.n_eqs) lz[k] = gl::mulp(lz[k], gl::prep(gl::e2(a.lq0[g][lo], a.lq1[g][lo])));
+        }
+    }
+    block_reduce<NS>(lz, lds);
+    constexpr u32 n_words = 2 * NS;
+    if (tid == 0)
+#pragma unroll
+        for (int k = 0; k < NS; k++) res[2 * k] = lz[k].c0, res[2 * k + 1] = lz[k].c1;
+    __syncthreads();
+    if (gridDim.x > 1) {
+        if (tid < n_words) st_agent(partial + (u64)tid * gridDim.x + blockIdx.x, res[tid]);
+        // (every wavefront's stores acknowledged before the workgroup's ticket is taken)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        if (!take_ticket(ff.counter, gridDim.x, &last_flag)) return;
+        // the last workgroup adds up the workgroups' words: a wavefront four words at a time, all their loads of a step in flight together
+        const u32 lane = tid & (WAVE - 1), wave = tid / WAVE;
+        for (u32 w0 = wave; w0 < n_words; w0 += 4 * (BLOCK / WAVE)) {
+            u64 sum[4] = {0, 0, 0, 0};
+            for (u32 b0 = lane; b0 < gridDim.x; b0 += 4 * WAVE) {
+                u64 x[4][4];
+#pragma unroll
+                for (u32 u = 0; u < 4; u++)
+#pragma unroll
+                    for (u32 c = 0; c < 4; c++) {
+                        const u32 w = w0 + c * (BLOCK / WAVE), b = b0 + u * WAVE;
+                        x[u][c] = w < n_words && b < gridDim.x ? ld_agent(partial + (u64)w * gridDim.x + b) : 0;
+                    }
+#pragma unroll
+                for (u32 u = 0; u < 4; u++)
+#pragma unroll
+                    for (u32 c = 0; c < 4; c++) sum[c] = gl::add(sum[c], x[u][c]);
+            }
+            wave_sum_field<4>(sum);
+#pragma unroll
+            for (u32 c = 0; c < 4; c++)
+                if (lane == WAVE - 1 && w0 + c * (BLOCK / WAVE) < n_words) res[w0 + c * (BLOCK / WAVE)] = sum[c];
+        }
+        __syncthreads();
+    }
+    if (tid == 0) {
+        if (ff.counter) *ff.counter = 0;
+        publish_words(ff.out_host, 0, res, n_words, ff.seq, WSUM_SEQ_SLOT, WSUM_CHK_SLOT);
+    }
+}
+
+// The sum of poly_kernel for rounds of few pairs, where a launch is one serial chain per thread: the work of a pair is
 // spread over 2^split_log adjacent lanes.  First the pair's tables are divided among the lanes (each loads,
 // folds and stores its tables and leaves value and slope in LDS), then the (point, term) products are: lane l
 // takes every item q = point_position * n_terms + term with q = l mod 2^split_log, reading a factor at point t

@@ -1,5 +1,5 @@
 """The hot kernels' bodies on the CPU under the host sanitizers (tests/cpp/emu_prod_kernel.cpp, tests/cpp/emu_slice_kernel.cpp,
-tests/cpp/emu_poly_kernel.cpp, tests/cpp/emu_point_kernels.cpp): no GPU involved.  The programs are built and run side by side (a build under the
+tests/cpp/emu_poly_kernel.cpp, tests/cpp/emu_point_kernels.cpp, tests/cpp/emu_weighted_kernels.cpp): no GPU involved.  The programs are built and run side by side (a build under the
 sanitizers takes over a minute), once per test session; each test then reads its program's outcome."""
 import os
 import shutil
@@ -12,7 +12,7 @@ CLANG = "/opt/rocm/llvm/bin/clang++"
 needs_clang = pytest.mark.skipif(not os.path.exists(CLANG), reason="needs clang (ext_vector_type, -ftrivial-auto-var-init)")
 
 PROGRAMS = {"prod": ("emu_prod_kernel.cpp", ["quick"]), "slice": ("emu_slice_kernel.cpp", []), "poly": ("emu_poly_kernel.cpp", []),
-            "point": ("emu_point_kernels.cpp", [])}
+            "point": ("emu_point_kernels.cpp", []), "weighted": ("emu_weighted_kernels.cpp", [])}
 
 
 @pytest.fixture(scope="module")
@@ -74,3 +74,9 @@ def test_poly_kernel_body_under_host_sanitizers(outcomes):
 def test_point_kernel_bodies_under_host_sanitizers(outcomes):
     # partial evaluations, evaluations at a point, combined tables: every kernel that takes its weights from a point
     _check(outcomes["point"])
+
+
+@needs_clang
+def test_weighted_sum_kernel_bodies_under_host_sanitizers(outcomes):
+    # sums over several eq factors: a round that is a launch of its own, and the resident rounds
+    _check(outcomes["weighted"])
