@@ -1652,19 +1652,26 @@ struct dps_sc {
     const u64 *eq_c0, *eq_c1;  // its storage (level 0 at entry 0)
     E2 fast_coeff;
     E2 eq_scalar;       // product of eq1(rho_i, r_{i+1}) over the bound variables
-    // A sum over several eq factors (wsum_kernel): every term has one of them, all in closed form.  In order of their polynomials' degrees, highest first;
-    // p(1) of a round gives the first one's sum at 1
+    // A sum over two or three eq factors (wsum_kernel, slice_kernel with SliceArgsParts): every term has one of them, all in closed form.  In order of
+    // their polynomials' degrees, highest first; p(1) of a round gives the first one's sum at 1
     struct WeightedEq {
         u32 k;                        // the eq table as registered
         std::shared_ptr<EqInfo> info;
         const u64 *c0, *c1;           // its storage (level 0 at entry 0)
         u32 degree;                   // of the polynomial it weights
         E2 scalar;                    // product of eq1(rho_i, r_{i+1}) over the bound variables
-        u32 op_begin, op_end;         // the polynomial's program in h_poly_ops
-        bool base_program;            // ... all of whose coefficients are in the base field
-        u32 off_q, off_d;             // where a resident trip's sums lie (dpk::SliceArgsEqs)
+        bool base_program;            // all coefficients of its program are in the base field
+        u32 off_q, off_d;             // where a resident trip's sums lie (dpk::SliceArgsParts)
     };
     std::vector<WeightedEq> weq;
+    struct ProgramPart {
+        u32 op_begin, op_end, of;     // operations in h_poly_ops; the polynomial
+    };
+    std::vector<ProgramPart> weq_parts;
+    // A sum of several terms with one common eq factor (fast_eq): its rounds that are launches of their own run by a program all the same, as if it were
+    // the only entry of weq; the resident rounds run term by term
+    bool one_program = false;
+    WeightedEq one;
     u32 weq_sums1 = 0, weq_sums2 = 0; // of a trip of one round, of two
     bool closed_eq(u32 k) const
     {
@@ -1835,23 +1842,26 @@ size_t slice_area_off(const dps_ctx *ctx) { return ctx->pinned_words / 2 + 64 + 
 
 // The sizes of a resident launch's arguments: a product's, and by its tables and terms a sum's (`shorter`: some table has fewer
 // variables than the sum)
-enum SliceSize { SLICE_PRODUCT, SLICE_FEW, SLICE_MANY, SLICE_EQS };
-SliceSize slice_size(bool sum, size_t n_tabs, size_t n_terms, bool shorter, size_t n_eqs)
+enum SliceSize { SLICE_PRODUCT, SLICE_FEW, SLICE_MANY, SLICE_PARTS_FEW, SLICE_PARTS_MANY };
+constexpr bool slice_parts(SliceSize s) { return s == SLICE_PARTS_FEW || s == SLICE_PARTS_MANY; }
+// (`n_ops`: of the programs of a sum that runs by them, else 0)
+SliceSize slice_size(bool sum, size_t n_tabs, size_t n_terms, bool shorter, size_t n_ops)
 {
-    if (n_eqs) return SLICE_EQS;
+    if (n_ops) return n_tabs <= 8 && n_ops <= (size_t)dpk::SliceArgsPartsFew::OPS && !shorter ? SLICE_PARTS_FEW : SLICE_PARTS_MANY;
     if (!sum) return SLICE_PRODUCT;
     return n_tabs <= (size_t)dpk::SL_FEW_TABS && n_terms <= (size_t)dpk::SL_FEW_TERMS && !shorter ? SLICE_FEW : SLICE_MANY;
 }
 template <SliceSize SIZE>
 using SliceArgsFor = std::conditional_t<SIZE == SLICE_PRODUCT, dpk::SliceArgsProduct,
-                                        std::conditional_t<SIZE == SLICE_FEW, dpk::SliceArgsFew, std::conditional_t<SIZE == SLICE_EQS, dpk::SliceArgsEqs, dpk::SliceArgs>>>;
+                                        std::conditional_t<SIZE == SLICE_FEW, dpk::SliceArgsFew, std::conditional_t<SIZE == SLICE_PARTS_FEW, dpk::SliceArgsPartsFew,
+                                                                                               std::conditional_t<SIZE == SLICE_PARTS_MANY, dpk::SliceArgsPartsMany, dpk::SliceArgs>>>>;
 template <int NF, bool EQ, SliceSize SIZE>
 constexpr auto slice_variant = &dpk::slice_kernel<NF, EQ, SIZE != SLICE_PRODUCT, dpk::SL_BLOCK, SliceArgsFor<SIZE>>;
 template <SliceSize SIZE>
 size_t slice_lds_bytes(u32 n_tabs, u32 cap, bool eq)
 {
     // (several eq factors: sized for as many as there can be)
-    return (size_t)dpk::slice_lds_words(n_tabs, cap, dpk::SL_BLOCK, SIZE == SLICE_EQS ? dpk::SL_MAX_EQS : eq, SliceArgsFor<SIZE>::TERMS) * 8;
+    return (size_t)dpk::slice_lds_words(n_tabs, cap, dpk::SL_BLOCK, slice_parts(SIZE) ? dpk::SL_MAX_EQS : eq, SliceArgsFor<SIZE>::TERMS) * 8;
 }
 
 // A workgroup of a resident launch may take most of a compute unit's LDS (it is alone there: 1024 threads); more than
@@ -1880,7 +1890,8 @@ u32 slice_lds_granted(dps_ctx *ctx)
 #define SLICE_VARIANTS(SK)                                                                                              \
     SK(1, true, SLICE_PRODUCT) SK(2, true, SLICE_PRODUCT) SK(2, false, SLICE_PRODUCT) SK(3, false, SLICE_PRODUCT)       \
     SLICE_SUM_VARIANTS(SK, SLICE_FEW) SLICE_SUM_VARIANTS(SK, SLICE_MANY)                                                \
-    SK(2, true, SLICE_EQS) SK(3, true, SLICE_EQS) SK(4, true, SLICE_EQS)
+    SK(2, true, SLICE_PARTS_FEW) SK(3, true, SLICE_PARTS_FEW) SK(4, true, SLICE_PARTS_FEW)                              \
+    SK(2, true, SLICE_PARTS_MANY) SK(3, true, SLICE_PARTS_MANY) SK(4, true, SLICE_PARTS_MANY)
 template <SliceSize SIZE>
 int32_t launch_slice(dps_ctx *ctx, u32 nf, bool eq, u32 workgroups, u32 n_tabs, u32 cap, const SliceArgsFor<SIZE> &a)
 {
@@ -2022,18 +2033,27 @@ int32_t launch_poly_dispatch(dps_ctx *ctx, u32 nf, bool eq, bool skip1, const dp
     return DPS_OK;
 }
 
-// (the compiled variants over base-field tables are those of two factors)
-bool wsum_general(u32 n_eqs, u32 second_degree) { return n_eqs > 2 || second_degree > 1; }
+// dpk::wsum_kernel's REST (base-field tables unfolded: compiled for one or two factors)
+int wsum_rest_kind(u32 n_eqs, u32 second_degree) { return n_eqs < 2 ? 0 : n_eqs > 2 || second_degree > 1 ? 2 : 1; }
 template <int NF, bool SKIP1>
 void launch_wsum_degree(dps_ctx *ctx, bool base, const dpk::WsumArgs &a, u32 blocks, u64 *partial, const dpk::FastFin &ff)
 {
     const size_t table = (size_t)dpk::BLOCK * 8;  // a limb of the values or slopes of a table
-    if (wsum_general(a.n_eqs, a.degree[1]))
-        dpk::wsum_kernel<NF, SKIP1, false, true><<<blocks, dpk::BLOCK, a.n_tabs * 4 * table, ctx->stream>>>(a, partial, ff);
-    else if (base)
-        dpk::wsum_kernel<NF, SKIP1, true, false><<<blocks, dpk::BLOCK, a.n_tabs * 2 * table, ctx->stream>>>(a, partial, ff);
-    else
-        dpk::wsum_kernel<NF, SKIP1, false, false><<<blocks, dpk::BLOCK, a.n_tabs * 4 * table, ctx->stream>>>(a, partial, ff);
+    switch (wsum_rest_kind(a.n_eqs, a.degree[1])) {
+    case 0:
+        if (base)
+            dpk::wsum_kernel<NF, SKIP1, true, 0><<<blocks, dpk::BLOCK, a.n_tabs * 2 * table, ctx->stream>>>(a, partial, ff);
+        else
+            dpk::wsum_kernel<NF, SKIP1, false, 0><<<blocks, dpk::BLOCK, a.n_tabs * 4 * table, ctx->stream>>>(a, partial, ff);
+        break;
+    case 1:
+        if (base)
+            dpk::wsum_kernel<NF, SKIP1, true, 1><<<blocks, dpk::BLOCK, a.n_tabs * 2 * table, ctx->stream>>>(a, partial, ff);
+        else
+            dpk::wsum_kernel<NF, SKIP1, false, 1><<<blocks, dpk::BLOCK, a.n_tabs * 4 * table, ctx->stream>>>(a, partial, ff);
+        break;
+    default: dpk::wsum_kernel<NF, SKIP1, false, 2><<<blocks, dpk::BLOCK, a.n_tabs * 4 * table, ctx->stream>>>(a, partial, ff);
+    }
 }
 int32_t launch_wsum(dps_ctx *ctx, bool skip1, bool base, const dpk::WsumArgs &a, u32 blocks, u64 *partial, const dpk::FastFin &ff)
 {
@@ -2179,70 +2199,106 @@ u32 product_blocks(u64 n_pairs)
 
 namespace {
 
-// Nested (Horner) form of a group's terms: the table found in most of the remaining terms is factored out of
-// them, recursively.  Appends the program to `ops`; returns its number of products.
-struct HornerTerm {
+// Nested (Horner) form of a sum of terms: the table found in most of the remaining terms is factored out of them, recursively.
+constexpr u32 MAX_PROGRAM_TERMS = 64, NO_TABLE = ~0u;
+struct ProgramTerm {
     E2 coeff;
-    std::vector<uint8_t> slots;  // remaining factors
+    uint8_t n, slot[DPS_MAX_FACTORS];  // remaining factors, as slots below SL_MAX_TABS
 };
 
-u32 horner_build(std::vector<HornerTerm> ts, u32 depth, std::vector<dpk::PolyOp> &ops)
+dpk::PolyOp program_op(u32 kind, u32 d, u32 slot, E2 c)
 {
-    auto make = [](u32 kind, u32 d, u32 slot, E2 c) {
-        dpk::PolyOp op;
-        memset(&op, 0, sizeof op);
-        op.c0 = c.c0;
-        op.c1 = c.c1;
-        op.w = gl::mul_small(c.c1, (u32)gl::W);
-        const u32 cls = c.c1 ? dpk::POLY_COEFF_ANY : c.c0 == 1 ? dpk::POLY_COEFF_ONE : c.c0 == gl::P - 1 ? dpk::POLY_COEFF_MINUS_ONE : dpk::POLY_COEFF_BASE;
-        op.code = kind | d << 2 | (kind == dpk::POLY_OP_LEAF ? cls : 0) << 6 | slot << 8;
-        return op;
-    };
+    dpk::PolyOp op;
+    memset(&op, 0, sizeof op);
+    op.c0 = c.c0;
+    op.c1 = c.c1;
+    op.w = gl::mul_small(c.c1, (u32)gl::W);
+    const u32 cls = c.c1 ? dpk::POLY_COEFF_ANY : c.c0 == 1 ? dpk::POLY_COEFF_ONE : c.c0 == gl::P - 1 ? dpk::POLY_COEFF_MINUS_ONE : dpk::POLY_COEFF_BASE;
+    op.code = kind | d << 2 | (kind == dpk::POLY_OP_LEAF ? cls : 0) << 6 | slot << 8;
+    return op;
+}
+
+// Appends the operations of the node of depth `depth` with these terms, each of at least one factor (their order is not kept); returns
+// its number of products.  `ends`: where the operations of each of its children end.
+u32 program_build(ProgramTerm *t, u32 n, u32 depth, std::vector<dpk::PolyOp> &ops, std::vector<u32> *ends = nullptr)
+{
     u32 products = 0;
-    // terms that end at this node were added to the node's constant by the caller
-    ts.erase(std::remove_if(ts.begin(), ts.end(), [](const HornerTerm &t) { return t.slots.empty(); }), ts.end());
-    while (!ts.empty()) {
-        // slots are positions within a group: fewer than POLY_MAXT
-        u32 count[dpk::POLY_MAXT] = {0};
-        for (const HornerTerm &t : ts) {
-            u32 seen = 0;
-            for (uint8_t sl : t.slots)
-                if (!((seen >> sl) & 1)) {
-                    seen |= 1u << sl;
-                    count[sl]++;
-                }
-        }
-        u32 best = 0;
-        for (u32 sl = 1; sl < (u32)dpk::POLY_MAXT; sl++)
-            if (count[sl] > count[best]) best = sl;
-        std::vector<HornerTerm> sub, rest;
-        for (HornerTerm &t : ts) {
-            auto it = std::find(t.slots.begin(), t.slots.end(), (uint8_t)best);
-            if (it == t.slots.end()) {
-                rest.push_back(std::move(t));
+    while (n) {
+        uint8_t count[dpk::SL_MAX_TABS] = {0};
+        u32 best = t[0].slot[0];
+        for (u32 i = 0; i < n; i++)
+            for (u32 f = 0; f < t[i].n; f++) {
+                const u32 sl = t[i].slot[f];
+                bool again = false;
+                for (u32 q = 0; q < f; q++) again = again || t[i].slot[q] == sl;
+                if (again) continue;
+                count[sl]++;
+                if (count[sl] > count[best] || (count[sl] == count[best] && sl < best)) best = sl;
+            }
+        // its terms to the front, those that end here behind the others among them
+        u32 inner = 0, with = 0;
+        E2 ending = gl::e2_zero();
+        for (u32 i = 0; i < n; i++) {
+            ProgramTerm &p = t[i];
+            u32 f = 0;
+            while (f < p.n && p.slot[f] != best) f++;
+            if (f == p.n) continue;
+            p.slot[f] = p.slot[--p.n];
+            if (p.n) {
+                std::swap(t[i], t[with]);
+                std::swap(t[with++], t[inner++]);
             } else {
-                t.slots.erase(it);
-                sub.push_back(std::move(t));
+                ending = gl::add(ending, p.coeff);
+                std::swap(t[i], t[with++]);
             }
         }
-        E2 ends = gl::e2_zero();
-        bool inner = false;
-        for (const HornerTerm &t : sub) {
-            if (t.slots.empty())
-                ends = gl::add(ends, t.coeff);
-            else
-                inner = true;
-        }
-        if (!inner) {
-            ops.push_back(make(dpk::POLY_OP_LEAF, depth, best, ends));
+        if (inner) {
+            ops.push_back(program_op(dpk::POLY_OP_ENTER, depth + 1, 0, ending));
+            products += program_build(t, inner, depth + 1, ops);
+            ops.push_back(program_op(dpk::POLY_OP_LEAVE, depth + 1, best, gl::e2_zero()));
         } else {
-            ops.push_back(make(dpk::POLY_OP_ENTER, depth + 1, 0, ends));
-            products += horner_build(std::move(sub), depth + 1, ops);
-            ops.push_back(make(dpk::POLY_OP_LEAVE, depth + 1, best, gl::e2_zero()));
+            ops.push_back(program_op(dpk::POLY_OP_LEAF, depth, best, ending));
         }
+        if (ends) ends->push_back((u32)ops.size());
         products++;
-        ts = std::move(rest);
+        t += with, n -= with;
     }
+    return products;
+}
+
+// A whole program: its first operation enters the root with the constant.  `most`: parts it may be cut into, between children of the root
+// (each enters a root of its own); `ends`: where the parts' operations end.  Returns the number of products.
+u32 program_root(ProgramTerm *t, u32 n, u32 most, std::vector<dpk::PolyOp> &ops, std::vector<u32> *ends)
+{
+    E2 root = gl::e2_zero();
+    u32 m = 0;
+    for (u32 i = 0; i < n; i++)
+        if (t[i].n)
+            std::swap(t[i], t[m++]);
+        else
+            root = gl::add(root, t[i].coeff);
+    const size_t begin = ops.size();
+    ops.push_back(program_op(dpk::POLY_OP_ENTER, 0, 0, root));
+    if (most < 2) return program_build(t, m, 0, ops);
+    std::vector<u32> children;
+    const u32 products = program_build(t, m, 0, ops, &children);
+    // parts of whole children, about as many operations in each
+    const u32 parts = std::min<u32>(most, std::max<u32>(1, (u32)children.size())), all = (u32)(ops.size() - begin - 1);
+    std::vector<dpk::PolyOp> cut;
+    u32 from = (u32)begin + 1, child = 0;
+    for (u32 q = 0; q < parts; q++) {
+        u32 to = from;
+        const u32 goal = (u32)begin + 1 + (u32)((u64)all * (q + 1) / parts);
+        // (at least one child a part, and one left for every part to come)
+        while (child < children.size() && (to == from || children[child] <= goal) && (children.size() - child > parts - q - 1)) to = children[child++];
+        if (q + 1 == parts && child < children.size()) to = children.back(), child = (u32)children.size();
+        cut.push_back(q == 0 ? ops[begin] : program_op(dpk::POLY_OP_ENTER, 0, 0, gl::e2_zero()));
+        cut.insert(cut.end(), ops.begin() + from, ops.begin() + to);
+        if (ends) ends->push_back((u32)(begin + cut.size()));
+        from = to;
+    }
+    ops.resize(begin);
+    ops.insert(ops.end(), cut.begin(), cut.end());
     return products;
 }
 
@@ -2286,6 +2342,9 @@ constexpr u32 SLICE_MIN_PAIRS = 32;
 constexpr u32 SLICE_SMALL_SUM_WORKGROUPS = 128;
 constexpr u32 SLICE_ONE_WORKGROUP_TERM_PAIRS = 512;  // pairs x terms up to which one workgroup takes the whole sum
 constexpr u32 SLICE_MAX_WORKGROUPS = 256;
+// Most pairs a workgroup is given of a product, and of a sum of several terms: more would make more rounds resident, but a trip's arithmetic is a
+// workgroup's alone (with 512 pairs of a 3-term sum the first trip took 75 us where a launch for the round and a trip of 128 pairs take 66)
+constexpr u32 SLICE_PRODUCT_PAIRS = 512, SLICE_SUM_PAIRS = 128;
 // the rounds a resident launch leaves to the host: at most so many, and so many extension multiplications in all
 // (measured: 2 to 6 rounds and 400 to 3000 multiplications differ by a few percent; these were the best over the benchmark configurations)
 constexpr u32 HOST_TAIL_MAX_ROUNDS = 5;
@@ -2355,8 +2414,8 @@ u32 slice_counter_sets_log(u32 W)
 u32 slice_second_round_passes(const dps_sc *sc, u32 n_quads)
 {
     if (!sc->weq.empty()) {
-        // (every factor has its own lanes; a lane takes a quad at one challenge)
-        const u32 per = ((u32)dpk::SL_BLOCK / (u32)sc->weq.size()) & ~63u;
+        // (every part has its own lanes; a lane takes a quad at one challenge)
+        const u32 per = ((u32)dpk::SL_BLOCK / (u32)sc->weq_parts.size()) & ~63u;
         u32 most = 0;
         for (const dps_sc::WeightedEq &w : sc->weq) most = std::max(most, (n_quads * (w.degree + 1) + per - 1) / per);
         return most;
@@ -2383,11 +2442,9 @@ void plan_resident_rounds(dps_sc *sc, u32 n_tabs, u32 n_mles)
         const E2 rho = (sc->weq.empty() ? sc->eq_info : sc->weq[0].info)->point[round - 1];
         return !(rho.c0 == 0 && rho.c1 == 0);
     };
-    const u32 pairs_fit = slice_pairs_per_workgroup(sc->ctx, slice_size(sc->poly, n_tabs, sc->slice_terms.size(), sc->slice_shorter, sc->weq.size()), sc->fast_nf, has_eq, n_tabs);
+    const u32 pairs_fit = slice_pairs_per_workgroup(sc->ctx, slice_size(sc->poly, n_tabs, sc->slice_terms.size(), sc->slice_shorter, sc->weq.empty() ? 0 : sc->h_poly_ops.size()), sc->fast_nf, has_eq, n_tabs);
     if (pairs_fit == 0) return;
-    // (more pairs per workgroup would make more rounds resident, but a trip's arithmetic is a workgroup's alone: with 512
-    // pairs of a 3-term sum the first trip took 75 us where a launch for the round and a trip of 128 pairs take 66)
-    const u32 per_wg_max = std::min<u32>(pairs_fit, sc->poly ? 128 : 512);
+    const u32 per_wg_max = std::min<u32>(pairs_fit, sc->poly ? SLICE_SUM_PAIRS : SLICE_PRODUCT_PAIRS);
     auto pairs_of = [&](u32 round) { return (u64)1 << (n - round); };
     u32 j = first_ok;
     while (pairs_of(j) > (u64)per_wg_max * SLICE_MAX_WORKGROUPS) j++;
@@ -2520,7 +2577,8 @@ struct SessionSetup {
 
     void detect_product();
     bool closed_form_eq_factor();
-    bool several_eq_factors();
+    bool weighted_programs();
+    bool adopt_programs(dps_sc::WeightedEq *eqs, u32 n_eqs, std::vector<dpk::PolyOp> &&ops);
     bool group_terms();
     void adopt_groups();
     void nested_programs();
@@ -2629,83 +2687,96 @@ bool SessionSetup::closed_form_eq_factor()
     return ok;
 }
 
-// A sum each of whose terms has one eq table, two or three of them in all, times polynomials of degree 4 at most over up to POLY_MAXT
+// A sum each of whose terms has one eq table, up to three of them in all, times polynomials of degree 4 at most over up to POLY_MAXT
 // other tables, all of full size: the eq factors in closed form, a nested program each for the polynomials (wsum_kernel).  What
-// does not fit (degrees, numbers of operations and sums) runs as before, with the eq tables as tables.
-bool SessionSetup::several_eq_factors()
+// does not fit (degrees, numbers of operations and sums) runs with the eq tables as tables among the others, or a single eq table in closed
+// form term by term.  (Linking an activation of 2^21 entries, two factors of degrees 3 and 1 over two tables: 684 -> 412 us; its rounds of 2^20 .. 2^17
+// pairs 158, 92, 66, 47 -> 59, 53, 40, 30 us, the resident ones 205 -> 141.)
+// One eq factor: the same programs in the rounds that are launches of their own (rounds of 2^19 .. 2^16 pairs of a fraction-sum layer 52, 38, 30, 25 ->
+// 46, 36, 29, 21 us); resident its rounds stay with the terms, which are spread over more lanes (a trip of two rounds 8.5 .. 10 us, 15 .. 16 by a program).
+bool SessionSetup::weighted_programs()
 {
-    std::vector<dps_sc::WeightedEq> eqs;
-    std::vector<u32> tabs, eq_of_term;
-    for (const dps_term &t : sc->terms) {
-        int e = -1;
+    if (sc->n_terms < 2 || sc->n_terms > MAX_PROGRAM_TERMS) return false;
+    dps_sc::WeightedEq eqs[dpk::WSUM_MAX_EQS];
+    u32 n_eqs = 0, tabs[dpk::POLY_MAXT], n_tabs = 0, eq_of_term[MAX_PROGRAM_TERMS];
+    for (u32 ti = 0; ti < sc->n_terms; ti++) {
+        const dps_term &t = sc->terms[ti];
+        u32 e = NO_TABLE;
         for (u32 f = 0; f < t.n_factors; f++) {
             const u32 k = t.factors[f];
             const dps_mle *h = mles[k];
             if (nv0[k] != n_vars) return false;
             if (h->eq && h->eq->m == n_vars && h->kind == DPS_EXT2) {
-                if (e >= 0) return false;
-                e = (int)k;
-            } else if (std::find(tabs.begin(), tabs.end(), k) == tabs.end()) {
-                tabs.push_back(k);
+                if (e != NO_TABLE) return false;
+                e = k;
+            } else if (std::find(tabs, tabs + n_tabs, k) == tabs + n_tabs) {
+                if (n_tabs == (u32)dpk::POLY_MAXT) return false;
+                tabs[n_tabs++] = k;
             }
         }
-        if (e < 0) return false;
-        size_t g = 0;
-        while (g < eqs.size() && eqs[g].k != (u32)e) g++;
-        if (g == eqs.size()) {
-            if (eqs.size() == dpk::WSUM_MAX_EQS) return false;
-            eqs.push_back(dps_sc::WeightedEq{(u32)e, mles[e]->eq, mles[e]->p0(), mles[e]->p1(), 0, gl::e2_one(), 0, 0, true, 0, 0});
+        if (e == NO_TABLE) return false;
+        u32 g = 0;
+        while (g < n_eqs && eqs[g].k != e) g++;
+        if (g == n_eqs) {
+            if (n_eqs == dpk::WSUM_MAX_EQS) return false;
+            eqs[n_eqs++] = dps_sc::WeightedEq{e, mles[e]->eq, mles[e]->p0(), mles[e]->p1(), 0, gl::e2_one(), true, 0, 0};
         }
         eqs[g].degree = std::max(eqs[g].degree, t.n_factors - 1);
-        eq_of_term.push_back((u32)e);
+        eq_of_term[ti] = e;
     }
-    if (eqs.size() < 2 || tabs.empty() || tabs.size() > (size_t)dpk::POLY_MAXT || n_mles != tabs.size() + eqs.size()) return false;
-    std::stable_sort(eqs.begin(), eqs.end(), [](const auto &x, const auto &y) { return x.degree > y.degree; });
-    if (eqs[0].degree < 2 || eqs[0].degree > 4 || eqs.back().degree < 1) return false;
+    if (!n_tabs || n_mles != n_tabs + n_eqs) return false;
+    std::stable_sort(eqs, eqs + n_eqs, [](const auto &x, const auto &y) { return x.degree > y.degree; });
+    if (eqs[0].degree < 2 || eqs[0].degree > 4 || eqs[n_eqs - 1].degree < 1) return false;
     std::vector<dpk::PolyOp> ops;
-    for (dps_sc::WeightedEq &w : eqs) {
-        std::vector<HornerTerm> ts;
-        dpk::PolyOp enter;
-        memset(&enter, 0, sizeof enter);
-        enter.code = dpk::POLY_OP_ENTER;
+    for (u32 g = 0; g < n_eqs; g++) {
+        ProgramTerm ts[MAX_PROGRAM_TERMS];
+        u32 n = 0;
         for (u32 ti = 0; ti < sc->n_terms; ti++) {
-            if (eq_of_term[ti] != w.k) continue;
+            if (eq_of_term[ti] != eqs[g].k) continue;
             const dps_term &t = sc->terms[ti];
-            HornerTerm ht;
-            ht.coeff = gl::e2(t.coeff[0], t.coeff[1]);
-            w.base_program = w.base_program && t.coeff[1] == 0;
+            ProgramTerm &p = ts[n++];
+            p.coeff = gl::e2(t.coeff[0], t.coeff[1]);
+            eqs[g].base_program = eqs[g].base_program && t.coeff[1] == 0;
+            p.n = 0;
             for (u32 f = 0; f < t.n_factors; f++)
-                if (t.factors[f] != w.k) ht.slots.push_back((uint8_t)(std::find(tabs.begin(), tabs.end(), t.factors[f]) - tabs.begin()));
-            if (ht.slots.empty()) {
-                const E2 c = gl::add(gl::e2(enter.c0, enter.c1), ht.coeff);
-                enter.c0 = c.c0, enter.c1 = c.c1;
-            }
-            ts.push_back(std::move(ht));
+                if (t.factors[f] != eqs[g].k) p.slot[p.n++] = (uint8_t)(std::find(tabs, tabs + n_tabs, t.factors[f]) - tabs);
         }
-        w.op_begin = (u32)ops.size();
-        ops.push_back(enter);
-        horner_build(std::move(ts), 0, ops);
-        w.op_end = (u32)ops.size();
+        const u32 begin = (u32)ops.size();
+        program_root(ts, n, 1, ops, nullptr);
+        if (n_eqs > 1) sc->weq_parts.push_back(dps_sc::ProgramPart{begin, (u32)ops.size(), g});
     }
-    if (ops.size() > (size_t)dpk::SL_EQS_OPS) return false;
-    // the places of a trip's sums
-    u32 sums = 0;
-    for (dps_sc::WeightedEq &w : eqs) w.off_q = sums, sums += w.degree + 1;
-    sc->weq_sums1 = sums;
-    for (size_t g = 0; g < eqs.size(); g++) {
-        eqs[g].off_d = sums;
-        sums += (g == 0 ? eqs[g].degree : eqs[g].degree + 1) * (eqs[g].degree + 1);
+    if (n_eqs == 1) {
+        if (ops.size() <= (size_t)dpk::SL_PARTS_OPS) {
+            sc->one_program = true;
+            sc->one = eqs[0];
+            sc->h_poly_ops = std::move(ops);
+        }
+        return false;
     }
-    sc->weq_sums2 = sums;
-    if (sc->weq_sums1 > (u32)dpk::SL_MAX_SUMS) return false;
-    sc->weq = std::move(eqs);
-    sc->h_poly_ops = std::move(ops);
-    nf = sc->weq[0].degree;
-    groups.assign(1, tabs);
+    if (!adopt_programs(eqs, n_eqs, std::move(ops))) return false;
+    nf = eqs[0].degree;
+    groups.assign(1, std::vector<u32>(tabs, tabs + n_tabs));
     tb.assign(1, 0);
     te.assign(1, sc->n_terms);
     sc->poly_op_begin.assign(1, 0);
     sc->poly_op_end.assign(1, 0);
+    return true;
+}
+
+// The session takes the programs written down (their parts are in weq_parts): the places of a trip's sums.  False: too many of something.
+bool SessionSetup::adopt_programs(dps_sc::WeightedEq *eqs, u32 n_eqs, std::vector<dpk::PolyOp> &&ops)
+{
+    u32 sums = 0;
+    for (u32 g = 0; g < n_eqs; g++) eqs[g].off_q = sums, sums += eqs[g].degree + 1;
+    sc->weq_sums1 = sums;
+    for (u32 g = 0; g < n_eqs; g++) eqs[g].off_d = sums, sums += (g == 0 ? eqs[g].degree : eqs[g].degree + 1) * (eqs[g].degree + 1);
+    sc->weq_sums2 = sums;
+    if (ops.size() > (size_t)dpk::SL_PARTS_OPS || sc->weq_sums1 > (u32)dpk::SL_MAX_SUMS) {
+        sc->weq_parts.clear();
+        return false;
+    }
+    sc->weq.assign(eqs, eqs + n_eqs);
+    sc->h_poly_ops = std::move(ops);
     return true;
 }
 
@@ -2800,25 +2871,17 @@ void SessionSetup::nested_programs()
     std::vector<dpk::PolyOp> all_ops;
     u32 plain = 0, nested = 0;
     for (size_t g = 0; g < groups.size() && use_ops; g++) {
-        std::vector<HornerTerm> ts;
-        E2 root = gl::e2_zero();
+        std::vector<ProgramTerm> ts(te[g] - tb[g]);
         for (u32 ti = tb[g]; ti < te[g]; ti++) {
             const dpk::PolyTerm &pt = poly_terms[ti];
-            HornerTerm ht;
-            ht.coeff = gl::e2(pt.c0, pt.c1);
-            ht.slots.assign(pt.slot, pt.slot + pt.n_factors);
-            if (ht.slots.empty()) root = gl::add(root, ht.coeff);
+            ProgramTerm &p = ts[ti - tb[g]];
+            p.coeff = gl::e2(pt.c0, pt.c1);
+            p.n = (uint8_t)pt.n_factors;
+            std::copy(pt.slot, pt.slot + pt.n_factors, p.slot);
             plain += pt.n_factors;  // n_factors - 1 products and one for the coefficient
-            ts.push_back(std::move(ht));
         }
         std::vector<dpk::PolyOp> ops;
-        dpk::PolyOp enter;
-        memset(&enter, 0, sizeof enter);
-        enter.c0 = root.c0;
-        enter.c1 = root.c1;
-        enter.code = dpk::POLY_OP_ENTER;
-        ops.push_back(enter);
-        nested += horner_build(std::move(ts), 0, ops);
+        nested += program_root(ts.data(), (u32)ts.size(), 1, ops, nullptr);
         if (ops.size() > (size_t)dpk::POLY_LDS_OPS) use_ops = false;
         sc->poly_op_begin[g] = (u32)all_ops.size();
         all_ops.insert(all_ops.end(), ops.begin(), ops.end());
@@ -2838,15 +2901,24 @@ void SessionSetup::detect_multi_term()
     sc->poly_max_tabs = 0;
     sc->d_poly_groups = nullptr;
     sc->d_poly_terms = nullptr;
+    sc->one_program = false;
     if (sc->fast || sc->n_terms < 1 || n_vars < 1) return;
     if (!closed_form_eq_factor()) return;
-    if (eq < 0 && several_eq_factors()) {
+    // (one eq factor, no round large enough for a program: nothing to do)
+    const bool only_resident = eq >= 0 && 1ull << (n_vars - 1) < POLY_SPLIT_MAX_PAIRS;
+    if (!only_resident && weighted_programs()) {
+        eq = -1;
         adopt_groups();
         return;
     }
     if (!group_terms()) return;
     adopt_groups();
-    nested_programs();
+    if (sc->one_program) {
+        sc->poly_op_begin.assign(groups.size(), 0);
+        sc->poly_op_end.assign(groups.size(), 0);
+    } else {
+        nested_programs();
+    }
 }
 
 int32_t SessionSetup::plan_and_ready_tables()
@@ -2892,9 +2964,6 @@ int32_t SessionSetup::plan_and_ready_tables()
                 dpk::SliceTerm tm;
                 memset(&tm, 0, sizeof tm);
                 tm.c0 = t.coeff[0], tm.c1 = t.coeff[1], tm.w = gl::mul_small(t.coeff[1], (u32)gl::W);
-                for (size_t g = 0; g < sc->weq.size(); g++)
-                    for (u32 f = 0; f < t.n_factors; f++)
-                        if (t.factors[f] == sc->weq[g].k) tm.eq = (u32)g;
                 for (u32 f = 0; f < t.n_factors; f++)
                     if (!sc->closed_eq(t.factors[f])) tm.slot[tm.n_factors++] = (uint8_t)(std::find(ids.begin(), ids.end(), t.factors[f]) - ids.begin());
                 sc->slice_terms.push_back(tm);
@@ -3174,7 +3243,7 @@ void SessionSetup::launch_limits()
     // (the launch of the first two rounds: 18 words a workgroup where the others have at most 16)
     if (sc->pair12) sc->max_blocks = std::max<u32>(sc->max_blocks, (PAIR12_BLOCKS * 2 * dpk::PAIR12_SUMS + 2 * dpk::MAX_PTS - 1) / (2 * dpk::MAX_PTS));
     for (const dps_sc::QuadStep &q : sc->quads) sc->max_blocks = std::max<u32>(sc->max_blocks, q.blocks);
-    if (!sc->weq.empty()) sc->max_blocks *= (2 * dpk::WSUM_MAX_SUMS + 2 * dpk::MAX_PTS - 1) / (2 * dpk::MAX_PTS);
+    if (!sc->weq.empty() || sc->one_program) sc->max_blocks *= (2 * dpk::WSUM_MAX_SUMS + 2 * dpk::MAX_PTS - 1) / (2 * dpk::MAX_PTS);
     sc->poly_split_cap = 0;
     sc->poly_finish_in_kernel = false;
     if (sc->poly) {
@@ -3932,7 +4001,26 @@ std::vector<E2> host_pair_weights(const EqInfo &eq, u32 j, u32 n_vars, u32 n_pai
     return weight;
 }
 
-// The sums q_g(t), t = 0 .. degree of factor g, of a round of a sum over several eq factors on the tables the host holds (q_0(1) left
+// A program on the host, its root's value in `acc` (dpk::poly_walk)
+E2 host_walk(const std::vector<dpk::PolyOp> &ops, u32 &pc, u32 end, E2 acc, const E2 *val)
+{
+    while (pc < end) {
+        const dpk::PolyOp &o = ops[pc];
+        const u32 kind = o.code & 3, cls = (o.code >> 6) & 3, sl = o.code >> 8;
+        if (kind == dpk::POLY_OP_LEAVE) break;
+        pc++;
+        if (kind == dpk::POLY_OP_LEAF) {
+            const E2 t = val[sl];
+            acc = gl::add(acc, cls == dpk::POLY_COEFF_ONE ? t : cls == dpk::POLY_COEFF_MINUS_ONE ? gl::neg(t) : cls == dpk::POLY_COEFF_BASE ? gl::mul_base(t, o.c0) : gl::mul(t, gl::e2(o.c0, o.c1)));
+        } else {
+            const E2 child = host_walk(ops, pc, end, gl::e2(o.c0, o.c1), val);
+            acc = gl::add(acc, gl::mul(child, val[ops[pc++].code >> 8]));
+        }
+    }
+    return acc;
+}
+
+// The sums q_g(t), t = 0 .. degree of factor g, of a round of a sum that runs by programs on the tables the host holds (q_0(1) left
 // out when it comes from the claim), factor g's from q[g * MAX_PTS] on
 void host_tail_weighted_sums(dps_sc *sc, u32 j, bool skip1, E2 *q)
 {
@@ -3942,7 +4030,7 @@ void host_tail_weighted_sums(dps_sc *sc, u32 j, bool skip1, E2 *q)
         weight[g] = host_pair_weights(*sc->weq[g].info, j, sc->n_vars, n_pairs);
         for (u32 t = 0; t <= sc->weq[g].degree; t++) q[g * dpk::MAX_PTS + t] = gl::e2_zero();
     }
-    E2 val[dpk::POLY_MAXT], d[dpk::POLY_MAXT];
+    E2 val[dpk::SL_MAX_TABS], d[dpk::SL_MAX_TABS];
     for (u32 p = 0; p < n_pairs; p++) {
         for (u32 f = 0; f < n_tabs; f++) {
             val[f] = sc->host_state[(size_t)f * len + 2 * p];
@@ -3952,11 +4040,11 @@ void host_tail_weighted_sums(dps_sc *sc, u32 j, bool skip1, E2 *q)
             if (t > 0)
                 for (u32 f = 0; f < n_tabs; f++) val[f] = gl::add(val[f], d[f]);
             E2 poly[dpk::WSUM_MAX_EQS] = {};
-            for (const dpk::SliceTerm &tm : sc->slice_terms) {
-                if (t > sc->weq[tm.eq].degree || (tm.eq == 0 && t == 1 && skip1)) continue;
-                E2 prod = gl::e2(tm.c0, tm.c1);
-                for (u32 k = 0; k < tm.n_factors; k++) prod = gl::mul(prod, val[tm.slot[k]]);
-                poly[tm.eq] = gl::add(poly[tm.eq], prod);
+            for (const dps_sc::ProgramPart &part : sc->weq_parts) {
+                if (t > sc->weq[part.of].degree || (part.of == 0 && t == 1 && skip1)) continue;
+                const dpk::PolyOp &root = sc->h_poly_ops[part.op_begin];
+                u32 pc = part.op_begin + 1;
+                poly[part.of] = gl::add(poly[part.of], host_walk(sc->h_poly_ops, pc, part.op_end, gl::e2(root.c0, root.c1), val));
             }
             for (size_t g = 0; g < sc->weq.size(); g++)
                 if (t <= sc->weq[g].degree) q[g * dpk::MAX_PTS + t] = gl::add(q[g * dpk::MAX_PTS + t], gl::mul(poly[g], weight[g][p]));
@@ -4059,9 +4147,11 @@ struct FusedRound {
     int32_t take_weighted_sums();
     int32_t launch_weighted(u32 jj, bool skip1_jj, bool ahead, u64 seq_jj);
     bool weighted() const { return !sc->weq.empty(); }
+    // a round of so many pairs that is a launch of its own runs by a program
+    bool by_program(u64 pairs) const { return weighted() || (sc->one_program && pairs >= POLY_SPLIT_MAX_PAIRS); }
     Plan plan_round(u32 jj, bool skip1_jj) const;
     int32_t launch_round(u32 jj, const Plan &p, bool skip1_jj, bool ahead, u64 seq_jj);
-    u32 slots_of(const Plan &p) const { return weighted() ? 0 : p.reside ? (n_groups > 1 ? n_groups : 0) : slots_for(p.blocks * n_groups); }
+    u32 slots_of(const Plan &p) const { return by_program(p.n_pairs) ? 0 : p.reside ? (n_groups > 1 ? n_groups : 0) : slots_for(p.blocks * n_groups); }
     int32_t multi_term_round();
     int32_t product_launch_ahead(u32 ahead = 1);
     int32_t product_round();
@@ -4093,7 +4183,8 @@ int32_t FusedRound::begin()
         a.ra1 = sc->prev_chal.c1;
         CHK(launch_folds(sc, j, true, challenge));
         if (has_eq) sc->eq_scalar = gl::mul(sc->eq_scalar, h_eq1(sc->eq_info->point[j - 2], r));
-        for (dps_sc::WeightedEq &w : sc->weq) w.scalar = gl::mul(w.scalar, h_eq1(w.info->point[j - 2], r));
+        for (dps_sc::WeightedEq &w : sc->weq)
+            w.scalar = gl::mul(w.scalar, h_eq1(w.info->point[j - 2], r));
     }
     // scale(t) = coeff * S * eq1(rho_{j-1}, t).  Only whether scale(1) vanishes matters to the kernel (it then has to
     // evaluate t = 1); everything else about the message is worked out while the kernel runs (prepare_message).
@@ -4214,7 +4305,9 @@ void FusedRound::form_message(const E2 *q)
 void FusedRound::form_weighted_message(E2 *q)
 {
         const size_t G = sc->weq.size();
-        auto scale = [&](size_t g, u32 t) { return gl::mul(sc->weq[g].scalar, h_eq1(sc->weq[g].info->point[j - 1], gl::e2(t, 0))); };
+        auto scaled = [&](size_t g, u32 t) {
+            return gl::mul(gl::mul(sc->weq[g].scalar, h_eq1(sc->weq[g].info->point[j - 1], gl::e2(t, 0))), q[g * dpk::MAX_PTS + t]);
+        };
         auto beyond = [&](size_t g, u32 t) {
             const u32 d = sc->weq[g].degree;
             E2 v = gl::e2_zero();
@@ -4227,7 +4320,7 @@ void FusedRound::form_weighted_message(E2 *q)
             for (size_t g = 0; g < G; g++) {
                 if (g == 0 && t == 1 && a.skip1) continue;
                 if (t > sc->weq[g].degree) q[g * dpk::MAX_PTS + t] = beyond(g, t);
-                v = gl::add(v, gl::mul(scale(g, t), q[g * dpk::MAX_PTS + t]));
+                v = gl::add(v, scaled(g, t));
             }
             if (t == 1 && a.skip1) {
                 const E2 p1 = gl::sub(sc->claim, msg[0]);
@@ -4248,17 +4341,21 @@ int32_t FusedRound::take_weighted_sums()
 {
         prepare_message();
         const int n0 = (int)nf + (a.skip1 ? 0 : 1);
-        const bool general = wsum_general((u32)sc->weq.size(), sc->weq[1].degree);
+        const int rest = wsum_rest_kind((u32)sc->weq.size(), sc->weq.size() > 1 ? sc->weq[1].degree : 0);
         u64 w[2 * dpk::WSUM_MAX_SUMS];
-        CHK(wait_result_at(ctx, ctx->res_off, fa.seq, 0, 2 * (u32)dpk::wsum_sums((int)nf, a.skip1 != 0, general), w, dpk::WSUM_SEQ_SLOT, dpk::WSUM_CHK_SLOT));
+        CHK(wait_result_at(ctx, ctx->res_off, fa.seq, 0, 2 * (u32)dpk::wsum_sums((int)nf, a.skip1 != 0, rest), w, dpk::WSUM_SEQ_SLOT, dpk::WSUM_CHK_SLOT));
         E2 q[dpk::WSUM_MAX_EQS * dpk::MAX_PTS];
+        q[1] = gl::e2_zero();
         for (int i = 0; i < n0; i++) q[a.skip1 && i > 0 ? i + 1 : i] = gl::e2(w[2 * i], w[2 * i + 1]);
         for (size_t g = 1; g < sc->weq.size(); g++)
             for (u32 t = 0; t <= sc->weq[g].degree; t++) {
-                const int i = n0 + (int)(g - 1) * dpk::wsum_rest((int)nf, general) + (int)t;
+                const int i = n0 + (int)(g - 1) * dpk::wsum_rest((int)nf, rest) + (int)t;
                 q[g * dpk::MAX_PTS + t] = gl::e2(w[2 * i], w[2 * i + 1]);
             }
-        form_weighted_message(q);
+        if (weighted())
+            form_weighted_message(q);
+        else
+            form_message(q);
         return DPS_OK;
 }
 
@@ -4315,7 +4412,7 @@ int32_t FusedRound::end_waiting_launch()
 bool FusedRound::admit_stages()
 {
         u32 widest = 1;
-        const SliceSize size = slice_size(sc->poly, sc->slice_ids.size(), sc->slice_terms.size(), sc->slice_shorter, sc->weq.size());
+        const SliceSize size = slice_size(sc->poly, sc->slice_ids.size(), sc->slice_terms.size(), sc->slice_shorter, sc->weq.empty() ? 0 : sc->h_poly_ops.size());
         for (const dps_sc::Stage &st : sc->stages) {
             widest = std::max(widest, st.W);
             if (slice_workgroups_per_cu(ctx, size, sc->fast_nf, sc->fast_eq >= 0 || weighted(), (u32)sc->slice_ids.size(), st.cap) < 1) return false;
@@ -4327,8 +4424,9 @@ bool FusedRound::admit_stages()
 // round has the sequence number seq0 (a round's call takes one number whether or not it makes a trip).
 int32_t FusedRound::launch_stages_at(u64 seq0, u32 first_go)
 {
-        switch (slice_size(sc->poly, sc->slice_ids.size(), sc->slice_terms.size(), sc->slice_shorter, sc->weq.size())) {
-        case SLICE_EQS: return launch_stages_of<SLICE_EQS>(seq0, first_go);
+        switch (slice_size(sc->poly, sc->slice_ids.size(), sc->slice_terms.size(), sc->slice_shorter, sc->weq.empty() ? 0 : sc->h_poly_ops.size())) {
+        case SLICE_PARTS_FEW: return launch_stages_of<SLICE_PARTS_FEW>(seq0, first_go);
+        case SLICE_PARTS_MANY: return launch_stages_of<SLICE_PARTS_MANY>(seq0, first_go);
         case SLICE_PRODUCT: return launch_stages_of<SLICE_PRODUCT>(seq0, first_go);
         case SLICE_FEW: return launch_stages_of<SLICE_FEW>(seq0, first_go);
         default: return launch_stages_of<SLICE_MANY>(seq0, first_go);
@@ -4385,16 +4483,20 @@ int32_t FusedRound::launch_stages_of(u64 seq0, u32 first_go)
             sa.hw0 = st.h0[n_tabs];
             sa.hw1 = st.h1[n_tabs];
             sa.n_tabs = n_tabs;
-            if constexpr (SIZE == SLICE_EQS) {
+            if constexpr (slice_parts(SIZE)) {
                 // (the programs in the terms' place)
                 memcpy(static_cast<void *>(sa.terms), sc->h_poly_ops.data(), sc->h_poly_ops.size() * sizeof(dpk::PolyOp));
                 sa.n_eqs = (u32)sc->weq.size();
+                sa.n_parts = (u32)sc->weq_parts.size();
+                for (u32 q = 0; q < sa.n_parts; q++) {
+                    const dps_sc::ProgramPart &part = sc->weq_parts[q];
+                    sa.op_begin[q] = (uint8_t)part.op_begin, sa.op_end[q] = (uint8_t)part.op_end, sa.part_of[q] = (uint8_t)part.of;
+                }
                 sa.hw_stride = si + 1 < sc->stages.size() ? (u32)(round_up((size_t)sc->stages[si + 1].src_len * 8, 256) / 8) : 0;
-                for (u32 g = 0; g < sa.n_eqs; g++) {
+                for (u32 g = 0; g < (u32)sc->weq.size(); g++) {
                     const dps_sc::WeightedEq &w = sc->weq[g];
                     sa.geq0[g] = w.c0, sa.geq1[g] = w.c1;
                     sa.degree[g] = w.degree, sa.off_q[g] = w.off_q, sa.off_d[g] = w.off_d;
-                    sa.op_begin[g] = w.op_begin, sa.op_end[g] = w.op_end;
                 }
                 sa.n_sums1 = sc->weq_sums1, sa.n_sums2 = sc->weq_sums2;
             } else if (SIZE != SLICE_PRODUCT) {
@@ -4575,7 +4677,7 @@ FusedRound::Plan FusedRound::plan_round(u32 jj, bool skip1_jj) const
 {
         Plan p;
         p.n_pairs = 1ull << (sc->n_vars - jj);
-        p.split = p.n_pairs <= POLY_SPLIT_MAX_PAIRS && !weighted();
+        p.split = p.n_pairs <= POLY_SPLIT_MAX_PAIRS && !by_program(p.n_pairs);
         p.split_log = 0;
         p.blocks = blocks_for_pairs(p.n_pairs);
         if (p.split) poly_split_plan(p.n_pairs, sc->poly_split_cap, n_groups <= POLY_RAW_MAX_GROUPS, &p.split_log, &p.blocks);
@@ -4590,7 +4692,7 @@ FusedRound::Plan FusedRound::plan_round(u32 jj, bool skip1_jj) const
 // waits for the mail of sequence number `seq_jj` and takes the challenge and the message's scalars from it.
 int32_t FusedRound::launch_round(u32 jj, const Plan &p, bool skip1_jj, bool ahead, u64 seq_jj)
 {
-        if (weighted()) return launch_weighted(jj, skip1_jj, ahead, seq_jj);
+        if (by_program(p.n_pairs)) return launch_weighted(jj, skip1_jj, ahead, seq_jj);
         dpk::PolyArgs pa;
         pa.groups = sc->d_poly_groups + (size_t)(jj - 1) * n_groups;
         pa.terms = sc->d_poly_terms;
@@ -4690,16 +4792,20 @@ int32_t FusedRound::launch_weighted(u32 jj, bool skip1_jj, bool ahead, u64 seq_j
             base = base && pg.tab[k].mode == dpk::POLY_PAIR && !pg.tab[k].s1;
         }
         wa.n_tabs = pg.n_tabs;
-        wa.n_eqs = (u32)sc->weq.size();
+        const dps_sc::WeightedEq *eqs = weighted() ? sc->weq.data() : &sc->one;
+        wa.n_eqs = weighted() ? (u32)sc->weq.size() : 1;
         const bool fact = poly_round_weights_factored(sc, jj);
         const u64 off = eq_level_off(sc->n_vars, jj), lo = fact ? eq_low_off(sc->n_vars, jj) : 0, hi = fact ? eq_level_off(sc->n_vars, jj + dpk::EQ_LO_BITS) : 0;
         for (u32 g = 0; g < wa.n_eqs; g++) {
-            const dps_sc::WeightedEq &w = sc->weq[g];
-            wa.op_begin[g] = w.op_begin, wa.op_end[g] = w.op_end, wa.degree[g] = w.degree;
+            const dps_sc::WeightedEq &w = eqs[g];
+            wa.degree[g] = w.degree;
             if (w.base_program) wa.base_program |= 1u << g;
             wa.q0[g] = w.c0 + off, wa.q1[g] = w.c1 + off;
             if (fact) wa.lq0[g] = w.c0 + lo, wa.lq1[g] = w.c1 + lo, wa.hq0[g] = w.c0 + hi, wa.hq1[g] = w.c1 + hi;
         }
+        // (weighted programs are not cut: a part for every factor)
+        if (!weighted()) wa.op_end[0] = (u32)sc->h_poly_ops.size();
+        for (const dps_sc::ProgramPart &q : sc->weq_parts) wa.op_begin[q.of] = q.op_begin, wa.op_end[q.of] = q.op_end;
         std::copy(sc->h_poly_ops.begin(), sc->h_poly_ops.end(), wa.ops);
         wa.n_pairs = 1ull << (sc->n_vars - jj);
         wa.r0 = ahead ? 0 : a.r0;
@@ -4789,7 +4895,7 @@ int32_t FusedRound::multi_term_round()
             }
         }
     }
-    int32_t rc = weighted() ? take_weighted_sums() : take_sums(slots_now);
+    int32_t rc = by_program(n_pairs) ? take_weighted_sums() : take_sums(slots_now);
     if (rc != DPS_OK) {
         // a launch that left without publishing may have taken some of its tickets and written some of its tables
         sc->broken = true;
