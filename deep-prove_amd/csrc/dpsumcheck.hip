@@ -1652,7 +1652,7 @@ struct dps_sc {
     const u64 *eq_c0, *eq_c1;  // its storage (level 0 at entry 0)
     E2 fast_coeff;
     E2 eq_scalar;       // product of eq1(rho_i, r_{i+1}) over the bound variables
-    // A sum over two or three eq factors (wsum_kernel, slice_kernel with SliceArgsParts): every term has one of them, all in closed form.  In order of
+    // A sum over two or three eq factors (wsum_kernel, slice_kernel with SliceArgsEqs): every term has one of them, all in closed form.  In order of
     // their polynomials' degrees, highest first; p(1) of a round gives the first one's sum at 1
     struct WeightedEq {
         u32 k;                        // the eq table as registered
@@ -1660,14 +1660,11 @@ struct dps_sc {
         const u64 *c0, *c1;           // its storage (level 0 at entry 0)
         u32 degree;                   // of the polynomial it weights
         E2 scalar;                    // product of eq1(rho_i, r_{i+1}) over the bound variables
-        bool base_program;            // all coefficients of its program are in the base field
-        u32 off_q, off_d;             // where a resident trip's sums lie (dpk::SliceArgsParts)
+        u32 op_begin, op_end;         // the polynomial's program in h_poly_ops
+        bool base_program;            // ... all of whose coefficients are in the base field
+        u32 off_q, off_d;             // where a resident trip's sums lie (dpk::SliceArgsEqs)
     };
     std::vector<WeightedEq> weq;
-    struct ProgramPart {
-        u32 op_begin, op_end, of;     // operations in h_poly_ops; the polynomial
-    };
-    std::vector<ProgramPart> weq_parts;
     // A sum of several terms with one common eq factor (fast_eq): its rounds that are launches of their own run by a program all the same, as if it were
     // the only entry of weq; the resident rounds run term by term
     bool one_program = false;
@@ -1842,26 +1839,23 @@ size_t slice_area_off(const dps_ctx *ctx) { return ctx->pinned_words / 2 + 64 + 
 
 // The sizes of a resident launch's arguments: a product's, and by its tables and terms a sum's (`shorter`: some table has fewer
 // variables than the sum)
-enum SliceSize { SLICE_PRODUCT, SLICE_FEW, SLICE_MANY, SLICE_PARTS_FEW, SLICE_PARTS_MANY };
-constexpr bool slice_parts(SliceSize s) { return s == SLICE_PARTS_FEW || s == SLICE_PARTS_MANY; }
-// (`n_ops`: of the programs of a sum that runs by them, else 0)
-SliceSize slice_size(bool sum, size_t n_tabs, size_t n_terms, bool shorter, size_t n_ops)
+enum SliceSize { SLICE_PRODUCT, SLICE_FEW, SLICE_MANY, SLICE_EQS };
+SliceSize slice_size(bool sum, size_t n_tabs, size_t n_terms, bool shorter, bool eqs)
 {
-    if (n_ops) return n_tabs <= 8 && n_ops <= (size_t)dpk::SliceArgsPartsFew::OPS && !shorter ? SLICE_PARTS_FEW : SLICE_PARTS_MANY;
+    if (eqs) return SLICE_EQS;
     if (!sum) return SLICE_PRODUCT;
     return n_tabs <= (size_t)dpk::SL_FEW_TABS && n_terms <= (size_t)dpk::SL_FEW_TERMS && !shorter ? SLICE_FEW : SLICE_MANY;
 }
 template <SliceSize SIZE>
 using SliceArgsFor = std::conditional_t<SIZE == SLICE_PRODUCT, dpk::SliceArgsProduct,
-                                        std::conditional_t<SIZE == SLICE_FEW, dpk::SliceArgsFew, std::conditional_t<SIZE == SLICE_PARTS_FEW, dpk::SliceArgsPartsFew,
-                                                                                               std::conditional_t<SIZE == SLICE_PARTS_MANY, dpk::SliceArgsPartsMany, dpk::SliceArgs>>>>;
+                                        std::conditional_t<SIZE == SLICE_FEW, dpk::SliceArgsFew, std::conditional_t<SIZE == SLICE_EQS, dpk::SliceArgsEqs, dpk::SliceArgs>>>;
 template <int NF, bool EQ, SliceSize SIZE>
 constexpr auto slice_variant = &dpk::slice_kernel<NF, EQ, SIZE != SLICE_PRODUCT, dpk::SL_BLOCK, SliceArgsFor<SIZE>>;
 template <SliceSize SIZE>
 size_t slice_lds_bytes(u32 n_tabs, u32 cap, bool eq)
 {
     // (several eq factors: sized for as many as there can be)
-    return (size_t)dpk::slice_lds_words(n_tabs, cap, dpk::SL_BLOCK, slice_parts(SIZE) ? dpk::SL_MAX_EQS : eq, SliceArgsFor<SIZE>::TERMS) * 8;
+    return (size_t)dpk::slice_lds_words(n_tabs, cap, dpk::SL_BLOCK, SIZE == SLICE_EQS ? dpk::SL_MAX_EQS : eq, SliceArgsFor<SIZE>::TERMS) * 8;
 }
 
 // A workgroup of a resident launch may take most of a compute unit's LDS (it is alone there: 1024 threads); more than
@@ -1890,8 +1884,7 @@ u32 slice_lds_granted(dps_ctx *ctx)
 #define SLICE_VARIANTS(SK)                                                                                              \
     SK(1, true, SLICE_PRODUCT) SK(2, true, SLICE_PRODUCT) SK(2, false, SLICE_PRODUCT) SK(3, false, SLICE_PRODUCT)       \
     SLICE_SUM_VARIANTS(SK, SLICE_FEW) SLICE_SUM_VARIANTS(SK, SLICE_MANY)                                                \
-    SK(2, true, SLICE_PARTS_FEW) SK(3, true, SLICE_PARTS_FEW) SK(4, true, SLICE_PARTS_FEW)                              \
-    SK(2, true, SLICE_PARTS_MANY) SK(3, true, SLICE_PARTS_MANY) SK(4, true, SLICE_PARTS_MANY)
+    SK(2, true, SLICE_EQS) SK(3, true, SLICE_EQS) SK(4, true, SLICE_EQS)
 template <SliceSize SIZE>
 int32_t launch_slice(dps_ctx *ctx, u32 nf, bool eq, u32 workgroups, u32 n_tabs, u32 cap, const SliceArgsFor<SIZE> &a)
 {
@@ -2219,8 +2212,8 @@ dpk::PolyOp program_op(u32 kind, u32 d, u32 slot, E2 c)
 }
 
 // Appends the operations of the node of depth `depth` with these terms, each of at least one factor (their order is not kept); returns
-// its number of products.  `ends`: where the operations of each of its children end.
-u32 program_build(ProgramTerm *t, u32 n, u32 depth, std::vector<dpk::PolyOp> &ops, std::vector<u32> *ends = nullptr)
+// its number of products.
+u32 program_build(ProgramTerm *t, u32 n, u32 depth, std::vector<dpk::PolyOp> &ops)
 {
     u32 products = 0;
     while (n) {
@@ -2259,16 +2252,14 @@ u32 program_build(ProgramTerm *t, u32 n, u32 depth, std::vector<dpk::PolyOp> &op
         } else {
             ops.push_back(program_op(dpk::POLY_OP_LEAF, depth, best, ending));
         }
-        if (ends) ends->push_back((u32)ops.size());
         products++;
         t += with, n -= with;
     }
     return products;
 }
 
-// A whole program: its first operation enters the root with the constant.  `most`: parts it may be cut into, between children of the root
-// (each enters a root of its own); `ends`: where the parts' operations end.  Returns the number of products.
-u32 program_root(ProgramTerm *t, u32 n, u32 most, std::vector<dpk::PolyOp> &ops, std::vector<u32> *ends)
+// A whole program: its first operation enters the root with the constant.  Returns the number of products.
+u32 program_root(ProgramTerm *t, u32 n, std::vector<dpk::PolyOp> &ops)
 {
     E2 root = gl::e2_zero();
     u32 m = 0;
@@ -2277,29 +2268,8 @@ u32 program_root(ProgramTerm *t, u32 n, u32 most, std::vector<dpk::PolyOp> &ops,
             std::swap(t[i], t[m++]);
         else
             root = gl::add(root, t[i].coeff);
-    const size_t begin = ops.size();
     ops.push_back(program_op(dpk::POLY_OP_ENTER, 0, 0, root));
-    if (most < 2) return program_build(t, m, 0, ops);
-    std::vector<u32> children;
-    const u32 products = program_build(t, m, 0, ops, &children);
-    // parts of whole children, about as many operations in each
-    const u32 parts = std::min<u32>(most, std::max<u32>(1, (u32)children.size())), all = (u32)(ops.size() - begin - 1);
-    std::vector<dpk::PolyOp> cut;
-    u32 from = (u32)begin + 1, child = 0;
-    for (u32 q = 0; q < parts; q++) {
-        u32 to = from;
-        const u32 goal = (u32)begin + 1 + (u32)((u64)all * (q + 1) / parts);
-        // (at least one child a part, and one left for every part to come)
-        while (child < children.size() && (to == from || children[child] <= goal) && (children.size() - child > parts - q - 1)) to = children[child++];
-        if (q + 1 == parts && child < children.size()) to = children.back(), child = (u32)children.size();
-        cut.push_back(q == 0 ? ops[begin] : program_op(dpk::POLY_OP_ENTER, 0, 0, gl::e2_zero()));
-        cut.insert(cut.end(), ops.begin() + from, ops.begin() + to);
-        if (ends) ends->push_back((u32)(begin + cut.size()));
-        from = to;
-    }
-    ops.resize(begin);
-    ops.insert(ops.end(), cut.begin(), cut.end());
-    return products;
+    return program_build(t, m, 0, ops);
 }
 
 // one staged upload of all descriptors; not waited for (the staging vector lives as long as the session)
@@ -2414,8 +2384,8 @@ u32 slice_counter_sets_log(u32 W)
 u32 slice_second_round_passes(const dps_sc *sc, u32 n_quads)
 {
     if (!sc->weq.empty()) {
-        // (every part has its own lanes; a lane takes a quad at one challenge)
-        const u32 per = ((u32)dpk::SL_BLOCK / (u32)sc->weq_parts.size()) & ~63u;
+        // (every factor has its own lanes; a lane takes a quad at one challenge)
+        const u32 per = ((u32)dpk::SL_BLOCK / (u32)sc->weq.size()) & ~63u;
         u32 most = 0;
         for (const dps_sc::WeightedEq &w : sc->weq) most = std::max(most, (n_quads * (w.degree + 1) + per - 1) / per);
         return most;
@@ -2442,7 +2412,7 @@ void plan_resident_rounds(dps_sc *sc, u32 n_tabs, u32 n_mles)
         const E2 rho = (sc->weq.empty() ? sc->eq_info : sc->weq[0].info)->point[round - 1];
         return !(rho.c0 == 0 && rho.c1 == 0);
     };
-    const u32 pairs_fit = slice_pairs_per_workgroup(sc->ctx, slice_size(sc->poly, n_tabs, sc->slice_terms.size(), sc->slice_shorter, sc->weq.empty() ? 0 : sc->h_poly_ops.size()), sc->fast_nf, has_eq, n_tabs);
+    const u32 pairs_fit = slice_pairs_per_workgroup(sc->ctx, slice_size(sc->poly, n_tabs, sc->slice_terms.size(), sc->slice_shorter, !sc->weq.empty()), sc->fast_nf, has_eq, n_tabs);
     if (pairs_fit == 0) return;
     const u32 per_wg_max = std::min<u32>(pairs_fit, sc->poly ? SLICE_SUM_PAIRS : SLICE_PRODUCT_PAIRS);
     auto pairs_of = [&](u32 round) { return (u64)1 << (n - round); };
@@ -2578,7 +2548,6 @@ struct SessionSetup {
     void detect_product();
     bool closed_form_eq_factor();
     bool weighted_programs();
-    bool adopt_programs(dps_sc::WeightedEq *eqs, u32 n_eqs, std::vector<dpk::PolyOp> &&ops);
     bool group_terms();
     void adopt_groups();
     void nested_programs();
@@ -2693,7 +2662,7 @@ bool SessionSetup::closed_form_eq_factor()
 // form term by term.  (Linking an activation of 2^21 entries, two factors of degrees 3 and 1 over two tables: 684 -> 412 us; its rounds of 2^20 .. 2^17
 // pairs 158, 92, 66, 47 -> 59, 53, 40, 30 us, the resident ones 205 -> 141.)
 // One eq factor: the same programs in the rounds that are launches of their own (rounds of 2^19 .. 2^16 pairs of a fraction-sum layer 52, 38, 30, 25 ->
-// 46, 36, 29, 21 us); resident its rounds stay with the terms, which are spread over more lanes (a trip of two rounds 8.5 .. 10 us, 15 .. 16 by a program).
+// 43, 34, 28, 20 us); resident its rounds stay with the terms, which are spread over more lanes (a trip of two rounds 8.5 .. 10 us, 15 .. 16 by a program).
 bool SessionSetup::weighted_programs()
 {
     if (sc->n_terms < 2 || sc->n_terms > MAX_PROGRAM_TERMS) return false;
@@ -2741,42 +2710,32 @@ bool SessionSetup::weighted_programs()
             for (u32 f = 0; f < t.n_factors; f++)
                 if (t.factors[f] != eqs[g].k) p.slot[p.n++] = (uint8_t)(std::find(tabs, tabs + n_tabs, t.factors[f]) - tabs);
         }
-        const u32 begin = (u32)ops.size();
-        program_root(ts, n, 1, ops, nullptr);
-        if (n_eqs > 1) sc->weq_parts.push_back(dps_sc::ProgramPart{begin, (u32)ops.size(), g});
+        eqs[g].op_begin = (u32)ops.size();
+        program_root(ts, n, ops);
+        eqs[g].op_end = (u32)ops.size();
     }
+    if (ops.size() > (size_t)dpk::SL_EQS_OPS) return false;
     if (n_eqs == 1) {
-        if (ops.size() <= (size_t)dpk::SL_PARTS_OPS) {
-            sc->one_program = true;
-            sc->one = eqs[0];
-            sc->h_poly_ops = std::move(ops);
-        }
+        sc->one_program = true;
+        sc->one = eqs[0];
+        sc->h_poly_ops = std::move(ops);
         return false;
     }
-    if (!adopt_programs(eqs, n_eqs, std::move(ops))) return false;
+    // the places of a resident trip's sums
+    u32 sums = 0;
+    for (u32 g = 0; g < n_eqs; g++) eqs[g].off_q = sums, sums += eqs[g].degree + 1;
+    sc->weq_sums1 = sums;
+    for (u32 g = 0; g < n_eqs; g++) eqs[g].off_d = sums, sums += (g == 0 ? eqs[g].degree : eqs[g].degree + 1) * (eqs[g].degree + 1);
+    sc->weq_sums2 = sums;
+    if (sc->weq_sums1 > (u32)dpk::SL_MAX_SUMS) return false;
+    sc->weq.assign(eqs, eqs + n_eqs);
+    sc->h_poly_ops = std::move(ops);
     nf = eqs[0].degree;
     groups.assign(1, std::vector<u32>(tabs, tabs + n_tabs));
     tb.assign(1, 0);
     te.assign(1, sc->n_terms);
     sc->poly_op_begin.assign(1, 0);
     sc->poly_op_end.assign(1, 0);
-    return true;
-}
-
-// The session takes the programs written down (their parts are in weq_parts): the places of a trip's sums.  False: too many of something.
-bool SessionSetup::adopt_programs(dps_sc::WeightedEq *eqs, u32 n_eqs, std::vector<dpk::PolyOp> &&ops)
-{
-    u32 sums = 0;
-    for (u32 g = 0; g < n_eqs; g++) eqs[g].off_q = sums, sums += eqs[g].degree + 1;
-    sc->weq_sums1 = sums;
-    for (u32 g = 0; g < n_eqs; g++) eqs[g].off_d = sums, sums += (g == 0 ? eqs[g].degree : eqs[g].degree + 1) * (eqs[g].degree + 1);
-    sc->weq_sums2 = sums;
-    if (ops.size() > (size_t)dpk::SL_PARTS_OPS || sc->weq_sums1 > (u32)dpk::SL_MAX_SUMS) {
-        sc->weq_parts.clear();
-        return false;
-    }
-    sc->weq.assign(eqs, eqs + n_eqs);
-    sc->h_poly_ops = std::move(ops);
     return true;
 }
 
@@ -2881,7 +2840,7 @@ void SessionSetup::nested_programs()
             plain += pt.n_factors;  // n_factors - 1 products and one for the coefficient
         }
         std::vector<dpk::PolyOp> ops;
-        nested += program_root(ts.data(), (u32)ts.size(), 1, ops, nullptr);
+        nested += program_root(ts.data(), (u32)ts.size(), ops);
         if (ops.size() > (size_t)dpk::POLY_LDS_OPS) use_ops = false;
         sc->poly_op_begin[g] = (u32)all_ops.size();
         all_ops.insert(all_ops.end(), ops.begin(), ops.end());
@@ -4039,15 +3998,14 @@ void host_tail_weighted_sums(dps_sc *sc, u32 j, bool skip1, E2 *q)
         for (u32 t = 0; t <= sc->fast_nf; t++) {
             if (t > 0)
                 for (u32 f = 0; f < n_tabs; f++) val[f] = gl::add(val[f], d[f]);
-            E2 poly[dpk::WSUM_MAX_EQS] = {};
-            for (const dps_sc::ProgramPart &part : sc->weq_parts) {
-                if (t > sc->weq[part.of].degree || (part.of == 0 && t == 1 && skip1)) continue;
-                const dpk::PolyOp &root = sc->h_poly_ops[part.op_begin];
-                u32 pc = part.op_begin + 1;
-                poly[part.of] = gl::add(poly[part.of], host_walk(sc->h_poly_ops, pc, part.op_end, gl::e2(root.c0, root.c1), val));
+            for (size_t g = 0; g < sc->weq.size(); g++) {
+                const dps_sc::WeightedEq &w = sc->weq[g];
+                if (t > w.degree || (g == 0 && t == 1 && skip1)) continue;
+                const dpk::PolyOp &root = sc->h_poly_ops[w.op_begin];
+                u32 pc = w.op_begin + 1;
+                const E2 poly = host_walk(sc->h_poly_ops, pc, w.op_end, gl::e2(root.c0, root.c1), val);
+                q[g * dpk::MAX_PTS + t] = gl::add(q[g * dpk::MAX_PTS + t], gl::mul(poly, weight[g][p]));
             }
-            for (size_t g = 0; g < sc->weq.size(); g++)
-                if (t <= sc->weq[g].degree) q[g * dpk::MAX_PTS + t] = gl::add(q[g * dpk::MAX_PTS + t], gl::mul(poly[g], weight[g][p]));
         }
     }
 }
@@ -4412,7 +4370,7 @@ int32_t FusedRound::end_waiting_launch()
 bool FusedRound::admit_stages()
 {
         u32 widest = 1;
-        const SliceSize size = slice_size(sc->poly, sc->slice_ids.size(), sc->slice_terms.size(), sc->slice_shorter, sc->weq.empty() ? 0 : sc->h_poly_ops.size());
+        const SliceSize size = slice_size(sc->poly, sc->slice_ids.size(), sc->slice_terms.size(), sc->slice_shorter, !sc->weq.empty());
         for (const dps_sc::Stage &st : sc->stages) {
             widest = std::max(widest, st.W);
             if (slice_workgroups_per_cu(ctx, size, sc->fast_nf, sc->fast_eq >= 0 || weighted(), (u32)sc->slice_ids.size(), st.cap) < 1) return false;
@@ -4424,9 +4382,8 @@ bool FusedRound::admit_stages()
 // round has the sequence number seq0 (a round's call takes one number whether or not it makes a trip).
 int32_t FusedRound::launch_stages_at(u64 seq0, u32 first_go)
 {
-        switch (slice_size(sc->poly, sc->slice_ids.size(), sc->slice_terms.size(), sc->slice_shorter, sc->weq.empty() ? 0 : sc->h_poly_ops.size())) {
-        case SLICE_PARTS_FEW: return launch_stages_of<SLICE_PARTS_FEW>(seq0, first_go);
-        case SLICE_PARTS_MANY: return launch_stages_of<SLICE_PARTS_MANY>(seq0, first_go);
+        switch (slice_size(sc->poly, sc->slice_ids.size(), sc->slice_terms.size(), sc->slice_shorter, !sc->weq.empty())) {
+        case SLICE_EQS: return launch_stages_of<SLICE_EQS>(seq0, first_go);
         case SLICE_PRODUCT: return launch_stages_of<SLICE_PRODUCT>(seq0, first_go);
         case SLICE_FEW: return launch_stages_of<SLICE_FEW>(seq0, first_go);
         default: return launch_stages_of<SLICE_MANY>(seq0, first_go);
@@ -4483,19 +4440,15 @@ int32_t FusedRound::launch_stages_of(u64 seq0, u32 first_go)
             sa.hw0 = st.h0[n_tabs];
             sa.hw1 = st.h1[n_tabs];
             sa.n_tabs = n_tabs;
-            if constexpr (slice_parts(SIZE)) {
+            if constexpr (SIZE == SLICE_EQS) {
                 // (the programs in the terms' place)
                 memcpy(static_cast<void *>(sa.terms), sc->h_poly_ops.data(), sc->h_poly_ops.size() * sizeof(dpk::PolyOp));
                 sa.n_eqs = (u32)sc->weq.size();
-                sa.n_parts = (u32)sc->weq_parts.size();
-                for (u32 q = 0; q < sa.n_parts; q++) {
-                    const dps_sc::ProgramPart &part = sc->weq_parts[q];
-                    sa.op_begin[q] = (uint8_t)part.op_begin, sa.op_end[q] = (uint8_t)part.op_end, sa.part_of[q] = (uint8_t)part.of;
-                }
                 sa.hw_stride = si + 1 < sc->stages.size() ? (u32)(round_up((size_t)sc->stages[si + 1].src_len * 8, 256) / 8) : 0;
-                for (u32 g = 0; g < (u32)sc->weq.size(); g++) {
+                for (u32 g = 0; g < sa.n_eqs; g++) {
                     const dps_sc::WeightedEq &w = sc->weq[g];
                     sa.geq0[g] = w.c0, sa.geq1[g] = w.c1;
+                    sa.op_begin[g] = w.op_begin, sa.op_end[g] = w.op_end;
                     sa.degree[g] = w.degree, sa.off_q[g] = w.off_q, sa.off_d[g] = w.off_d;
                 }
                 sa.n_sums1 = sc->weq_sums1, sa.n_sums2 = sc->weq_sums2;
@@ -4798,14 +4751,11 @@ int32_t FusedRound::launch_weighted(u32 jj, bool skip1_jj, bool ahead, u64 seq_j
         const u64 off = eq_level_off(sc->n_vars, jj), lo = fact ? eq_low_off(sc->n_vars, jj) : 0, hi = fact ? eq_level_off(sc->n_vars, jj + dpk::EQ_LO_BITS) : 0;
         for (u32 g = 0; g < wa.n_eqs; g++) {
             const dps_sc::WeightedEq &w = eqs[g];
-            wa.degree[g] = w.degree;
+            wa.op_begin[g] = w.op_begin, wa.op_end[g] = w.op_end, wa.degree[g] = w.degree;
             if (w.base_program) wa.base_program |= 1u << g;
             wa.q0[g] = w.c0 + off, wa.q1[g] = w.c1 + off;
             if (fact) wa.lq0[g] = w.c0 + lo, wa.lq1[g] = w.c1 + lo, wa.hq0[g] = w.c0 + hi, wa.hq1[g] = w.c1 + hi;
         }
-        // (weighted programs are not cut: a part for every factor)
-        if (!weighted()) wa.op_end[0] = (u32)sc->h_poly_ops.size();
-        for (const dps_sc::ProgramPart &q : sc->weq_parts) wa.op_begin[q.of] = q.op_begin, wa.op_end[q.of] = q.op_end;
         std::copy(sc->h_poly_ops.begin(), sc->h_poly_ops.end(), wa.ops);
         wa.n_pairs = 1ull << (sc->n_vars - jj);
         wa.r0 = ahead ? 0 : a.r0;

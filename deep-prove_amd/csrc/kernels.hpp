@@ -1698,7 +1698,7 @@ struct SliceTerm {
 template <int TABS_, int TERMS_, bool LACKS_>
 struct SliceArgsOf {
     static constexpr int TABS = TABS_, TERMS = TERMS_;
-    static constexpr u32 EQS = 0;  // (SliceArgsParts: eq factors of a sum given as programs)
+    static constexpr u32 EQS = 0;  // (SliceArgsEqs: several eq factors)
     static constexpr bool LACKS = LACKS_;  // tables of fewer variables are among them
     const u64 *s0[TABS];
     const u64 *s1[TABS];         // the tables before the folds that are pending when the launch starts: src_len entries each
@@ -1742,28 +1742,21 @@ struct SliceArgsOf {
 using SliceArgs = SliceArgsOf<SL_MAX_TABS, SL_MAX_TERMS, true>;
 using SliceArgsFew = SliceArgsOf<SL_FEW_TABS, SL_FEW_TERMS, false>;
 using SliceArgsProduct = SliceArgsOf<4, 1, false>;  // (at most 3 tables, no terms)
-// A sum given as nested programs: sum_g eq(rho_g, x) P_g(x) with up to three eq factors and polynomials P_g over shared tables (wsum_kernel
-// says why they are kept apart), or one polynomial without an eq factor of its own (n_eqs = 0).  A program may be cut into parts at its
-// root; every part has lanes of its own, whole wavefronts of them, so that a wavefront runs one program.  The
-// programs lie in the terms' place.  Sums: P_g's q_g(t), t = 0 .. degree[g], from off_q[g] on; with a trip of two rounds, from off_d[g] on,
-// those of the second round at its points (t = 0, 2, .. for the first polynomial, whose t = 1 comes from the claim, t = 0, 1, 2, .. for the
-// others), each at the challenges 0 .. degree[g] (a polynomial of that degree in the challenge).
-constexpr u32 SL_MAX_EQS = 3, SL_MAX_PARTS = 8;
-template <int TABS_, int OPS_, bool LACKS_>
-struct SliceArgsParts : SliceArgsOf<TABS_, OPS_ * (int)sizeof(PolyOp) / (int)sizeof(SliceTerm) + 1, LACKS_> {
+// A sum over several eq factors, sum_g eq(rho_g, x) P_g(x) with polynomials P_g over shared tables (wsum_kernel says why they are kept
+// apart).  The weights of every factor live in LDS; P_g is a nested program in the terms' place, walked by lanes of its own, whole
+// wavefronts of them, so that a wavefront runs one program.  Sums: P_g's q_g(t), t = 0 .. degree[g], from off_q[g] on; with a trip of two
+// rounds, from off_d[g] on, those of the second round at its points (t = 0, 2, .. for the first factor, whose t = 1 comes from
+// the claim, t = 0, 1, 2, .. for the others), each at the challenges 0 .. degree[g] (a polynomial of that degree in the challenge).
+constexpr u32 SL_MAX_EQS = 3;
+constexpr int SL_EQS_OPS = 64;
+struct SliceArgsEqs : SliceArgsOf<8, SL_EQS_OPS * (int)sizeof(PolyOp) / (int)sizeof(SliceTerm) + 1, false> {
     static constexpr u32 EQS = SL_MAX_EQS;
-    static constexpr int OPS = OPS_;
-    u32 n_parts, n_eqs, hw_stride;      // hw0, hw1: hw_stride words for every eq factor
-    u32 n_sums1, n_sums2;               // of a trip of one round, of two
+    u32 n_eqs, hw_stride;               // hw0, hw1: hw_stride words for every factor
     const u64 *geq0[SL_MAX_EQS], *geq1[SL_MAX_EQS];
-    u32 degree[SL_MAX_EQS], off_q[SL_MAX_EQS], off_d[SL_MAX_EQS];
-    uint8_t op_begin[SL_MAX_PARTS], op_end[SL_MAX_PARTS], part_of[SL_MAX_PARTS];  // a part's operations; the polynomial it is a part of
+    u32 degree[SL_MAX_EQS], off_q[SL_MAX_EQS], off_d[SL_MAX_EQS], op_begin[SL_MAX_EQS], op_end[SL_MAX_EQS];
+    u32 n_sums1, n_sums2;               // of a trip of one round, of two
 };
-using SliceArgsPartsFew = SliceArgsParts<8, 32, false>;
-using SliceArgsPartsMany = SliceArgsParts<SL_MAX_TABS, 64, true>;
-constexpr int SL_PARTS_OPS = SliceArgsPartsMany::OPS;
-static_assert(sizeof(SliceArgsPartsMany) <= 4096 && sizeof(SliceArgsPartsMany::terms) >= SL_PARTS_OPS * sizeof(PolyOp) &&
-                  sizeof(SliceArgsPartsFew::terms) >= SliceArgsPartsFew::OPS * sizeof(PolyOp), "kernel arguments");
+static_assert(sizeof(SliceArgsEqs) <= 4096 && sizeof(SliceArgsEqs::terms) >= SL_EQS_OPS * sizeof(PolyOp), "kernel arguments");
 static_assert(sizeof(SliceArgs) <= 4096, "kernel arguments");
 
 // dynamic LDS of slice_kernel, in 64-bit words: counters per wavefront, mailbox copy, flags, the terms, then the two table buffers
@@ -1819,7 +1812,7 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
     // same two buffers: read once when the launch starts, and from round to round the weight of a pair is the sum of the
     // weights of the two pairs it is made of (R_{j+1}(p) = R_j(2p) + R_j(2p + 1)), so a fold of the tables is an add here.
     // (several eq factors: `g` is the factor, their weights follow one another)
-    static_assert(ARGS::EQS == 0 || (EQ && TERMS), "programs belong to a sum of several terms");
+    static_assert(ARGS::EQS == 0 || (EQ && TERMS), "several eq factors belong to a sum of several terms");
     u32 n_eqs = 1;
     if constexpr (ARGS::EQS > 0) n_eqs = a.n_eqs;
     u64 *const wts_big = buf_small + (size_t)nt * 2 * (cap / 2), *const wts_small = wts_big + n_eqs * 2 * sl_weights_cap(cap);
@@ -1831,7 +1824,7 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
         // the programs, in the terms' place
         const u64 *src = reinterpret_cast<const u64 *>(a.terms);
         u64 *dst = dyn + SL_LDS_TERMS;
-        for (u32 w = tid; w < a.op_end[a.n_parts - 1] * (u32)(sizeof(PolyOp) / 8); w += BLOCK) dst[w] = src[w];
+        for (u32 w = tid; w < a.op_end[a.n_eqs - 1] * (u32)(sizeof(PolyOp) / 8); w += BLOCK) dst[w] = src[w];
     } else if (TERMS) {
         // the terms are read per pair and point: staged in LDS once (visible after the first wait's barrier)
         const u64 *src = reinterpret_cast<const u64 *>(a.terms);
@@ -2122,13 +2115,12 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
         // and spread over the lanes; every unit's value goes into the point's counters, where the pieces add up.
         // ---- round j: pairs of the state; units taken from the last thread down, those of the quads from the first up ----
         if constexpr (ARGS::EQS > 0) {
-            // This wavefront's part, and this lane's place among the lanes of that part.  A unit of work is a pair, or with a trip of two
+            // This wavefront's factor, and this lane's place among the lanes of that factor.  A unit of work is a pair, or with a trip of two
             // rounds a quad at one challenge (first the pairs, then the quads challenge by challenge): a lane walks the program at
-            // all of its polynomial's points, and where a wavefront's units are of one kind it adds its sums up before they go into the
+            // all of its factor's points, and where a wavefront's units are of one kind it adds its sums up before they go into the
             // counters (a counter that every lane adds to serves them one after the other).
-            const u32 per = (BLOCK / a.n_parts) & ~(u32)(WAVE - 1);
-            const u32 part = __builtin_amdgcn_readfirstlane(tid / per), l = tid - part * per;
-            const u32 g = part < a.n_parts ? a.part_of[part] : 0;
+            const u32 per = (BLOCK / n_eqs) & ~(u32)(WAVE - 1);
+            const u32 g = __builtin_amdgcn_readfirstlane(tid / per), l = tid - g * per;
             auto units = [&](auto n_points, auto skips, auto program_degree) {
                 constexpr int N = decltype(n_points)::value, DEG = decltype(program_degree)::value;
                 constexpr bool SKIP = decltype(skips)::value;
@@ -2150,9 +2142,9 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
                         return wsum_points<N, SKIP>(lo, gl::sub(hi, lo));
                     };
                     E2 out[N];
-                    wsum_program<DEG>(a.op_begin[part], a.op_end[part], out, [&](u32 o) -> const PolyOp & { return ops[o]; }, table);
+                    wsum_program<DEG>(a.op_begin[g], a.op_end[g], out, [&](u32 o) -> const PolyOp & { return ops[o]; }, table);
                     E2 w = gl::e2_zero();
-                    if (mine && n_eqs) w = pair ? weight(big, at, g) : gl::add(weight(big, 2 * at, g), weight(big, 2 * at + 1, g));
+                    if (mine) w = pair ? weight(big, at, g) : gl::add(weight(big, 2 * at, g), weight(big, 2 * at + 1, g));
                     const gl::E2P wp = gl::prep(w);
                     // where the sums of point i go: those of pairs from off_q on, those of quads from off_d on
                     const u32 kind = !mine ? ~0u : pair ? 0 : 1 + smp;
@@ -2163,7 +2155,7 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
                         const u32 ti = g == 0 && t > 1 ? t - 1 : t;
                         const bool wanted = mine && t <= d && (pair ? !(g == 0 && t == 1 && skip1) : !(g == 0 && t == 1));
                         const u32 idx = pair ? a.off_q[g] + t : a.off_d[g] + smp * npt + ti;
-                        const E2 x = n_eqs ? gl::mulp(out[i], wp) : out[i];
+                        const E2 x = gl::mulp(out[i], wp);
                         if (alike)
                             flush_wave(idx, x, wanted);
                         else if (wanted)
@@ -2171,14 +2163,13 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
                     }
                 }
             };
-            // (the first polynomial is of the highest degree, NF)
-            if (part >= a.n_parts) {
-            } else if (g == 0) {
+            // (the first factor's polynomial is of the highest degree, NF)
+            if (g == 0) {
                 if (skip1)
                     units(std::integral_constant<int, NF>{}, std::true_type{}, std::integral_constant<int, NF>{});
                 else
                     units(std::integral_constant<int, NF + 1>{}, std::false_type{}, std::integral_constant<int, NF>{});
-            } else {
+            } else if (g < n_eqs) {
                 if (a.degree[g] == 1)
                     units(std::integral_constant<int, 2>{}, std::false_type{}, std::integral_constant<int, 1>{});
                 else
@@ -2639,7 +2630,7 @@ struct WsumArgs {
     u32 wait_first, spin_limit;
     const u64 *mail;
     u64 *relay;
-    PolyOp ops[SL_PARTS_OPS];
+    PolyOp ops[SL_EQS_OPS];
 };
 static_assert(sizeof(WsumArgs) <= 4000, "kernel arguments");
 template <int NF, bool SKIP1, bool BASE, int REST>

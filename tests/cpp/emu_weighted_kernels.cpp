@@ -1,5 +1,5 @@
 // Sums over several eq factors, sum_g eq(rho_g, x) P_g(x), on the CPU through tests/cpp/emu/hip/hip_runtime.h under the host sanitizers:
-// wsum_kernel (a round that is a launch of its own) and slice_kernel with SliceArgsParts (the rounds resident in LDS, one or two a trip).
+// wsum_kernel (a round that is a launch of its own) and slice_kernel with SliceArgsEqs (the rounds resident in LDS, one or two a trip).
 // Every sum is compared with q_g(t) = sum_x' R_g(x') P_g(t, x') worked out by plain loops from the terms, R_g from its definition.
 // The programs are built by the rule the library uses, from terms that are also evaluated one by one.
 #include <algorithm>
@@ -199,23 +199,13 @@ static void run_round(const char *name, u32 log_pairs, u32 blocks, u32 n_tabs, s
 
 // ---- slice_kernel: all rounds from round 1, `wide` workgroups and then one ----
 template <int NF>
-static void run_resident(const char *name, u32 n_vars, u32 wide, u32 n_tabs, std::vector<std::vector<Term>> polys, u32 base_tabs, bool doubles, u32 last_left,
-                         std::vector<std::vector<Term>> parts = {}, std::vector<u32> lacks = {})
+static void run_resident(const char *name, u32 n_vars, u32 wide, u32 n_tabs, std::vector<std::vector<Term>> polys, u32 base_tabs, bool doubles, u32 last_left)
 {
-    // (`parts`: of the single polynomial, which then has no eq factor; `lacks`: variables that tables do not have)
-    const bool plain = !parts.empty();
     const u32 G = (u32)polys.size(), n_gpu = n_vars - last_left;
     std::vector<Table> state(n_tabs, Table((size_t)1 << n_vars));
     std::vector<std::vector<u64>> s0(n_tabs), s1(n_tabs), h0(n_tabs), h1(n_tabs);
     for (u32 f = 0; f < n_tabs; f++)
-    {
-        const u32 lack = lacks.empty() ? 0 : lacks[f];
-        for (size_t i = 0; i < state[f].size() >> lack; i++) {
-            const E2 x = f < base_tabs ? gl::e2(felt(), 0) : felt2();
-            s0[f].push_back(x.c0), s1[f].push_back(x.c1);
-        }
-        for (size_t i = 0; i < state[f].size(); i++) state[f][i] = gl::e2(s0[f][i >> lack], s1[f][i >> lack]);
-    }
+        for (E2 &x : state[f]) x = f < base_tabs ? gl::e2(felt(), 0) : felt2(), s0[f].push_back(x.c0), s1[f].push_back(x.c1);
     std::vector<std::vector<E2>> rho(G);
     std::vector<std::vector<u64>> e0(G, std::vector<u64>((size_t)2 << n_vars)), e1 = e0;
     for (u32 g = 0; g < G; g++) {
@@ -227,20 +217,16 @@ static void run_resident(const char *name, u32 n_vars, u32 wide, u32 n_tabs, std
                 e0[g][off] = v.c0, e1[g][off] = v.c1;
             }
     }
-    dpk::SliceArgsPartsMany a;
+    dpk::SliceArgsEqs a;
     memset(&a, 0, sizeof a);
     std::vector<dpk::PolyOp> ops;
     u32 sums = 0;
-    a.n_eqs = plain ? 0 : G;
-    for (auto &part : plain ? parts : polys) {
-        auto p = program_of(part);
-        a.op_begin[a.n_parts] = (uint8_t)ops.size();
-        ops.insert(ops.end(), p.begin(), p.end());
-        a.op_end[a.n_parts] = (uint8_t)ops.size();
-        a.part_of[a.n_parts] = (uint8_t)(plain ? 0 : a.n_parts);
-        a.n_parts++;
-    }
+    a.n_eqs = G;
     for (u32 g = 0; g < G; g++) {
+        auto p = program_of(polys[g]);
+        a.op_begin[g] = (u32)ops.size();
+        ops.insert(ops.end(), p.begin(), p.end());
+        a.op_end[g] = (u32)ops.size();
         a.degree[g] = degree_of(polys[g]);
         a.off_q[g] = sums;
         sums += a.degree[g] + 1;
@@ -284,7 +270,6 @@ static void run_resident(const char *name, u32 n_vars, u32 wide, u32 n_tabs, std
         h0[f].assign(handed + 1, 0), h1[f].assign(handed + 1, 0);
         a.s0[f] = s0[f].data(), a.s1[f] = f < base_tabs ? nullptr : s1[f].data();
         a.h0[f] = h0[f].data(), a.h1[f] = h1[f].data();
-        if (!lacks.empty() && lacks[f]) a.lacks[f] = (uint8_t)(lacks[f] + 1), a.any_lacks = 1;
     }
     std::vector<u64> mail(64, 0), relay(dpk::MAIL_RELAY_WORDS, 0), area(dpk::SL_AREA_WORDS, 0), fin(dpk::SL_FIN_AREA_WORDS, 0),
         gctr((size_t)dpk::SL_MAX_GROUPS * dpk::SL_GROUP_WORDS * dpk::SL_CTR_STRIDE, 0);
@@ -295,7 +280,7 @@ static void run_resident(const char *name, u32 n_vars, u32 wide, u32 n_tabs, std
     gridDim = dim3(wide), blockDim = dim3(dpk::BLOCK);
     std::vector<std::thread> th;
     std::vector<std::unique_ptr<emu::Group>> groups;
-    std::vector<std::vector<u64>> lds(wide, std::vector<u64>(dpk::slice_lds_words(n_tabs, cap, dpk::BLOCK, G, dpk::SliceArgsPartsMany::TERMS), 0xAAAAAAAAAAAAAAAAull));
+    std::vector<std::vector<u64>> lds(wide, std::vector<u64>(dpk::slice_lds_words(n_tabs, cap, dpk::BLOCK, G, dpk::SliceArgsEqs::TERMS), 0xAAAAAAAAAAAAAAAAull));
     for (u32 b = 0; b < wide; b++) {
         groups.emplace_back(new emu::Group());
         groups.back()->reset(dpk::BLOCK);
@@ -306,7 +291,7 @@ static void run_resident(const char *name, u32 n_vars, u32 wide, u32 n_tabs, std
                 emu::group = g;
                 threadIdx = dim3(t);
                 blockIdx = dim3(b, 0, 0);
-                dpk::slice_kernel<NF, true, true, dpk::BLOCK, dpk::SliceArgsPartsMany>(a);
+                dpk::slice_kernel<NF, true, true, dpk::BLOCK, dpk::SliceArgsEqs>(a);
             });
     }
     bool ok = true;
@@ -356,7 +341,7 @@ static void run_resident(const char *name, u32 n_vars, u32 wide, u32 n_tabs, std
         };
         auto direct = [&](const std::vector<Table> &tabs, u32 round, u32 g, u32 t) {
             E2 v = gl::e2_zero();
-            for (size_t p = 0; p < tabs[0].size() / 2; p++) v = gl::add(v, plain ? eval(polys[g], tabs, p, t) : gl::mul(eq_at(rho[g], round, n_vars - round, p), eval(polys[g], tabs, p, t)));
+            for (size_t p = 0; p < tabs[0].size() / 2; p++) v = gl::add(v, gl::mul(eq_at(rho[g], round, n_vars - round, p), eval(polys[g], tabs, p, t)));
             return v;
         };
         for (u32 g = 0; g < G && ok; g++) {
@@ -402,17 +387,13 @@ int main()
     run_round<3, true, false, 1>("extension tables folded on the way in", 8, 1, 2, {lp, ll}, true, false);
     run_round<4, true, false, 2>("three factors of degrees 4, 2 and 1", 9, 3, 4, {p4, p2, p1}, true, false);
     run_round<4, false, false, 2>("the same unfolded, every point, one pair", 0, 1, 4, {p4, p2, p1}, false, false);
+    run_round<3, true, false, 0>("one factor, extension tables folded on the way in", 9, 2, 4, {lp}, true, false);
+    run_round<3, false, true, 0>("the same unfolded over base tables, every point", 6, 1, 4, {lp}, false, true);
     run_round<2, true, false, 2>("degrees 2 and 2 over base tables", 7, 1, 4, {p2, p2}, false, true);
     run_resident<3>("resident, two factors, trips of two rounds", 7, 1, 2, {lp, ll}, 2, true, 0);
     run_resident<3>("resident, one round a trip, the last two rounds left out", 6, 1, 2, {lp, ll}, 1, false, 2);
     run_resident<3>("resident, four workgroups, then one", 9, 4, 2, {lp, ll}, 0, true, 2);
     run_resident<2>("resident, degrees 2 and 2, more pairs than lanes", 10, 1, 4, {p2, p2}, 4, true, 3);
-    const std::vector<Term> a1{{felt2(), {0, 1, 4}}, {felt2(), {1, 1, 4}}}, a2{{felt2(), {2, 3, 5}}, {felt2(), {}}}, a3{{one, {0, 5}}};
-    std::vector<Term> all = a1;
-    for (auto &x : {a2, a3}) all.insert(all.end(), x.begin(), x.end());
-    run_resident<3>("resident, one polynomial in three parts, no eq factor", 8, 1, 6, {all}, 2, true, 2, {a1, a2, a3});
-    run_resident<3>("the same over four workgroups, tables of fewer variables", 9, 4, 6, {all}, 1, true, 2, {a1, a2, a3}, {0, 0, 3, 1, 0, 8});
-    run_resident<2>("one eq factor, four workgroups", 8, 4, 4, {p2}, 0, true, 2);
     run_resident<4>("resident, three factors of degrees 4, 2 and 1, two workgroups", 7, 2, 4, {p4, p2, p1}, 1, false, 1);
     printf("%s\n", failures ? "FAILED" : "all cases ok");
     return failures ? 1 : 0;
