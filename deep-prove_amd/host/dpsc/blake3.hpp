@@ -29,8 +29,8 @@ inline constexpr RoundIndex make_round_index()
         for (int i = 0; i < 4; i++) {
             r.idx[k][i] = S[k][2 * i];           // first words of the column step's four G
             r.idx[k][4 + i] = S[k][2 * i + 1];   // their second words
-            r.idx[k][8 + i] = S[k][8 + 2 * i];   // the diagonal step's
-            r.idx[k][12 + i] = S[k][9 + 2 * i];
+            r.idx[k][8 + i] = S[k][8 + 2 * ((i + 3) % 4)];   // the diagonal step's, lane i the diagonal through word 4 + i
+            r.idx[k][12 + i] = S[k][9 + 2 * ((i + 3) % 4)];
         }
     return r;
 }
@@ -188,26 +188,28 @@ private:
         const __m128i cv_lo = _mm_loadu_si128((const __m128i *)cv), cv_hi = _mm_loadu_si128((const __m128i *)(cv + 4));
         __m128i r0 = cv_lo, r1 = cv_hi, r2 = _mm_loadu_si128((const __m128i *)IV);
         __m128i r3 = _mm_set_epi32((int)flags, (int)block_len, (int)(uint32_t)(counter >> 32), (int)(uint32_t)counter);
+// (r1 is what a step waits for: the message words go onto r0 first, and between a column and a diagonal step the other three
+// rows are rotated against it)
 #define DPSC_G(mx, my)                             \
-    r0 = _mm_add_epi32(_mm_add_epi32(r0, r1), mx); \
+    r0 = _mm_add_epi32(_mm_add_epi32(r0, mx), r1); \
     r3 = _mm_ror_epi32(_mm_xor_si128(r3, r0), 16); \
     r2 = _mm_add_epi32(r2, r3);                    \
     r1 = _mm_ror_epi32(_mm_xor_si128(r1, r2), 12); \
-    r0 = _mm_add_epi32(_mm_add_epi32(r0, r1), my); \
+    r0 = _mm_add_epi32(_mm_add_epi32(r0, my), r1); \
     r3 = _mm_ror_epi32(_mm_xor_si128(r3, r0), 8);  \
     r2 = _mm_add_epi32(r2, r3);                    \
     r1 = _mm_ror_epi32(_mm_xor_si128(r1, r2), 7);
         for (int k = 0; k < 7; k++) {
             const __m512i p = _mm512_permutexvar_epi32(_mm512_load_si512(ri.idx[k]), m);
             DPSC_G(_mm512_castsi512_si128(p), _mm512_extracti32x4_epi32(p, 1))
-            // lane i of the rows now holds words i, 4 + (i + 1) % 4, 8 + (i + 2) % 4, 12 + (i + 3) % 4: the diagonals
-            r1 = _mm_shuffle_epi32(r1, _MM_SHUFFLE(0, 3, 2, 1));
-            r2 = _mm_shuffle_epi32(r2, _MM_SHUFFLE(1, 0, 3, 2));
-            r3 = _mm_shuffle_epi32(r3, _MM_SHUFFLE(2, 1, 0, 3));
+            // lane i of the rows now holds words (i + 3) % 4, 4 + i, 8 + (i + 1) % 4, 12 + (i + 2) % 4: the diagonals, the one through word 4 + i in lane i
+            r0 = _mm_shuffle_epi32(r0, _MM_SHUFFLE(2, 1, 0, 3));
+            r2 = _mm_shuffle_epi32(r2, _MM_SHUFFLE(0, 3, 2, 1));
+            r3 = _mm_shuffle_epi32(r3, _MM_SHUFFLE(1, 0, 3, 2));
             DPSC_G(_mm512_extracti32x4_epi32(p, 2), _mm512_extracti32x4_epi32(p, 3))
-            r1 = _mm_shuffle_epi32(r1, _MM_SHUFFLE(2, 1, 0, 3));
-            r2 = _mm_shuffle_epi32(r2, _MM_SHUFFLE(1, 0, 3, 2));
-            r3 = _mm_shuffle_epi32(r3, _MM_SHUFFLE(0, 3, 2, 1));
+            r0 = _mm_shuffle_epi32(r0, _MM_SHUFFLE(0, 3, 2, 1));
+            r2 = _mm_shuffle_epi32(r2, _MM_SHUFFLE(2, 1, 0, 3));
+            r3 = _mm_shuffle_epi32(r3, _MM_SHUFFLE(1, 0, 3, 2));
         }
 #undef DPSC_G
         _mm_storeu_si128((__m128i *)out, _mm_xor_si128(r0, r2));

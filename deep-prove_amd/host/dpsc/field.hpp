@@ -121,27 +121,49 @@ inline std::vector<F> eq_evals_host(const F *point, size_t m)
     return t;
 }
 
-// value at r of the polynomial with the given evaluations at 0..d (the Lagrange denominators, k! (d - k)! up to the sign,
-// are inverted together: one inversion a call)
+// 1 / prod_{m != k, m <= d} (k - m): the Lagrange denominators over the nodes 0..d, for the degrees round messages have
+constexpr size_t LAGRANGE_MAX_DEGREE = 8;
+struct LagrangeDenominators {
+    uint64_t inv[LAGRANGE_MAX_DEGREE + 1][LAGRANGE_MAX_DEGREE + 1];
+    LagrangeDenominators()
+    {
+        for (size_t d = 0; d <= LAGRANGE_MAX_DEGREE; d++)
+            for (size_t k = 0; k <= d; k++) {
+                uint64_t den = 1;
+                for (size_t m = 0; m <= d; m++)
+                    if (m != k) den = Fp::mul(den, Fp::sub(k, m));
+                inv[d][k] = Fp::inv(den);
+            }
+    }
+};
+
+// value at r of the polynomial with the given evaluations at 0..d
 inline F interpolate_uni(const F *evals, size_t d, const F &r)
 {
-    std::vector<uint64_t> den(d + 1, 1), before(d + 1);
-    for (size_t k = 0; k <= d; k++)
-        for (size_t m = 0; m <= d; m++)
-            if (m != k) den[k] = Fp::mul(den[k], Fp::sub(k, m));
-    uint64_t all = 1;
+    static const LagrangeDenominators table;
+    // prod_{m < k} (r - m) on the way up, prod_{m > k} (r - m) on the way down
+    std::vector<F> below_long;
+    F below_short[LAGRANGE_MAX_DEGREE + 1], *below = below_short;
+    if (d > LAGRANGE_MAX_DEGREE) below_long.resize(d + 1), below = below_long.data();
+    F run = F::one();
     for (size_t k = 0; k <= d; k++) {
-        before[k] = all;
-        all = Fp::mul(all, den[k]);
+        below[k] = run;
+        run *= r - F::from_u64(k);
     }
-    uint64_t inv = Fp::inv(all);
-    F acc = F::zero();
+    F acc = F::zero(), above = F::one();
     for (size_t k = d + 1; k-- > 0;) {
-        F num(Fp::mul(inv, before[k]), 0);  // 1 / den[k]
-        inv = Fp::mul(inv, den[k]);
-        for (size_t m = 0; m <= d; m++)
-            if (m != k) num *= r - F::from_u64(m);
-        acc += num * evals[k];
+        uint64_t w;
+        if (d <= LAGRANGE_MAX_DEGREE) {
+            w = table.inv[d][k];
+        } else {
+            uint64_t den = 1;
+            for (size_t m = 0; m <= d; m++)
+                if (m != k) den = Fp::mul(den, Fp::sub(k, m));
+            w = Fp::inv(den);
+        }
+        const F basis = below[k] * above;
+        acc += F(Fp::mul(basis.c0, w), Fp::mul(basis.c1, w)) * evals[k];
+        above *= r - F::from_u64(k);
     }
     return acc;
 }

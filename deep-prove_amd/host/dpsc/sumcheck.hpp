@@ -82,17 +82,17 @@ public:
         vp.num_vars = num_vars_;
         for (auto *p : mles_) vp.mles.push_back(p->raw());
         for (auto &e : exprs) {
-            for (auto &m : e.to_monomials(challenges)) {
-                if (m.wits.size() > DPS_MAX_FACTORS) throw Error(DPS_ERR_UNSUPPORTED, "to_virtual_polys: too many factors in a product");
+            e.for_each_monomial(challenges, [&](const F &coeff, const uint16_t *wits, size_t n) {
+                if (n > DPS_MAX_FACTORS) throw Error(DPS_ERR_UNSUPPORTED, "to_virtual_polys: too many factors in a product");
                 dps_term t;
                 memset(&t, 0, sizeof t);
-                t.coeff[0] = m.coeff.c0;
-                t.coeff[1] = m.coeff.c1;
-                t.n_factors = (uint32_t)m.wits.size();
-                for (size_t i = 0; i < m.wits.size(); i++) t.factors[i] = m.wits[i];
+                t.coeff[0] = coeff.c0;
+                t.coeff[1] = coeff.c1;
+                t.n_factors = (uint32_t)n;
+                for (size_t i = 0; i < n; i++) t.factors[i] = wits[i];
                 vp.degree = std::max<uint32_t>(vp.degree, t.n_factors);
                 vp.terms.push_back(t);
-            }
+            });
         }
         return vp;
     }
