@@ -2307,10 +2307,15 @@ namespace {
 // (measured with 128, 64, 32, 16: 8 products over 16 tables 0.130, 0.119, 0.114, 0.111 ms; the fraction-tree proof 3.37, 3.30,
 // 3.28, 3.38 ms -- more workgroups cost little since their sums go into several sets of counters)
 constexpr u32 SLICE_MIN_PAIRS = 32;
+// A sum of several terms is cut further, into up to SLICE_SUM_WORKGROUPS workgroups, while one has more than this many pairs times terms (a lane each, with some of the
+// points: the first trip then is one pass over them): 26 fraction-sum layers of up to 2^15 entries 1460 -> 1400 us, those of 2^21 3140 -> 3100, the products of
+// an attention layer over 2^12 entries 201 -> 181.  Finer (4 pairs) those were 1420 .. 1440, 3150 and 180 .. 185 us; with 64 workgroups 16 products
+// over 32 tables of 2^11 entries are 5 us slower (290 -> 295), with 32 they stay as they were.
+constexpr u32 SLICE_SUM_TERM_PAIRS = 128, SLICE_SUM_MIN_PAIRS = 8, SLICE_SUM_WORKGROUPS = 32;
 // ... and a sum that could be cut finer takes half the device at most, so that two such sums of two contexts find room
 // side by side (a launch that fills the device alone sends every other context's resident rounds back to launches of their own)
 constexpr u32 SLICE_SMALL_SUM_WORKGROUPS = 128;
-constexpr u32 SLICE_ONE_WORKGROUP_TERM_PAIRS = 512;  // pairs x terms up to which one workgroup takes the whole sum
+constexpr u32 SLICE_ONE_WORKGROUP_TERM_PAIRS = 512;  // pairs x terms up to which one workgroup takes the whole sum (sums of several terms: SLICE_SUM_TERM_PAIRS)
 constexpr u32 SLICE_MAX_WORKGROUPS = 256;
 // Most pairs a workgroup is given of a product, and of a sum of several terms: more would make more rounds resident, but a trip's arithmetic is a
 // workgroup's alone (with 512 pairs of a 3-term sum the first trip took 75 us where a launch for the round and a trip of 128 pairs take 66)
@@ -2418,12 +2423,12 @@ void plan_resident_rounds(dps_sc *sc, u32 n_tabs, u32 n_mles)
     auto pairs_of = [&](u32 round) { return (u64)1 << (n - round); };
     u32 j = first_ok;
     while (pairs_of(j) > (u64)per_wg_max * SLICE_MAX_WORKGROUPS) j++;
-    // (a small sum stays with one workgroup -- 128 pairs of three terms: four workgroups were 7 us slower over the eight
-    // rounds; 128 pairs of eight terms over 16 tables: four workgroups were 13 us faster)
-    const u64 term_pairs = pairs_of(j) * (sc->poly ? std::max<size_t>(sc->slice_terms.size(), 1) : 1);
-    const u32 per_wg = term_pairs <= SLICE_ONE_WORKGROUP_TERM_PAIRS && pairs_of(j) <= per_wg_max
-                           ? (u32)pairs_of(j)
-                           : (u32)std::min<u64>(per_wg_max, std::max<u64>(SLICE_MIN_PAIRS, pairs_of(j) / SLICE_SMALL_SUM_WORKGROUPS));
+    // (a sum small enough stays with one workgroup: no handing over)
+    const u32 n_terms = sc->poly && sc->weq.empty() ? (u32)sc->slice_terms.size() : 1;
+    u32 per_wg = (u32)std::min<u64>(per_wg_max, std::max<u64>(SLICE_MIN_PAIRS, pairs_of(j) / SLICE_SMALL_SUM_WORKGROUPS));
+    if (n_terms > 1)
+        while (per_wg > SLICE_SUM_MIN_PAIRS && per_wg * n_terms > SLICE_SUM_TERM_PAIRS && pairs_of(j) / per_wg < SLICE_SUM_WORKGROUPS) per_wg >>= 1;
+    if (pairs_of(j) * n_terms <= (n_terms > 1 ? SLICE_SUM_TERM_PAIRS : SLICE_ONE_WORKGROUP_TERM_PAIRS) && pairs_of(j) <= per_wg_max) per_wg = (u32)pairs_of(j);
     sc->tail_j0 = j;
     // The last rounds are the host's: a trip costs the way to the GPU and back and a workgroup's barriers whatever it
     // carries, a round of a few pairs costs the host a microsecond.  As many rounds as stay below HOST_TAIL_MULTS
