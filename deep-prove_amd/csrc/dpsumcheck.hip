@@ -1721,6 +1721,9 @@ struct dps_sc {
     u64 tail_seq0;
     void *scratch;      // one pool block holding every ping-pong buffer
     void *dev_block;    // descriptors, partials, per-round result
+    bool described;            // the descriptors of every round's launch are worked out (else of round 1 only: SessionSetup::run)
+    void *late_block = nullptr;  // ... behind dps_sc_begin: where they lie then
+    void *desc_block = nullptr;  // where the descriptors lie
     // precomputed descriptors (device)
     std::vector<u32> fold_off, fold_cnt;            // per step j = 2..n_vars+1: all tables that fold
     std::vector<u32> fold_extra_off, fold_extra_cnt;  // same, without the fast term's tables
@@ -2273,8 +2276,10 @@ u32 program_root(ProgramTerm *t, u32 n, std::vector<dpk::PolyOp> &ops)
 }
 
 // one staged upload of all descriptors; not waited for (the staging vector lives as long as the session)
+int32_t describe_now(dps_sc *sc);
 int32_t ensure_descs(dps_sc *sc)
 {
+    CHK(describe_now(sc));
     if (sc->descs_uploaded || sc->stage.empty()) return DPS_OK;
     dps_ctx *ctx = sc->ctx;
     const void *from = sc->stage.data();
@@ -2289,7 +2294,7 @@ int32_t ensure_descs(dps_sc *sc)
         memcpy(ctx->h_desc_stage, sc->stage.data(), sc->stage.size());
         from = ctx->h_desc_stage;
     }
-    hipError_t e = hipMemcpyAsync(sc->dev_block, from, sc->stage.size(), hipMemcpyHostToDevice, ctx->stream);
+    hipError_t e = hipMemcpyAsync(sc->desc_block, from, sc->stage.size(), hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess && staged) {
         e = hipEventRecord(ctx->desc_event, ctx->stream);
         ctx->desc_pending = e == hipSuccess;
@@ -2496,8 +2501,8 @@ void plan_resident_rounds(dps_sc *sc, u32 n_tabs, u32 n_mles)
 }
 
 // The session's resident launch found no place on the device (admit_waiting_launch): the rounds it would have run, and
-// those the host would have worked out behind it, are launches of their own like the rounds before them.  Every
-// round's launch was described at set-up whatever the plan, and the eq levels those rounds read are built.
+// those the host would have worked out behind it, are launches of their own like the rounds before them.  The
+// descriptors of their launches are there or are made now (describe_now), and the eq levels those rounds read are built.
 void drop_resident_plan(dps_sc *sc)
 {
     sc->stages.clear();
@@ -2562,11 +2567,13 @@ struct SessionSetup {
     void fold_step(u32 j);
     void poly_groups_of_round(u32 j);
     void term_descs_of_round(u32 j);
-    void describe_rounds();
+    void describe_rounds(u32 steps);
     int32_t plan_first_two_rounds();
     void launch_limits();
+    size_t descriptor_bytes();
+    char *place_descriptors(char *p);
     int32_t allocate_device_block();
-    int32_t stage_descriptors();
+    void stage_descriptors();
     int32_t run();
 };
 
@@ -3175,9 +3182,10 @@ void SessionSetup::term_descs_of_round(u32 j)
     }
 }
 
-// a dry run of the rounds: every descriptor the launches will need
-void SessionSetup::describe_rounds()
+// a dry run of the first `steps` rounds (with the last fold n_vars + 1): every descriptor their launches will need
+void SessionSetup::describe_rounds(u32 steps)
 {
+    sc->described = steps > n_vars;
     sim = sc->m;
     sc->fold_off.assign(n_vars + 2, 0);
     sc->fold_cnt.assign(n_vars + 2, 0);
@@ -3188,13 +3196,16 @@ void SessionSetup::describe_rounds()
     sc->fast_nb.assign(n_vars + 2, 0);
     pre0.assign(n_mles, nullptr), pre1.assign(n_mles, nullptr);
     folded.assign(n_mles, 0);
-    for (u32 j = 1; j <= n_vars + 1; j++) {
+    for (u32 j = 1; j <= steps; j++) {
         std::fill(folded.begin(), folded.end(), 0);
         fold_step(j);
         if (j <= n_vars && sc->poly) poly_groups_of_round(j);
         if (j <= n_vars && !sc->fast && !sc->poly) term_descs_of_round(j);
     }
 
+    sc->h_poly_groups = poly_groups;
+    sc->h_poly_terms = poly_terms;
+    if (!sc->described) return;
     for (const dps_term &t : sc->terms) fins.push_back(dpk::FinTerm{t.coeff[0], t.coeff[1], t.n_factors, 0});
 
     for (u32 k = 0; k < n_mles; k++) gath.push_back(dpk::GatherDesc{sim[k].c0, sim[k].c1});
@@ -3231,25 +3242,23 @@ void SessionSetup::launch_limits()
     }
 }
 
-int32_t SessionSetup::allocate_device_block()
+size_t SessionSetup::descriptor_bytes()
 {
     bytes_fold = round_up(folds.size() * sizeof(dpk::FoldDesc), 256);
     bytes_fold_x = round_up(folds_extra.size() * sizeof(dpk::FoldDesc), 256);
     bytes_terms = round_up(tdescs.size() * sizeof(dpk::TermDesc), 256);
     bytes_fin = round_up(fins.size() * sizeof(dpk::FinTerm), 256);
     bytes_gath = round_up(gath.size() * sizeof(dpk::GatherDesc), 256);
-    size_t bytes_partial = round_up((size_t)std::max<u32>(sc->n_terms, 1) * sc->max_blocks * 2 * dpk::MAX_PTS * 8, 256);
-    size_t bytes_result = round_up((2 * dpk::MAX_PTS + 2 * (size_t)n_mles) * 8, 256) + 256;
     bytes_pg = round_up(poly_groups.size() * sizeof(dpk::PolyGroup), 256);
     bytes_pt = round_up(poly_terms.size() * sizeof(dpk::PolyTerm), 256);
     bytes_po = round_up(sc->h_poly_ops.size() * sizeof(dpk::PolyOp), 256);
-    // what a resident stage that does not run to the last round leaves for the next: two limb arrays per table
-    size_t bytes_hand = 0;
-    const u32 slice_tabs = (u32)sc->slice_ids.size();
-    for (size_t i = 0; i + 1 < sc->stages.size(); i++) bytes_hand += round_up((size_t)sc->stages[i + 1].src_len * 8, 256) * 2 * (slice_tabs + std::max<size_t>(1, sc->weq.size()));
-    size_t total = bytes_fold + bytes_fold_x + bytes_terms + bytes_fin + bytes_gath + bytes_pg + bytes_pt + bytes_po + bytes_partial + bytes_result + bytes_hand;
-    CHK(pool_alloc(ctx, total, &sc->dev_block));
-    char *p = (char *)sc->dev_block;
+    return bytes_fold + bytes_fold_x + bytes_terms + bytes_fin + bytes_gath + bytes_pg + bytes_pt + bytes_po;
+}
+
+// Their places from `p` on; returns what lies behind them
+char *SessionSetup::place_descriptors(char *p)
+{
+    sc->desc_block = p;
     sc->d_fold = (dpk::FoldDesc *)p;
     p += bytes_fold;
     sc->d_fold_extra = (dpk::FoldDesc *)p;
@@ -3265,7 +3274,21 @@ int32_t SessionSetup::allocate_device_block()
     sc->d_poly_terms = (dpk::PolyTerm *)p;
     p += bytes_pt;
     sc->d_poly_ops = (dpk::PolyOp *)p;
-    p += bytes_po;
+    return p + bytes_po;
+}
+
+int32_t SessionSetup::allocate_device_block()
+{
+    const size_t bytes_desc = sc->described ? descriptor_bytes() : 0;
+    size_t bytes_partial = round_up((size_t)std::max<u32>(sc->n_terms, 1) * sc->max_blocks * 2 * dpk::MAX_PTS * 8, 256);
+    size_t bytes_result = round_up((2 * dpk::MAX_PTS + 2 * (size_t)n_mles) * 8, 256) + 256;
+    // what a resident stage that does not run to the last round leaves for the next: two limb arrays per table
+    size_t bytes_hand = 0;
+    const u32 slice_tabs = (u32)sc->slice_ids.size();
+    for (size_t i = 0; i + 1 < sc->stages.size(); i++) bytes_hand += round_up((size_t)sc->stages[i + 1].src_len * 8, 256) * 2 * (slice_tabs + std::max<size_t>(1, sc->weq.size()));
+    CHK(pool_alloc(ctx, bytes_desc + bytes_partial + bytes_result + bytes_hand, &sc->dev_block));
+    char *p = (char *)sc->dev_block;
+    if (sc->described) p = place_descriptors(p);
     sc->d_partial = (u64 *)p;
     p += bytes_partial;
     sc->d_result = (u64 *)p;
@@ -3285,13 +3308,11 @@ int32_t SessionSetup::allocate_device_block()
     return DPS_OK;
 }
 
-int32_t SessionSetup::stage_descriptors()
+void SessionSetup::stage_descriptors()
 {
     // one staged upload of all descriptors
     std::vector<char> &stage = sc->stage;  // lives as long as the session: the upload is not waited for
     stage.assign(bytes_fold + bytes_fold_x + bytes_terms + bytes_fin + bytes_gath + bytes_pg + bytes_pt + bytes_po, 0);
-    sc->h_poly_groups = poly_groups;
-    sc->h_poly_terms = poly_terms;
     char *q = stage.data();
     if (!folds.empty()) memcpy(q, folds.data(), folds.size() * sizeof(dpk::FoldDesc));
     q += bytes_fold;
@@ -3308,16 +3329,7 @@ int32_t SessionSetup::stage_descriptors()
     if (!poly_terms.empty()) memcpy(q, poly_terms.data(), poly_terms.size() * sizeof(dpk::PolyTerm));
     q += bytes_pt;
     if (!sc->h_poly_ops.empty()) memcpy(q, sc->h_poly_ops.data(), sc->h_poly_ops.size() * sizeof(dpk::PolyOp));
-    // Sessions whose launches carry their descriptors themselves (a product session that ends in the resident kernel; a
-    // single group of terms, inline in the kernel arguments or staged in pinned memory for the resident launch) upload
-    // nothing unless a step outside that flow needs the block (ensure_descs).
     sc->descs_uploaded = false;
-    const bool self_contained = (sc->fast && sc->tail_j0) || sc->tail_j0 == 1 ||
-                                (sc->poly && sc->poly_tabs.size() == 1 && sc->h_poly_terms.size() <= (size_t)dpk::POLY_LDS_TERMS);
-    if (!self_contained) {
-        CHK(ensure_descs(sc));
-    }
-    return DPS_OK;
 }
 
 // eq * f * g over two base-field tables, large enough for the factored eq weights: rounds 1 and 2 are one launch that
@@ -3367,11 +3379,39 @@ int32_t SessionSetup::run()
     detect_multi_term();
     CHK(plan_and_ready_tables());
     CHK(layout_scratch());
-    describe_rounds();
+    // A sum that is resident, or the host's, from round 1 on with every table of it needs no launch but the one of round 1: the others are worked out when one
+    // is needed all the same (describe_now).  16 products over 32 tables of 11 variables were set up in 41 us, fraction-sum layers in 2.5 .. 3.3.
+    bool later = n_vars >= 1 && (sc->host_only || sc->tail_j0 == 1);
+    for (u32 k = 0; k < n_mles && later; k++) later = (in_fast(k) || sc->closed_eq(k)) && !zpad_of(k);
+    describe_rounds(later ? 1 : n_vars + 1);
     CHK(plan_first_two_rounds());
     launch_limits();
     CHK(allocate_device_block());
-    return stage_descriptors();
+    sc->descs_uploaded = false;
+    if (later) return DPS_OK;
+    stage_descriptors();
+    // Sessions whose launches carry their descriptors themselves (a product session that ends in the resident kernel; a
+    // single group of terms, inline in the kernel arguments or staged in pinned memory for the resident launch) upload
+    // nothing unless a step outside that flow needs the block (ensure_descs).
+    const bool self_contained = (sc->fast && sc->tail_j0) || sc->tail_j0 == 1 ||
+                                (sc->poly && sc->poly_tabs.size() == 1 && sc->h_poly_terms.size() <= (size_t)dpk::POLY_LDS_TERMS);
+    return self_contained ? (int32_t)DPS_OK : ensure_descs(sc);
+}
+
+// What dps_sc_begin left out, from the tables' layout and the groups the session keeps
+int32_t describe_now(dps_sc *sc)
+{
+    if (sc->described || sc->inner) return DPS_OK;
+    SessionSetup su;
+    su.ctx = sc->ctx, su.sc = sc, su.n_vars = sc->n_vars, su.mles = nullptr, su.n_mles = sc->n_mles;
+    su.poly_terms = sc->h_poly_terms;
+    su.describe_rounds(sc->n_vars + 1);
+    sc->described = false;  // (until they have a place)
+    CHK(pool_alloc(sc->ctx, std::max<size_t>(su.descriptor_bytes(), 256), &sc->late_block));
+    su.place_descriptors((char *)sc->late_block);
+    su.stage_descriptors();
+    sc->described = true;
+    return DPS_OK;
 }
 
 }  // namespace
@@ -3767,6 +3807,9 @@ namespace {
 int32_t launch_folds(dps_sc *sc, u32 step, bool extra_only, const u64 *chal)
 {
     dps_ctx *ctx = sc->ctx;
+    // (a session not described has no tables but those its kernel folds)
+    if (!sc->described && extra_only && step <= sc->n_vars) return DPS_OK;
+    CHK(describe_now(sc));
     u32 cnt = extra_only ? sc->fold_extra_cnt[step] : sc->fold_cnt[step];
     if (!cnt) return DPS_OK;
     CHK(ensure_descs(sc));
@@ -5238,6 +5281,7 @@ extern "C" int32_t dps_sc_round(dps_sc *sc, const uint64_t *challenge, uint64_t 
         if (sc->tail_j0 && j == sc->tail_j0 && !sc->tail_running && !fr.admit_stages()) {
             if (!sc->quads.empty()) CHK(fr.catch_up_after_quads());
             drop_resident_plan(sc);
+            CHK(describe_now(sc));
         }
         if ((sc->tail_j0 && j >= sc->tail_j0) || sc->host_only) return fr.resident_round();
         if (sc->pair12 && j == 1) return fr.first_two_rounds_launch();
@@ -5370,6 +5414,7 @@ extern "C" int32_t dps_sc_free(dps_sc *sc)
     drop_combined(sc);
     pool_free(ctx, sc->scratch);
     pool_free(ctx, sc->dev_block);
+    pool_free(ctx, sc->late_block);
     delete sc;
     return DPS_OK;
 }
