@@ -1777,7 +1777,26 @@ __host__ __device__ constexpr u32 slice_lds_words(u32 n_tabs, u32 cap, u32 blk, 
 // A workgroup of these launches is 1024 threads: what a round costs here is the longest chain of dependent field
 // multiplications in any one lane, and with more lanes each has fewer units of work behind one another.
 constexpr int SL_BLOCK = 1024;
-constexpr int SL_PRE = 2;  // items (table, entry) a thread of a launch made ahead asks for before it waits for its first mail
+// Entries a thread asks for before it waits for a mail, of those it takes up from device memory (of a sum of several terms one: the kernel has no registers
+// for more)
+template <bool TERMS>
+constexpr int sl_pre = TERMS ? 1 : 2;
+
+// The first FRONT bytes of a kernel's arguments and what lies around their end (ALL bytes, behind them the launch's sizes), asked for in one go: the compiler
+// loads an argument where control first needs it, and a kernel that branches on them pays the way to memory for line after line.
+template <size_t FRONT, size_t ALL>
+__device__ __forceinline__ void touch_arguments()
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    const auto *p = (const __attribute__((address_space(4))) u32 *)__builtin_amdgcn_kernarg_segment_ptr();
+    constexpr u32 LINE = 64 / 4, LAST = (u32)((FRONT - 4) / 4);
+#define DPK_WORD(i) "s"(p[(i) * LINE < LAST ? (i) * LINE : LAST])
+    asm volatile("" ::DPK_WORD(0), DPK_WORD(1), DPK_WORD(2), DPK_WORD(3), DPK_WORD(4), DPK_WORD(5), DPK_WORD(6), DPK_WORD(7), DPK_WORD(8), DPK_WORD(9), DPK_WORD(10),
+                 DPK_WORD(11), DPK_WORD(12), DPK_WORD(13), DPK_WORD(14), DPK_WORD(15), DPK_WORD(16), DPK_WORD(17), DPK_WORD(18), DPK_WORD(19), "s"(p[ALL / 4 - LINE]),
+                 "s"(p[ALL / 4 - 1]), "s"(p[ALL / 4]));
+#undef DPK_WORD
+#endif
+}
 
 // NF: tables of the product, or with TERMS the largest number of factors of a term (the degree of the polynomial summed)
 // BLK: threads of a workgroup (SL_BLOCK in the library; the kernel's CPU test runs smaller ones)
@@ -1792,7 +1811,9 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
     constexpr int NSMP = NF + 1;        // samples of that round's sums as a polynomial in the challenge: 0..NF-1, leading coefficient
     constexpr int NS = NP + NSMP * NPT; // extension sums per trip
     static_assert(NS <= SL_MAX_SUMS && 4 * NS <= BLK, "sums per trip fit the result area, their counters one lane each");
+    constexpr int SL_PRE = sl_pre<TERMS>;
     extern __shared__ u64 dyn[];
+    touch_arguments<sizeof(ARGS) - sizeof(a.terms), sizeof(ARGS)>();
     u64 *const ctr = dyn + SL_LDS_CTR;  // [wavefront][4 * SL_MAX_SUMS]
     u64 *const box = dyn + SL_LDS_BOX;
     int *const ok_flag = reinterpret_cast<int *>(dyn + SL_LDS_FLAGS);
@@ -1820,17 +1841,11 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
         return big ? wts_big + (size_t)(2 * g + limb) * sl_weights_cap(cap) : wts_small + (size_t)(2 * g + limb) * sl_weights_cap(cap / 2);
     };
     auto weight = [&](bool big, u32 p, u32 g = 0) { return gl::e2(wts(big, 0, g)[p], wts(big, 1, g)[p]); };
-    if constexpr (ARGS::EQS > 0) {
-        // the programs, in the terms' place
-        const u64 *src = reinterpret_cast<const u64 *>(a.terms);
-        u64 *dst = dyn + SL_LDS_TERMS;
-        for (u32 w = tid; w < a.op_end[a.n_eqs - 1] * (u32)(sizeof(PolyOp) / 8); w += BLOCK) dst[w] = src[w];
-    } else if (TERMS) {
-        // the terms are read per pair and point: staged in LDS once (visible after the first wait's barrier)
-        const u64 *src = reinterpret_cast<const u64 *>(a.terms);
-        u64 *dst = dyn + SL_LDS_TERMS;
-        for (u32 w = tid; w < a.n_terms * (u32)(sizeof(SliceTerm) / 8); w += BLOCK) dst[w] = src[w];
-    }
+    // the terms (the programs of several eq factors) are read per pair and point: staged in LDS once.  Asked for here, stored with the first trip
+    u32 term_words = TERMS ? a.n_terms * (u32)(sizeof(SliceTerm) / 8) : 0u;
+    if constexpr (ARGS::EQS > 0) term_words = a.op_end[a.n_eqs - 1] * (u32)(sizeof(PolyOp) / 8);
+    u64 term_word = 0;
+    if (TERMS && tid < term_words) term_word = reinterpret_cast<const u64 *>(a.terms)[tid];
 
     // lanes that share a pair (a quad) at one evaluation point split the terms among them
     const u32 p_split = TERMS ? a.n_terms : 1u;
@@ -1894,28 +1909,67 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
         trip_seq = a.seq0 + (j - a.j0);
         bool skip1;
         E2 rb_ = gl::e2_zero(), ra_ = gl::e2_zero();
-        // A launch made ahead of its first round finds its sources complete (the launch before it on the stream has ended)
-        // but not yet its challenges: the entries this thread will fold are asked for before it waits for the mail, so
-        // that they cross from device memory during the wait (up to SL_PRE items a thread; more are loaded after the mail).
+        // What a thread takes up from device memory is asked for in one go, and before it waits for a mail: the sources are complete (the launch
+        // before this one on the stream has ended; the gate), only the challenges are not known yet.  Up to SL_PRE entries a thread, the eq weights behind
+        // them; more entries are loaded after the mail.
+        u64 pre_w[2] = {0, 0};
+        if (EQ && ARGS::EQS == 0 && k == 0 && tid < (len >> 1)) {
+            const u64 e0 = ((2ull << a.n_vars) - (2ull << (a.n_vars - j))) + (u64)wg * (len >> 1) + tid;
+            pre_w[0] = a.eq0[e0], pre_w[1] = a.eq1[e0];
+        }
         U64x2 pre[SL_PRE][4];
-        const bool have_pre = k == 0 && !a.first_go && pend >= 1 && (nt << len_log) <= (u32)(SL_PRE * BLOCK) && !(ARGS::LACKS && a.any_lacks);
-        if (have_pre) {
+        const bool takes_up = k == 0 || regroup;
+        if (takes_up) {
             const u64 base = (u64)wg * src_each;
 #pragma unroll
             for (int sidx = 0; sidx < SL_PRE; sidx++) {
                 const u32 u = tid + (u32)sidx * BLOCK;
                 if (u < (nt << len_log)) {
                     const u32 f = u >> len_log, i = u & (len - 1);
-                    const u64 *p0 = a.s0[f], *p1 = a.s1[f];
-                    const u64 e = base + ((u64)i << pend);
-                    pre[sidx][0] = ld2(p0 + e);
-                    pre[sidx][2] = p1 ? ld2(p1 + e) : U64x2{0, 0};
-                    if (pend == 2) {
-                        pre[sidx][1] = ld2(p0 + e + 2);
-                        pre[sidx][3] = ld2(p1 + e + 2);
+                    const u64 *p0 = regroup ? a.h0[f] : a.s0[f], *p1 = regroup ? a.h1[f] : a.s1[f];
+                    const bool shorter = ARGS::LACKS && k == 0 && a.any_lacks && a.lacks[f];
+                    if (pend == 0 || shorter) {
+                        const u64 e = shorter ? ((base >> pend) + i) >> (a.lacks[f] - 1) : base + i;
+                        pre[sidx][0].x = p0[e];
+                        pre[sidx][2].x = p1 ? p1[e] : 0;
+                    } else {
+                        const u64 e = base + ((u64)i << pend);
+                        pre[sidx][0] = ld2(p0 + e);
+                        pre[sidx][2] = p1 ? ld2(p1 + e) : U64x2{0, 0};
+                        if (pend == 2) {
+                            pre[sidx][1] = ld2(p0 + e + 2);
+                            pre[sidx][3] = ld2(p1 + e + 2);
+                        }
                     }
                 }
             }
+        }
+        // the weights of round j's pairs, from the eq table's level of that round, or from what the workgroups left, added up in runs of 2^pend
+        if (EQ && takes_up)
+            for (u32 g = 0; g < n_eqs; g++) {
+                const u64 *q0 = a.eq0, *q1 = a.eq1;
+                u64 stride = 0;
+                if constexpr (ARGS::EQS > 0) q0 = a.geq0[g], q1 = a.geq1[g], stride = a.hw_stride;
+                const u64 e0 = ((2ull << a.n_vars) - (2ull << (a.n_vars - j))) + (u64)wg * (len >> 1);
+                for (u32 i = tid; i < (len >> 1); i += BLOCK) {
+                    E2 v;
+                    if (ARGS::EQS == 0 && k == 0 && i < (u32)BLOCK) {
+                        v = gl::e2(pre_w[0], pre_w[1]);
+                    } else if (k == 0) {
+                        v = gl::e2(q0[e0 + i], q1[e0 + i]);
+                    } else {
+                        const u64 e = (u64)g * stride + ((u64)i << pend);
+                        v = gl::e2(a.hw0[e], a.hw1[e]);
+                        for (u32 q = 1; q < (1u << pend); q++) v = gl::add(v, gl::e2(a.hw0[e + q], a.hw1[e + q]));
+                    }
+                    wts(true, 0, g)[i] = v.c0;
+                    wts(true, 1, g)[i] = v.c1;
+                }
+            }
+        if (TERMS && k == 0) {
+            u64 *dst = dyn + SL_LDS_TERMS;
+            if (tid < term_words) dst[tid] = term_word;
+            for (u32 w = tid + BLOCK; w < term_words; w += BLOCK) dst[w] = reinterpret_cast<const u64 *>(a.terms)[w];
         }
         if (k == 0 && a.first_go) {
             // a launch made for round 1, when it is that round's turn: nothing is pending, whether t = 1 is evaluated came
@@ -1933,8 +1987,8 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
         }
         const gl::E2P rb = gl::prep(rb_), ra = gl::prep(ra_);
         // ---- the pending folds ----
-        if (have_pre) {
-            // (the entries asked for before the wait)
+        if (takes_up) {
+            // (the entries asked for)
 #pragma unroll
             for (int sidx = 0; sidx < SL_PRE; sidx++) {
                 const u32 u = tid + (u32)sidx * BLOCK;
@@ -1942,8 +1996,10 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
                     const u32 f = u >> len_log, i = u & (len - 1);
                     const U64x2 x0 = pre[sidx][0], x1 = pre[sidx][2];
                     E2 v;
-                    if (pend == 1) {
-                        v = a.s1[f] ? fold1p(gl::e2(x0.x, x1.x), gl::e2(x0.y, x1.y), rb) : fold1_base(x0.x, x0.y, rb_);
+                    if (pend == 0 || (ARGS::LACKS && k == 0 && a.any_lacks && a.lacks[f])) {
+                        v = gl::e2(x0.x, x1.x);
+                    } else if (pend == 1) {
+                        v = fold1p(gl::e2(x0.x, x1.x), gl::e2(x0.y, x1.y), rb);
                     } else {
                         const U64x2 y0 = pre[sidx][1], y1 = pre[sidx][3];
                         v = fold1p(fold1p(gl::e2(x0.x, x1.x), gl::e2(x0.y, x1.y), ra), fold1p(gl::e2(y0.x, y1.x), gl::e2(y0.y, y1.y), ra), rb);
@@ -1952,11 +2008,10 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
                     tab(true, f, 1)[i] = v.c1;
                 }
             }
-        } else if (k == 0 || regroup) {
             // from device memory: entry i of the state is the source's entry i (nothing pending), or is made of its entries
             // 2i, 2i+1 (one fold) or 4i..4i+3 (two)
             const u64 base = (u64)wg * src_each;
-            for (u32 u = tid; u < (nt << len_log); u += BLOCK) {
+            for (u32 u = tid + SL_PRE * BLOCK; u < (nt << len_log); u += BLOCK) {
                 const u32 f = u >> len_log, i = u & (len - 1);
                 const u64 *p0 = regroup ? a.h0[f] : a.s0[f], *p1 = regroup ? a.h1[f] : a.s1[f];
                 E2 v;
@@ -2005,40 +2060,6 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
                         wts(!in_big, 1, g)[i] = v.c1;
                     }
             in_big = !in_big;
-        }
-        if constexpr (ARGS::EQS > 0) {
-            if (k == 0 || regroup)
-                for (u32 g = 0; g < n_eqs; g++) {
-                    const u64 e0 = ((2ull << a.n_vars) - (2ull << (a.n_vars - j))) + (u64)wg * (len >> 1);
-                    for (u32 i = tid; i < (len >> 1); i += BLOCK) {
-                        E2 v;
-                        if (k == 0) {
-                            v = gl::e2(a.geq0[g][e0 + i], a.geq1[g][e0 + i]);
-                        } else {
-                            const u64 e = (u64)g * a.hw_stride + ((u64)i << pend);
-                            v = gl::e2(a.hw0[e], a.hw1[e]);
-                            for (u32 q = 1; q < (1u << pend); q++) v = gl::add(v, gl::e2(a.hw0[e + q], a.hw1[e + q]));
-                        }
-                        wts(true, 0, g)[i] = v.c0;
-                        wts(true, 1, g)[i] = v.c1;
-                    }
-                }
-        } else if (EQ && k == 0) {
-            // the weights of round j's pairs, from the eq table's level of that round
-            const u64 e0 = ((2ull << a.n_vars) - (2ull << (a.n_vars - j))) + (u64)wg * (len >> 1);
-            for (u32 i = tid; i < (len >> 1); i += BLOCK) {
-                wts(true, 0)[i] = a.eq0[e0 + i];
-                wts(true, 1)[i] = a.eq1[e0 + i];
-            }
-        } else if (EQ && regroup) {
-            // ... or from what the workgroups left, added up in runs of 2^pend
-            for (u32 i = tid; i < (len >> 1); i += BLOCK) {
-                const u64 e = (u64)i << pend;
-                E2 v = gl::e2(a.hw0[e], a.hw1[e]);
-                for (u32 q = 1; q < (1u << pend); q++) v = gl::add(v, gl::e2(a.hw0[e + q], a.hw1[e + q]));
-                wts(true, 0)[i] = v.c0;
-                wts(true, 1)[i] = v.c1;
-            }
         }
         // this wavefront's counters start the trip at zero
         u32 ns = NS;  // sums of this trip
@@ -2163,8 +2184,44 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
                     }
                 }
             };
+            // Where the factor's lanes are enough for it a unit is one point of a pair, or of a quad at one challenge: the chain of a walk at one
+            // point instead of four in turn (two tables, degrees 3 and 1: trips 15 .. 16 -> 13.5 .. 15 us, the last workgroup's three 19, 13, 12 -> 16, 12, 9).
+            // Units of one sum lie side by side, points of pairs first.
+            const u32 dg = g < n_eqs ? a.degree[g] : 0, ptsq = g == 0 && skip1 ? dg : dg + 1, ptsd = g == 0 ? dg : dg + 1;
+            const u32 n_points = ptsq * (len >> 1) + (dbl ? (dg + 1) * ptsd * (len >> 2) : 0);
+            auto point_units = [&](auto program_degree) {
+                constexpr int DEG = decltype(program_degree)::value;
+                const PolyOp *ops = reinterpret_cast<const PolyOp *>(lterms);
+                const bool mine = l < n_points, pair = !mine || l < ptsq * (len >> 1);
+                const u32 v = !mine ? 0 : pair ? l : l - ptsq * (len >> 1), run_log = pair ? len_log - 1 : len_log - 2;
+                const u32 q = v >> run_log, at = v & ((1u << run_log) - 1), smp = pair ? 0 : q / ptsd, ti = pair ? q : q - smp * ptsd;
+                const u32 t = ti > 0 && g == 0 && (!pair || skip1) ? ti + 1 : ti;
+                auto table = [&](u32 f) {
+                    E2 lo, hi;
+                    if (pair) {
+                        lo = ent(f, 2 * at), hi = ent(f, 2 * at + 1);
+                    } else {
+                        lo = line_at(ent(f, 4 * at), ent(f, 4 * at + 1), smp), hi = line_at(ent(f, 4 * at + 2), ent(f, 4 * at + 3), smp);
+                    }
+                    return WsumPoints<E2, 1>{{line_at(lo, hi, t)}};
+                };
+                E2 out[1];
+                wsum_program<DEG>(a.op_begin[g], a.op_end[g], out, [&](u32 o) -> const PolyOp & { return ops[o]; }, table);
+                const E2 w = pair ? weight(big, at, g) : gl::add(weight(big, 2 * at, g), weight(big, 2 * at + 1, g));
+                const u32 idx = !mine ? ~0u : pair ? a.off_q[g] + t : a.off_d[g] + q;
+                const E2 x = gl::mulp(out[0], gl::prep(w));
+                if (__shfl(idx, 0, WAVE) == __shfl(idx, WAVE - 1, WAVE))
+                    flush_wave(idx, x, mine);
+                else if (mine)
+                    flush(idx, x);
+            };
             // (the first factor's polynomial is of the highest degree, NF)
-            if (g == 0) {
+            if (g < n_eqs && n_points <= per) {
+                if (a.degree[g] == 1)
+                    point_units(std::integral_constant<int, 1>{});
+                else
+                    point_units(std::integral_constant<int, NF>{});
+            } else if (g == 0) {
                 if (skip1)
                     units(std::integral_constant<int, NF>{}, std::true_type{}, std::integral_constant<int, NF>{});
                 else
