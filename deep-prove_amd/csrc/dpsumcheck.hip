@@ -2320,7 +2320,9 @@ constexpr u32 SLICE_SUM_TERM_PAIRS = 128, SLICE_SUM_MIN_PAIRS = 8, SLICE_SUM_WOR
 // ... and a sum that could be cut finer takes half the device at most, so that two such sums of two contexts find room
 // side by side (a launch that fills the device alone sends every other context's resident rounds back to launches of their own)
 constexpr u32 SLICE_SMALL_SUM_WORKGROUPS = 128;
-constexpr u32 SLICE_ONE_WORKGROUP_TERM_PAIRS = 512;  // pairs x terms up to which one workgroup takes the whole sum (sums of several terms: SLICE_SUM_TERM_PAIRS)
+// Pairs of a product up to which one workgroup takes the whole sum (sums of several terms: SLICE_SUM_TERM_PAIRS).  With all 512 of a sum of 10 variables its first trip
+// is 7.5 us of arithmetic: with 512, 256, 128, 64, 32 pairs that sum is 63.7, 62.9, 61.9, 62.3, 63.4 us, two of 9 and 10 variables 87.3, 84.5, 84.8, 83.8, 84.6.
+constexpr u32 SLICE_ONE_WORKGROUP_PAIRS = 128;
 constexpr u32 SLICE_MAX_WORKGROUPS = 256;
 // Most pairs a workgroup is given of a product, and of a sum of several terms: more would make more rounds resident, but a trip's arithmetic is a
 // workgroup's alone (with 512 pairs of a 3-term sum the first trip took 75 us where a launch for the round and a trip of 128 pairs take 66)
@@ -2433,7 +2435,7 @@ void plan_resident_rounds(dps_sc *sc, u32 n_tabs, u32 n_mles)
     u32 per_wg = (u32)std::min<u64>(per_wg_max, std::max<u64>(SLICE_MIN_PAIRS, pairs_of(j) / SLICE_SMALL_SUM_WORKGROUPS));
     if (n_terms > 1)
         while (per_wg > SLICE_SUM_MIN_PAIRS && per_wg * n_terms > SLICE_SUM_TERM_PAIRS && pairs_of(j) / per_wg < SLICE_SUM_WORKGROUPS) per_wg >>= 1;
-    if (pairs_of(j) * n_terms <= (n_terms > 1 ? SLICE_SUM_TERM_PAIRS : SLICE_ONE_WORKGROUP_TERM_PAIRS) && pairs_of(j) <= per_wg_max) per_wg = (u32)pairs_of(j);
+    if (pairs_of(j) * n_terms <= (n_terms > 1 ? SLICE_SUM_TERM_PAIRS : SLICE_ONE_WORKGROUP_PAIRS) && pairs_of(j) <= per_wg_max) per_wg = (u32)pairs_of(j);
     sc->tail_j0 = j;
     // The last rounds are the host's: a trip costs the way to the GPU and back and a workgroup's barriers whatever it
     // carries, a round of a few pairs costs the host a microsecond.  As many rounds as stay below HOST_TAIL_MULTS

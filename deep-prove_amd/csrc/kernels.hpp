@@ -1769,10 +1769,13 @@ __host__ __device__ constexpr u32 sl_lds_tables(u32 blk, u32 terms) { return sl_
 static_assert(sizeof(SliceTerm) % 8 == 0, "terms are copied as 64-bit words");
 // (`eq`: the weights of the eq factor, one per pair of a table's entries, are kept like a table of half the size)
 __host__ __device__ constexpr u32 sl_weights_cap(u32 cap) { return cap / 2 > 0 ? cap / 2 : 1; }
+// A table's two limb arrays of `cap` entries and a word: lanes that share a pair read the same entry of different tables, which with a stride of a power of
+// two would all lie in one bank (16 products over 32 tables, 32 pairs a workgroup: first trip 34 -> 26 us)
+__host__ __device__ constexpr u32 sl_table_stride(u32 cap) { return 2 * cap + 1; }
 // (`eq`: how many eq factors there are)
 __host__ __device__ constexpr u32 slice_lds_words(u32 n_tabs, u32 cap, u32 blk, u32 eq, u32 terms = SL_MAX_TERMS)
 {
-    return sl_lds_tables(blk, terms) + n_tabs * 2 * (cap + cap / 2) + eq * 2 * (sl_weights_cap(cap) + sl_weights_cap(cap / 2));
+    return sl_lds_tables(blk, terms) + n_tabs * (sl_table_stride(cap) + sl_table_stride(cap / 2)) + eq * 2 * (sl_weights_cap(cap) + sl_weights_cap(cap / 2));
 }
 // A workgroup of these launches is 1024 threads: what a round costs here is the longest chain of dependent field
 // multiplications in any one lane, and with more lanes each has fewer units of work behind one another.
@@ -1826,9 +1829,11 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
     const u32 cap = len;
     u32 len_log = (u32)__builtin_ctz(len);      // a workgroup's share is a power of two
     // two buffers per limb array: `cap` entries and half of that; a fold reads one and writes the other
-    u64 *const buf_big = dyn + SL_LDS_TABLES, *const buf_small = buf_big + (size_t)nt * 2 * cap;
+    u64 *const buf_big = dyn + SL_LDS_TABLES, *const buf_small = buf_big + (size_t)nt * sl_table_stride(cap);
     bool in_big = true;  // where the current state is
-    auto tab = [&](bool big, u32 f, int limb) -> u64 * { return big ? buf_big + (size_t)(f * 2 + limb) * cap : buf_small + (size_t)(f * 2 + limb) * (cap / 2); };
+    auto tab = [&](bool big, u32 f, int limb) -> u64 * {
+        return big ? buf_big + (size_t)f * sl_table_stride(cap) + (size_t)limb * cap : buf_small + (size_t)f * sl_table_stride(cap / 2) + (size_t)limb * (cap / 2);
+    };
     // The weights of the eq factor, R_j(p) = eq(rho_{j+1..}, p) for the pairs p of round j, live beside the tables in the
     // same two buffers: read once when the launch starts, and from round to round the weight of a pair is the sum of the
     // weights of the two pairs it is made of (R_{j+1}(p) = R_j(2p) + R_j(2p + 1)), so a fold of the tables is an add here.
@@ -1836,7 +1841,7 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
     static_assert(ARGS::EQS == 0 || (EQ && TERMS), "several eq factors belong to a sum of several terms");
     u32 n_eqs = 1;
     if constexpr (ARGS::EQS > 0) n_eqs = a.n_eqs;
-    u64 *const wts_big = buf_small + (size_t)nt * 2 * (cap / 2), *const wts_small = wts_big + n_eqs * 2 * sl_weights_cap(cap);
+    u64 *const wts_big = buf_small + (size_t)nt * sl_table_stride(cap / 2), *const wts_small = wts_big + n_eqs * 2 * sl_weights_cap(cap);
     auto wts = [&](bool big, int limb, u32 g = 0) -> u64 * {
         return big ? wts_big + (size_t)(2 * g + limb) * sl_weights_cap(cap) : wts_small + (size_t)(2 * g + limb) * sl_weights_cap(cap / 2);
     };
@@ -1850,6 +1855,17 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
     // lanes that share a pair (a quad) at one evaluation point split the terms among them
     const u32 p_split = TERMS ? a.n_terms : 1u;
     const u32 q_split = TERMS ? (a.n_terms * (u32)(NPT * NSMP) <= (u32)BLOCK ? a.n_terms : 1u) : 1u;
+    // A trip of two rounds has twice as many pairs as quads.  So many quads, and twice as many pairs, are taken side by side, the pairs by the last lanes and the quads by
+    // the first: the lanes' passes over both are then the same (64 pairs of three terms of degree 3: two passes where all lanes for the one and then for the other
+    // were three).  [0] every point, [1] t = 1 left out.  0: all lanes for the pairs, then all for the quads, where that would leave more than an eighth of the lanes
+    // without work, or a quad's lanes take all its terms and a pair's do not.
+    const u32 q_lanes = q_split * (u32)(NPT * NSMP);
+    auto side = [&](u32 points) {
+        if (ARGS::EQS > 0) return 0u;  // (lanes by factor, and no terms)
+        const u32 lanes = q_lanes + 2 * p_split * points, n = (u32)BLOCK / lanes;
+        return q_split == p_split && n * lanes >= (u32)BLOCK / 8 * 7 ? n : 0u;
+    };
+    const u32 q_side[2] = {side(NP), side(NP - 1)};
     u32 j = a.j0, pend = a.pend0;
     u64 trip_seq = a.seq0;
     u32 Wc = W;  // workgroups still at work
@@ -2235,10 +2251,13 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
         } else {
             const u32 n_pairs = len >> 1;
             const u32 rt = BLOCK - 1 - tid;
-            const u32 m0 = rt % p_split, t = (rt / p_split) % (u32)NP, slot = rt / (p_split * (u32)NP), n_slots = BLOCK / (p_split * (u32)NP);
+            const u32 m0 = rt % p_split, rest = rt / p_split, slot = skip1 ? rest / (u32)(NP - 1) : rest / (u32)NP;
+            const u32 ti = skip1 ? rest % (u32)(NP - 1) : rest % (u32)NP, t = skip1 && ti > 0 ? ti + 1 : ti;
+            const u32 side_by_side = skip1 ? q_side[1] : q_side[0];
+            const u32 n_slots = dbl && side_by_side ? 2 * side_by_side : skip1 ? BLOCK / (p_split * (u32)(NP - 1)) : BLOCK / (p_split * (u32)NP);
             E2 acc = gl::e2_zero();
             bool any = false;
-            if (slot < n_slots && !(t == 1 && skip1)) {
+            if (slot < n_slots) {
                 for (u32 p = slot; p < n_pairs; p += n_slots) {
                     any = true;
                     const E2 g = poly_of([&](u32 f) { return line_at(ent(f, 2 * p), ent(f, 2 * p + 1), t); }, false, m0, p_split);
@@ -2252,7 +2271,7 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
             const u32 n_quads = len >> 2;
             // a lane keeps one sample at one point (of some of the terms)
             const u32 m0 = tid % q_split, ti = (tid / q_split) % (u32)NPT, smp = (tid / (q_split * (u32)NPT)) % (u32)NSMP;
-            const u32 slot = tid / (q_split * (u32)(NPT * NSMP)), n_slots = BLOCK / (q_split * (u32)(NPT * NSMP));
+            const u32 side_by_side = skip1 ? q_side[1] : q_side[0], slot = tid / q_lanes, n_slots = side_by_side ? side_by_side : BLOCK / q_lanes;
             const u32 t = ti == 0 ? 0 : ti + 1;  // points t = 0, 2, .., NF
             E2 acc = gl::e2_zero();
             bool any = false;
