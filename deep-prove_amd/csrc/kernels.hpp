@@ -4077,6 +4077,11 @@ __global__ void __launch_bounds__(LOGUP_TAIL_BLOCK) logup_tail_kernel(LogupTailB
     constexpr u32 CAP = 1u << LOGUP_TAIL_BITS;
     // numerators (two limb arrays) and denominators (two) of a level: CAP entries each in `big`, half of that in `small`
     __shared__ u64 big[4 * CAP], small_[2 * CAP];
+    // An output entry is four words, numerator and denominator of two limbs each, and a lane makes one of them, whole wavefronts the same: a level is as long as
+    // one lane's chain of products, and that is four of the base field and a reduction instead of three of the extension (ten levels 21.8 -> 18.4 us)
+    constexpr u32 PART = LOGUP_TAIL_BLOCK / 4;
+    const u32 word = __builtin_amdgcn_readfirstlane(threadIdx.x / PART);
+    const bool den = word >= 2, limb = (word & 1) != 0;
     u32 cur = (u32)a.first_cur;
     for (u32 l = 0; l < a.n_levels; l++, cur >>= 1) {
         const u32 prev = 2 * cur;
@@ -4085,8 +4090,8 @@ __global__ void __launch_bounds__(LOGUP_TAIL_BLOCK) logup_tail_kernel(LogupTailB
         const u64 *src = to_big ? small_ : big;
         u64 *dst = to_big ? big : small_;
         const u64 *g0 = a.c0 + a.off[l], *g1 = a.c1 + a.off[l];
-        u64 *n0 = a.c0 + a.off[l + 1], *n1 = a.c1 + a.off[l + 1], *d0 = n0 + cur, *d1 = n1 + cur;
-        for (u32 i = threadIdx.x; i < cur; i += LOGUP_TAIL_BLOCK) {
+        u64 *const out = (limb ? a.c1 : a.c0) + a.off[l + 1] + (den ? cur : 0);
+        for (u32 i = threadIdx.x & (PART - 1); i < cur; i += PART) {
             E2 nl, nh, dl, dh;
             if (l == 0) {
                 nl = gl::e2(g0[i], g1[i]), nh = gl::e2(g0[i + cur], g1[i + cur]);
@@ -4095,23 +4100,21 @@ __global__ void __launch_bounds__(LOGUP_TAIL_BLOCK) logup_tail_kernel(LogupTailB
                 nl = gl::e2(src[i], src[cap_s + i]), nh = gl::e2(src[i + cur], src[cap_s + i + cur]);
                 dl = gl::e2(src[2 * cap_s + i], src[3 * cap_s + i]), dh = gl::e2(src[2 * cap_s + i + cur], src[3 * cap_s + i + cur]);
             }
-            const E2 num = gl::add(gl::mul(nl, dh), gl::mul(nh, dl));
-            const E2 den = gl::mul(dl, dh);
-            n0[i] = num.c0;
-            n1[i] = num.c1;
-            d0[i] = den.c0;
-            d1[i] = den.c1;
-            dst[i] = num.c0;
-            dst[cap_d + i] = num.c1;
-            dst[2 * cap_d + i] = den.c0;
-            dst[3 * cap_d + i] = den.c1;
-            if (a.shadow && cur <= LOGUP_SHADOW_MAX) {
-                u64 *sh = a.shadow + logup_shadow_off(cur);
-                st_sys(sh + i, num.c0);
-                st_sys(sh + cur + i, num.c1);
-                st_sys(sh + 2 * cur + i, den.c0);
-                st_sys(sh + 3 * cur + i, den.c1);
+            gl::Acc sum = gl::acc_zero();
+            auto add_product = [&](E2 x, E2 y) {
+                gl::acc_prod(sum, x.c0, limb ? y.c1 : y.c0);
+                gl::acc_prod(sum, x.c1, limb ? y.c0 : gl::mul_small(y.c1, (u32)gl::W));
+            };
+            if (den) {
+                add_product(dl, dh);
+            } else {
+                add_product(nl, dh);
+                add_product(nh, dl);
             }
+            const u64 v = gl::acc_reduce(sum);
+            out[i] = v;
+            dst[word * cap_d + i] = v;
+            if (a.shadow && cur <= LOGUP_SHADOW_MAX) st_sys(a.shadow + logup_shadow_off(cur) + word * cur + i, v);
         }
         __syncthreads();
     }
