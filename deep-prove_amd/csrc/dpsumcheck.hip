@@ -2328,9 +2328,10 @@ constexpr u32 SLICE_MAX_WORKGROUPS = 256;
 // workgroup's alone (with 512 pairs of a 3-term sum the first trip took 75 us where a launch for the round and a trip of 128 pairs take 66)
 constexpr u32 SLICE_PRODUCT_PAIRS = 512, SLICE_SUM_PAIRS = 128;
 // the rounds a resident launch leaves to the host: at most so many, and so many extension multiplications in all
-// (measured: 2 to 6 rounds and 400 to 3000 multiplications differ by a few percent; these were the best over the benchmark configurations)
+// (2 to 6 rounds and 400 to 3000 multiplications differ by a few percent: with 400, 800, 1200, 1800 the products of an attention layer over 2^12 entries take 182, 179,
+// 174, 173 us, 26 fraction-sum layers of up to 2^15 entries 1377, 1350, 1333, 1348, those of 2^21 3147, 3084, 3082, 3099)
 constexpr u32 HOST_TAIL_MAX_ROUNDS = 5;
-constexpr u64 HOST_TAIL_MULTS = 800;
+constexpr u64 HOST_TAIL_MULTS = 1200;
 
 // eq * f * g over two base-field tables, large enough for the factored eq weights: rounds 1 and 2 can be one launch
 // that reads the tables once and writes nothing (pair12_kernel).  `first_resident`: the first round of the resident
