@@ -2320,9 +2320,9 @@ constexpr u32 SLICE_SUM_TERM_PAIRS = 128, SLICE_SUM_MIN_PAIRS = 8, SLICE_SUM_WOR
 // ... and a sum that could be cut finer takes half the device at most, so that two such sums of two contexts find room
 // side by side (a launch that fills the device alone sends every other context's resident rounds back to launches of their own)
 constexpr u32 SLICE_SMALL_SUM_WORKGROUPS = 128;
-// Pairs of a product up to which one workgroup takes the whole sum (sums of several terms: SLICE_SUM_TERM_PAIRS).  With all 512 of a sum of 10 variables its first trip
-// is 7.5 us of arithmetic: with 512, 256, 128, 64, 32 pairs that sum is 63.7, 62.9, 61.9, 62.3, 63.4 us, two of 9 and 10 variables 87.3, 84.5, 84.8, 83.8, 84.6.
-constexpr u32 SLICE_ONE_WORKGROUP_PAIRS = 128;
+// Pairs of a product up to which one workgroup takes the whole sum (sums of several terms: SLICE_SUM_TERM_PAIRS).  All 512 of a sum of 10 variables are 7.5 us of
+// arithmetic in its first trip: cut into workgroups of 32 that sum takes 46.9 us instead of 50.9, but the one of 9 variables 45.6, whole 40.3.
+constexpr u32 SLICE_ONE_WORKGROUP_PAIRS = 256;
 constexpr u32 SLICE_MAX_WORKGROUPS = 256;
 // Most pairs a workgroup is given of a product, and of a sum of several terms: more would make more rounds resident, but a trip's arithmetic is a
 // workgroup's alone (with 512 pairs of a 3-term sum the first trip took 75 us where a launch for the round and a trip of 128 pairs take 66)
@@ -3383,7 +3383,8 @@ int32_t SessionSetup::run()
     CHK(plan_and_ready_tables());
     CHK(layout_scratch());
     // A sum that is resident, or the host's, from round 1 on with every table of it needs no launch but the one of round 1: the others are worked out when one
-    // is needed all the same (describe_now).  16 products over 32 tables of 11 variables were set up in 41 us, fraction-sum layers in 2.5 .. 3.3.
+    // is needed all the same (describe_now).  Setting 16 products over 32 tables of 11 variables up: 41 -> 34 us; 26 fraction-sum layers of up to
+    // 2^15 entries 1448 -> 1414.
     bool later = n_vars >= 1 && (sc->host_only || sc->tail_j0 == 1);
     for (u32 k = 0; k < n_mles && later; k++) later = (in_fast(k) || sc->closed_eq(k)) && !zpad_of(k);
     describe_rounds(later ? 1 : n_vars + 1);
