@@ -2152,102 +2152,51 @@ __global__ void __launch_bounds__(BLK) slice_kernel(ARGS a)
         // and spread over the lanes; every unit's value goes into the point's counters, where the pieces add up.
         // ---- round j: pairs of the state; units taken from the last thread down, those of the quads from the first up ----
         if constexpr (ARGS::EQS > 0) {
-            // This wavefront's factor, and this lane's place among the lanes of that factor.  A unit of work is a pair, or with a trip of two
-            // rounds a quad at one challenge (first the pairs, then the quads challenge by challenge): a lane walks the program at
-            // all of its factor's points, and where a wavefront's units are of one kind it adds its sums up before they go into the
-            // counters (a counter that every lane adds to serves them one after the other).
+            // This wavefront's factor, and this lane's place among the lanes of that factor.  A unit of work is one point of a pair, or with a
+            // trip of two rounds one point of a quad at one challenge; units of one sum lie side by side, points of pairs first, and a wavefront
+            // all of whose units are of one sum adds them up before they go into the counters (a counter that every lane adds to serves them one
+            // after the other).  (A lane that walks the program at all points of a pair keeps a value a point and level of the program: at degree 4
+            // that is more than the 128 registers a thread of 1024 can have.  With such walks beside the ones at a point this kernel spilled 149 of them and
+            // kept 3.4 KB a lane in scratch memory; without, it has 96 registers at every degree: linking a gated activation (degrees 4 and 1) of 2^8,
+            // 2^16, 2^20 entries 256, 632, 800 -> 110, 232, 423 us, degrees 3 and 1 of 2^16 entries 172 -> 170.)
             const u32 per = (BLOCK / n_eqs) & ~(u32)(WAVE - 1);
             const u32 g = __builtin_amdgcn_readfirstlane(tid / per), l = tid - g * per;
-            auto units = [&](auto n_points, auto skips, auto program_degree) {
-                constexpr int N = decltype(n_points)::value, DEG = decltype(program_degree)::value;
-                constexpr bool SKIP = decltype(skips)::value;
+            const u32 dg = g < n_eqs ? a.degree[g] : 0, ptsq = g == 0 && skip1 ? dg : dg + 1, ptsd = g == 0 ? dg : dg + 1;
+            const u32 n_units = g < n_eqs ? ptsq * (len >> 1) + (dbl ? (dg + 1) * ptsd * (len >> 2) : 0) : 0;
+            auto units = [&](auto program_degree) {
+                constexpr int DEG = decltype(program_degree)::value;
                 const PolyOp *ops = reinterpret_cast<const PolyOp *>(lterms);
-                const u32 d = a.degree[g], npt = g == 0 ? d : d + 1;  // (points of a round that takes p(1) from its claim)
-                const u32 n_pairs = len >> 1, n_quads = len >> 2, n_units = n_pairs + (dbl ? n_quads * (d + 1) : 0);
-                const u32 quads_log = len_log >= 2 ? len_log - 2 : 0;
                 for (u32 base = 0; base < n_units; base += per) {
                     const u32 u = base + l;
-                    const bool mine = u < n_units, pair = u < n_pairs;
-                    const u32 v = pair || !mine ? 0 : u - n_pairs, smp = v >> quads_log, at = !mine ? 0 : pair ? u : v & (n_quads - 1);
+                    const bool mine = u < n_units, pair = !mine || u < ptsq * (len >> 1);
+                    const u32 v = !mine ? 0 : pair ? u : u - ptsq * (len >> 1), run_log = pair ? len_log - 1 : len_log - 2;
+                    const u32 q = v >> run_log, at = v & ((1u << run_log) - 1), smp = pair ? 0 : q / ptsd, ti = pair ? q : q - smp * ptsd;
+                    const u32 t = ti > 0 && g == 0 && (!pair || skip1) ? ti + 1 : ti;
                     auto table = [&](u32 f) {
                         E2 lo, hi;
-                        if (pair || !mine) {
+                        if (pair) {
                             lo = ent(f, 2 * at), hi = ent(f, 2 * at + 1);
                         } else {
                             lo = line_at(ent(f, 4 * at), ent(f, 4 * at + 1), smp), hi = line_at(ent(f, 4 * at + 2), ent(f, 4 * at + 3), smp);
                         }
-                        return wsum_points<N, SKIP>(lo, gl::sub(hi, lo));
+                        return WsumPoints<E2, 1>{{line_at(lo, hi, t)}};
                     };
-                    E2 out[N];
+                    E2 out[1];
                     wsum_program<DEG>(a.op_begin[g], a.op_end[g], out, [&](u32 o) -> const PolyOp & { return ops[o]; }, table);
-                    E2 w = gl::e2_zero();
-                    if (mine) w = pair ? weight(big, at, g) : gl::add(weight(big, 2 * at, g), weight(big, 2 * at + 1, g));
-                    const gl::E2P wp = gl::prep(w);
-                    // where the sums of point i go: those of pairs from off_q on, those of quads from off_d on
-                    const u32 kind = !mine ? ~0u : pair ? 0 : 1 + smp;
-                    const bool alike = __shfl(kind, 0, WAVE) == __shfl(kind, WAVE - 1, WAVE);
-#pragma unroll
-                    for (int i = 0; i < N; i++) {
-                        const u32 t = SKIP && i > 0 ? (u32)i + 1 : (u32)i;
-                        const u32 ti = g == 0 && t > 1 ? t - 1 : t;
-                        const bool wanted = mine && t <= d && (pair ? !(g == 0 && t == 1 && skip1) : !(g == 0 && t == 1));
-                        const u32 idx = pair ? a.off_q[g] + t : a.off_d[g] + smp * npt + ti;
-                        const E2 x = gl::mulp(out[i], wp);
-                        if (alike)
-                            flush_wave(idx, x, wanted);
-                        else if (wanted)
-                            flush(idx, x);
-                    }
+                    const E2 w = pair ? weight(big, at, g) : gl::add(weight(big, 2 * at, g), weight(big, 2 * at + 1, g));
+                    const u32 idx = !mine ? ~0u : pair ? a.off_q[g] + t : a.off_d[g] + q;
+                    const E2 x = gl::mulp(out[0], gl::prep(w));
+                    if (__shfl(idx, 0, WAVE) == __shfl(idx, WAVE - 1, WAVE))
+                        flush_wave(idx, x, mine);
+                    else if (mine)
+                        flush(idx, x);
                 }
             };
-            // Where the factor's lanes are enough for it a unit is one point of a pair, or of a quad at one challenge: the chain of a walk at one
-            // point instead of four in turn (two tables, degrees 3 and 1: trips 15 .. 16 -> 13.5 .. 15 us, the last workgroup's three 19, 13, 12 -> 16, 12, 9).
-            // Units of one sum lie side by side, points of pairs first.
-            const u32 dg = g < n_eqs ? a.degree[g] : 0, ptsq = g == 0 && skip1 ? dg : dg + 1, ptsd = g == 0 ? dg : dg + 1;
-            const u32 n_points = ptsq * (len >> 1) + (dbl ? (dg + 1) * ptsd * (len >> 2) : 0);
-            auto point_units = [&](auto program_degree) {
-                constexpr int DEG = decltype(program_degree)::value;
-                const PolyOp *ops = reinterpret_cast<const PolyOp *>(lterms);
-                const bool mine = l < n_points, pair = !mine || l < ptsq * (len >> 1);
-                const u32 v = !mine ? 0 : pair ? l : l - ptsq * (len >> 1), run_log = pair ? len_log - 1 : len_log - 2;
-                const u32 q = v >> run_log, at = v & ((1u << run_log) - 1), smp = pair ? 0 : q / ptsd, ti = pair ? q : q - smp * ptsd;
-                const u32 t = ti > 0 && g == 0 && (!pair || skip1) ? ti + 1 : ti;
-                auto table = [&](u32 f) {
-                    E2 lo, hi;
-                    if (pair) {
-                        lo = ent(f, 2 * at), hi = ent(f, 2 * at + 1);
-                    } else {
-                        lo = line_at(ent(f, 4 * at), ent(f, 4 * at + 1), smp), hi = line_at(ent(f, 4 * at + 2), ent(f, 4 * at + 3), smp);
-                    }
-                    return WsumPoints<E2, 1>{{line_at(lo, hi, t)}};
-                };
-                E2 out[1];
-                wsum_program<DEG>(a.op_begin[g], a.op_end[g], out, [&](u32 o) -> const PolyOp & { return ops[o]; }, table);
-                const E2 w = pair ? weight(big, at, g) : gl::add(weight(big, 2 * at, g), weight(big, 2 * at + 1, g));
-                const u32 idx = !mine ? ~0u : pair ? a.off_q[g] + t : a.off_d[g] + q;
-                const E2 x = gl::mulp(out[0], gl::prep(w));
-                if (__shfl(idx, 0, WAVE) == __shfl(idx, WAVE - 1, WAVE))
-                    flush_wave(idx, x, mine);
-                else if (mine)
-                    flush(idx, x);
-            };
             // (the first factor's polynomial is of the highest degree, NF)
-            if (g < n_eqs && n_points <= per) {
-                if (a.degree[g] == 1)
-                    point_units(std::integral_constant<int, 1>{});
-                else
-                    point_units(std::integral_constant<int, NF>{});
-            } else if (g == 0) {
-                if (skip1)
-                    units(std::integral_constant<int, NF>{}, std::true_type{}, std::integral_constant<int, NF>{});
-                else
-                    units(std::integral_constant<int, NF + 1>{}, std::false_type{}, std::integral_constant<int, NF>{});
-            } else if (g < n_eqs) {
-                if (a.degree[g] == 1)
-                    units(std::integral_constant<int, 2>{}, std::false_type{}, std::integral_constant<int, 1>{});
-                else
-                    units(std::integral_constant<int, NF + 1>{}, std::false_type{}, std::integral_constant<int, NF>{});
-            }
+            if (dg == 1)
+                units(std::integral_constant<int, 1>{});
+            else
+                units(std::integral_constant<int, NF>{});
         } else {
             const u32 n_pairs = len >> 1;
             const u32 rt = BLOCK - 1 - tid;
