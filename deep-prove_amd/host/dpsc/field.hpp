@@ -150,16 +150,22 @@ inline F interpolate_uni(const F *evals, size_t d, const F &r)
         below[k] = run;
         run *= r - F::from_u64(k);
     }
+    // (a message of more points than the table's -- a proof that is only verified here: 1 / k! from one inversion, the denominator k! (d - k)! up to the sign)
+    std::vector<uint64_t> inv_fact;
+    if (d > LAGRANGE_MAX_DEGREE) {
+        inv_fact.assign(d + 1, 1);
+        for (size_t k = 2; k <= d; k++) inv_fact[d] = Fp::mul(inv_fact[d], k);
+        inv_fact[d] = Fp::inv(inv_fact[d]);
+        for (size_t k = d; k > 0; k--) inv_fact[k - 1] = Fp::mul(inv_fact[k], k);
+    }
     F acc = F::zero(), above = F::one();
     for (size_t k = d + 1; k-- > 0;) {
         uint64_t w;
         if (d <= LAGRANGE_MAX_DEGREE) {
             w = table.inv[d][k];
         } else {
-            uint64_t den = 1;
-            for (size_t m = 0; m <= d; m++)
-                if (m != k) den = Fp::mul(den, Fp::sub(k, m));
-            w = Fp::inv(den);
+            w = Fp::mul(inv_fact[k], inv_fact[d - k]);
+            if ((d - k) % 2) w = Fp::neg(w);
         }
         const F basis = below[k] * above;
         acc += F(Fp::mul(basis.c0, w), Fp::mul(basis.c1, w)) * evals[k];

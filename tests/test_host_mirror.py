@@ -7,8 +7,9 @@ import subprocess
 import numpy as np
 import pytest
 
+from pyfield import interpolate
 from test_oracle_field import BLAKE3_KAT
-from util import rand_e2
+from util import from_E2, rand_e2, to_E2
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -65,6 +66,16 @@ def test_verifier_accepts_checker_proof_and_rejects_tampering(dp, orc):
     bad[4, 2, 1] ^= np.uint64(1)
     rc, _, _ = dp.Context.sumcheck_verify(ctx_free, claim, bad, dp.Transcript())
     assert rc != 0
+
+
+@pytest.mark.parametrize("degree", list(range(1, 10)) + [12, 17])
+def test_verifier_evaluates_messages_of_any_degree(dp, degree):
+    # one round: what is left to check is the message's polynomial at the challenge (degrees on both sides of the kept denominators' limit)
+    msg = rand_e2(degree + 1, 500 + degree)
+    values = to_E2(msg)
+    claim = from_E2([values[0] + values[1]])[0]
+    rc, point, expected = dp.Context.sumcheck_verify(dp.Context.__new__(dp.Context), claim, msg[None], dp.Transcript())
+    assert rc == 0 and to_E2(expected)[0] == interpolate(values, to_E2(point)[0])
 
 
 def test_expression_flattening_cpp(tmp_path):
