@@ -89,6 +89,42 @@ int main()
             bad++;
         }
     }
+    // products of more tables than the short form of a monomial holds, repeated tables, merging and cancelling monomials of products of sums
+    {
+        auto power = [](uint16_t id, int n) {
+            Expression e = Expression::WitIn(id);
+            for (int i = 1; i < n; i++) e = e * Expression::WitIn(id);
+            return e;
+        };
+        Expression long_product = Expression::Constant(rnd());
+        for (uint16_t i = 0; i < 11; i++) long_product = long_product * Expression::WitIn((uint16_t)((7 * i) % 11));
+        bad += check("eleven_tables", long_product, 11, 0, 11);
+        bad += check("nine_times_one_table", power(1, 9), 2, 0, 9);
+        const Expression a = Expression::WitIn(3), b = Expression::WitIn(1), c = Expression::Challenge(0, 2, one, zero);
+        const Expression e = (a + b) * (a - b) + c * (b * a + a * b) + (a + Expression::Constant(rnd())) * (b + c) * power(0, 2) - power(2, 4) * power(4, 4);
+        bad += check("products_of_sums", e, 5, 1, 8);
+        // the same monomials in the same order whether or not a product beside them is too long for the short form
+        for (int rep = 0; rep < 5; rep++) {
+            const std::vector<F> ch{rnd()};
+            const auto with_short = e.to_monomials(ch), with_long = (e + power(5, 9)).to_monomials(ch);
+            bool ok = with_long.size() == with_short.size() + 1;
+            size_t at = 0;
+            for (auto &m : with_long) {
+                if (m.wits == std::vector<uint16_t>(9, 5)) continue;
+                ok = ok && at < with_short.size() && m.wits == with_short[at].wits && m.coeff == with_short[at].coeff;
+                at++;
+            }
+            for (size_t i = 0; i + 1 < with_short.size(); i++) ok = ok && with_short[i].wits < with_short[i + 1].wits;
+            for (auto &m : with_short) ok = ok && std::is_sorted(m.wits.begin(), m.wits.end()) && !m.coeff.is_zero();
+            // (a + b)(a - b): the mixed products cancel, those of 2 c a b are one monomial
+            for (auto &m : with_short)
+                if (m.wits == std::vector<uint16_t>{1, 3}) ok = ok && m.coeff == (ch[0] * ch[0]) + (ch[0] * ch[0]);
+            if (!ok) {
+                printf("FAIL long and short monomials differ\n");
+                bad++;
+            }
+        }
+    }
     // Challenge(id, pow, scalar, offset) = scalar * chal^pow + offset
     {
         F s = rnd(), o = rnd(), ch = rnd();
