@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "kernels.hpp"
+#include "program.hpp"
 
 using gl::E2;
 using gl::u32;
@@ -2195,86 +2196,6 @@ u32 product_blocks(u64 n_pairs)
 
 namespace {
 
-// Nested (Horner) form of a sum of terms: the table found in most of the remaining terms is factored out of them, recursively.
-constexpr u32 MAX_PROGRAM_TERMS = 64, NO_TABLE = ~0u;
-struct ProgramTerm {
-    E2 coeff;
-    uint8_t n, slot[DPS_MAX_FACTORS];  // remaining factors, as slots below SL_MAX_TABS
-};
-
-dpk::PolyOp program_op(u32 kind, u32 d, u32 slot, E2 c)
-{
-    dpk::PolyOp op;
-    memset(&op, 0, sizeof op);
-    op.c0 = c.c0;
-    op.c1 = c.c1;
-    op.w = gl::mul_small(c.c1, (u32)gl::W);
-    const u32 cls = c.c1 ? dpk::POLY_COEFF_ANY : c.c0 == 1 ? dpk::POLY_COEFF_ONE : c.c0 == gl::P - 1 ? dpk::POLY_COEFF_MINUS_ONE : dpk::POLY_COEFF_BASE;
-    op.code = kind | d << 2 | (kind == dpk::POLY_OP_LEAF ? cls : 0) << 6 | slot << 8;
-    return op;
-}
-
-// Appends the operations of the node of depth `depth` with these terms, each of at least one factor (their order is not kept); returns
-// its number of products.
-u32 program_build(ProgramTerm *t, u32 n, u32 depth, std::vector<dpk::PolyOp> &ops)
-{
-    u32 products = 0;
-    while (n) {
-        uint8_t count[dpk::SL_MAX_TABS] = {0};
-        u32 best = t[0].slot[0];
-        for (u32 i = 0; i < n; i++)
-            for (u32 f = 0; f < t[i].n; f++) {
-                const u32 sl = t[i].slot[f];
-                bool again = false;
-                for (u32 q = 0; q < f; q++) again = again || t[i].slot[q] == sl;
-                if (again) continue;
-                count[sl]++;
-                if (count[sl] > count[best] || (count[sl] == count[best] && sl < best)) best = sl;
-            }
-        // its terms to the front, those that end here behind the others among them
-        u32 inner = 0, with = 0;
-        E2 ending = gl::e2_zero();
-        for (u32 i = 0; i < n; i++) {
-            ProgramTerm &p = t[i];
-            u32 f = 0;
-            while (f < p.n && p.slot[f] != best) f++;
-            if (f == p.n) continue;
-            p.slot[f] = p.slot[--p.n];
-            if (p.n) {
-                std::swap(t[i], t[with]);
-                std::swap(t[with++], t[inner++]);
-            } else {
-                ending = gl::add(ending, p.coeff);
-                std::swap(t[i], t[with++]);
-            }
-        }
-        if (inner) {
-            ops.push_back(program_op(dpk::POLY_OP_ENTER, depth + 1, 0, ending));
-            products += program_build(t, inner, depth + 1, ops);
-            ops.push_back(program_op(dpk::POLY_OP_LEAVE, depth + 1, best, gl::e2_zero()));
-        } else {
-            ops.push_back(program_op(dpk::POLY_OP_LEAF, depth, best, ending));
-        }
-        products++;
-        t += with, n -= with;
-    }
-    return products;
-}
-
-// A whole program: its first operation enters the root with the constant.  Returns the number of products.
-u32 program_root(ProgramTerm *t, u32 n, std::vector<dpk::PolyOp> &ops)
-{
-    E2 root = gl::e2_zero();
-    u32 m = 0;
-    for (u32 i = 0; i < n; i++)
-        if (t[i].n)
-            std::swap(t[i], t[m++]);
-        else
-            root = gl::add(root, t[i].coeff);
-    ops.push_back(program_op(dpk::POLY_OP_ENTER, 0, 0, root));
-    return program_build(t, m, 0, ops);
-}
-
 // one staged upload of all descriptors; not waited for (the staging vector lives as long as the session)
 int32_t describe_now(dps_sc *sc);
 int32_t ensure_descs(dps_sc *sc)
@@ -2671,6 +2592,8 @@ bool SessionSetup::closed_form_eq_factor()
     return ok;
 }
 
+constexpr u32 MAX_PROGRAM_TERMS = 64, NO_TABLE = ~0u;
+
 // A sum each of whose terms has one eq table, up to three of them in all, times polynomials of degree 4 at most over up to POLY_MAXT
 // other tables, all of full size: the eq factors in closed form, a nested program each for the polynomials (wsum_kernel).  What
 // does not fit (degrees, numbers of operations and sums) runs with the eq tables as tables among the others, or a single eq table in closed
@@ -2713,12 +2636,12 @@ bool SessionSetup::weighted_programs()
     if (eqs[0].degree < 2 || eqs[0].degree > 4 || eqs[n_eqs - 1].degree < 1) return false;
     std::vector<dpk::PolyOp> ops;
     for (u32 g = 0; g < n_eqs; g++) {
-        ProgramTerm ts[MAX_PROGRAM_TERMS];
+        dpk::ProgramTerm ts[MAX_PROGRAM_TERMS];
         u32 n = 0;
         for (u32 ti = 0; ti < sc->n_terms; ti++) {
             if (eq_of_term[ti] != eqs[g].k) continue;
             const dps_term &t = sc->terms[ti];
-            ProgramTerm &p = ts[n++];
+            dpk::ProgramTerm &p = ts[n++];
             p.coeff = gl::e2(t.coeff[0], t.coeff[1]);
             eqs[g].base_program = eqs[g].base_program && t.coeff[1] == 0;
             p.n = 0;
@@ -2726,7 +2649,7 @@ bool SessionSetup::weighted_programs()
                 if (t.factors[f] != eqs[g].k) p.slot[p.n++] = (uint8_t)(std::find(tabs, tabs + n_tabs, t.factors[f]) - tabs);
         }
         eqs[g].op_begin = (u32)ops.size();
-        program_root(ts, n, ops);
+        dpk::program_root(ts, n, ops);
         eqs[g].op_end = (u32)ops.size();
     }
     if (ops.size() > (size_t)dpk::SL_EQS_OPS) return false;
@@ -2845,17 +2768,17 @@ void SessionSetup::nested_programs()
     std::vector<dpk::PolyOp> all_ops;
     u32 plain = 0, nested = 0;
     for (size_t g = 0; g < groups.size() && use_ops; g++) {
-        std::vector<ProgramTerm> ts(te[g] - tb[g]);
+        std::vector<dpk::ProgramTerm> ts(te[g] - tb[g]);
         for (u32 ti = tb[g]; ti < te[g]; ti++) {
             const dpk::PolyTerm &pt = poly_terms[ti];
-            ProgramTerm &p = ts[ti - tb[g]];
+            dpk::ProgramTerm &p = ts[ti - tb[g]];
             p.coeff = gl::e2(pt.c0, pt.c1);
             p.n = (uint8_t)pt.n_factors;
             std::copy(pt.slot, pt.slot + pt.n_factors, p.slot);
             plain += pt.n_factors;  // n_factors - 1 products and one for the coefficient
         }
         std::vector<dpk::PolyOp> ops;
-        nested += program_root(ts.data(), (u32)ts.size(), ops);
+        nested += dpk::program_root(ts.data(), (u32)ts.size(), ops);
         if (ops.size() > (size_t)dpk::POLY_LDS_OPS) use_ops = false;
         sc->poly_op_begin[g] = (u32)all_ops.size();
         all_ops.insert(all_ops.end(), ops.begin(), ops.end());

@@ -1,7 +1,8 @@
 // Sums over several eq factors, sum_g eq(rho_g, x) P_g(x), on the CPU through tests/cpp/emu/hip/hip_runtime.h under the host sanitizers:
 // wsum_kernel (a round that is a launch of its own) and slice_kernel with SliceArgsEqs (the rounds resident in LDS, one or two a trip).
 // Every sum is compared with q_g(t) = sum_x' R_g(x') P_g(t, x') worked out by plain loops from the terms, R_g from its definition.
-// The programs are built by the rule the library uses, from terms that are also evaluated one by one.
+// The programs are built as the library builds them (program.hpp), from terms that are also evaluated one by one; programs of random lists of
+// terms are walked by a plain stack machine besides.
 #include <algorithm>
 #include <chrono>
 #include <memory>
@@ -10,6 +11,7 @@
 
 #include "dpsumcheck.h"
 #include "kernels.hpp"
+#include "program.hpp"
 
 using gl::E2;
 using gl::u32;
@@ -43,55 +45,16 @@ struct Term {
     E2 coeff;
     std::vector<u32> slots;
 };
-static dpk::PolyOp make_op(u32 kind, u32 depth, u32 slot, E2 c)
-{
-    dpk::PolyOp op;
-    memset(&op, 0, sizeof op);
-    op.c0 = c.c0, op.c1 = c.c1, op.w = gl::mul_small(c.c1, (u32)gl::W);
-    const u32 cls = c.c1 ? dpk::POLY_COEFF_ANY : c.c0 == 1 ? dpk::POLY_COEFF_ONE : c.c0 == gl::P - 1 ? dpk::POLY_COEFF_MINUS_ONE : dpk::POLY_COEFF_BASE;
-    op.code = kind | depth << 2 | (kind == dpk::POLY_OP_LEAF ? cls : 0) << 6 | slot << 8;
-    return op;
-}
-static void build(std::vector<Term> ts, u32 depth, std::vector<dpk::PolyOp> &ops)
-{
-    ts.erase(std::remove_if(ts.begin(), ts.end(), [](const Term &t) { return t.slots.empty(); }), ts.end());
-    while (!ts.empty()) {
-        const u32 best = ts[0].slots[0];
-        std::vector<Term> sub, rest;
-        for (Term &t : ts) {
-            auto it = std::find(t.slots.begin(), t.slots.end(), best);
-            if (it == t.slots.end()) {
-                rest.push_back(t);
-            } else {
-                t.slots.erase(it);
-                sub.push_back(t);
-            }
-        }
-        E2 ends = gl::e2_zero();
-        bool inner = false;
-        for (const Term &t : sub) {
-            if (t.slots.empty())
-                ends = gl::add(ends, t.coeff);
-            else
-                inner = true;
-        }
-        if (!inner) {
-            ops.push_back(make_op(dpk::POLY_OP_LEAF, depth, best, ends));
-        } else {
-            ops.push_back(make_op(dpk::POLY_OP_ENTER, depth + 1, 0, ends));
-            build(sub, depth + 1, ops);
-            ops.push_back(make_op(dpk::POLY_OP_LEAVE, depth + 1, best, gl::e2_zero()));
-        }
-        ts = rest;
-    }
-}
 static std::vector<dpk::PolyOp> program_of(const std::vector<Term> &terms)
 {
-    E2 root = gl::e2_zero();
-    for (const Term &t : terms)
-        if (t.slots.empty()) root = gl::add(root, t.coeff);
-    std::vector<dpk::PolyOp> ops{make_op(dpk::POLY_OP_ENTER, 0, 0, root)};
-    build(terms, 0, ops);
+    std::vector<dpk::ProgramTerm> ts(terms.size());
+    for (size_t i = 0; i < terms.size(); i++) {
+        ts[i].coeff = terms[i].coeff;
+        ts[i].n = (uint8_t)terms[i].slots.size();
+        for (size_t f = 0; f < terms[i].slots.size(); f++) ts[i].slot[f] = (uint8_t)terms[i].slots[f];
+    }
+    std::vector<dpk::PolyOp> ops;
+    dpk::program_root(ts.data(), (u32)ts.size(), ops);
     return ops;
 }
 static E2 eval(const std::vector<Term> &terms, const std::vector<Table> &tabs, size_t pair, u64 t)
@@ -120,9 +83,63 @@ static E2 eq_at(const std::vector<E2> &rho, u32 first, u32 bits, u64 i)
 
 static int failures = 0;
 
+// ---- programs of random lists of terms: the value, the depth, the coefficients' classes and the number of products ----
+static void check_programs()
+{
+    bool ok = true;
+    for (u32 rep = 0; rep < 3000 && ok; rep++) {
+        const u32 n_tabs = 1 + (u32)(splitmix() % (rep % 3 == 0 ? (u32)dpk::SL_MAX_TABS : 4u)), n_terms = (u32)(splitmix() % 65), most = 1 + (u32)(splitmix() % DPS_MAX_DEGREE);
+        std::vector<E2> val;
+        for (u32 k = 0; k < n_tabs; k++) val.push_back(felt2());
+        std::vector<Term> terms;
+        E2 want = gl::e2_zero();
+        u32 degree = 0, factors = 0;
+        for (u32 i = 0; i < n_terms; i++) {
+            const u32 cls = (u32)(splitmix() % 4);
+            Term t{cls == 0 ? felt2() : gl::e2(cls == 1 ? 1 : cls == 2 ? gl::P - 1 : felt(), 0), {}};
+            for (u32 f = (u32)(splitmix() % (most + 1)); f > 0; f--) t.slots.push_back((u32)(splitmix() % n_tabs));
+            E2 prod = t.coeff;
+            for (u32 sl : t.slots) prod = gl::mul(prod, val[sl]);
+            want = gl::add(want, prod);
+            degree = std::max(degree, (u32)t.slots.size()), factors += (u32)t.slots.size();
+            terms.push_back(t);
+        }
+        const std::vector<dpk::PolyOp> ops = program_of(terms);
+        std::vector<E2> acc;
+        u32 products = 0;
+        for (const dpk::PolyOp &o : ops) {
+            const u32 kind = o.code & 3, depth = (o.code >> 2) & 15, cls = (o.code >> 6) & 3, slot = o.code >> 8;
+            const E2 c = gl::e2(o.c0, o.c1);
+            if (kind == dpk::POLY_OP_ENTER) {
+                ok = ok && acc.size() == depth && (depth == 0 || depth < degree);
+                acc.push_back(c);
+            } else if (kind == dpk::POLY_OP_LEAF) {
+                ok = ok && acc.size() == depth + 1 && slot < n_tabs && o.w == gl::mul_small(c.c1, (u32)gl::W) &&
+                     cls == (c.c1 ? dpk::POLY_COEFF_ANY : c.c0 == 1 ? dpk::POLY_COEFF_ONE : c.c0 == gl::P - 1 ? dpk::POLY_COEFF_MINUS_ONE : dpk::POLY_COEFF_BASE);
+                if (ok) acc.back() = gl::add(acc.back(), gl::mul(val[slot], c)), products++;
+            } else {
+                ok = ok && acc.size() == depth + 1 && depth > 0 && slot < n_tabs;
+                if (!ok) break;
+                const E2 child = acc.back();
+                acc.pop_back();
+                acc.back() = gl::add(acc.back(), gl::mul(child, val[slot])), products++;
+            }
+        }
+        ok = ok && acc.size() == 1 && gl::eq(acc[0], want) && products <= factors;
+        if (!ok) printf("program %u: %u terms over %u tables\n", rep, n_terms, n_tabs);
+    }
+    printf("%-60s : %s\n", "programs of random lists of terms", ok ? "ok" : "MISMATCH");
+    if (!ok) failures++;
+}
+
 // ---- wsum_kernel: one round over 2^log_pairs pairs by `blocks` workgroups ----
+struct Launch {
+    bool factored = false;     // the weights as products of a low and a high table
+    int mail = 0;              // a launch made ahead: 1, the challenge comes by mail, 2, by mail through the relay
+    std::vector<u32> only{};   // workgroups that are run (none: all), whose partial sums are compared instead of the launch's
+};
 template <int NF, bool SKIP1, bool BASE, int REST>
-static void run_round(const char *name, u32 log_pairs, u32 blocks, u32 n_tabs, std::vector<std::vector<Term>> polys, bool folds, bool base_tabs)
+static void run_round(const char *name, u32 log_pairs, u32 blocks, u32 n_tabs, std::vector<std::vector<Term>> polys, bool folds, bool base_tabs, Launch how = Launch())
 {
     constexpr int NS = dpk::wsum_sums(NF, SKIP1, REST);
     const size_t n_pairs = (size_t)1 << log_pairs;
@@ -154,19 +171,41 @@ static void run_round(const char *name, u32 log_pairs, u32 blocks, u32 n_tabs, s
     }
     std::copy(ops.begin(), ops.end(), a.ops);
     std::vector<std::vector<E2>> rho(G), R(G);
-    std::vector<std::vector<u64>> q0(G), q1(G);
+    std::vector<std::vector<u64>> q0(G), q1(G), lq0(G), lq1(G), hq0(G), hq1(G);
+    const size_t lows = (size_t)1 << dpk::EQ_LO_BITS;
     for (u32 g = 0; g < G; g++) {
+        if (how.factored) {
+            // (the streamed table is not to be read)
+            for (size_t i = 0; i < lows; i++) lq0[g].push_back(felt()), lq1[g].push_back(felt());
+            for (size_t i = 0; i < (n_pairs + lows - 1) / lows; i++) hq0[g].push_back(felt()), hq1[g].push_back(felt());
+            for (size_t i = 0; i < n_pairs; i++)
+                R[g].push_back(gl::mul(gl::e2(hq0[g][i / lows], hq1[g][i / lows]), gl::e2(lq0[g][i % lows], lq1[g][i % lows])));
+            a.lq0[g] = lq0[g].data(), a.lq1[g] = lq1[g].data(), a.hq0[g] = hq0[g].data(), a.hq1[g] = hq1[g].data();
+            continue;
+        }
         for (u32 v = 0; v < log_pairs; v++) rho[g].push_back(felt2());
         for (size_t i = 0; i < n_pairs; i++) R[g].push_back(eq_at(rho[g], 0, log_pairs, i)), q0[g].push_back(R[g][i].c0), q1[g].push_back(R[g][i].c1);
         a.q0[g] = q0[g].data(), a.q1[g] = q1[g].data();
     }
-    std::vector<u64> partial((size_t)2 * NS * blocks, 0), out(64, 0), dyn((size_t)n_tabs * (BASE ? 2 : 4) * dpk::BLOCK);
+    std::vector<u64> partial((size_t)2 * NS * blocks, 0), out(64, 0), dyn((size_t)n_tabs * (BASE ? 2 : 4) * dpk::BLOCK), mail(64, 0), relay(dpk::MAIL_RELAY_WORDS, 0);
     u32 counter = 0;
+    if (how.mail) {
+        // the mail is there before the launch (workgroups run one after the other here); the arguments hold no challenge
+        a.r0 = a.r1 = 0x1234;
+        a.wait_first = 1, a.mail = mail.data(), a.relay = how.mail == 2 ? relay.data() : nullptr, a.spin_limit = 1u << 30;
+        mail[dpk::MAIL_R] = r.c0, mail[dpk::MAIL_R + 1] = r.c1, mail[dpk::MAIL_SKIP1] = SKIP1 ? 1 : 0;
+        u64 chk = 17;
+        for (u32 m = dpk::MAIL_R; m < (u32)dpk::MAIL_WORDS; m++) chk ^= dpk::mail_mix(mail[m], m);
+        mail[dpk::MAIL_CHK] = chk, mail[dpk::MAIL_SEQ] = 17;
+    }
     dpk::FastFin ff;
     memset(&ff, 0, sizeof ff);
     ff.partial = partial.data(), ff.n_blocks = blocks, ff.out_host = out.data(), ff.seq = 17, ff.counter = &counter;
     gridDim = dim3(blocks), blockDim = dim3(dpk::BLOCK);
-    for (u32 b = 0; b < blocks; b++) {
+    const bool whole = how.only.empty();
+    if (whole)
+        for (u32 b = 0; b < blocks; b++) how.only.push_back(b);
+    for (u32 b : how.only) {
         emu::default_group.reset(dpk::BLOCK);
         emu::default_group.dyn = dyn.data();
         std::vector<std::thread> th;
@@ -178,21 +217,34 @@ static void run_round(const char *name, u32 log_pairs, u32 blocks, u32 n_tabs, s
             });
         for (auto &x : th) x.join();
     }
-    bool ok = out[dpk::WSUM_SEQ_SLOT] == 17 && counter == 0;
-    u64 chk = 17;
-    for (u32 i = 0; i < 2 * NS; i++) chk ^= dpk::rotl64(out[i], i + 1);
-    ok = ok && chk == out[dpk::WSUM_CHK_SLOT];
-    const u32 n0 = SKIP1 ? NF : NF + 1;
-    for (u32 g = 0; g < G; g++)
-        for (u32 t = 0; t <= a.degree[g]; t++) {
-            if (g == 0 && t == 1 && SKIP1) continue;
-            const u32 s = g == 0 ? (SKIP1 && t > 0 ? t - 1 : t) : n0 + (g - 1) * dpk::wsum_rest(NF, REST) + t;
-            E2 want = gl::e2_zero();
-            for (size_t i = 0; i < n_pairs; i++) want = gl::add(want, gl::mul(R[g][i], eval(polys[g], tabs, i, t)));
-            if (!gl::eq(want, gl::e2(out[2 * s], out[2 * s + 1]))) ok = false, printf("%s: factor %u point %u\n", name, g, t);
-        }
-    for (u32 k = 0; k < n_tabs && folds; k++)
-        for (size_t i = 0; i < 2 * n_pairs; i++) ok = ok && d0[k][i] == tabs[k][i].c0 && d1[k][i] == tabs[k][i].c1;
+    bool ok = true;
+    if (whole) {
+        ok = out[dpk::WSUM_SEQ_SLOT] == 17 && counter == 0;
+        u64 chk = 17;
+        for (u32 i = 0; i < 2 * NS; i++) chk ^= dpk::rotl64(out[i], i + 1);
+        ok = ok && chk == out[dpk::WSUM_CHK_SLOT];
+    }
+    const size_t stride = (size_t)blocks * dpk::BLOCK;
+    // sum of the pairs of workgroups [b, b + n)
+    auto compare = [&](u32 b, u32 n, auto &&word) {
+        const u32 n0 = SKIP1 ? NF : NF + 1;
+        for (u32 g = 0; g < G; g++)
+            for (u32 t = 0; t <= a.degree[g]; t++) {
+                if (g == 0 && t == 1 && SKIP1) continue;
+                const u32 s = g == 0 ? (SKIP1 && t > 0 ? t - 1 : t) : n0 + (g - 1) * dpk::wsum_rest(NF, REST) + t;
+                E2 want = gl::e2_zero();
+                for (size_t first = (size_t)b * dpk::BLOCK; first < n_pairs; first += stride)
+                    for (size_t i = first; i < std::min(n_pairs, first + (size_t)n * dpk::BLOCK); i++) want = gl::add(want, gl::mul(R[g][i], eval(polys[g], tabs, i, t)));
+                if (!gl::eq(want, gl::e2(word(2 * s), word(2 * s + 1)))) ok = false, printf("%s: workgroup %u factor %u point %u\n", name, b, g, t);
+            }
+        for (u32 k = 0; k < n_tabs && folds; k++)
+            for (size_t first = (size_t)b * dpk::BLOCK; first < n_pairs; first += stride)
+                for (size_t i = 2 * first; i < 2 * std::min(n_pairs, first + (size_t)n * dpk::BLOCK); i++) ok = ok && d0[k][i] == tabs[k][i].c0 && d1[k][i] == tabs[k][i].c1;
+    };
+    if (whole)
+        compare(0, blocks, [&](u32 w) { return out[w]; });
+    else
+        for (u32 b : how.only) compare(b, 1, [&](u32 w) { return partial[(size_t)w * blocks + b]; });
     printf("%-60s 2^%u pairs, %u workgroups : %s\n", name, log_pairs, blocks, ok ? "ok" : "MISMATCH");
     if (!ok) failures++;
 }
@@ -381,6 +433,7 @@ int main()
     // the linking sum's shape: v - b^2 v + c b^2 + d b, and s v + s' b
     const std::vector<Term> lp{{one, {0}}, {minus, {1, 1, 0}}, {half, {1, 1}}, {gl::e2(77, 0), {1}}}, ll{{felt2(), {0}}, {felt2(), {1}}};
     const std::vector<Term> p4{{felt2(), {0, 1, 2, 2}}, {felt2(), {2, 3}}, {felt2(), {}}, {one, {3}}}, p2{{felt2(), {0, 3}}, {minus, {1}}}, p1{{half, {2}}, {felt2(), {}}};
+    check_programs();
     run_round<3, false, true, 1>("two factors, base tables", 9, 2, 2, {lp, ll}, false, true);
     run_round<3, true, true, 1>("the same, p(1) from the claim, a single workgroup", 5, 1, 2, {lp, ll}, false, true);
     run_round<3, true, false, 1>("base tables folded on the way in", 9, 2, 2, {lp, ll}, true, true);
@@ -390,6 +443,18 @@ int main()
     run_round<3, true, false, 0>("one factor, extension tables folded on the way in", 9, 2, 4, {lp}, true, false);
     run_round<3, false, true, 0>("the same unfolded over base tables, every point", 6, 1, 4, {lp}, false, true);
     run_round<2, true, false, 2>("degrees 2 and 2 over base tables", 7, 1, 4, {p2, p2}, false, true);
+    // a lane takes several pairs, one behind the other
+    run_round<3, true, false, 1>("two factors, several pairs a lane", 10, 2, 2, {lp, ll}, true, true);
+    run_round<3, false, false, 1>("the same, every point, the challenge by mail", 10, 1, 2, {lp, ll}, true, true, {.mail = 1});
+    run_round<4, true, false, 2>("three factors, several pairs a lane, mail through the relay", 10, 3, 4, {p4, p2, p1}, true, false, {.mail = 2});
+    run_round<4, false, false, 2>("the same, every point", 9, 1, 4, {p4, p2, p1}, true, false);
+    run_round<2, true, false, 2>("degrees 2 and 2, several pairs a lane", 9, 1, 4, {p2, p2}, true, false);
+    run_round<3, false, true, 0>("one factor unfolded, several pairs a lane", 9, 1, 4, {lp}, false, true);
+    // the weights as a low and a high table: workgroups of a launch whose stride is a run of the low table, two runs of pairs
+    run_round<3, true, true, 1>("two factors, base tables, factored weights", 17, 256, 2, {lp, ll}, false, true, {.factored = true, .only = {0, 255}});
+    run_round<3, false, false, 1>("two factors folded, every point, factored weights", 17, 256, 2, {lp, ll}, true, false, {.factored = true, .mail = 2, .only = {0, 77}});
+    run_round<4, true, false, 2>("three factors folded, factored weights", 17, 256, 4, {p4, p2, p1}, true, false, {.factored = true, .only = {0, 255}});
+    run_round<3, true, false, 0>("one factor folded, factored weights", 17, 256, 4, {lp}, true, false, {.factored = true, .only = {0, 128}});
     run_resident<3>("resident, two factors, trips of two rounds", 7, 1, 2, {lp, ll}, 2, true, 0);
     run_resident<3>("resident, one round a trip, the last two rounds left out", 6, 1, 2, {lp, ll}, 1, false, 2);
     run_resident<3>("resident, four workgroups, then one", 9, 4, 2, {lp, ll}, 0, true, 2);

@@ -19,7 +19,8 @@ PROGRAMS = {"prod": ("emu_prod_kernel.cpp", ["quick"]), "slice": ("emu_slice_ker
 def outcomes(tmp_path_factory):
     tmp_path = tmp_path_factory.mktemp("emu")
     csrc = os.path.join(ROOT, "deep-prove_amd", "csrc")
-    shutil.copy(os.path.join(csrc, "gl.hpp"), tmp_path / "gl.hpp")
+    for header in ("gl.hpp", "program.hpp"):
+        shutil.copy(os.path.join(csrc, header), tmp_path / header)
     text = open(os.path.join(csrc, "kernels.hpp")).read()
     # dynamic LDS has no host spelling: the emulation hands every workgroup a buffer of its own
     assert "extern __shared__ u64 dyn[];" in text
