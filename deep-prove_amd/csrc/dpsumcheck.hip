@@ -171,7 +171,8 @@ constexpr int MAX_DEVICES = 64;
 // fits an untouched one, so launches admitted together are placed together, in whatever order their workgroups
 // arrive), up to the device's number of compute units.  A launch that does not get its place is not made: a round
 // that would have been launched ahead is launched when its challenge is there, and a session whose resident launch
-// is refused runs the same rounds as launches of their own.  The results are the same bits either way.
+// is refused makes one of fewer workgroups or makes it some rounds later (FusedRound::seat_stages); the rounds before it are launches of
+// their own.  The results are the same bits either way.
 // Launches that wait for nothing (all others) come and go by themselves and are not counted.
 // ---------------------------------------------------------------------------
 struct DeviceLedger {
@@ -205,6 +206,18 @@ bool admit_waiting_launch(dps_ctx *ctx, u32 workgroups, bool together)
     l.used += want;
     ctx->units_held = (u32)want;
     return true;
+}
+
+// compute units the device has for waiting launches, and those that none of another context holds
+struct Units {
+    u32 all, free;
+};
+Units units_of(dps_ctx *ctx)
+{
+    DeviceLedger &l = ledger_of(ctx->device);
+    std::lock_guard<std::mutex> lock(l.mu);
+    const int budget = std::max(0, l.limit >= 0 ? std::min(l.limit, l.total) : l.total);
+    return Units{(u32)budget, (u32)std::max(0, budget - (l.used - (int)ctx->units_held))};
 }
 
 // the context's waiting launch has had its last mail (or was told to leave and has left): its place is free again
@@ -1724,6 +1737,7 @@ struct dps_sc {
     void *dev_block;    // descriptors, partials, per-round result
     bool described;            // the descriptors of every round's launch are worked out (else of round 1 only: SessionSetup::run)
     void *late_block = nullptr;  // ... behind dps_sc_begin: where they lie then
+    void *late_hand = nullptr;   // what the stages of a plan made behind dps_sc_begin leave for the next (plan_again)
     void *desc_block = nullptr;  // where the descriptors lie
     // precomputed descriptors (device)
     std::vector<u32> fold_off, fold_cnt;            // per step j = 2..n_vars+1: all tables that fold
@@ -2335,11 +2349,12 @@ constexpr u32 SLICE_SECOND_ROUND_BUDGET = 10;
 // Which rounds of a session are resident, in which launches, and how they pair up into trips.  `n_tabs`: tables in LDS.
 // A trip covers two rounds when the second one's p(1) can come from the claim (its eq coordinate is not zero) and the
 // workgroups still hold a quad each.  The first resident round is the first whose pairs fit 256 workgroups.
-void plan_resident_rounds(dps_sc *sc, u32 n_tabs, u32 n_mles)
+// `first`, `most`: for a plan made in the place of that one (plan_again), the first round it may begin with and the workgroups there are;
+// the rounds before it are launches of a round each.
+void plan_resident_rounds(dps_sc *sc, u32 n_tabs, u32 n_mles, u32 first = 0, u32 most = SLICE_MAX_WORKGROUPS)
 {
     const u32 n = sc->n_vars;
     const bool has_eq = sc->fast_eq >= 0 || !sc->weq.empty();
-    const u32 first_ok = 1;
     auto claim_gives_p1 = [&](u32 round) {
         if (sc->fast_coeff.c0 == 0 && sc->fast_coeff.c1 == 0) return false;
         if (!has_eq) return true;
@@ -2350,14 +2365,15 @@ void plan_resident_rounds(dps_sc *sc, u32 n_tabs, u32 n_mles)
     if (pairs_fit == 0) return;
     const u32 per_wg_max = std::min<u32>(pairs_fit, sc->poly ? SLICE_SUM_PAIRS : SLICE_PRODUCT_PAIRS);
     auto pairs_of = [&](u32 round) { return (u64)1 << (n - round); };
-    u32 j = first_ok;
-    while (pairs_of(j) > (u64)per_wg_max * SLICE_MAX_WORKGROUPS) j++;
+    u32 j = std::max<u32>(first, 1);
+    while (pairs_of(j) > (u64)per_wg_max * most) j++;
     // (a sum small enough stays with one workgroup: no handing over)
     const u32 n_terms = sc->poly && sc->weq.empty() ? (u32)sc->slice_terms.size() : 1;
     u32 per_wg = (u32)std::min<u64>(per_wg_max, std::max<u64>(SLICE_MIN_PAIRS, pairs_of(j) / SLICE_SMALL_SUM_WORKGROUPS));
     if (n_terms > 1)
         while (per_wg > SLICE_SUM_MIN_PAIRS && per_wg * n_terms > SLICE_SUM_TERM_PAIRS && pairs_of(j) / per_wg < SLICE_SUM_WORKGROUPS) per_wg >>= 1;
     if (pairs_of(j) * n_terms <= (n_terms > 1 ? SLICE_SUM_TERM_PAIRS : SLICE_ONE_WORKGROUP_PAIRS) && pairs_of(j) <= per_wg_max) per_wg = (u32)pairs_of(j);
+    while (pairs_of(j) / per_wg > most) per_wg <<= 1;
     sc->tail_j0 = j;
     // The last rounds are the host's: a trip costs the way to the GPU and back and a workgroup's barriers whatever it
     // carries, a round of a few pairs costs the host a microsecond.  As many rounds as stay below HOST_TAIL_MULTS
@@ -2384,7 +2400,7 @@ void plan_resident_rounds(dps_sc *sc, u32 n_tabs, u32 n_mles)
     for (u32 r = n_gpu + 1; r <= n; r++) sc->round_kind[r] = 4;
     // a launch that starts with round 1 has nothing to fold first; one behind a launch that covered two rounds
     // (quad_kernel) finds the state of two rounds ago
-    u32 pend = j == 1 ? 0 : (!sc->poly && quad_launches_fit(sc, n_mles, j) ? 2 : 1);
+    u32 pend = j == 1 ? 0 : (first == 0 && !sc->poly && quad_launches_fit(sc, n_mles, j) ? 2 : 1);
     u64 entries = (u64)1 << (n - j + 1 + pend);  // of the tables the stage to come starts from (before its pending folds)
     auto add_stage = [&](u32 W) {
         dps_sc::Stage st;
@@ -2424,9 +2440,9 @@ void plan_resident_rounds(dps_sc *sc, u32 n_tabs, u32 n_mles)
     while (j <= n_gpu) add_stage(1);
 }
 
-// The session's resident launch found no place on the device (admit_waiting_launch): the rounds it would have run, and
-// those the host would have worked out behind it, are launches of their own like the rounds before them.  The
-// descriptors of their launches are there or are made now (describe_now), and the eq levels those rounds read are built.
+// The rounds the session's resident launch would have run, and those the host would have worked out behind it, are launches of their own
+// like the rounds before them.  The descriptors of their launches are there or are made now (describe_now), and the eq levels those
+// rounds read are built.
 void drop_resident_plan(dps_sc *sc)
 {
     sc->stages.clear();
@@ -2438,6 +2454,49 @@ void drop_resident_plan(dps_sc *sc)
     for (uint8_t &k : sc->round_kind)
         if (k <= 4) k = 0;
     std::fill(sc->round_wide.begin(), sc->round_wide.end(), 0);
+}
+
+size_t hand_over_bytes(const dps_sc *sc)
+{
+    size_t bytes = 0;
+    for (size_t i = 0; i + 1 < sc->stages.size(); i++)
+        bytes += round_up((size_t)sc->stages[i + 1].src_len * 8, 256) * 2 * (sc->slice_ids.size() + std::max<size_t>(1, sc->weq.size()));
+    return bytes;
+}
+// what a resident stage that does not run to the last round leaves for the next, from `p` on: two limb arrays per table
+void place_hand_over(dps_sc *sc, char *p)
+{
+    const u32 slice_tabs = (u32)sc->slice_ids.size();
+    for (size_t i = 0; i + 1 < sc->stages.size(); i++) {
+        const size_t limb = round_up((size_t)sc->stages[i + 1].src_len * 8, 256);
+        for (u32 f = 0; f <= slice_tabs; f++) {
+            // (behind the tables the eq weights, one factor's behind the other's)
+            const size_t n = f < slice_tabs ? 1 : std::max<size_t>(1, sc->weq.size());
+            sc->stages[i].h0[f] = (u64 *)p;
+            p += n * limb;
+            sc->stages[i].h1[f] = (u64 *)p;
+            p += n * limb;
+        }
+    }
+}
+
+int32_t describe_now(dps_sc *sc);
+
+// Another plan in the place of the session's, beginning with round `first` at the earliest and with at most `most` workgroups; without
+// memory for what its launches leave one another there is none.
+void plan_again(dps_sc *sc, u32 first, u32 most)
+{
+    drop_resident_plan(sc);
+    if (first > sc->n_vars || !most) return;
+    plan_resident_rounds(sc, (u32)sc->slice_ids.size(), sc->n_mles, first, most);
+    const size_t bytes = hand_over_bytes(sc);
+    if (!bytes) return;
+    pool_free(sc->ctx, sc->late_hand);
+    sc->late_hand = nullptr;
+    if (pool_alloc(sc->ctx, bytes, &sc->late_hand) == DPS_OK)
+        place_hand_over(sc, (char *)sc->late_hand);
+    else
+        drop_resident_plan(sc);
 }
 
 }  // namespace
@@ -3208,28 +3267,14 @@ int32_t SessionSetup::allocate_device_block()
     const size_t bytes_desc = sc->described ? descriptor_bytes() : 0;
     size_t bytes_partial = round_up((size_t)std::max<u32>(sc->n_terms, 1) * sc->max_blocks * 2 * dpk::MAX_PTS * 8, 256);
     size_t bytes_result = round_up((2 * dpk::MAX_PTS + 2 * (size_t)n_mles) * 8, 256) + 256;
-    // what a resident stage that does not run to the last round leaves for the next: two limb arrays per table
-    size_t bytes_hand = 0;
-    const u32 slice_tabs = (u32)sc->slice_ids.size();
-    for (size_t i = 0; i + 1 < sc->stages.size(); i++) bytes_hand += round_up((size_t)sc->stages[i + 1].src_len * 8, 256) * 2 * (slice_tabs + std::max<size_t>(1, sc->weq.size()));
-    CHK(pool_alloc(ctx, bytes_desc + bytes_partial + bytes_result + bytes_hand, &sc->dev_block));
+    CHK(pool_alloc(ctx, bytes_desc + bytes_partial + bytes_result + hand_over_bytes(sc), &sc->dev_block));
     char *p = (char *)sc->dev_block;
     if (sc->described) p = place_descriptors(p);
     sc->d_partial = (u64 *)p;
     p += bytes_partial;
     sc->d_result = (u64 *)p;
     p += bytes_result;
-    for (size_t i = 0; i + 1 < sc->stages.size(); i++) {
-        const size_t limb = round_up((size_t)sc->stages[i + 1].src_len * 8, 256);
-        for (u32 f = 0; f <= slice_tabs; f++) {
-            // (behind the tables the eq weights, one factor's behind the other's)
-            const size_t n = f < slice_tabs ? 1 : std::max<size_t>(1, sc->weq.size());
-            sc->stages[i].h0[f] = (u64 *)p;
-            p += n * limb;
-            sc->stages[i].h1[f] = (u64 *)p;
-            p += n * limb;
-        }
-    }
+    place_hand_over(sc, p);
     sc->d_counter = ctx->d_counter;
     return DPS_OK;
 }
@@ -4072,6 +4117,7 @@ struct FusedRound {
     int32_t take_sums(u32 n_slots);
     int32_t end_waiting_launch();
     bool admit_stages();
+    int32_t seat_stages(u32 jj, bool *seated);
     int32_t launch_stages_at(u64 seq0, u32 first_go = 0);
     template <SliceSize SIZE>
     int32_t launch_stages_of(u64 seq0, u32 first_go);
@@ -4353,6 +4399,26 @@ bool FusedRound::admit_stages()
         return admit_waiting_launch(ctx, widest, true);
 }
 
+// Whether the resident rounds begin with round jj = tail_j0.  Where their launch finds no place: fewer workgroups that take more pairs each, if
+// the compute units that are free now are enough for that; else round jj is a launch of its own, and the plan begins with the round after
+// it, which asks again.  With 8 compute units for waiting launches, every round a launch of its own / this, us: a product of 2^10 entries 153 / 62,
+// attention over 2^12 entries 284 / 175, linking a softmax of 2^12 and 2^16 entries 465 / 188 and 620 / 340, 2^22 lookups 4910 / 3680; eight contexts on
+// eight threads, each linking a softmax of 2^16 entries (which asks for all 256): 1250 / 655 us a proof.
+int32_t FusedRound::seat_stages(u32 jj, bool *seated)
+{
+        *seated = admit_stages();
+        if (*seated) return DPS_OK;
+        const Units units = units_of(ctx);
+        u32 most = 1;
+        while (2 * most <= std::min(units.free, SLICE_MAX_WORKGROUPS)) most *= 2;
+        if (units.free) {
+            plan_again(sc, jj, most);
+            *seated = sc->tail_j0 == jj && admit_stages();
+        }
+        if (!*seated) plan_again(sc, jj + 1, units.all ? SLICE_MAX_WORKGROUPS : 0);
+        return sc->tail_j0 == 1 ? (int32_t)DPS_OK : describe_now(sc);
+}
+
 // The launches of the resident rounds, queued one behind the other: the trip that starts at the first resident
 // round has the sequence number seq0 (a round's call takes one number whether or not it makes a trip).
 int32_t FusedRound::launch_stages_at(u64 seq0, u32 first_go)
@@ -4400,7 +4466,7 @@ int32_t FusedRound::launch_stages_of(u64 seq0, u32 first_go)
                         sa.lacks[f] = (uint8_t)(tb.mode == dpk::POLY_BCAST ? tb.shift + 2 : 1);
                         sa.any_lacks = 1;
                     }
-                } else if (!sc->quads.empty()) {
+                } else if (st.pend0 == 2) {
                     // the state of two rounds ago, as the last launch of two rounds left it
                     sa.s0[f] = sc->quads.back().d0[f];
                     sa.s1[f] = sc->quads.back().d1[f];
@@ -4611,7 +4677,8 @@ FusedRound::Plan FusedRound::plan_round(u32 jj, bool skip1_jj) const
         if (p.split) poly_split_plan(p.n_pairs, sc->poly_split_cap, n_groups <= POLY_RAW_MAX_GROUPS, &p.split_log, &p.blocks);
         // a single workgroup (per group) from here on: it stays for the remaining rounds
         // (several groups stay only with their tables in LDS: they must not read each other's stores)
-        p.reside = p.split && n_groups <= POLY_RAW_MAX_GROUPS && p.blocks == 1 && skip1_jj && jj < sc->n_vars &&
+        // (and only where no resident launch of all tables is planned)
+        p.reside = p.split && !sc->tail_j0 && n_groups <= POLY_RAW_MAX_GROUPS && p.blocks == 1 && skip1_jj && jj < sc->n_vars &&
                    sc->n_vars - jj + 1 <= (u32)dpk::POLY_RES_ROUNDS && (n_groups == 1 || poly_split_state_ok(ctx, nf, has_eq, true));
         return p;
 }
@@ -4798,14 +4865,13 @@ int32_t FusedRound::multi_term_round()
                 skip1_next = !(rho.c0 == 0 && rho.c1 == 0);
             }
             const Plan pn = plan_round(j + 1, skip1_next);
-            if (sc->tail_j0 && j + 1 == sc->tail_j0) {
+            bool seated = false;
+            if (sc->tail_j0 && j + 1 == sc->tail_j0) CHK(seat_stages(j + 1, &seated));
+            if (seated) {
                 // the rounds from here on are resident: their launches are queued now and wait for their first mail
-                // (when the device has room for them now; else the next round asks again)
-                if (admit_stages()) {
-                    CHK(launch_stages_at(ctx->seq + 1));
-                    sc->wait_fresh = true;
-                    sc->ahead_at = std::chrono::steady_clock::now();
-                }
+                CHK(launch_stages_at(ctx->seq + 1));
+                sc->wait_fresh = true;
+                sc->ahead_at = std::chrono::steady_clock::now();
             } else if (admit_waiting_launch(ctx, pn.blocks * std::max<u32>(n_groups, 1), pn.reside)) {
                 CHK(launch_round(j + 1, pn, skip1_next, true, ctx->seq + 1));
                 sc->tail_running = true;
@@ -4847,13 +4913,19 @@ int32_t FusedRound::product_launch_ahead(u32 ahead)
     if (jn <= sc->n_vars && !ctx->profiling && !sc->no_ahead) {
         const u64 next_seq = ctx->seq + ahead;
         const u64 pairs_n = 1ull << (sc->n_vars - jn);
-        bool made = false;
+        bool made = false, seated = false;
         if (sc->tail_j0 && jn == sc->tail_j0) {
-            // (when the device has room for the resident launches now; else the next round asks again)
-            if (admit_stages()) {
-                CHK(launch_stages_at(next_seq));
-                made = true;
+            if (sc->stages[0].pend0 == 2) {
+                // (behind launches of two rounds each the tables are two folds behind, which no other launch takes up: the round itself asks again)
+                seated = admit_stages();
+                if (!seated) return DPS_OK;
+            } else {
+                CHK(seat_stages(jn, &seated));
             }
+        }
+        if (seated) {
+            CHK(launch_stages_at(next_seq));
+            made = true;
         } else if (const dps_sc::QuadStep *q = quad_at(jn)) {
             // the next two rounds are one launch
             if (admit_waiting_launch(ctx, q->blocks, false)) {
@@ -5205,10 +5277,13 @@ extern "C" int32_t dps_sc_round(dps_sc *sc, const uint64_t *challenge, uint64_t 
         CHK(fr.begin());
         // the resident rounds begin here and their launch is not on the GPU yet: with no place for it on the device
         // these rounds are launches of their own
-        if (sc->tail_j0 && j == sc->tail_j0 && !sc->tail_running && !fr.admit_stages()) {
-            if (!sc->quads.empty()) CHK(fr.catch_up_after_quads());
-            drop_resident_plan(sc);
-            CHK(describe_now(sc));
+        if (sc->tail_j0 && j == sc->tail_j0 && !sc->tail_running) {
+            bool seated = false;
+            if (sc->stages[0].pend0 == 2) {
+                seated = fr.admit_stages();
+                if (!seated) CHK(fr.catch_up_after_quads());
+            }
+            if (!seated) CHK(fr.seat_stages(j, &seated));
         }
         if ((sc->tail_j0 && j >= sc->tail_j0) || sc->host_only) return fr.resident_round();
         if (sc->pair12 && j == 1) return fr.first_two_rounds_launch();
@@ -5342,6 +5417,7 @@ extern "C" int32_t dps_sc_free(dps_sc *sc)
     pool_free(ctx, sc->scratch);
     pool_free(ctx, sc->dev_block);
     pool_free(ctx, sc->late_block);
+    pool_free(ctx, sc->late_hand);
     delete sc;
     return DPS_OK;
 }

@@ -47,6 +47,15 @@ def _stacked(orc, n, seed, pairs=8):
     return up, lambda: list(tabs), terms
 
 
+def _linking(orc, n, seed, factors=2):
+    """sums over several eq factors, each times a polynomial of its own over two tables"""
+    tabs, points = [rand_e2(1 << n, seed + k) for k in range(2)], [rand_e2(n, seed + 10 + g) for g in range(factors)]
+    polys = [[[0], [0, 1, 1], [1]], [[0], [1]], [[0, 1]]][:factors]
+    up = lambda c: [c.mle_from_ext2(t) for t in tabs] + [c.eq_build(r) for r in points]  # noqa: E731
+    terms = [(np.array([seed % 91 + k + 1, g], dtype=np.uint64), fs + [2 + g]) for g, poly in enumerate(polys) for k, fs in enumerate(poly)]
+    return up, lambda: tabs + [orc.eq_evals(r) for r in points], terms
+
+
 def _reference(orc, n, host_tables, terms, label):
     return orc.sc_prove(n, host_tables(), terms, orc.OracleTranscript(label))
 
@@ -87,6 +96,35 @@ def test_rounds_without_a_place_on_the_device(dp, orc, budget):
         ctx.close()
     used, cap = dp.resident_budget(0)
     assert used == 0 and cap > 0
+
+
+@pytest.mark.parametrize("budget", [1, 3, 8, 40])
+def test_a_resident_launch_that_finds_few_places_takes_them(dp, orc, budget):
+    """A sum whose resident launch asks for more workgroups than there are places is resident all the same: with fewer workgroups, from the first
+    round whose pairs they can take on.  From the rounds' launches made as they come (profiled) and from launches made ahead."""
+    shapes = [("product", 10, _product(orc, 10, 45000)), ("product", 18, _product(orc, 18, 45100)), ("product", 22, _product(orc, 22, 45200)),
+              ("layer", 9, _layer(orc, 9, 45300)), ("layer", 17, _layer(orc, 17, 45400)), ("stacked", 10, _stacked(orc, 10, 45500)),
+              ("two factors", 9, _linking(orc, 9, 45600)), ("two factors", 17, _linking(orc, 17, 45700)), ("three factors", 13, _linking(orc, 13, 45800, 3))]
+    ctx = dp.Context(0)
+    try:
+        dp.set_resident_budget(0, budget)
+        for kind, n, (up, host_tables, terms) in shapes:
+            ref = _reference(orc, n, host_tables, terms, b"few")
+            gpu = up(ctx)
+            for profiled in (True, False):
+                ctx.profile(profiled)
+                ctx.profile_reset()
+                assert _same(ctx.sumcheck_prove(n, gpu, terms, dp.Transcript(b"few")), ref), (kind, n, budget)
+                if profiled:
+                    made = {k: v["launches"] for k, v in ctx.profile_read().items()}
+                    assert made["tail"] > 0, (kind, n, budget, made)
+                    # (the rounds before: those of more pairs than the places take, 512 a workgroup of a product, 128 of another sum)
+                    before = sum(made[k] for k in ("eval_first", "fold_eval", "eval_terms"))
+                    assert before <= max(0, n - 1 - (9 if kind == "product" else 7) - (budget.bit_length() - 1)), (kind, n, budget, made)
+                assert dp.resident_budget(0)[0] == 0
+    finally:
+        dp.set_resident_budget(0, -1)
+        ctx.close()
 
 
 def test_a_session_left_midway_gives_its_place_back(dp, orc):
