@@ -4563,7 +4563,8 @@ int32_t FusedRound::resident_round()
         for (size_t g = 0; g < sc->weq.size(); g++) {
             const dps_sc::WeightedEq &w = sc->weq[g];
             const u32 d = w.degree, npt = g == 0 ? d : d + 1;
-            for (u32 ti = 0; ti < npt; ti++) wq[g * dpk::MAX_PTS + (g == 0 && ti > 0 ? ti + 1 : ti)] = gl::e2_zero();
+            // (the first factor's point 1 too: where its scalar has become zero it is not solved for, and is read)
+            for (u32 t = 0; t <= d; t++) wq[g * dpk::MAX_PTS + t] = gl::e2_zero();
             for (u32 k = 0; k <= d; k++) {
                 E2 basis = gl::e2(ctx->h_inv_den[d][k], 0);
                 for (u32 m = 0; m <= d; m++)
