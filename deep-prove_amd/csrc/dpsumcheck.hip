@@ -2712,6 +2712,11 @@ bool SessionSetup::weighted_programs()
         eqs[g].op_end = (u32)ops.size();
     }
     if (ops.size() > (size_t)dpk::SL_EQS_OPS) return false;
+    // Their gain is in the resident rounds.  Where the device has no compute unit for those, programs that a lane walks one behind the other (three, or two of
+    // degree 2 and more) lose to the eq tables as tables, whose small rounds spread a pair over lanes: linking a softmax of 2^8 / 2^12 / 2^16 / 2^20
+    // entries 355 / 500 / 680 / 975 us and 315 / 455 / 615 / 995, a normalisation 525 / 775 / 1040 / 1560 and 385 / 595 / 825 / 1475.  An activation's
+    // two of degrees 3 and 1 do not: 275 / 365 / 470 / 640 and 290 / 400 / 530 / 810.
+    if (n_eqs > 1 && wsum_rest_kind(n_eqs, eqs[1].degree) == 2 && !units_of(ctx).all) return false;
     if (n_eqs == 1) {
         sc->one_program = true;
         sc->one = eqs[0];
