@@ -2331,13 +2331,6 @@ u32 slice_counter_sets_log(u32 W)
 // point for some of the terms (slice_kernel's q_split), the lanes of a pass cover BLOCK / (q_split NF (NF + 1)) quads
 u32 slice_second_round_passes(const dps_sc *sc, u32 n_quads)
 {
-    if (!sc->weq.empty()) {
-        // (every factor has its own lanes; a lane takes a quad at one challenge)
-        const u32 per = ((u32)dpk::SL_BLOCK / (u32)sc->weq.size()) & ~63u;
-        u32 most = 0;
-        for (const dps_sc::WeightedEq &w : sc->weq) most = std::max(most, (n_quads * (w.degree + 1) + per - 1) / per);
-        return most;
-    }
     const u32 nf = sc->fast_nf, per_quad_pts = nf * (nf + 1);
     const u32 n_terms = sc->poly ? (u32)sc->slice_terms.size() : 1;
     const u32 q_split = n_terms * per_quad_pts <= (u32)dpk::SL_BLOCK ? n_terms : 1;
@@ -2415,9 +2408,12 @@ void plan_resident_rounds(dps_sc *sc, u32 n_tabs, u32 n_mles, u32 first = 0, u32
             bool dbl = len >= 4 && j + 1 <= n_gpu && claim_gives_p1(j + 1);
             // The second round's sums are (NF + 1) NF evaluations a quad where a trip of its own takes NF a pair: worth it while
             // the lanes take a workgroup's quads in a few passes (a pass is a chain of about NF + 1 dependent products), that
-            // is while it costs less than the trip it saves.  Measured on the degree-4 linking sum (7 terms: two-round
-            // trips from 32 entries a workgroup on, 0.83 -> 0.72 ms) and on 8 products over 16 tables (0.145 -> 0.135 ms).
-            if (dbl && slice_second_round_passes(sc, (u32)(len >> 2)) * (sc->fast_nf + 1) > SLICE_SECOND_ROUND_BUDGET) dbl = false;
+            // is while it costs less than the trip it saves.  Measured on a sum of degree 4 and 7 terms (two-round trips from 32 entries a workgroup
+            // on, 0.83 -> 0.72 ms) and on 8 products over 16 tables (0.145 -> 0.135 ms).  Several eq factors, whose lanes take a point each of
+            // a quad at one challenge: whenever the sums fit.  With at most 128 pairs a workgroup that is up to two passes more for every factor; allowing
+            // no more, one, two of them, factors of degrees 3 and 1 over 2^13 .. 2^16 entries take 127, 139, 155, 172 / 128, 145, 161, 179 / 129,
+            // 146, 156, 171 us, of 2 and 1 over 2^16 143 / 137 / 137, of 2, 1 and 1 171 / 161 / 161.
+            if (dbl && sc->weq.empty() && slice_second_round_passes(sc, (u32)(len >> 2)) * (sc->fast_nf + 1) > SLICE_SECOND_ROUND_BUDGET) dbl = false;
             if (W > 1 && j + 1 == n_gpu) dbl = false;  // the last trip is the single workgroup's
             if (!sc->weq.empty() && sc->weq_sums2 > (u32)dpk::SL_MAX_SUMS) dbl = false;
             if (dbl) st.dbl_mask |= 1u << st.n_trips;

@@ -3,11 +3,12 @@ zkml/src/lookup/operation/inputs/variant.rs:222-348, written out as terms), agai
 launches (a sum of one variable, all rounds resident, one launch before the resident ones, factored weights), base and extension
 tables, rounds that evaluate t = 1, and no room for resident launches."""
 import importlib
+import time
 
 import numpy as np
 import pytest
 
-from util import from_E2, rand_base, rand_e2, to_E2
+from util import rand_base, rand_e2
 
 pytestmark = pytest.mark.gpu
 
@@ -94,20 +95,40 @@ def test_claim_known_before_round_one(dp, ctx, orc, n):
     _prove(dp, ctx, orc, n, "beb", THREE_LOW, 1400 + n, zero_at=(1,), claimed=True)
 
 
-@pytest.mark.parametrize("kinds,polys", [("be", LINKING), ("beb", THREE_LOW), ("beeb", THREE)])
-@pytest.mark.parametrize("at", [0, 1, 2, 3])
-def test_challenge_that_makes_the_eq_factors_vanish(dp, ctx, orc, kinds, polys, at):
-    # the points' coordinate `at` is 1 and so is nothing of eq(rho, .) left at the challenge 0: the messages that follow take p(1) from a first factor of scalar zero
-    n = 8
-    dev, host, terms = _instance(dp, ctx, orc, n, kinds, polys, 1500 + at, one_at=(at,))
-    tables, s, challenge = [to_E2(t) for t in host], ctx.session(n, dev, terms), None
+@pytest.mark.parametrize("kinds,polys", [("be", LINKING), ("beb", THREE_LOW), ("beeb", THREE), ("be", LINKING[:1])])
+@pytest.mark.parametrize("n,at", [(8, 0), (8, 1), (8, 2), (8, 3), (19, 0), (19, 1), (19, 2)])
+def test_challenge_that_makes_the_eq_factors_vanish(dp, ctx, orc, kinds, polys, n, at):
+    # the points' coordinate `at` is 1 and so is nothing of eq(rho, .) left at the challenge 0: the messages that follow take p(1) from a first factor of scalar zero,
+    # and a launch made ahead that leaves t = 1 out is not the one that is needed
+    dev, tables, terms = _instance(dp, ctx, orc, n, kinds, polys, 1500 + n + at, one_at=(at,))
+    s, challenge = ctx.session(n, dev, terms), None
     for j in range(n):
-        message = orc.sc_round_poly(n - j, [from_E2(t) for t in tables], [n - j] * len(tables), terms)
+        message = orc.sc_round_poly(n - j, tables, [n - j] * len(tables), terms)
         assert (s.round(challenge) == message).all(), j
         challenge = np.zeros(2, dtype=np.uint64) if j == at else rand_e2(1, 1600 + j)[0]
-        r = to_E2(challenge)[0]
-        tables = [[a + r * (b - a) for a, b in zip(t[::2], t[1::2])] for t in tables]
-    assert (s.finish(challenge) == from_E2([t[0] for t in tables])).all()
+        tables = [orc.mle_fix_low(t, challenge[None]) for t in tables]
+    assert (s.finish(challenge) == np.concatenate([t.reshape(1, 2) for t in tables])).all()
+
+
+@pytest.mark.parametrize("kinds,polys", [("be", LINKING), ("beeb", THREE)])
+@pytest.mark.parametrize("how", ["other call", "slow caller"])
+def test_launch_made_ahead_steps_aside(dp, ctx, orc, kinds, polys, how):
+    # rounds 1 .. 3 of 19 variables (more than 2^15 pairs) are launches, the rest resident: before each of them has its challenge another call needs the context, or the caller
+    # takes longer than the launch waits
+    n = 19
+    dev, host, terms = _instance(dp, ctx, orc, n, kinds, polys, 1700)
+    proof, point, finals = orc.sc_prove(n, host, terms, orc.OracleTranscript(b"aside"))
+    for after in (1, 2, 3):
+        s, challenge = ctx.session(n, dev, terms), None
+        for j in range(n):
+            assert (s.round(challenge) == proof[j]).all(), (after, j)
+            challenge = point[j]
+            if j + 1 == after and how == "other call":
+                assert (ctx.eq_build(point[:3]).download() == orc.eq_evals(point[:3])).all()
+            elif j + 1 == after:
+                time.sleep(0.3)
+        assert (s.finish(challenge) == finals).all()
+        del s
 
 
 @pytest.mark.parametrize("n,zero_at", [(6, (0, 3)), (11, (2,)), (17, (0, 1, 5))])
