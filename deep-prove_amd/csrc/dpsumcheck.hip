@@ -2652,8 +2652,9 @@ constexpr u32 MAX_PROGRAM_TERMS = 64, NO_TABLE = ~0u;
 // A sum each of whose terms has one eq table, up to three of them in all, times polynomials of degree 4 at most over up to POLY_MAXT
 // other tables, all of full size: the eq factors in closed form, a nested program each for the polynomials (wsum_kernel).  What
 // does not fit (degrees, numbers of operations and sums) runs with the eq tables as tables among the others, or a single eq table in closed
-// form term by term.  (Linking an activation of 2^21 entries, two factors of degrees 3 and 1 over two tables: 684 -> 412 us; its rounds of 2^20 .. 2^17
-// pairs 158, 92, 66, 47 -> 59, 53, 40, 30 us, the resident ones 205 -> 141.)
+// form term by term.  (Linking an activation of 2^21 entries, two factors of degrees 3 and 1 over two tables: 686 -> 399 us; its rounds of 2^20 .. 2^16
+// pairs 158, 92, 66, 47, 46 -> 68, 53, 40, 30, 24 us, the resident ones 211 -> 117.  Degrees 4 and 1, 2^8 / 2^14 / 2^20 entries:
+// 215 / 403 / 836 -> 111 / 191 / 422; 3, 3 and 1: 119 / 228 / 677 -> 113 / 192 / 528; 4, 4 and 2: 317 / 600 / 1370 -> 148 / 250 / 807.)
 // One eq factor: the same programs in the rounds that are launches of their own (rounds of 2^19 .. 2^16 pairs of a fraction-sum layer 52, 38, 30, 25 ->
 // 43, 34, 28, 20 us); resident its rounds stay with the terms, which are spread over more lanes (a trip of two rounds 8.5 .. 10 us, 15 .. 16 by a program).
 bool SessionSetup::weighted_programs()
@@ -5277,8 +5278,7 @@ extern "C" int32_t dps_sc_round(dps_sc *sc, const uint64_t *challenge, uint64_t 
         fr.sc = sc, fr.ctx = ctx, fr.j = j, fr.challenge = challenge, fr.evals_out = evals_out;
         fr.n_pairs = n_pairs, fr.blocks = blocks, fr.cst = cst, fr.fa = fa;
         CHK(fr.begin());
-        // the resident rounds begin here and their launch is not on the GPU yet: with no place for it on the device
-        // these rounds are launches of their own
+        // the resident rounds begin here and their launch is not on the GPU yet: as planned, or as there is a place for it
         if (sc->tail_j0 && j == sc->tail_j0 && !sc->tail_running) {
             bool seated = false;
             if (sc->stages[0].pend0 == 2) {

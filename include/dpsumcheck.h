@@ -74,7 +74,8 @@ int32_t dps_ctx_sync(dps_ctx *ctx);
  * host takes its turn (the resident launches of the late rounds, the launches made ahead of their round); launches of
  * that kind from different contexts share the device through a process-wide ledger, one compute unit per workgroup,
  * so that those admitted are always placed together and none waits for room another holds.  A launch that finds no
- * place is not made and its rounds run as ordinary launches: same results, bit for bit, more launches.
+ * place is made with fewer workgroups or some rounds later, and the rounds before it run as ordinary launches: same results, bit for
+ * bit, more launches.
  * dps_device_set_resident_budget caps what all contexts of this process together may hold on `device` (compute units;
  * -1: the whole device, the default; 0: no launch ever waits on the GPU) -- for a GPU shared with other work.
  * dps_device_resident_budget reads the ledger: units held now, and the cap in force (-1 before the first context). */

@@ -89,6 +89,19 @@ def test_many_tables_without_resident_launches(dp, ctx, orc, case):
         dp.set_resident_budget(0, -1)
 
 
+@pytest.mark.parametrize("case", [0, 1, 3, 7, 8, 9, 10, 11])
+@pytest.mark.parametrize("budget", [1, 2, 5])
+def test_many_tables_in_few_workgroups(dp, ctx, orc, case, budget):
+    # the resident launch in as many workgroups as there are places, behind rounds that are launches: tables one and several variables short of its first round too
+    n, table_vars, base, n_terms, deg = CASES[case]
+    gpu, host, terms = _instance(ctx, orc, 700 + case, table_vars, base, n_terms, deg)
+    dp.set_resident_budget(0, budget)
+    try:
+        _check(dp, ctx, orc, n, gpu, host, terms)
+    finally:
+        dp.set_resident_budget(0, -1)
+
+
 @pytest.mark.parametrize("tables,n_terms,eq,short", [(16, 24, False, False), (17, 24, False, False), (16, 25, False, False), (16, 24, True, False),
                                                      (17, 25, True, False), (4, 3, True, True), (16, 24, False, True)])
 def test_sizes_of_the_arguments(dp, ctx, orc, tables, n_terms, eq, short):

@@ -3,7 +3,7 @@
 The reference proves the chunks of a model concurrently from a thread pool (zkml/src/graph/executor.rs:148,
 zkml/src/iop/mod.rs:268-279), so several sessions are live at once from different threads.  Launches that stay on the
 GPU between the host's turns (resident launches, launches made ahead) take their place in a process-wide ledger of the
-device first; one that finds no place is not made and its rounds run as ordinary launches.  Checked here: the proofs
+device first; one that finds no place is made with fewer workgroups or some rounds later, and the rounds before it run as ordinary launches.  Checked here: the proofs
 are the checker's bits whatever the ledger allows, from one thread with the budget cut down and from four threads
 that contend for the whole device."""
 import importlib
