@@ -4408,7 +4408,7 @@ bool FusedRound::admit_stages()
 // eight threads, each linking a softmax of 2^16 entries (which asks for all 256): 1250 / 655 us a proof.
 int32_t FusedRound::seat_stages(u32 jj, bool *seated)
 {
-        *seated = admit_stages();
+        *seated = sc->tail_j0 == jj && admit_stages();
         if (*seated) return DPS_OK;
         const Units units = units_of(ctx);
         u32 most = 1;
@@ -5283,7 +5283,11 @@ extern "C" int32_t dps_sc_round(dps_sc *sc, const uint64_t *challenge, uint64_t 
             bool seated = false;
             if (sc->stages[0].pend0 == 2) {
                 seated = fr.admit_stages();
-                if (!seated) CHK(fr.catch_up_after_quads());
+                if (!seated) {
+                    // (the plan counts on tables that are two folds behind, and they no longer are: this one may not be asked for again)
+                    CHK(fr.catch_up_after_quads());
+                    plan_again(sc, j, SLICE_MAX_WORKGROUPS);
+                }
             }
             if (!seated) CHK(fr.seat_stages(j, &seated));
         }

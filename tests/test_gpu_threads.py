@@ -127,6 +127,37 @@ def test_a_resident_launch_that_finds_few_places_takes_them(dp, orc, budget):
         ctx.close()
 
 
+@pytest.mark.parametrize("kind,n,times", [("product", 24, 1500), ("product", 22, 500), ("layer", 17, 500), ("stacked", 17, 200), ("linking", 17, 500)])
+def test_a_place_that_comes_and_goes(dp, orc, kind, n, times):
+    """Another thread gives the device's compute units back and takes them away again all the time, so that a launch that has just been refused finds its
+    place a moment later, and a session plans its rounds again and again.  A product of 24 variables has two launches of two rounds each: where the resident
+    launch behind them is refused a fold is caught up on, into the tables they wrote, and what is planned from there on takes the tables as they are then
+    (asked for again, the first plan would read them as they were: about one proof in 150).  The reference is the proof without another thread, which the
+    other tests compare with the checker's."""
+    up, _, terms = {"product": _product, "layer": _layer, "stacked": _stacked, "linking": _linking}[kind](orc, n, 46000)
+    ctx = dp.Context(0)
+    stop = threading.Event()
+
+    def toggle():
+        while not stop.is_set():
+            for units in (0, -1, 0, 9, 0, 100):
+                dp.set_resident_budget(0, units)
+
+    thread = threading.Thread(target=toggle)
+    try:
+        gpu = up(ctx)
+        ref = ctx.sumcheck_prove(n, gpu, terms, dp.Transcript(b"goes"))
+        thread.start()
+        for k in range(times):
+            assert _same(ctx.sumcheck_prove(n, gpu, terms, dp.Transcript(b"goes")), ref), k
+    finally:
+        stop.set()
+        if thread.ident is not None:
+            thread.join()
+        dp.set_resident_budget(0, -1)
+        ctx.close()
+
+
 def test_a_session_left_midway_gives_its_place_back(dp, orc):
     ctx = dp.Context(0)
     up, _, terms = _product(orc, 16, 42000)
