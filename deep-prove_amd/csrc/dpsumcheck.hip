@@ -4691,6 +4691,8 @@ FusedRound::Plan FusedRound::plan_round(u32 jj, bool skip1_jj) const
 int32_t FusedRound::launch_round(u32 jj, const Plan &p, bool skip1_jj, bool ahead, u64 seq_jj)
 {
         if (by_program(p.n_pairs)) return launch_weighted(jj, skip1_jj, ahead, seq_jj);
+        // (before their places are read: a session that has not described its launches gets them here)
+        if (!inline_descs) CHK(ensure_descs(sc));
         dpk::PolyArgs pa;
         pa.groups = sc->d_poly_groups + (size_t)(jj - 1) * n_groups;
         pa.terms = sc->d_poly_terms;
@@ -4704,8 +4706,6 @@ int32_t FusedRound::launch_round(u32 jj, const Plan &p, bool skip1_jj, bool ahea
                 memcpy(pa.o0, sc->h_poly_ops.data(), sc->h_poly_ops.size() * sizeof(dpk::PolyOp));
             else
                 std::copy(sc->h_poly_terms.begin(), sc->h_poly_terms.end(), pa.t0);
-        } else {
-            CHK(ensure_descs(sc));
         }
         pa.q0 = pa.q1 = nullptr;
         pa.lq0 = pa.lq1 = pa.hq0 = pa.hq1 = nullptr;
@@ -4747,7 +4747,6 @@ int32_t FusedRound::launch_round(u32 jj, const Plan &p, bool skip1_jj, bool ahea
             pa.last_round = sc->n_vars;
             if (n_groups > 1) {
                 // one resident workgroup per group, each publishing its own sums
-                CHK(ensure_descs(sc));
                 pa.groups = sc->d_poly_groups + (size_t)(jj - 1) * n_groups;
                 pa.group_stride = n_groups;
                 pa.raw_out = ctx->d_pinned + poly_raw_off(ctx);

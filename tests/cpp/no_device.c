@@ -74,9 +74,15 @@ int hipMemset(void *d, int v, size_t n) { return (void)d, (void)v, (void)n, 0; }
 int hipMemsetAsync(void *d, int v, size_t n, void *stream) { return (void)d, (void)v, (void)n, (void)stream, 0; }
 int hipFuncSetAttribute(const void *f, int attribute, int value) { return (void)f, (void)attribute, (void)value, 0; }
 int hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *f, int block, size_t lds) { return (void)f, (void)block, (void)lds, *n = 1, 0; }
+// the last launch's first argument: its first word (a pointer, in structures that begin with one)
+static uint64_t launches, first_word;
+uint64_t no_device_launches(void) { return launches; }
+uint64_t no_device_first_word(void) { return first_word; }
 int hipLaunchKernel(const void *f, dim3 grid, dim3 block, void **args, size_t lds, void *stream)
 {
-    return (void)f, (void)grid, (void)block, (void)args, (void)lds, (void)stream, 0;
+    launches++;
+    memcpy(&first_word, args[0], 8);
+    return (void)f, (void)grid, (void)block, (void)lds, (void)stream, 0;
 }
 int hipGetLastError(void) { return 0; }
 const char *hipGetErrorString(int e) { return (void)e, "no device"; }

@@ -27,7 +27,7 @@ def run(no_device):
     def go(body):
         text = "import ctypes, importlib, sys\nimport numpy as np\n"
         text += "dev = ctypes.CDLL(%r, ctypes.RTLD_GLOBAL)\n" % str(no_device)  # (before the library: its calls are found here)
-        text += "for f in ('no_device_in_use', 'no_device_most'): getattr(dev, f).restype = ctypes.c_int64\n"
+        text += "for f in ('no_device_in_use', 'no_device_most', 'no_device_launches', 'no_device_first_word'): getattr(dev, f).restype = ctypes.c_int64\n"
         text += "dev.no_device_budget.argtypes = [ctypes.c_int64]\n"
         text += "sys.path.insert(0, %r)\ndp = importlib.import_module('deep-prove_amd')\n" % ROOT + body
         res = subprocess.run([sys.executable, "-c", text], stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True, timeout=300)
@@ -71,6 +71,37 @@ except dp.DpsError as e:
     assert e.status == 3, e  # out of memory
 dev.no_device_budget(1 << 60)
 s = ctx.session(n, tabs, terms)
+print("done")
+""")
+
+
+def test_a_round_asked_for_again_when_its_descriptors_did_not_fit(run):
+    # 8 products over 16 tables, several groups of them: planned to be resident from round 1, so only round 1 is described.  Without a place on the device the
+    # launches read descriptors from device memory; where those do not fit the call fails, and the next one finds memory for them
+    run("""
+n = 9
+one = np.array([1, 0], dtype=np.uint64)
+ctx = dp.Context(0)
+z = np.zeros((1 << n, 2), dtype=np.uint64)
+tabs = [ctx.mle_from_ext2(z) for _ in range(16)]
+s = ctx.session(n, tabs, [(one, [h, 8 + h]) for h in range(8)])
+dp.set_resident_budget(0, 0)
+dev.no_device_budget(dev.no_device_in_use())
+launches = dev.no_device_launches()
+try:
+    s.round(None)
+    raise SystemExit("a round without memory")
+except dp.DpsError as e:
+    assert e.status == 3, e  # out of memory
+assert dev.no_device_launches() == launches
+dev.no_device_budget(1 << 60)
+try:
+    s.round(None)
+    raise SystemExit("a result without a device")
+except dp.DpsError as e:
+    assert e.status == 2, e
+assert dev.no_device_launches() == launches + 1
+assert dev.no_device_first_word() != 0, "the launch has no descriptors"
 print("done")
 """)
 
