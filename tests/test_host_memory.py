@@ -106,6 +106,33 @@ print("done")
 """)
 
 
+def test_sums_over_three_eq_factors_without_a_compute_unit_take_them_as_tables(run):
+    # sum_g eq_g P_g over two tables.  In closed form the eq tables are never folded and have no buffers; as tables they do (3/4 of 2^n entries each)
+    run("""
+n = 16
+one = np.array([1, 0], dtype=np.uint64)
+ctx = dp.Context(0)
+tabs = [ctx.mle_from_ext2(np.zeros((1 << n, 2), dtype=np.uint64)) for _ in range(2)]
+eqs = [ctx.eq_build(np.full((n, 2), g + 1, dtype=np.uint64)) for g in range(3)]
+polys = {"softmax": [[[0], [0, 1, 1]], [[0], [1, 1, 1]], [[0, 1]]], "two cubics": [[[0], [0, 1, 1]], [[0], [1, 1, 1]]], "activation": [[[0], [0, 1, 1]], [[0], [1]]]}
+def taken(ps):
+    terms = [(one, fs + [2 + g]) for g, poly in enumerate(ps) for fs in poly]
+    before = dev.no_device_in_use()
+    s = ctx.session(n, tabs + eqs[:len(ps)], terms)
+    bytes_ = dev.no_device_in_use() - before
+    ctx.keep = getattr(ctx, "keep", []) + [s]  # (so that no session finds another's memory)
+    return bytes_
+folded = 16 * (3 << n) // 4
+with_units = {k: taken(ps) for k, ps in polys.items()}
+dp.set_resident_budget(0, 0)
+without = {k: taken(ps) for k, ps in polys.items()}
+for k, ps in polys.items():
+    more = without[k] - with_units[k]
+    assert (more >= folded * len(ps)) == (k != "activation"), (k, more, folded)
+print("done")
+""")
+
+
 def test_a_logup_circuit_is_complete_as_its_constructor_leaves_it(no_device, tmp_path):
     exe, lib = tmp_path / "test_logup_circuit", os.path.join(ROOT, "deep-prove_amd", "lib")
     # (linked before the library: its calls are found in the runtime without a device)
